@@ -19,6 +19,7 @@
 
 #include "lt_internal.h"
 #include "lt_kernels.h"
+#include "lt_flat.h"
 #include "lt_mlp.h"
 #include "lt_sched.h"
 
@@ -169,6 +170,12 @@ struct Engine {
     uint64_t slot_sz = 0;        // bytes per slot (256-aligned)
     bool slot_packed = false;    // slots keep columns packed (pack_partitions = 2)
     uint8_t *d_slots = nullptr;
+    // One raw slot per partition: the slots are slices of one rowptr and one
+    // col array (at most as many bytes), which run_flat walks directly.
+    bool flat = false;
+    uint64_t *flat_rowptr = nullptr;   // [V+1], in d_slots
+    uint32_t *flat_col = nullptr;      // [E], in d_slots
+    uint32_t *d_rowptr32 = nullptr;    // [V+1] copy of flat_rowptr once every partition is cached (E < 2^32)
     std::vector<int32_t> slot_of;      // partition -> slot or -1
     std::vector<int32_t> part_in_slot; // slot -> partition or -1
     std::vector<uint32_t> free_slots;
@@ -274,7 +281,7 @@ struct Engine {
 
     ~Engine();
     lt_status init(const lt_graph *g_, const lt_partition *p_, const lt_config *c);
-    lt_status ensure_pool(uint64_t walkers);
+    lt_status ensure_pool(uint64_t walkers, bool check_only = false);
     lt_status ensure_outputs(const RunSpec &rs, bool want_endpoints, bool want_moves);
     lt_status run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoints_out, uint32_t *moves_out);
 
@@ -298,7 +305,7 @@ struct Engine {
     void record(uint32_t p, int kind, int32_t loaded, int32_t evicted);
     lt_status evict(uint32_t p);
     lt_status load_async(uint32_t p);
-    lt_status copy_partition(uint32_t p, uint8_t *base);
+    lt_status copy_partition(uint32_t p, uint64_t *rp, uint32_t *cp);
     lt_status fetch_partition(uint32_t p, uint64_t *rowptr_out, uint32_t *col_out);
     // Bit streams of p's slot whose column part starts at cp: past the block
     // headers when the slot holds p's block image, nullptr for raw columns.
@@ -307,7 +314,20 @@ struct Engine {
         const uint64_t nblk = (part.edge_off[p + 1] - part.edge_off[p] + kBlockEdges - 1) / kBlockEdges;
         return cp + 2 * (nblk + 1);
     }
+    // Where p's cached rowptr and col slices lie.
+    void slot_ptrs(uint32_t p, uint64_t **rp, uint32_t **cp) const {
+        if (flat) {
+            *rp = flat_rowptr + part.node_off[p];
+            *cp = flat_col + part.edge_off[p];
+        } else {
+            uint8_t *base = d_slots + (size_t)slot_of[p] * slot_sz;
+            *rp = (uint64_t *)base;
+            *cp = (uint32_t *)(base + ((uint64_t)part.node_off[p + 1] - part.node_off[p] + 1) * 8);
+        }
+    }
     lt_status set_table(uint32_t p, bool present);
+    bool can_run_flat() const;
+    lt_status run_flat(const RunSpec &rs);
     lt_status scheduler_loop();
     lt_status scheduler_loop_learned();
     lt_status scheduler_loop_device();
@@ -347,6 +367,7 @@ Engine::~Engine() {
     dfree(d_col_tab);
     dfree(d_words_tab);
     dfree(d_slots);
+    dfree(d_rowptr32);
     dfree(q.slab);
     dfree(q.frame);
     dfree(q.free_stack);
@@ -509,7 +530,15 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
     if (nslots == P) rp_resident = false;  // nothing is zero-copied with every partition cached
     if (rp_resident && nslots >= rp_slots + 2) nslots -= rp_slots;
     else rp_resident = false;
-    LT_TRY(dmalloc(&d_slots, (size_t)nslots * slot_bytes));
+    flat = nslots == P && !slot_packed && !cfg.device_schedule;
+    if (flat) {
+        const size_t rp_size = (rp_bytes + 255) & ~(size_t)255;
+        LT_TRY(dmalloc(&d_slots, rp_size + 4 * (size_t)g->E));
+        flat_rowptr = (uint64_t *)d_slots;
+        flat_col = (uint32_t *)(d_slots + rp_size);
+    } else {
+        LT_TRY(dmalloc(&d_slots, (size_t)nslots * slot_bytes));
+    }
     slot_of.assign(P, -1);
     part_in_slot.assign(nslots, -1);
     resident.assign(P, 0);
@@ -600,12 +629,9 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
 // Size the chunk pool for `walkers` queued walkers: every queue may hold a
 // partly filled chunk, the slice being consumed keeps its chunks until the
 // fix-up, and allocation races may strand up to kLostCap chunks per launch.
-lt_status Engine::ensure_pool(uint64_t walkers) {
+// check_only: refuse what the queues could not hold, allocate nothing.
+lt_status Engine::ensure_pool(uint64_t walkers, bool check_only) {
     if (walkers <= wcap && q.slab) return LT_OK;
-    dfree(q.slab);
-    dfree(q.frame);
-    dfree(q.free_stack);
-    dfree(q.lost);
     const uint64_t wchunks = (walkers + kChunk - 1) / kChunk;
     // one launch holds at most `held` source chunks while filling new ones
     const uint64_t held = cfg.device_schedule ? wchunks + 1 : std::min<uint64_t>(slice, wchunks + 1);
@@ -615,6 +641,11 @@ lt_status Engine::ensure_pool(uint64_t walkers) {
         set_error("%llu walkers exceed the queue limits; lower -b", (unsigned long long)walkers);
         return LT_E_ARG;
     }
+    if (check_only) return LT_OK;
+    dfree(q.slab);
+    dfree(q.frame);
+    dfree(q.free_stack);
+    dfree(q.lost);
     q.nchunks = (uint32_t)nchunks;
     q.maxc = (uint32_t)maxc;
     LT_TRY(dmalloc(&q.slab, (size_t)nchunks * kChunk));
@@ -683,9 +714,11 @@ lt_status Engine::set_table(uint32_t p, bool present) {
     const uint64_t *rp = nullptr;
     const uint32_t *cp = nullptr, *wp = nullptr;
     if (present) {
-        uint8_t *base = d_slots + (size_t)slot_of[p] * slot_sz;
-        rp = (const uint64_t *)base;
-        cp = (const uint32_t *)(base + ((uint64_t)part.node_off[p + 1] - part.node_off[p] + 1) * 8);
+        uint64_t *r;
+        uint32_t *c;
+        slot_ptrs(p, &r, &c);
+        rp = r;
+        cp = c;
         wp = slot_words(p, cp);
     }
     set_table_kernel<<<1, 64, 0, s_compute>>>(d_rowptr_tab, d_col_tab, d_words_tab, p, rp, cp, wp);
@@ -715,20 +748,23 @@ lt_status Engine::load_async(uint32_t p) {
     const uint32_t s = free_slots.back();
     free_slots.pop_back();
     hipEvent_t t = t_load.begin(s_dma);
-    LT_TRY(copy_partition(p, d_slots + (size_t)s * slot_sz));
-    t_load.end(t, s_copy);
     slot_of[p] = (int32_t)s;
     part_in_slot[s] = (int32_t)p;
+    uint64_t *rp;
+    uint32_t *cp;
+    slot_ptrs(p, &rp, &cp);
+    LT_TRY(copy_partition(p, rp, cp));
+    t_load.end(t, s_copy);
     return LT_OK;
 }
 
-// Slot bytes of partition p: the rowptr slice, then the col slice, either
+// Slot bytes of partition p: the rowptr slice at rp and the col slice at cp, either
 // copied as is, or copied gap-coded into a staging buffer and unpacked from
 // there, or (block slots) its block image copied into the slot, where it stays.
 // The DMAs run on s_dma; s_copy waits for them (and unpacks), so the load is
 // complete when s_copy reaches this point.  A staging buffer is refilled only
 // after the unpack of its previous image.  Block slots copy on s_copy alone.
-lt_status Engine::copy_partition(uint32_t p, uint8_t *base) {
+lt_status Engine::copy_partition(uint32_t p, uint64_t *rp, uint32_t *cp) {
     const uint32_t nb = part.node_off[p], ne = part.node_off[p + 1];
     const uint64_t eb = part.edge_off[p], ee = part.edge_off[p + 1];
     const size_t rbytes = ((size_t)ne - nb + 1) * 8, cbytes = (size_t)(ee - eb) * 4;
@@ -736,13 +772,13 @@ lt_status Engine::copy_partition(uint32_t p, uint8_t *base) {
     uint32_t k = 0;
     if (packed && slot_packed) {  // the block image is the slot's column part
         if (rp_resident) {
-            LT_HIP(hipMemcpyAsync(base, d_rowptr_all + nb, rbytes, hipMemcpyDeviceToDevice, s_copy));
+            LT_HIP(hipMemcpyAsync(rp, d_rowptr_all + nb, rbytes, hipMemcpyDeviceToDevice, s_copy));
         } else {
-            LT_HIP(hipMemcpyAsync(base, g->rowptr + nb, rbytes, hipMemcpyHostToDevice, s_copy));
+            LT_HIP(hipMemcpyAsync(rp, g->rowptr + nb, rbytes, hipMemcpyHostToDevice, s_copy));
             st.h2d_bytes_explicit += rbytes;
             st.h2d_bytes_unpacked += rbytes;
         }
-        LT_HIP(hipMemcpyAsync(base + rbytes, pk->host + pk->off[p], pk->size[p], hipMemcpyHostToDevice, s_copy));
+        LT_HIP(hipMemcpyAsync(cp, pk->host + pk->off[p], pk->size[p], hipMemcpyHostToDevice, s_copy));
         st.h2d_bytes_unpacked += cbytes;
         st.h2d_bytes_explicit += pk->size[p];
         st.packed_image_bytes += pk->size[p];
@@ -755,9 +791,9 @@ lt_status Engine::copy_partition(uint32_t p, uint8_t *base) {
         if (stage_used[k] && s_dma != s_copy) LT_HIP(hipStreamWaitEvent(s_dma, stage_free[k], 0));
     }
     if (rp_resident) {
-        LT_HIP(hipMemcpyAsync(base, d_rowptr_all + nb, rbytes, hipMemcpyDeviceToDevice, s_dma));
+        LT_HIP(hipMemcpyAsync(rp, d_rowptr_all + nb, rbytes, hipMemcpyDeviceToDevice, s_dma));
     } else {
-        LT_HIP(hipMemcpyAsync(base, g->rowptr + nb, rbytes, hipMemcpyHostToDevice, s_dma));
+        LT_HIP(hipMemcpyAsync(rp, g->rowptr + nb, rbytes, hipMemcpyHostToDevice, s_dma));
         st.h2d_bytes_explicit += rbytes;
         st.h2d_bytes_unpacked += rbytes;
     }
@@ -772,7 +808,7 @@ lt_status Engine::copy_partition(uint32_t p, uint8_t *base) {
             LT_HIP(hipStreamWaitEvent(s_copy, ev_dma, 0));
         }
         unpack_kernel<<<(unsigned)((waves + 3) / 4), 256, 0, s_copy>>>(
-            d_stage[k], (uint32_t)n, ee - eb, nwords, pk->vbits, (const uint64_t *)base, (uint32_t *)(base + rbytes));
+            d_stage[k], (uint32_t)n, ee - eb, nwords, pk->vbits, rp, cp);
         LT_HIP(hipGetLastError());
         LT_HIP(hipEventRecord(stage_free[k], s_copy));
         stage_used[k] = true;
@@ -780,7 +816,7 @@ lt_status Engine::copy_partition(uint32_t p, uint8_t *base) {
         st.packed_image_bytes += pk->size[p];
         st.packed_col_bytes += cbytes;
     } else {
-        if (cbytes) LT_HIP(hipMemcpyAsync(base + rbytes, g->col + eb, cbytes, hipMemcpyHostToDevice, s_dma));
+        if (cbytes) LT_HIP(hipMemcpyAsync(cp, g->col + eb, cbytes, hipMemcpyHostToDevice, s_dma));
         st.h2d_bytes_explicit += cbytes;
         if (s_dma != s_copy) {
             LT_HIP(hipEventRecord(ev_dma, s_dma));
@@ -805,7 +841,7 @@ lt_status Engine::fetch_partition(uint32_t p, uint64_t *rowptr_out, uint32_t *co
     uint8_t *buf = nullptr;
     LT_TRY(dmalloc(&buf, rn * 8 + m * 4));
     const lt_stats keep = st;
-    lt_status rc = copy_partition(p, buf);
+    lt_status rc = copy_partition(p, (uint64_t *)buf, (uint32_t *)(buf + rn * 8));
     st = keep;
     hipError_t e = rc == LT_OK ? hipStreamSynchronize(s_copy) : hipSuccess;
     if (rc == LT_OK && e == hipSuccess) e = hipMemcpy(rowptr_out, buf, rn * 8, hipMemcpyDeviceToHost);
@@ -879,10 +915,12 @@ lt_status Engine::process(uint32_t p, bool zerocopy, uint64_t walkers) {
         a.rowptr = zc_rowptr + part.node_off[p];
         a.col = zc_col + part.edge_off[p];
     } else {
-        const uint8_t *base = d_slots + (size_t)slot_of[p] * slot_sz;
-        a.rowptr = (const uint64_t *)base;
-        a.col = (const uint32_t *)(base + ((uint64_t)part.node_off[p + 1] - part.node_off[p] + 1) * 8);
-        a.words = slot_words(p, a.col);
+        uint64_t *rp;
+        uint32_t *cp;
+        slot_ptrs(p, &rp, &cp);
+        a.rowptr = rp;
+        a.col = cp;
+        a.words = slot_words(p, cp);
     }
     EventTimer &phase = zerocopy ? t_zc : t_compute;
     hipEvent_t tp = phase.begin(s_compute);
@@ -1752,6 +1790,66 @@ lt_status Engine::scheduler_loop_device() {
     return LT_OK;
 }
 
+// Whether the job can walk the flat arrays: every partition cached, walkers
+// allowed to walk through all of them in one launch (span resident with
+// batches, or a single partition), all of them on the device at once, and no
+// decision trace or append ablation asked for.  Edge numbers have to fit 32 bits.
+bool Engine::can_run_flat() const {
+    if (!flat || g->E > 0xFFFFFFFFull || cfg.record_trace || cfg.append_mode != 0 || spill_on) return false;
+    if (P > 1 && (cfg.span != LT_SPAN_RESIDENT || res_batch <= 1)) return false;
+    for (uint32_t p = 0; p < P; p++)
+        if (!resident[p]) return false;
+    return true;
+}
+
+// Eight workgroups per CU: the kernels hold few registers, and the lanes of a
+// small job should all have one walker before any has two.
+static void launch_flat(const FlatArgs &a, int app, int num_cu, hipStream_t s) {
+    const uint64_t n = a.id_hi - a.id_lo;
+    const int grid = (int)std::min<uint64_t>((n + kBlock - 1) / kBlock, (uint64_t)8 * num_cu);
+    if (app == APP_PAGERANK) flat_walk_kernel<APP_PAGERANK><<<grid, kBlock, 0, s>>>(a);
+    else if (app == APP_PPR) flat_ppr_kernel<<<grid, kBlock, 0, s>>>(a);
+    else flat_walk_kernel<APP_GENERIC><<<grid, kBlock, 0, s>>>(a);
+}
+
+// Walkers of one launch: as many as a queue slice of the default size holds,
+// which keeps the per-lane event counts far below 2^32.
+constexpr uint64_t kFlatPiece = (uint64_t)kSliceChunks * kChunk;
+
+// The whole job over the flat arrays: walkers are created, walked and finished
+// in registers, so the queues are not touched.  Row offsets are read as 32
+// bits, which halves the lines that the hot rows take in L2.
+lt_status Engine::run_flat(const RunSpec &rs) {
+    if (!d_rowptr32) {  // kept: slots of a flat cache are never evicted
+        LT_TRY(dmalloc(&d_rowptr32, (size_t)V + 1));
+        narrow_rowptr_kernel<<<std::min<int>(8 * num_cu, (int)(V / 256 + 1)), 256, 0, s_compute>>>(
+            flat_rowptr, d_rowptr32, (size_t)V + 1);
+        LT_HIP(hipGetLastError());
+    }
+    FlatArgs a{};
+    a.app = app;
+    a.rowptr = d_rowptr32;
+    a.col = flat_col;
+    a.stats = d_stats;
+    hipEvent_t tp = t_compute.begin(s_compute);
+    for (uint64_t lo = 0; lo < rs.total; lo += kFlatPiece) {
+        a.id_lo = lo;
+        a.id_hi = std::min<uint64_t>(rs.total, lo + kFlatPiece);
+        hipEvent_t tk = t_kernel.begin(s_compute);
+        launch_flat(a, app_kind, num_cu, s_compute);
+        LT_HIP(hipGetLastError());
+        t_kernel.end(tk, s_compute);
+        st.kernel_launches++;
+    }
+    t_compute.end(tp, s_compute);
+    LT_HIP(spin_stream(s_compute));
+    w_run = rs.total;
+    st.iterations = st.explicit_iterations = st.computing_calls = 1;
+    st.resident_batched = P - 1;
+    for (uint32_t p = 0; p < P; p++) last_use[p] = ++use_clock;
+    return LT_OK;
+}
+
 lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoints_out, uint32_t *moves_out) {
     LT_HIP(hipSetDevice(device));
     memset(&st, 0, sizeof(st));
@@ -1782,7 +1880,8 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
     // partitions (capped cache, PPR around its sources); with every partition
     // resident the visits spread over all of V and one array is faster.
     count_copies = rs.app != APP_GENERIC && (nslots < P || rs.app == APP_PPR) ? kCountCopies : 1;
-    LT_TRY(ensure_pool(std::max<uint64_t>(cap, 1)));
+    const bool walk_flat = can_run_flat();
+    LT_TRY(ensure_pool(std::max<uint64_t>(cap, 1), walk_flat));  // a flat job keeps the queues' limits
     LT_TRY(ensure_outputs(rs, endpoints_out != nullptr, moves_out != nullptr));
 
     app_kind = rs.app;
@@ -1819,7 +1918,13 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
         LT_HIP(hipMemsetAsync(d_paths, 0xFF, 4 * (size_t)rs.total * (rs.length + 1), s_compute));
 
     double running_ms = 0;
-    for (uint64_t id0 = 0; id0 < rs.total; id0 += wave) {
+    if (walk_flat) {
+        LT_HIP(hipStreamSynchronize(s_compute));
+        const auto t0 = std::chrono::steady_clock::now();
+        LT_TRY(run_flat(rs));
+        running_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    }
+    for (uint64_t id0 = walk_flat ? rs.total : 0; id0 < rs.total; id0 += wave) {
         const uint64_t id1 = std::min<uint64_t>(rs.total, id0 + wave);
         // createWalkers: untimed, as in the reference (src/LightTraffic.h:33-44)
         reset_queues_kernel<<<1024, 256, 0, s_compute>>>(q, P);
@@ -1872,8 +1977,8 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
         LT_HIP(hipStreamSynchronize(s_compute));
         running_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     }
-    LT_TRY(read_meta());
-    for (uint32_t i = 0; i < P; i++)
+    if (!walk_flat) LT_TRY(read_meta());
+    for (uint32_t i = 0; !walk_flat && i < P; i++)
         if (counts[i]) {
             set_error("partition %u still holds %llu walkers after the run", i, (unsigned long long)counts[i]);
             return LT_E_INTERNAL;
