@@ -12,6 +12,7 @@
 #include <stdint.h>
 
 #include "lt_rng.h"
+#include "lt_visits.h"
 
 namespace lt {
 
@@ -54,7 +55,9 @@ struct Queues {
     uint32_t *free_stack;  // [nchunks]
     PoolCtl *ctl;
     uint32_t *lost;        // [kLostCap]
-    uint32_t *packed;      // [P + 4]: the P queue lengths, then PoolCtl (one D2H per decision)
+    uint32_t *packed;      // [P + 4 + kLogRegions]: the P queue lengths, PoolCtl, the fill of the
+                           // visit log's regions (one D2H per decision)
+    const unsigned long long *vcur;  // cursors of the visit log, or nullptr
     uint32_t maxc;         // chunk slots per partition
     uint32_t nchunks;
     uint32_t P;
@@ -86,6 +89,9 @@ struct AppArgs {
     uint32_t source;      // single-source ppr
     uint32_t *counts;     // u32[V] or, with counts_stride = V, u32[kCountCopies][V]; or nullptr
     uint64_t counts_stride;  // 0: one count array; V: workgroup b counts into copy b % kCountCopies
+    uint32_t *vlog;       // visit log (VisitLog), or nullptr: visits are added to counts directly
+    unsigned long long *vcur;  // its cursors
+    uint32_t vcap;        // entries per region
     uint32_t *endpoints;  // u32[N] indexed by walker id, or nullptr
     uint32_t *moves_out;  // u32[N] (genericwalk), or nullptr
     uint32_t *paths;      // genericwalk: u32[N][length + 1], vertex after k moves at [id][k], or nullptr

@@ -233,6 +233,16 @@ struct Engine {
     uint32_t *d_counts = nullptr;
     size_t counts_cap = 0;
     uint32_t count_copies = 1;  // 1 or kCountCopies arrays of V counts
+    // Visit log of the running job (lt_visits.h) and the scratch it is counted with.
+    uint32_t nbins = 0;
+    VisitLog vl{};
+    VisitScratch vs{};
+    unsigned long long *d_vcur = nullptr;
+    uint64_t vlog_cap = 0;                       // entries allocated
+    uint64_t vrun_cap = 0, vpartial_cap = 0;     // words
+    uint32_t vregion = 0;                        // entries per region of the running job, 0 = no log
+    lt_status ensure_log(uint64_t visits, bool queued);
+    lt_status count_log(uint32_t n, uint32_t most);
     uint32_t *d_endpoints = nullptr;
     size_t endpoints_cap = 0;
     uint32_t *d_moves = nullptr;
@@ -378,6 +388,13 @@ Engine::~Engine() {
     dfree(d_plan);
     if (h_plan) (void)hipHostFree(h_plan);
     dfree(d_counts);
+    dfree(vl.log);
+    dfree(d_vcur);
+    dfree(vs.sorted);
+    dfree(vs.run);
+    dfree(vs.total);
+    dfree(vs.unit_off);
+    dfree(vs.partial);
     dfree(d_endpoints);
     dfree(d_moves);
     dfree(d_paths);
@@ -591,11 +608,16 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
     // queue lengths one 128-byte line apart, then PoolCtl on its own line; the
     // fix-up kernel packs both into h_meta (pinned, mapped) for the host
     LT_TRY(dmalloc(&d_meta, (size_t)P * kQStride + kQStride));
-    LT_HIP(hipHostMalloc((void **)&h_meta, 4 * (P + 4), hipHostMallocMapped | hipHostMallocCoherent));
+    LT_HIP(hipHostMalloc((void **)&h_meta, 4 * (P + 4 + kLogRegions), hipHostMallocMapped | hipHostMallocCoherent));
     LT_HIP(hipHostGetDevicePointer((void **)&q.packed, h_meta, 0));
     q.qlen = d_meta;
     q.ctl = (PoolCtl *)(d_meta + (size_t)P * kQStride);
     q.P = P;
+    LT_TRY(dmalloc(&d_vcur, (size_t)kLogRegions * kCurStride));
+    LT_HIP(hipMemset(d_vcur, 0, sizeof(*d_vcur) * kLogRegions * kCurStride));
+    nbins = (uint32_t)(((uint64_t)V + kBin - 1) / kBin);
+    LT_TRY(dmalloc(&vs.total, nbins));
+    LT_TRY(dmalloc(&vs.unit_off, (size_t)nbins + 1));
     LT_TRY(dmalloc(&d_ds, 1));
     LT_TRY(dmalloc(&d_slot_of, P));
     LT_TRY(dmalloc(&d_part_in_slot, nslots));
@@ -691,6 +713,77 @@ lt_status Engine::ensure_outputs(const RunSpec &rs, bool want_endpoints, bool wa
     return LT_OK;
 }
 
+// Log for a job of `visits` visits, or none (vregion = 0).  A flat job has one from
+// kLogVisits on: below, the counters' atomics (27 G/s) cost less than the
+// launches that count a log, 10 to 30 us.  A job that goes through the queues walks
+// a few thousand visits a launch when it is small, and their atomics overlap
+// its other waits: 14 M visits in 900 launches took 33.0 ms directly and 35.0 with
+// a log, 103 M in 72 launches 18.4 and 15.1.  Above kMaxBins bins (67 M
+// vertices) the scatter's LDS does not hold a tile's histogram, and a device
+// that cannot hold a log counts directly.
+constexpr uint64_t kLogVisits = 1u << 18, kLogVisitsQueued = 1u << 24;
+constexpr uint64_t kLogMost = 1ull << 26;  // entries: 256 MB, and 128 MB sorted
+
+lt_status Engine::ensure_log(uint64_t visits, bool queued) {
+    vregion = 0;
+    if (visits < (queued ? kLogVisitsQueued : kLogVisits) || nbins > kMaxBins) return LT_OK;
+    // regions fill unevenly: a quarter more, and a launch's workgroups' buffers
+    visits = std::min(visits, kLogMost);
+    const uint64_t want = std::min(kLogMost, visits + visits / 4 + (1u << 20)) & ~(uint64_t)(kTile * kLogRegions - 1);
+    if (vlog_cap < want) {
+        dfree(vl.log);
+        dfree(vs.sorted);
+        vlog_cap = 0;
+        if (dmalloc(&vl.log, want) != LT_OK || dmalloc(&vs.sorted, want) != LT_OK) {
+            dfree(vl.log);
+            dfree(vs.sorted);
+            return LT_OK;
+        }
+        vlog_cap = want;
+    }
+    vregion = (uint32_t)(want / kLogRegions);
+    return LT_OK;
+}
+
+// Counts the log into d_counts and empties it: the n entries of a flat job's
+// log, or (n = 0) the regions, which hold at most `most` entries each.
+lt_status Engine::count_log(uint32_t n, uint32_t most) {
+    VisitLog l = vl;
+    l.cur = d_vcur;
+    l.cap = n ? 0 : vregion;
+    l.n = n;
+    const uint64_t entries = n ? n : (uint64_t)std::min(most, vregion) * kLogRegions;
+    if (entries == 0) return LT_OK;
+    l.tiles = (uint32_t)(((n ? n : entries / kLogRegions) + kTile - 1) / kTile);
+    const uint32_t ntiles = n ? l.tiles : l.tiles * kLogRegions;
+    const bool few = nbins <= kFewBins && ntiles * nbins <= 1024;
+    vs.unit = std::max<uint32_t>(kHistUnit, (uint32_t)(entries / 512));
+    const uint32_t units = few ? ntiles * nbins : (uint32_t)((entries + vs.unit - 1) / vs.unit) + nbins;
+    if (vpartial_cap < (uint64_t)units * kBin) {
+        dfree(vs.partial);
+        vpartial_cap = 0;
+        LT_TRY(dmalloc(&vs.partial, (size_t)units * kBin));
+        vpartial_cap = (uint64_t)units * kBin;
+    }
+    if (few) {
+        visit_hist_kernel<false><<<units, kVisitThreads, 0, s_compute>>>(l, vs, nbins, ntiles);
+    } else {
+        if (vrun_cap < (uint64_t)nbins * ntiles) {
+            dfree(vs.run);
+            vrun_cap = 0;
+            LT_TRY(dmalloc(&vs.run, (size_t)nbins * ntiles));
+            vrun_cap = (uint64_t)nbins * ntiles;
+        }
+        visit_tile_kernel<<<ntiles, kVisitThreads, 4 * kRepl * nbins, s_compute>>>(l, vs, nbins, ntiles);
+        visit_scan_kernel<<<nbins, kVisitThreads, 0, s_compute>>>(vs, ntiles);
+        visit_scatter_kernel<<<ntiles, kVisitThreads, scatter_lds(nbins), s_compute>>>(l, vs, nbins, ntiles);
+        visit_hist_kernel<true><<<units, kVisitThreads, 0, s_compute>>>(l, vs, nbins, ntiles);
+    }
+    visit_sum_kernel<<<(V + 255) / 256, 256, 0, s_compute>>>(l, vs, d_counts, V);
+    LT_HIP(hipGetLastError());
+    return LT_OK;
+}
+
 lt_status Engine::read_meta() {
     if (meta_dirty) {  // the last queue update on s_compute was not followed by a fix-up
         pack_meta_kernel<<<1, kBlock, 0, s_compute>>>(q);
@@ -706,6 +799,15 @@ lt_status Engine::read_meta() {
     for (uint32_t i = 0; i < P; i++) {
         dcounts[i] = h_meta[i];
         counts[i] = dcounts[i] + hcount[i];
+    }
+    if (vregion) {  // the log is counted before its fullest region is full
+        const uint32_t *cur = h_meta + P + 4;
+        const uint32_t most = *std::max_element(cur, cur + kLogRegions);
+        if (most >= vregion / 5 * 4) {
+            LT_TRY(count_log(0, most));
+            meta_dirty = true;
+            for (uint32_t r = 0; r < kLogRegions; r++) h_meta[P + 4 + r] = 0;
+        }
     }
     return LT_OK;
 }
@@ -1759,10 +1861,12 @@ lt_status Engine::scheduler_loop_device() {
     uint64_t launches = 0;
     while (true) {
         LT_HIP(hipGraphLaunch(exec, s_compute));
+        meta_dirty = false;  // each iteration ends with a fix-up
         launches++;
         LT_HIP(hipMemcpyAsync(&h, d_ds, sizeof(h), hipMemcpyDeviceToHost, s_compute));
         LT_HIP(hipStreamSynchronize(s_compute));
         if (h.choice < 0) break;
+        if (vregion) LT_TRY(read_meta());  // counts the visit log if it fills up
         if (launches > (1ull << 24)) {
             set_error("device schedule did not drain the queues");
             return LT_E_INTERNAL;
@@ -1832,14 +1936,20 @@ lt_status Engine::run_flat(const RunSpec &rs) {
     a.col = flat_col;
     a.stats = d_stats;
     hipEvent_t tp = t_compute.begin(s_compute);
-    for (uint64_t lo = 0; lo < rs.total; lo += kFlatPiece) {
+    // a launch's visits have to fit the log; walks too long for that count directly
+    uint64_t piece = kFlatPiece;
+    const uint64_t each = app_kind == APP_PAGERANK ? rs.length : 1, room = (uint64_t)vregion * kLogRegions;
+    if (a.app.vlog && room / each < std::min<uint64_t>(rs.total, 1u << 16)) a.app.vlog = nullptr;
+    if (a.app.vlog) piece = std::min(piece, room / each);
+    for (uint64_t lo = 0; lo < rs.total; lo += piece) {
         a.id_lo = lo;
-        a.id_hi = std::min<uint64_t>(rs.total, lo + kFlatPiece);
+        a.id_hi = std::min<uint64_t>(rs.total, lo + piece);
         hipEvent_t tk = t_kernel.begin(s_compute);
         launch_flat(a, app_kind, num_cu, s_compute);
         LT_HIP(hipGetLastError());
         t_kernel.end(tk, s_compute);
         st.kernel_launches++;
+        if (a.app.vlog) LT_TRY(count_log((uint32_t)((a.id_hi - lo) * each), 0));
     }
     t_compute.end(tp, s_compute);
     LT_HIP(spin_stream(s_compute));
@@ -1876,11 +1986,19 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
     spill_on = cap < rs.total && !cfg.device_schedule;
     dev_cap = cap;
     const uint64_t wave = spill_on ? rs.total : cap;
-    // Per-XCD count copies pay when the walkers of one launch stay in a few
-    // partitions (capped cache, PPR around its sources); with every partition
-    // resident the visits spread over all of V and one array is faster.
-    count_copies = rs.app != APP_GENERIC && (nslots < P || rs.app == APP_PPR) ? kCountCopies : 1;
+    const bool counting = rs.app != APP_GENERIC && counts_out;
+    uint64_t visits = rs.total;
+    if (rs.app == APP_PAGERANK && __builtin_mul_overflow(rs.total, (uint64_t)rs.length, &visits)) visits = UINT64_MAX;
     const bool walk_flat = can_run_flat();
+    if (counting) LT_TRY(ensure_log(visits, !walk_flat));
+    else vregion = 0;
+    // Without a log, copies of the counters, one per XCD: through the queues
+    // where the walkers of one launch stay in a few partitions (capped cache,
+    // PPR around its sources; one array measured 29 % slower there); for a flat
+    // job where clearing and adding up the copies of a small graph costs less than
+    // its hot vertices' atomics (5 G/s in one array, 27 G/s in copies).
+    const bool copies = walk_flat ? visits >= (1u << 16) && V <= (1u << 20) : nslots < P || rs.app == APP_PPR;
+    count_copies = counting && !vregion && copies ? kCountCopies : 1;
     LT_TRY(ensure_pool(std::max<uint64_t>(cap, 1), walk_flat));  // a flat job keeps the queues' limits
     LT_TRY(ensure_outputs(rs, endpoints_out != nullptr, moves_out != nullptr));
 
@@ -1890,8 +2008,12 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
     app.V = V;
     app.length = rs.length;
     app.source = rs.source;
-    app.counts = d_counts;
+    app.counts = counting ? d_counts : nullptr;
     app.counts_stride = count_copies > 1 ? V : 0;
+    app.vlog = vregion ? vl.log : nullptr;
+    app.vcur = d_vcur;
+    app.vcap = vregion;
+    q.vcur = vregion ? d_vcur : nullptr;
     app.endpoints = endpoints_out ? d_endpoints : nullptr;
     app.moves_out = moves_out ? d_moves : nullptr;
     app.paths = rs.paths_out ? d_paths : nullptr;
@@ -1911,7 +2033,8 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
         app.q_src = d_qsrc;
         app.nq = rs.nq;
     }
-    LT_HIP(hipMemsetAsync(d_counts, 0, 4 * (size_t)V * count_copies, s_compute));
+    if (vregion) LT_HIP(hipMemsetAsync(d_vcur, 0, sizeof(*d_vcur) * kLogRegions * kCurStride, s_compute));
+    if (counting) LT_HIP(hipMemsetAsync(d_counts, 0, 4 * (size_t)V * count_copies, s_compute));
     LT_HIP(hipMemsetAsync(d_stats, 0, 8 * (size_t)kNumStats * kStatSlots, s_compute));
     if (moves_out) LT_HIP(hipMemsetAsync(d_moves, 0, 4 * rs.total, s_compute));
     if (rs.paths_out)  // columns after an early stop stay 0xFFFFFFFF
@@ -1970,7 +2093,15 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
         const auto t1 = std::chrono::steady_clock::now();
         running_ms += std::chrono::duration<double, std::milli>(t1 - t0).count();
     }
-    if (count_copies > 1) {  // part of the walk's work, so inside the timed region
+    if (vregion && !walk_flat) {  // part of the walk's work, so inside the timed region
+        const auto t0 = std::chrono::steady_clock::now();
+        LT_TRY(read_meta());
+        const uint32_t *cur = h_meta + P + 4;
+        LT_TRY(count_log(0, *std::max_element(cur, cur + kLogRegions)));
+        LT_HIP(hipStreamSynchronize(s_compute));
+        running_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    }
+    if (count_copies > 1) {
         const auto t0 = std::chrono::steady_clock::now();
         sum_count_copies_kernel<<<std::max(1, 8 * num_cu), 256, 0, s_compute>>>(d_counts, V);
         LT_HIP(hipGetLastError());

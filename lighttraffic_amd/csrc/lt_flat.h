@@ -55,16 +55,7 @@ __global__ __launch_bounds__(kBlock) void flat_walk_kernel(FlatArgs a) {
     const uint64_t seed = a.app.seed;
     const uint32_t length = a.app.length;
     Counters ct;
-    if constexpr (APP == APP_PAGERANK) {
-        __shared__ uint32_t s_vkeys[kVisitSlots], s_vcnt[kVisitSlots];
-        for (uint32_t i = threadIdx.x; i < kVisitSlots; i += blockDim.x) {
-            s_vkeys[i] = kVisitEmpty;
-            s_vcnt[i] = 0;
-        }
-        __syncthreads();
-        ct.vkeys = s_vkeys;
-        ct.vcnt = s_vcnt;
-    }
+    const uint64_t n = a.id_hi - a.id_lo;
     const uint64_t stride = (uint64_t)gridDim.x * kBlock;
     for (uint64_t id = a.id_lo + (uint64_t)blockIdx.x * kBlock + threadIdx.x; id < a.id_hi; id += stride) {
         const u32x4 s = draw(seed, id, 0, TAG_START);
@@ -75,7 +66,9 @@ __global__ __launch_bounds__(kBlock) void flat_walk_kernel(FlatArgs a) {
             for (; left > 0; left--) {
                 // the draw does not wait for the vertex being read
                 const u32x4 x = draw(seed, id, left - 1, TAG_PAGERANK);
-                count_visit(a.app, cur, ct);
+                // every walker visits `length` vertices: its place in the log is known
+                if (a.app.vlog) __builtin_nontemporal_store(cur, &a.app.vlog[(length - left) * n + (id - a.id_lo)]);
+                else if (a.app.counts) count_direct(a.app, cur);
                 ct.visits++;
                 if (left == 1) break;
                 uint32_t b = 0, d = 0;
@@ -104,7 +97,6 @@ __global__ __launch_bounds__(kBlock) void flat_walk_kernel(FlatArgs a) {
         }
         if (a.app.endpoints) a.app.endpoints[id] = cur;
     }
-    if constexpr (APP == APP_PAGERANK) flush_visits(a.app, ct);
     flush_counters(ct, a.stats);
 }
 
@@ -115,16 +107,7 @@ __global__ __launch_bounds__(kBlock) void flat_walk_kernel(FlatArgs a) {
 __global__ __launch_bounds__(kBlock) void flat_ppr_kernel(FlatArgs a) {
     const uint32_t *rp = a.rowptr;
     Counters ct;
-    __shared__ uint32_t s_vkeys[kVisitSlots], s_vcnt[kVisitSlots];
     __shared__ uint32_t s_next;
-    if (a.app.counts) {  // uniform
-        for (uint32_t i = threadIdx.x; i < kVisitSlots; i += blockDim.x) {
-            s_vkeys[i] = kVisitEmpty;
-            s_vcnt[i] = 0;
-        }
-        ct.vkeys = s_vkeys;
-        ct.vcnt = s_vcnt;
-    }
     const uint64_t n = a.id_hi - a.id_lo, per = (n + gridDim.x - 1) / gridDim.x;
     const uint64_t lo = a.id_lo + (uint64_t)blockIdx.x * per;
     const uint32_t mine = lo < a.id_hi ? (uint32_t)min(per, a.id_hi - lo) : 0u;
@@ -167,14 +150,14 @@ __global__ __launch_bounds__(kBlock) void flat_ppr_kernel(FlatArgs a) {
             }
         }
         if (over) {
-            if (a.app.counts) count_visit(a.app, cur, ct);
+            if (a.app.vlog) a.app.vlog[id - a.id_lo] = cur;  // one visit per walker
+            else if (a.app.counts) count_direct(a.app, cur);
             ct.visits++;
             if (a.app.endpoints) a.app.endpoints[id] = cur;
             i = atomicAdd(&s_next, 1u);
             if (i < mine) start(i);
         }
     }
-    if (a.app.counts) flush_visits(a.app, ct);
     flush_counters(ct, a.stats);
 }
 

@@ -368,8 +368,7 @@ __device__ void block_append(const Queues &q, uint32_t P, const AppendLds &L, co
 // Per-thread event counts of one launch (far below 2^32), summed as u64.
 struct Counters {
     uint32_t moves = 0, tele = 0, visits = 0, resid = 0, zc_moves = 0, zc_reads = 0;
-    uint32_t passes = 0;  // workgroup passes since the launch began (uniform in a workgroup)
-    uint32_t *vkeys = nullptr, *vcnt = nullptr;  // workgroup visit table in LDS (walk kernels)
+    uint32_t *vbuf = nullptr, *vn = nullptr;  // workgroup visit buffer in LDS and its fill (walk kernels)
 };
 
 // Workgroup sum of the counters, added to slot blockIdx.x % kStatSlots, so
@@ -420,48 +419,51 @@ __device__ __forceinline__ uint32_t span_col(const Span &sp, uint64_t e) {
 
 __device__ __forceinline__ uint64_t walker_id(const Walker &w) { return ((uint64_t)w.id_hi << 32) | w.id_lo; }
 
-// Visits go to a workgroup table in LDS (open addressing, 4 probes) and reach
-// the global counters once per vertex every kVisitFlushPasses passes and at
-// the end of the launch (flush_visits); a vertex that finds no slot is
-// counted in global memory directly.  Flushing every pass instead cost 2 % of
-// the walk time of R-MAT s26 pagerank with an 8 GB cache; every 16, 64 passes
-// or only at the end measured the same.
-constexpr uint32_t kVisitSlots = 2048;
-constexpr uint32_t kVisitFlushPasses = 16;  // a power of two
-constexpr uint32_t kVisitEmpty = 0xFFFFFFFFu;
+// Visits go to the visit log: a workgroup collects a pass's visits in LDS
+// (consecutive lanes, one LDS atomic per wave) and copies them to its region of
+// the log after the pass, in one reservation (walk_walkers).  Visits that do not
+// fit the buffer are reserved in the log wave by wave, and those that do not fit
+// the log, or of a job without one, are added to the counters directly.
+constexpr uint32_t kVisitBuf = 4096;
 
-__device__ __forceinline__ void count_visit(const AppArgs &a, uint32_t v, Counters &ct) {
-    if (ct.vkeys) {
-        const uint32_t h = (v * 2654435761u) >> 21;  // 11 bits: kVisitSlots
-#pragma unroll
-        for (uint32_t probe = 0; probe < 4; probe++) {
-            const uint32_t i = (h + probe) & (kVisitSlots - 1);
-            uint32_t k = ct.vkeys[i];
-            if (k == kVisitEmpty) k = atomicCAS(&ct.vkeys[i], kVisitEmpty, v);
-            if (k == kVisitEmpty || k == v) {
-                atomicAdd(&ct.vcnt[i], 1u);
-                return;
-            }
-        }
-    }
+__device__ __forceinline__ void count_direct(const AppArgs &a, uint32_t v) {
     atomicAdd(&a.counts[(size_t)(blockIdx.x % kCountCopies) * a.counts_stride + v], 1u);
 }
 
-// Adds the workgroup's visit table to the global counters and empties it.
-// Collective over the workgroup.
-__device__ __forceinline__ void flush_visits(const AppArgs &a, const Counters &ct) {
-    if (!ct.vkeys) return;
-    __syncthreads();
-    uint32_t *g = a.counts + (size_t)(blockIdx.x % kCountCopies) * a.counts_stride;
-    for (uint32_t i = threadIdx.x; i < kVisitSlots; i += blockDim.x) {
-        const uint32_t k = ct.vkeys[i];
-        if (k != kVisitEmpty) {
-            atomicAdd(&g[k], ct.vcnt[i]);
-            ct.vkeys[i] = kVisitEmpty;
-            ct.vcnt[i] = 0;
+// First of n entries reserved in the workgroup's region (vcap: past its end).
+__device__ __forceinline__ uint32_t log_reserve(const AppArgs &a, uint32_t n) {
+    const unsigned long long at = atomicAdd(&a.vcur[(blockIdx.x % kLogRegions) * kCurStride], (unsigned long long)n);
+    return (uint32_t)min(at, (unsigned long long)a.vcap);
+}
+
+__device__ __forceinline__ uint32_t lanes_before(uint64_t mask) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+__device__ __forceinline__ void log_store(const AppArgs &a, uint32_t i, uint32_t v) {
+    if (i < a.vcap) a.vlog[(size_t)(blockIdx.x % kLogRegions) * a.vcap + i] = v;
+    else count_direct(a, v);
+}
+
+__device__ __forceinline__ void count_visit(const AppArgs &a, uint32_t v, Counters &ct) {
+    if (ct.vbuf) {
+        const uint64_t m = __ballot(1);
+        const uint32_t rank = lanes_before(m);
+        uint32_t i = 0;
+        if (rank == 0) i = atomicAdd(ct.vn, (uint32_t)__popcll(m));
+        i = (uint32_t)__builtin_amdgcn_readfirstlane((int)i) + rank;
+        if (i < kVisitBuf) {
+            ct.vbuf[i] = v;
+            return;
         }
+        const uint64_t o = __ballot(1);
+        const uint32_t orank = lanes_before(o);
+        uint32_t j = 0;
+        if (orank == 0) j = log_reserve(a, (uint32_t)__popcll(o));
+        log_store(a, (uint32_t)__builtin_amdgcn_readfirstlane((int)j) + orank, v);
+        return;
     }
-    __syncthreads();
+    if (a.counts) count_direct(a, v);
 }
 
 // One update of app/pagerank.cu:26-44: count the visit, then teleport with
@@ -496,7 +498,7 @@ __device__ __forceinline__ void step_pagerank(Walker &w, const Span &sp, const A
 // left; a vertex without neighbours is counted and ends the walk.
 __device__ __forceinline__ void step_ppr(Walker &w, const Span &sp, const AppArgs &a, Counters &ct) {
     if (w.step == 1) {
-        if (a.counts) count_visit(a, w.cur, ct);
+        count_visit(a, w.cur, ct);
         ct.visits++;
     }
     w.step -= 1;
@@ -509,7 +511,7 @@ __device__ __forceinline__ void step_ppr(Walker &w, const Span &sp, const AppArg
         ct.moves++;
         if (sp.zc) { ct.zc_moves++; ct.zc_reads += 1 + a.rp_host; }
     } else {
-        if (a.counts) count_visit(a, w.cur, ct);
+        count_visit(a, w.cur, ct);
         ct.visits++;
         w.step = 0;
         if (sp.zc) ct.zc_reads += a.rp_host;
@@ -603,10 +605,27 @@ __device__ __forceinline__ void walk_walkers(const WalkArgs &a, const AppendLds 
     for (int k = 0; k < WPT; k++) {
         if ((uint32_t)k * kBlock + threadIdx.x < nvalid) dst[k] = walk_residency<APP>(w[k], a, src, src_sp, ct);
     }
-    block_append<WPT>(a.q, a.pt.P, L, w, dst, s_wsum, a.append_mode);
     if constexpr (APP != APP_GENERIC) {  // genericwalk counts no visits
-        if ((++ct.passes & (kVisitFlushPasses - 1)) == 0) flush_visits(a.app, ct);
+        if (ct.vbuf) {  // uniform
+            // The log is reserved before the append and written after it, so
+            // the reservation's round trip overlaps the append's own.
+            __shared__ uint32_t s_at;
+            __syncthreads();
+            const uint32_t n = min(*ct.vn, kVisitBuf);
+            uint32_t at = 0;
+            if (threadIdx.x == kBlock - 1 && n) at = log_reserve(a.app, n);
+            block_append<WPT>(a.q, a.pt.P, L, w, dst, s_wsum, a.append_mode);
+            if (threadIdx.x == kBlock - 1) {
+                s_at = at;
+                *ct.vn = 0;
+            }
+            __syncthreads();
+            for (uint32_t i = threadIdx.x; i < n; i += kBlock) log_store(a.app, s_at + i, ct.vbuf[i]);
+            __syncthreads();
+            return;
+        }
     }
+    block_append<WPT>(a.q, a.pt.P, L, w, dst, s_wsum, a.append_mode);
 }
 
 // One workgroup pass: walkers [base, base + kBlock * WPT) of src's queue,
@@ -634,15 +653,12 @@ __global__ __launch_bounds__(kBlock) void walk_kernel(WalkArgs a) {
     const AppendLds L = carve_lds(smem, a.pt.P, WPT);
     Counters ct;
     if constexpr (APP != APP_GENERIC) {
-        __shared__ uint32_t s_vkeys[kVisitSlots], s_vcnt[kVisitSlots];
-        if (a.app.counts) {  // uniform
-            for (uint32_t i = threadIdx.x; i < kVisitSlots; i += blockDim.x) {
-                s_vkeys[i] = kVisitEmpty;
-                s_vcnt[i] = 0;
-            }
+        __shared__ uint32_t s_vbuf[kVisitBuf], s_vn;
+        if (a.app.vlog) {  // uniform
+            if (threadIdx.x == 0) s_vn = 0;
             __syncthreads();
-            ct.vkeys = s_vkeys;
-            ct.vcnt = s_vcnt;
+            ct.vbuf = s_vbuf;
+            ct.vn = &s_vn;
         }
     }
     if (a.nsrc) {  // batch: the whole queues of several partitions, each in the partition table
@@ -662,7 +678,6 @@ __global__ __launch_bounds__(kBlock) void walk_kernel(WalkArgs a) {
             const uint64_t local = base - a.voff[k], n = qlen_of(a.q, src);
             if (local < n) walk_pass<APP, WPT>(a, L, s_wsum, src, sp, local, n, ct);  // uniform per workgroup
         }
-        if constexpr (APP != APP_GENERIC) flush_visits(a.app, ct);
         flush_counters(ct, a.stats);
         return;
     }
@@ -683,7 +698,6 @@ __global__ __launch_bounds__(kBlock) void walk_kernel(WalkArgs a) {
                 walk_walkers<APP, WPT>(a, L, s_wsum, src, src_sp, a.hptr[k] + local,
                                        min(a.hn[k] - local, (uint32_t)BW), ct);
         }
-        if constexpr (APP != APP_GENERIC) flush_visits(a.app, ct);
         flush_counters(ct, a.stats);
         return;
     }
@@ -713,7 +727,6 @@ __global__ __launch_bounds__(kBlock) void walk_kernel(WalkArgs a) {
     src_sp.eb = a.pt.edge_off[src];
     for (uint64_t base = lo64 + (uint64_t)blockIdx.x * BW; base < hi64; base += (uint64_t)gridDim.x * BW)
         walk_pass<APP, WPT>(a, L, s_wsum, src, src_sp, base, hi64, ct);
-    if constexpr (APP != APP_GENERIC) flush_visits(a.app, ct);
     flush_counters(ct, a.stats);
 }
 
@@ -796,6 +809,8 @@ __device__ void pack_meta(const Queues &q) {
         q.packed[q.P + 2] = c.nlost;
         q.packed[q.P + 3] = c.overflow;
     }
+    if (q.vcur && threadIdx.x < kLogRegions)
+        q.packed[q.P + 4 + threadIdx.x] = (uint32_t)min(q.vcur[threadIdx.x * kCurStride], 0xFFFFFFFFull);
 }
 
 __global__ __launch_bounds__(kBlock) void pack_meta_kernel(Queues q) { pack_meta(q); }
