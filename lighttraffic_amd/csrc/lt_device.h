@@ -55,8 +55,9 @@ struct Queues {
     uint32_t *free_stack;  // [nchunks]
     PoolCtl *ctl;
     uint32_t *lost;        // [kLostCap]
-    uint32_t *packed;      // [P + 4 + kLogRegions]: the P queue lengths, PoolCtl, the fill of the
-                           // visit log's regions (one D2H per decision)
+    uint32_t *packed;      // [P + 5 + kLogRegions] in mapped host memory: the P queue lengths, PoolCtl, the
+                           // fill of the visit log's regions, and seq once the rest is written
+    uint32_t seq;          // names this launch's write of packed
     const unsigned long long *vcur;  // cursors of the visit log, or nullptr
     uint32_t maxc;         // chunk slots per partition
     uint32_t nchunks;
@@ -194,12 +195,33 @@ struct SpillArgs {
     Walker *const *hptr;     // host chunks, mapped for the device
 };
 
-// Table entries of a zero-copy batch.
-struct ZcBatch {
+// Partition table entries to set before a walk.
+constexpr uint32_t kTableBatch = 32;
+struct TableBatch {
     uint32_t n;
-    uint32_t part[kMaxZcBatch];
-    const uint64_t *rowptr[kMaxZcBatch];
-    const uint32_t *col[kMaxZcBatch];
+    uint32_t part[kTableBatch];
+    uint8_t zc[kTableBatch];  // 1: the entry points at host memory (zero-copy batch)
+    const uint64_t *rowptr[kTableBatch];  // nullptr: not resident
+    const uint32_t *col[kTableBatch];
+    const uint32_t *words[kTableBatch];
+};
+
+// Where the tables lie.
+struct Tables {
+    const uint64_t **rowptr;
+    const uint32_t **col;
+    const uint32_t **words;
+    uint8_t *zc;
+};
+
+// What a walk launch consumed (fixup_kernel): chunks [chunk_lo, chunk_hi) of
+// src[0]'s queue, or with n > 1 the whole queues of src[0..n).
+struct Consumed {
+    uint32_t n;  // 0: nothing
+    uint32_t src[kMaxZcBatch];
+    uint32_t chunk_lo, chunk_hi;
+    int last;    // the queues end with those chunks
+    int leave;   // src[] leave the partition table (zero-copy batch)
 };
 
 struct InitArgs {

@@ -114,16 +114,8 @@ struct EventTimer {
     }
 };
 
-// Waits on the scheduler's critical path poll instead of blocking: every
-// decision waits for the fix-up of the previous walk, and a blocking wait adds
-// its wake-up latency to each of them.
-static hipError_t spin_stream(hipStream_t st) {
-    hipError_t e;
-    while ((e = hipStreamQuery(st)) == hipErrorNotReady) {
-    }
-    return e;
-}
-
+// Waits for prefetch copies poll their events: a blocking wait adds its
+// wake-up latency to a decision.
 static hipError_t spin_event(hipEvent_t ev) {
     hipError_t e;
     while ((e = hipEventQuery(ev)) == hipErrorNotReady) {
@@ -307,7 +299,13 @@ struct Engine {
         return LT_OK;
     }
     bool meta_dirty = true;  // q.packed may be older than the queues
-    hipEvent_t ev_evicted = nullptr;  // table updates of prefetch evictions, awaited by the copy stream
+    uint32_t meta_seq = 0;   // of the last launch that writes q.packed
+    bool meta_seen = true;   // h_meta holds what that launch wrote
+    lt_status launch_fixup(const Consumed &d);
+    lt_status wait_meta();
+    TableBatch table_due{};  // table updates of the next walk launch
+    lt_status flush_tables();
+    Tables tables() const { return {d_rowptr_tab, d_col_tab, d_words_tab, d_zc_part}; }
     lt_status process(uint32_t p, bool zerocopy, uint64_t walkers_hint);
     lt_status process_zc(uint32_t c, const uint8_t *pending);
     lt_status walk_batch(const std::vector<uint32_t> &parts, bool zerocopy);
@@ -336,6 +334,7 @@ struct Engine {
         }
     }
     lt_status set_table(uint32_t p, bool present);
+    lt_status table_entry(uint32_t p, const uint64_t *rp, const uint32_t *cp, const uint32_t *wp, bool zc);
     bool can_run_flat() const;
     lt_status run_flat(const RunSpec &rs);
     lt_status scheduler_loop();
@@ -369,7 +368,6 @@ Engine::~Engine() {
     if (s_copy) (void)hipStreamSynchronize(s_copy);
     if (s_dma && s_dma != s_copy) (void)hipStreamSynchronize(s_dma);
     for (auto ev : pool_events) (void)hipEventDestroy(ev);
-    if (ev_evicted) (void)hipEventDestroy(ev_evicted);
     dfree(d_node_off);
     dfree(d_edge_off);
     dfree(d_lut);
@@ -392,8 +390,6 @@ Engine::~Engine() {
     dfree(d_vcur);
     dfree(vs.sorted);
     dfree(vs.run);
-    dfree(vs.total);
-    dfree(vs.unit_off);
     dfree(vs.partial);
     dfree(d_endpoints);
     dfree(d_moves);
@@ -608,20 +604,19 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
     // queue lengths one 128-byte line apart, then PoolCtl on its own line; the
     // fix-up kernel packs both into h_meta (pinned, mapped) for the host
     LT_TRY(dmalloc(&d_meta, (size_t)P * kQStride + kQStride));
-    LT_HIP(hipHostMalloc((void **)&h_meta, 4 * (P + 4 + kLogRegions), hipHostMallocMapped | hipHostMallocCoherent));
+    LT_HIP(hipHostMalloc((void **)&h_meta, 4 * (P + 5 + kLogRegions), hipHostMallocMapped | hipHostMallocCoherent));
+    memset(h_meta, 0, 4 * (P + 5 + kLogRegions));
     LT_HIP(hipHostGetDevicePointer((void **)&q.packed, h_meta, 0));
     q.qlen = d_meta;
     q.ctl = (PoolCtl *)(d_meta + (size_t)P * kQStride);
     q.P = P;
-    LT_TRY(dmalloc(&d_vcur, (size_t)kLogRegions * kCurStride));
-    LT_HIP(hipMemset(d_vcur, 0, sizeof(*d_vcur) * kLogRegions * kCurStride));
     nbins = (uint32_t)(((uint64_t)V + kBin - 1) / kBin);
-    LT_TRY(dmalloc(&vs.total, nbins));
-    LT_TRY(dmalloc(&vs.unit_off, (size_t)nbins + 1));
-    LT_TRY(dmalloc(&d_ds, 1));
-    LT_TRY(dmalloc(&d_slot_of, P));
-    LT_TRY(dmalloc(&d_part_in_slot, nslots));
-    LT_TRY(dmalloc(&d_resident, P));
+    if (cfg.device_schedule) {
+        LT_TRY(dmalloc(&d_ds, 1));
+        LT_TRY(dmalloc(&d_slot_of, P));
+        LT_TRY(dmalloc(&d_part_in_slot, nslots));
+        LT_TRY(dmalloc(&d_resident, P));
+    }
     LT_TRY(dmalloc(&d_zc_part, P));
     LT_HIP(hipMemset(d_zc_part, 0, P));
     zc_batch = cfg.zc_batch > 0 ? (uint32_t)cfg.zc_batch
@@ -727,6 +722,12 @@ constexpr uint64_t kLogMost = 1ull << 26;  // entries: 256 MB, and 128 MB sorted
 lt_status Engine::ensure_log(uint64_t visits, bool queued) {
     vregion = 0;
     if (visits < (queued ? kLogVisitsQueued : kLogVisits) || nbins > kMaxBins) return LT_OK;
+    if (!d_vcur) {
+        const size_t cur = (size_t)kLogRegions * kCurStride;  // cursors, then the bins' totals and first units
+        LT_TRY(dmalloc(&d_vcur, cur + nbins + 1));
+        vs.total = (uint32_t *)(d_vcur + cur);
+        vs.unit_off = vs.total + nbins;
+    }
     // regions fill unevenly: a quarter more, and a launch's workgroups' buffers
     visits = std::min(visits, kLogMost);
     const uint64_t want = std::min(kLogMost, visits + visits / 4 + (1u << 20)) & ~(uint64_t)(kTile * kLogRegions - 1);
@@ -784,13 +785,48 @@ lt_status Engine::count_log(uint32_t n, uint32_t most) {
     return LT_OK;
 }
 
+lt_status Engine::launch_fixup(const Consumed &d) {
+    q.seq = ++meta_seq;
+    fixup_kernel<<<1, kBlock, 0, s_compute>>>(q, d, tables(), nullptr);
+    LT_HIP(hipGetLastError());
+    meta_dirty = false;
+    meta_seen = false;
+    return LT_OK;
+}
+
+// Waits until h_meta holds what the last launch that packs it wrote, and so
+// until the walk before that launch is over.  Every decision waits here; the
+// host polls the number that the kernel writes: launch, fix-up and wait of a
+// small kernel take 10 us so, 27 us when hipStreamQuery is polled and 12 us with
+// hipStreamSynchronize.  A stream that ends or fails without the number being
+// written is found by the query made once in a while.
+lt_status Engine::wait_meta() {
+    if (meta_seen) return LT_OK;
+    const uint32_t *flag = h_meta + P + 4 + kLogRegions;
+    for (uint32_t it = 1; __atomic_load_n(flag, __ATOMIC_ACQUIRE) != meta_seq; it++) {
+        __builtin_ia32_pause();
+        if ((it & 0xFFFFF) == 0) {
+            const hipError_t e = hipStreamQuery(s_compute);
+            if (e == hipErrorNotReady) continue;
+            LT_HIP(e);
+            if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == meta_seq) break;
+            set_error("queue lengths were not written");
+            return LT_E_INTERNAL;
+        }
+    }
+    meta_seen = true;
+    return LT_OK;
+}
+
 lt_status Engine::read_meta() {
     if (meta_dirty) {  // the last queue update on s_compute was not followed by a fix-up
+        q.seq = ++meta_seq;
         pack_meta_kernel<<<1, kBlock, 0, s_compute>>>(q);
         LT_HIP(hipGetLastError());
         meta_dirty = false;
+        meta_seen = false;
     }
-    LT_HIP(spin_stream(s_compute));  // the last fix-up wrote h_meta
+    LT_TRY(wait_meta());
     const PoolCtl *c = (const PoolCtl *)(h_meta + P);
     if (c->overflow) {
         set_error("walker queue pool overflow (flags 0x%x, top %u)", c->overflow, c->top);
@@ -823,8 +859,31 @@ lt_status Engine::set_table(uint32_t p, bool present) {
         cp = c;
         wp = slot_words(p, cp);
     }
-    set_table_kernel<<<1, 64, 0, s_compute>>>(d_rowptr_tab, d_col_tab, d_words_tab, p, rp, cp, wp);
+    return table_entry(p, rp, cp, wp, false);
+}
+
+// Queue a table update for the next walk launch (flush_tables).
+lt_status Engine::table_entry(uint32_t p, const uint64_t *rp, const uint32_t *cp, const uint32_t *wp, bool zc) {
+    uint32_t k = 0;
+    while (k < table_due.n && table_due.part[k] != p) k++;  // the last update of a partition counts
+    if (k == kTableBatch) {
+        LT_TRY(flush_tables());
+        k = 0;
+    }
+    if (k == table_due.n) table_due.n++;
+    table_due.part[k] = p;
+    table_due.rowptr[k] = rp;
+    table_due.col[k] = cp;
+    table_due.words[k] = wp;
+    table_due.zc[k] = zc ? 1 : 0;
+    return LT_OK;
+}
+
+lt_status Engine::flush_tables() {
+    if (table_due.n == 0) return LT_OK;
+    set_tables_kernel<<<1, 64, 0, s_compute>>>(tables(), table_due);
     LT_HIP(hipGetLastError());
+    table_due.n = 0;
     return LT_OK;
 }
 
@@ -970,6 +1029,7 @@ static void launch_walk_app(const WalkArgs &a, int wpt, int grid, size_t lds, hi
 }
 
 lt_status Engine::launch_walk(const WalkArgs &a, uint64_t walkers, hipStream_t s) {
+    LT_TRY(flush_tables());
     const uint64_t fill = (uint64_t)num_cu * 4 * 6 * 64;  // threads for ~6 waves per SIMD
     const int wpt = cfg.walkers_per_thread > 0 ? cfg.walkers_per_thread
                     : walkers >= 4 * fill         ? 4
@@ -1038,10 +1098,13 @@ lt_status Engine::process(uint32_t p, bool zerocopy, uint64_t walkers) {
         LT_TRY(launch_walk(a, sw, s_compute));
         kt.end(tk, s_compute);
         st.zerocopy_launches += zerocopy ? 1 : 0;
-        fixup_kernel<<<1, kBlock, 0, s_compute>>>(q, p, (uint32_t)lo, last ? 0xFFFFFFFFu : (uint32_t)hi, last ? 1 : 0,
-                                                  nullptr);
-        LT_HIP(hipGetLastError());
-        meta_dirty = false;
+        Consumed d{};
+        d.n = 1;
+        d.src[0] = p;
+        d.chunk_lo = (uint32_t)lo;
+        d.chunk_hi = a.chunk_hi;
+        d.last = last ? 1 : 0;
+        LT_TRY(launch_fixup(d));
         st.kernel_launches++;
     }
     if (host) LT_TRY(process_host(p, a));
@@ -1147,11 +1210,13 @@ lt_status Engine::spill_round(const std::vector<uint32_t> &victims) {
     const int grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((prefix[nv] + 255) / 256, (uint64_t)num_cu * 8));
     spill_gather_kernel<<<grid, 256, 0, s_compute>>>(sa);
     LT_HIP(hipGetLastError());
+    sa.q.seq = ++meta_seq;
     release_queues_kernel<<<1, kBlock, 0, s_compute>>>(sa);
     LT_HIP(hipGetLastError());
     meta_dirty = false;
+    meta_seen = false;
     t_wevict.end(te, s_compute);
-    LT_HIP(spin_stream(s_compute));  // the plan and host chunks are final before they are reused
+    LT_TRY(wait_meta());  // the plan and host chunks are final before they are reused
     for (uint32_t k = 0; k < nv; k++) {
         hcount[victims[k]] += dcounts[victims[k]];
         dcounts[victims[k]] = 0;
@@ -1220,11 +1285,9 @@ lt_status Engine::process_host(uint32_t p, const WalkArgs &a) {
         hipEvent_t tk = t_kernel.begin(s_compute);
         LT_TRY(launch_walk(b, total, s_compute));
         t_kernel.end(tk, s_compute);
-        fixup_kernel<<<1, kBlock, 0, s_compute>>>(q, kEmpty, 0, 0, 0, nullptr);
-        LT_HIP(hipGetLastError());
-        meta_dirty = false;
+        LT_TRY(launch_fixup(Consumed{}));
         t_wload.end(tl, s_compute);
-        LT_HIP(spin_stream(s_compute));  // the pieces go back to the free list below
+        LT_TRY(wait_meta());  // the pieces go back to the free list below
         hhead[p] += total;
         hcount[p] -= total;
         while (!hq[p].empty() && (hhead[p] >= kChunk || hcount[p] == 0)) {
@@ -1326,39 +1389,30 @@ lt_status Engine::walk_batch(const std::vector<uint32_t> &parts, bool zerocopy) 
     a.span_resident = 1;
     a.stats = d_stats;
     a.ss = sched_state(false);
-    ZcBatch b{};
-    b.n = (uint32_t)parts.size();
-    a.nsrc = b.n;
+    Consumed d{};
+    d.n = a.nsrc = (uint32_t)parts.size();
+    d.chunk_hi = 0xFFFFFFFFu;
+    d.last = 1;
+    d.leave = zerocopy ? 1 : 0;
     a.src = parts[0];
     a.voff[0] = 0;
     uint64_t total = 0;
-    for (uint32_t k = 0; k < b.n; k++) {
+    for (uint32_t k = 0; k < d.n; k++) {
         const uint32_t p = parts[k];
-        b.part[k] = p;
-        b.rowptr[k] = zc_rowptr + part.node_off[p];
-        b.col[k] = zc_col + part.edge_off[p];
-        a.srcs[k] = p;
+        d.src[k] = a.srcs[k] = p;
+        if (zerocopy)
+            LT_TRY(table_entry(p, zc_rowptr + part.node_off[p], zc_col + part.edge_off[p], nullptr, true));
         a.voff[k + 1] = a.voff[k] + (counts[p] + kChunk - 1) / kChunk * kChunk;
         total += counts[p];
     }
     EventTimer &phase = zerocopy ? t_zc : t_compute;
     EventTimer &kt = zerocopy ? t_kzc : t_kernel;
     hipEvent_t tp = phase.begin(s_compute);
-    if (zerocopy) {
-        set_zc_tables_kernel<<<1, 64, 0, s_compute>>>(d_rowptr_tab, d_col_tab, d_zc_part, b, 1);
-        LT_HIP(hipGetLastError());
-    }
     hipEvent_t tk = kt.begin(s_compute);
     LT_TRY(launch_walk(a, total, s_compute));
     kt.end(tk, s_compute);
     st.zerocopy_launches += zerocopy ? 1 : 0;
-    for (uint32_t p : parts) fixup_kernel<<<1, kBlock, 0, s_compute>>>(q, p, 0, 0xFFFFFFFFu, 1, nullptr);
-    LT_HIP(hipGetLastError());
-    meta_dirty = false;
-    if (zerocopy) {
-        set_zc_tables_kernel<<<1, 64, 0, s_compute>>>(d_rowptr_tab, d_col_tab, d_zc_part, b, 0);
-        LT_HIP(hipGetLastError());
-    }
+    LT_TRY(launch_fixup(d));
     st.kernel_launches++;
     phase.end(tp, s_compute);
     return LT_OK;
@@ -1509,7 +1563,7 @@ lt_status Engine::run_partition(uint32_t p, int32_t &prev_loaded) {
                 st.computing_calls++;
                 record((uint32_t)c, 2, -1, -1);
                 LT_TRY(process_resident((uint32_t)c, 2, nullptr));
-                LT_HIP(hipStreamSynchronize(s_compute));
+                LT_TRY(wait_meta());
             }
             // the pipelined work changed the queues; p's count is re-read below
             LT_TRY(read_meta());
@@ -1543,7 +1597,6 @@ lt_status Engine::scheduler_loop() {
         prev = c;
         LT_TRY(run_partition((uint32_t)c, prev_loaded));
     }
-    LT_HIP(hipDeviceSynchronize());
     return LT_OK;
 }
 
@@ -1602,7 +1655,7 @@ lt_status Engine::scheduler_loop_learned() {
             st.computing_calls++;
             record((uint32_t)p2, 2, -1, -1);
             LT_TRY(process_resident((uint32_t)p2, 2, prefetched.data()));
-            LT_HIP(hipStreamSynchronize(s_compute));
+            LT_TRY(wait_meta());
         }
         return read_meta();
     };
@@ -1710,19 +1763,13 @@ lt_status Engine::scheduler_loop_learned() {
             // decision's, computed while its walk ran): no inference here on
             // the critical path unless they are far out of date
             if (!scores_recent() && !plain_victims) LT_TRY(infer_scores(c));
-            bool evicted_any = false;
+            // copies into the freed slots may start at once: no walk is running, and
+            // the next one is launched behind the table updates
             while ((scores_valid || plain_victims) && free_slots.size() < want) {
                 const int32_t v = learned_victim(c, -1);
                 if (v < 0) break;
                 LT_TRY(evict((uint32_t)v));
                 prefetched[v] = 0;
-                evicted_any = true;
-            }
-            if (evicted_any) {  // copies into the freed slots start after the table updates
-                if (!ev_evicted) LT_HIP(hipEventCreateWithFlags(&ev_evicted, hipEventDisableTiming));
-                LT_HIP(hipEventRecord(ev_evicted, s_compute));
-                LT_HIP(hipStreamWaitEvent(s_copy, ev_evicted, 0));
-                if (s_dma != s_copy) LT_HIP(hipStreamWaitEvent(s_dma, ev_evicted, 0));
             }
         }
         st.computing_calls++;
@@ -1760,9 +1807,7 @@ lt_status Engine::scheduler_loop_learned() {
         }
     }
     LT_TRY(retire(inflight.empty() ? -1 : inflight.back().part));
-    LT_TRY(infer_collect());
-    LT_HIP(hipDeviceSynchronize());
-    return LT_OK;
+    return infer_collect();
 }
 
 SchedState Engine::sched_state(bool device) const {
@@ -1846,7 +1891,7 @@ lt_status Engine::scheduler_loop_device() {
                 launch_walk_app<APP_GENERIC>(a, dwpt, walk_grid[APP_GENERIC][dwpt], lds_bytes(dwpt), s_compute);
                 break;
         }
-        fixup_kernel<<<1, kBlock, 0, s_compute>>>(q, kEmpty, 0, 0, 0, d_ds);
+        fixup_kernel<<<1, kBlock, 0, s_compute>>>(q, Consumed{}, tables(), d_ds);
     }
     hipError_t ce = hipStreamEndCapture(s_compute, &graph);
     if (ce != hipSuccess) {
@@ -1861,10 +1906,10 @@ lt_status Engine::scheduler_loop_device() {
     uint64_t launches = 0;
     while (true) {
         LT_HIP(hipGraphLaunch(exec, s_compute));
-        meta_dirty = false;  // each iteration ends with a fix-up
         launches++;
         LT_HIP(hipMemcpyAsync(&h, d_ds, sizeof(h), hipMemcpyDeviceToHost, s_compute));
         LT_HIP(hipStreamSynchronize(s_compute));
+        meta_dirty = true;
         if (h.choice < 0) break;
         if (vregion) LT_TRY(read_meta());  // counts the visit log if it fills up
         if (launches > (1ull << 24)) {
@@ -1952,7 +1997,7 @@ lt_status Engine::run_flat(const RunSpec &rs) {
         if (a.app.vlog) LT_TRY(count_log((uint32_t)((a.id_hi - lo) * each), 0));
     }
     t_compute.end(tp, s_compute);
-    LT_HIP(spin_stream(s_compute));
+    LT_HIP(hipStreamSynchronize(s_compute));
     w_run = rs.total;
     st.iterations = st.explicit_iterations = st.computing_calls = 1;
     st.resident_batched = P - 1;
@@ -2042,7 +2087,6 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
 
     double running_ms = 0;
     if (walk_flat) {
-        LT_HIP(hipStreamSynchronize(s_compute));
         const auto t0 = std::chrono::steady_clock::now();
         LT_TRY(run_flat(rs));
         running_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -2079,12 +2123,10 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
                 default: init_kernel<APP_GENERIC><<<grid, kBlock, lds_bytes(), s_compute>>>(ia); break;
             }
             LT_HIP(hipGetLastError());
-            fixup_kernel<<<1, kBlock, 0, s_compute>>>(q, kEmpty, 0, 0, 0, nullptr);
-            LT_HIP(hipGetLastError());
-            meta_dirty = false;
+            LT_TRY(launch_fixup(Consumed{}));
             lo += n;
         }
-        LT_HIP(hipStreamSynchronize(s_compute));
+        LT_TRY(wait_meta());
         const auto t0 = std::chrono::steady_clock::now();
         w_run = id1 - id0;
         if (cfg.device_schedule) LT_TRY(scheduler_loop_device());

@@ -798,60 +798,68 @@ __global__ __launch_bounds__(kBlock) void init_kernel(InitArgs a) {
     }
 }
 
-// Copy the queue lengths and PoolCtl into q.packed for the host's one D2H.
-// Collective over one workgroup; runs after every queue update of the stream.
+// Copy the queue lengths and PoolCtl into q.packed for the host, which polls
+// the sequence number behind them (Engine::wait_meta).  Collective over one
+// workgroup; runs after every queue update of the stream.  The words are
+// written through to the host, and every wave waits for its own before the
+// barrier, so the number is written last.
+__device__ __forceinline__ void to_host(uint32_t *p, uint32_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __device__ void pack_meta(const Queues &q) {
-    for (uint32_t i = threadIdx.x; i < q.P; i += blockDim.x) q.packed[i] = qlen_of(q, i);
-    if (threadIdx.x == 0) {
-        const PoolCtl c = *q.ctl;
-        q.packed[q.P] = c.top;
-        q.packed[q.P + 1] = c.popped;
-        q.packed[q.P + 2] = c.nlost;
-        q.packed[q.P + 3] = c.overflow;
-    }
+    for (uint32_t i = threadIdx.x; i < q.P; i += blockDim.x) to_host(&q.packed[i], qlen_of(q, i));
+    if (threadIdx.x < sizeof(PoolCtl) / 4) to_host(&q.packed[q.P + threadIdx.x], ((const uint32_t *)q.ctl)[threadIdx.x]);
     if (q.vcur && threadIdx.x < kLogRegions)
-        q.packed[q.P + 4 + threadIdx.x] = (uint32_t)min(q.vcur[threadIdx.x * kCurStride], 0xFFFFFFFFull);
+        to_host(&q.packed[q.P + 4 + threadIdx.x], (uint32_t)min(q.vcur[threadIdx.x * kCurStride], 0xFFFFFFFFull));
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x == 0)
+        __hip_atomic_store(&q.packed[q.P + 4 + kLogRegions], q.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __global__ __launch_bounds__(kBlock) void pack_meta_kernel(Queues q) { pack_meta(q); }
 
 // Return the popped-but-unused state of the pool, the lost chunks and the
-// consumed source chunks [chunk_lo, chunk_hi) to the free stack; clear the
-// source queue after its last slice; pack the queue lengths.  One workgroup.
-__global__ __launch_bounds__(kBlock) void fixup_kernel(Queues q, uint32_t src, uint32_t chunk_lo, uint32_t chunk_hi,
-                                                       int last, const DevSched *ds) {
-    __shared__ uint32_t s_top, s_nlost, s_cnt;
-    if (ds) {  // device-scheduled iteration: the whole queue of the choice was consumed
-        src = ds->choice < 0 ? kEmpty : (uint32_t)ds->choice;
-        chunk_lo = 0;
-        chunk_hi = 0xFFFFFFFFu;
-        last = 1;
+// consumed source chunks to the free stack; clear the source queues after their
+// last slice; take a zero-copy batch out of the partition table; pack the queue
+// lengths.  One workgroup.  A batch's sources share one launch: sixteen
+// launches of 4.4 us each followed a walk of sixteen queues before.
+__global__ __launch_bounds__(kBlock) void fixup_kernel(Queues q, Consumed d, Tables tab, const DevSched *ds) {
+    __shared__ uint32_t s_top, s_nlost, s_off[kMaxZcBatch + 1];
+    // a device-scheduled iteration consumed the whole queue of its choice
+    const int32_t choice = ds ? ds->choice : -1;
+    const uint32_t n = ds ? (choice < 0 ? 0u : 1u) : d.n;
+    const uint32_t lo = ds ? 0u : d.chunk_lo, most = ds ? 0xFFFFFFFFu : d.chunk_hi;
+    const auto src = [&](uint32_t k) { return ds ? (uint32_t)choice : d.src[k]; };
+    if (threadIdx.x < n) {
+        const uint32_t nch = (qlen_of(q, src(threadIdx.x)) + kChunk - 1) >> kChunkLog2;
+        const uint32_t hi = min(most, nch);
+        s_off[threadIdx.x + 1] = hi > lo ? hi - lo : 0;
     }
+    __syncthreads();
     if (threadIdx.x == 0) {
         PoolCtl c = *q.ctl;
         uint32_t popped = c.popped;
         if (popped > c.top) popped = c.top;
         uint32_t nlost = c.nlost < kLostCap ? c.nlost : kLostCap;
-        uint32_t cnt = 0;
-        if (src != kEmpty) {
-            const uint32_t nch = (qlen_of(q, src) + kChunk - 1) >> kChunkLog2;
-            const uint32_t hi = min(chunk_hi, nch);
-            cnt = hi > chunk_lo ? hi - chunk_lo : 0;
-        }
+        s_off[0] = 0;
+        for (uint32_t k = 0; k < n; k++) s_off[k + 1] += s_off[k];
         s_top = c.top - popped;
         s_nlost = nlost;
-        s_cnt = cnt;
-        if (s_top + nlost + cnt > q.nchunks) {
+        if (s_top + nlost + s_off[n] > q.nchunks) {
             q.ctl->overflow |= 16u;
             s_nlost = 0;
-            s_cnt = 0;
+            for (uint32_t k = 0; k <= n; k++) s_off[k] = 0;
         }
     }
     __syncthreads();
-    const uint32_t top = s_top, nlost = s_nlost, cnt = s_cnt;
+    const uint32_t top = s_top, nlost = s_nlost, cnt = s_off[n];
     for (uint32_t i = threadIdx.x; i < nlost; i += kBlock) q.free_stack[top + i] = q.lost[i];
+    uint32_t k = 0;
     for (uint32_t j = threadIdx.x; j < cnt; j += kBlock) {
-        uint32_t *f = &q.frame[(size_t)src * q.maxc + chunk_lo + j];
+        while (j >= s_off[k + 1]) k++;
+        uint32_t *f = &q.frame[(size_t)src(k) * q.maxc + lo + (j - s_off[k])];
         q.free_stack[top + nlost + j] = *f;
         *f = kEmpty;
     }
@@ -860,8 +868,17 @@ __global__ __launch_bounds__(kBlock) void fixup_kernel(Queues q, uint32_t src, u
         q.ctl->top = top + nlost + cnt;
         q.ctl->popped = 0;
         q.ctl->nlost = 0;
-        if (last && src != kEmpty) qlen_of(q, src) = 0;
     }
+    if (threadIdx.x < n) {
+        const uint32_t p = src(threadIdx.x);
+        if (ds || d.last) qlen_of(q, p) = 0;
+        if (!ds && d.leave) {
+            tab.rowptr[p] = nullptr;
+            tab.col[p] = nullptr;
+            tab.zc[p] = 0;
+        }
+    }
+    if (ds) return;  // no host waits for an iteration of the device loop
     __syncthreads();
     pack_meta(q);
 }
@@ -935,24 +952,15 @@ __global__ void reset_queues_kernel(Queues q, uint32_t P) {
     }
 }
 
-// Enter (on = 1) or remove a zero-copy batch's partitions in the partition table.
-__global__ void set_zc_tables_kernel(const uint64_t **rowptr_tab, const uint32_t **col_tab, uint8_t *zc_part,
-                                     ZcBatch b, int on) {
+// Partition table updates, all those due before a walk in one launch.
+__global__ void set_tables_kernel(Tables tab, TableBatch b) {
     const uint32_t k = threadIdx.x;
-    if (blockIdx.x == 0 && k < b.n) {
+    if (k < b.n) {
         const uint32_t p = b.part[k];
-        rowptr_tab[p] = on ? b.rowptr[k] : nullptr;
-        col_tab[p] = on ? b.col[k] : nullptr;
-        zc_part[p] = on ? 1 : 0;
-    }
-}
-
-__global__ void set_table_kernel(const uint64_t **rowptr_tab, const uint32_t **col_tab, const uint32_t **words_tab,
-                                 uint32_t p, const uint64_t *rp, const uint32_t *cp, const uint32_t *wp) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        rowptr_tab[p] = rp;
-        col_tab[p] = cp;
-        words_tab[p] = wp;
+        tab.rowptr[p] = b.rowptr[k];
+        tab.col[p] = b.col[k];
+        tab.words[p] = b.words[k];
+        tab.zc[p] = b.zc[k];
     }
 }
 
