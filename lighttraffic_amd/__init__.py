@@ -369,34 +369,35 @@ class Engine:
         self.partition = partition
         self.config = cfg
 
+    # Result arrays are not cleared first: a run that succeeds writes every word.
     def pagerank(self, w, l=10, runs=1, endpoints=False):
-        counts = np.zeros(self.graph.num_node, np.uint32)
-        ep = np.zeros(w * runs, np.uint32) if endpoints else None
+        counts = np.empty(self.graph.num_node, np.uint32)
+        ep = np.empty(w * runs, np.uint32) if endpoints else None
         _check(_lib.lt_run_pagerank(self._h, w, l, runs, counts.ctypes.data, _ptr(ep)), "lt_run_pagerank")
         return (counts, ep) if endpoints else counts
 
     def ppr(self, w, source=0, prob=0.15, endpoints=False):
-        counts = np.zeros(self.graph.num_node, np.uint32)
-        ep = np.zeros(w, np.uint32) if endpoints else None
+        counts = np.empty(self.graph.num_node, np.uint32)
+        ep = np.empty(w, np.uint32) if endpoints else None
         _check(_lib.lt_run_ppr(self._h, w, source, prob, counts.ctypes.data, _ptr(ep)), "lt_run_ppr")
         return (counts, ep) if endpoints else counts
 
     def genericwalk(self, w, l=10, runs=1, endpoints=True, moves=False):
-        ep = np.zeros(w * runs, np.uint32) if endpoints else None
-        mv = np.zeros(w * runs, np.uint32) if moves else None
+        ep = np.empty(w * runs, np.uint32) if endpoints else None
+        mv = np.empty(w * runs, np.uint32) if moves else None
         _check(_lib.lt_run_genericwalk(self._h, w, l, runs, _ptr(ep), _ptr(mv)), "lt_run_genericwalk")
         return ep, mv
 
     def genericwalk_paths(self, w, l=10, runs=1):
         """u32[w * runs, l + 1]: column k is the vertex after k moves, 0xFFFFFFFF after an early stop."""
-        paths = np.zeros((w * runs, l + 1), np.uint32)
+        paths = np.empty((w * runs, l + 1), np.uint32)
         _check(_lib.lt_run_genericwalk_paths(self._h, w, l, runs, paths.ctypes.data), "lt_run_genericwalk_paths")
         return paths
 
     def ppr_batch(self, sources, counts, prob=0.15, endpoints=True):
         sources = np.ascontiguousarray(sources, dtype=np.uint32)
         counts = np.ascontiguousarray(counts, dtype=np.uint64)
-        ep = np.zeros(int(counts.sum()), np.uint32) if endpoints else None
+        ep = np.empty(int(counts.sum()), np.uint32) if endpoints else None
         _check(_lib.lt_run_ppr_batch(self._h, len(sources), sources.ctypes.data, counts.ctypes.data, prob,
                                      _ptr(ep)), "lt_run_ppr_batch")
         return ep

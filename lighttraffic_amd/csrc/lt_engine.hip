@@ -21,6 +21,7 @@
 #include "lt_kernels.h"
 #include "lt_flat.h"
 #include "lt_mlp.h"
+#include "lt_results.h"
 #include "lt_sched.h"
 
 #define LT_HIP(call)                                                                                   \
@@ -122,6 +123,12 @@ static hipError_t spin_event(hipEvent_t ev) {
     }
     return e;
 }
+
+// h_out: kNumStats u64 of event counters, the job's time in ticks of the
+// device's wall clock, the sequence number, those of the ring's buffers, then small
+// results.
+constexpr uint32_t kOutTicks = 2 * kNumStats, kOutFlag = kOutTicks + 1, kOutRing = kOutFlag + 1, kOutData = 64;
+constexpr uint64_t kManyOut = 1u << 20;  // words: from here on threads help with the results
 
 struct RunSpec {
     int app = APP_PAGERANK;
@@ -245,6 +252,23 @@ struct Engine {
     uint32_t *d_qsrc = nullptr;
     size_t q_cap = 0;
     unsigned long long *d_stats = nullptr;
+    // Results on their way to the caller (lt_results.h).
+    static constexpr uint32_t kRing = 4;
+    static constexpr size_t kRingBytes = 2u << 20;
+    uint32_t *h_out = nullptr, *d_out = nullptr;  // pinned: event counters, sequence number, small results
+    uint32_t out_seq = 0;
+    int wall_khz = 100000;                        // rate of the device's wall clock
+    uint8_t *h_ring = nullptr, *d_ring = nullptr; // pinned: kRing buffers
+    uint32_t ring_seq[kRing] = {};                // of each buffer's last fill
+    std::vector<OutSeg> outs;                     // results of the running job
+    uint8_t *h_query = nullptr;                   // pinned staging of the query table
+    size_t query_cap = 0;
+    lt_status poll_host(const uint32_t *flag, uint32_t seq, const char *what);
+    lt_status finish_job(bool small);
+    lt_status ensure_ring();
+    lt_status mark_ring(uint32_t slot);
+    lt_status wait_ring(uint32_t slot);
+    lt_status copy_results(ResultHelpers &help);
 
     lt_stats st{};
     std::vector<lt_trace_rec> trace;
@@ -336,7 +360,8 @@ struct Engine {
     lt_status set_table(uint32_t p, bool present);
     lt_status table_entry(uint32_t p, const uint64_t *rp, const uint32_t *cp, const uint32_t *wp, bool zc);
     bool can_run_flat() const;
-    lt_status run_flat(const RunSpec &rs);
+    lt_status run_flat(const RunSpec &rs, ResultHelpers &help);
+    bool job_finished = false;  // run_flat has handed the job's results out
     lt_status scheduler_loop();
     lt_status scheduler_loop_learned();
     lt_status scheduler_loop_device();
@@ -397,6 +422,9 @@ Engine::~Engine() {
     dfree(d_qoff);
     dfree(d_qsrc);
     dfree(d_stats);
+    if (h_out) (void)hipHostFree(h_out);
+    if (h_ring) (void)hipHostFree(h_ring);
+    if (h_query) (void)hipHostFree(h_query);
     dfree(d_ds);
     dfree(d_slot_of);
     dfree(d_part_in_slot);
@@ -629,7 +657,12 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
     res_batch = std::min(res_batch, kMaxZcBatch);
     if (cfg.span != LT_SPAN_RESIDENT) res_batch = 1;
     slice = cfg.slice_chunks > 0 ? (uint32_t)cfg.slice_chunks : kSliceChunks;
-    LT_TRY(dmalloc(&d_stats, (size_t)kNumStats * kStatSlots));
+    LT_TRY(dmalloc(&d_stats, (size_t)kNumStats * kStatSlots + 1));
+    LT_HIP(hipHostMalloc((void **)&h_out, 4 * (kOutData + kSmallOut), hipHostMallocMapped | hipHostMallocCoherent));
+    memset(h_out, 0, 4 * kOutData);
+    LT_HIP(hipHostGetDevicePointer((void **)&d_out, h_out, 0));
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0) wall_khz = khz;
     counts.assign(P, 0);
     dcounts.assign(P, 0);
     hq.assign(P, {});
@@ -802,19 +835,23 @@ lt_status Engine::launch_fixup(const Consumed &d) {
 // written is found by the query made once in a while.
 lt_status Engine::wait_meta() {
     if (meta_seen) return LT_OK;
-    const uint32_t *flag = h_meta + P + 4 + kLogRegions;
-    for (uint32_t it = 1; __atomic_load_n(flag, __ATOMIC_ACQUIRE) != meta_seq; it++) {
+    LT_TRY(poll_host(h_meta + P + 4 + kLogRegions, meta_seq, "queue lengths"));
+    meta_seen = true;
+    return LT_OK;
+}
+
+lt_status Engine::poll_host(const uint32_t *flag, uint32_t seq, const char *what) {
+    for (uint32_t it = 1; __atomic_load_n(flag, __ATOMIC_ACQUIRE) != seq; it++) {
         __builtin_ia32_pause();
         if ((it & 0xFFFFF) == 0) {
             const hipError_t e = hipStreamQuery(s_compute);
             if (e == hipErrorNotReady) continue;
             LT_HIP(e);
-            if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == meta_seq) break;
-            set_error("queue lengths were not written");
+            if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == seq) break;
+            set_error("%s were not written", what);
             return LT_E_INTERNAL;
         }
     }
-    meta_seen = true;
     return LT_OK;
 }
 
@@ -1968,7 +2005,7 @@ constexpr uint64_t kFlatPiece = (uint64_t)kSliceChunks * kChunk;
 // The whole job over the flat arrays: walkers are created, walked and finished
 // in registers, so the queues are not touched.  Row offsets are read as 32
 // bits, which halves the lines that the hot rows take in L2.
-lt_status Engine::run_flat(const RunSpec &rs) {
+lt_status Engine::run_flat(const RunSpec &rs, ResultHelpers &help) {
     if (!d_rowptr32) {  // kept: slots of a flat cache are never evicted
         LT_TRY(dmalloc(&d_rowptr32, (size_t)V + 1));
         narrow_rowptr_kernel<<<std::min<int>(8 * num_cu, (int)(V / 256 + 1)), 256, 0, s_compute>>>(
@@ -1980,28 +2017,123 @@ lt_status Engine::run_flat(const RunSpec &rs) {
     a.rowptr = d_rowptr32;
     a.col = flat_col;
     a.stats = d_stats;
-    hipEvent_t tp = t_compute.begin(s_compute);
     // a launch's visits have to fit the log; walks too long for that count directly
     uint64_t piece = kFlatPiece;
     const uint64_t each = app_kind == APP_PAGERANK ? rs.length : 1, room = (uint64_t)vregion * kLogRegions;
     if (a.app.vlog && room / each < std::min<uint64_t>(rs.total, 1u << 16)) a.app.vlog = nullptr;
     if (a.app.vlog) piece = std::min(piece, room / each);
-    for (uint64_t lo = 0; lo < rs.total; lo += piece) {
-        a.id_lo = lo;
-        a.id_hi = std::min<uint64_t>(rs.total, lo + piece);
+    // Endpoints and moves of fixed-length walks are written by whole waves:
+    // straight into the ring, a launch per buffer, so that they reach the host while
+    // the next walkers walk.  (PPR lanes end one by one, and paths are written
+    // a word per row: those results stay on the device until the end.)
+    const uint32_t nout = (uint32_t)outs.size();
+    const bool ring = app_kind == APP_GENERIC && !a.app.paths && nout && nout * rs.total >= kManyOut;
+    constexpr uint32_t kTwo = kRing / 2;  // a launch takes two buffers: its last walkers leave
+                                          // the card half idle for some 10 us
+    if (ring) {
+        LT_TRY(ensure_ring());
+        piece = 2 * kRingBytes / 4 / nout;
+    }
+    const auto drain = [&](uint64_t k) -> lt_status {  // launch k's results to the caller
+        LT_TRY(wait_ring(k % kTwo));
+        const uint64_t n = std::min<uint64_t>(piece, rs.total - k * piece);
+        for (uint32_t o = 0; o < nout; o++)
+            help.copiers().copy(outs[o].dst + k * piece, h_ring + k % kTwo * 2 * kRingBytes + 4 * o * piece, 4 * n);
+        return LT_OK;
+    };
+    hipEvent_t tp = t_compute.begin(s_compute);
+    uint64_t k = 0, drained = 0;
+    for (; k * piece < rs.total; k++) {
+        a.id_lo = k * piece;
+        a.id_hi = std::min<uint64_t>(rs.total, a.id_lo + piece);
+        if (ring) {
+            for (; drained + kTwo <= k; drained++) LT_TRY(drain(drained));
+            uint32_t *at = (uint32_t *)(d_ring + k % kTwo * 2 * kRingBytes) - a.id_lo;
+            if (app.endpoints) a.app.endpoints = at;
+            if (app.moves_out) a.app.moves_out = at + (app.endpoints ? piece : 0);
+        }
         hipEvent_t tk = t_kernel.begin(s_compute);
         launch_flat(a, app_kind, num_cu, s_compute);
         LT_HIP(hipGetLastError());
         t_kernel.end(tk, s_compute);
         st.kernel_launches++;
-        if (a.app.vlog) LT_TRY(count_log((uint32_t)((a.id_hi - lo) * each), 0));
+        if (ring) LT_TRY(mark_ring(k % kTwo));
+        if (a.app.vlog) LT_TRY(count_log((uint32_t)((a.id_hi - a.id_lo) * each), 0));
+        if (k == 0) help.start(outs);
     }
     t_compute.end(tp, s_compute);
-    LT_HIP(hipStreamSynchronize(s_compute));
     w_run = rs.total;
     st.iterations = st.explicit_iterations = st.computing_calls = 1;
     st.resident_batched = P - 1;
     for (uint32_t p = 0; p < P; p++) last_use[p] = ++use_clock;
+    job_finished = ring;
+    if (ring) {
+        LT_TRY(finish_job(false));
+        for (; drained < k; drained++) LT_TRY(drain(drained));
+        LT_TRY(poll_host(h_out + kOutFlag, out_seq, "results"));
+    }
+    return LT_OK;
+}
+
+// Last kernels of a job: its small results and event counters into pinned
+// memory; waits for them, and so for the job's walks.
+lt_status Engine::finish_job(bool small) {
+    if (small && !outs.empty()) {
+        SmallOut o{};
+        o.n = (uint32_t)outs.size();
+        o.dst = d_out + kOutData;
+        for (uint32_t k = 0; k < o.n; k++) {
+            o.src[k] = outs[k].src;
+            o.end[k] = (k ? o.end[k - 1] : 0) + (uint32_t)outs[k].words;
+        }
+        small_out_kernel<<<(o.end[o.n - 1] + 255) / 256, 256, 0, s_compute>>>(o);
+    }
+    finish_kernel<<<1, kStatSlots, 0, s_compute>>>(d_stats, d_out, d_out + kOutFlag, ++out_seq);
+    LT_HIP(hipGetLastError());
+    if (!small) return LT_OK;  // copy_results first
+    LT_TRY(poll_host(h_out + kOutFlag, out_seq, "results"));
+    const uint32_t *from = h_out + kOutData;
+    for (const OutSeg &o : outs) {
+        memcpy(o.dst, from, 4 * o.words);
+        from += o.words;
+    }
+    return LT_OK;
+}
+
+lt_status Engine::ensure_ring() {
+    if (h_ring) return LT_OK;
+    LT_HIP(hipHostMalloc((void **)&h_ring, kRing * kRingBytes, hipHostMallocMapped | hipHostMallocCoherent));
+    LT_HIP(hipHostGetDevicePointer((void **)&d_ring, h_ring, 0));
+    return LT_OK;
+}
+
+// The ring buffer is full once the stream gets here.
+lt_status Engine::mark_ring(uint32_t slot) {
+    mark_kernel<<<1, 1, 0, s_compute>>>(d_out + kOutRing + slot, ++ring_seq[slot]);
+    LT_HIP(hipGetLastError());
+    return LT_OK;
+}
+
+lt_status Engine::wait_ring(uint32_t slot) { return poll_host(h_out + kOutRing + slot, ring_seq[slot], "results"); }
+
+// The results in pieces of a ring buffer's size: kernels fill the next buffers
+// while the team copies the oldest one out.
+lt_status Engine::copy_results(ResultHelpers &help) {
+    LT_TRY(ensure_ring());
+    std::vector<OutSeg> pieces;
+    for (const OutSeg &o : outs)
+        for (uint64_t at = 0; at < o.words; at += kRingBytes / 4)
+            pieces.push_back({o.dst + at, o.src + at, std::min<uint64_t>(kRingBytes / 4, o.words - at)});
+    for (size_t issued = 0, out = 0; out < pieces.size(); out++) {
+        for (; issued < pieces.size() && issued < out + kRing; issued++) {
+            const uint32_t slot = issued % kRing;
+            fill_ring_kernel<<<64, 256, 0, s_compute>>>(pieces[issued].src, (uint32_t *)(d_ring + slot * kRingBytes),
+                                                        pieces[issued].words);
+            LT_TRY(mark_ring(slot));
+        }
+        LT_TRY(wait_ring(out % kRing));
+        help.copiers().copy(pieces[out].dst, h_ring + out % kRing * kRingBytes, 4 * pieces[out].words);
+    }
     return LT_OK;
 }
 
@@ -2037,12 +2169,12 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
     const bool walk_flat = can_run_flat();
     if (counting) LT_TRY(ensure_log(visits, !walk_flat));
     else vregion = 0;
-    // Without a log, copies of the counters, one per XCD: through the queues
-    // where the walkers of one launch stay in a few partitions (capped cache,
-    // PPR around its sources; one array measured 29 % slower there); for a flat
-    // job where clearing and adding up the copies of a small graph costs less than
-    // its hot vertices' atomics (5 G/s in one array, 27 G/s in copies).
-    const bool copies = walk_flat ? visits >= (1u << 16) && V <= (1u << 20) : nslots < P || rs.app == APP_PPR;
+    // Without a log, copies of the counters, one per XCD: where the walkers of
+    // one launch stay in a few partitions (capped cache, PPR around its sources; one
+    // array measured 29 % slower there), and where clearing and adding up the
+    // copies of a small graph costs less than its hot vertices' atomics (5 G/s in
+    // one array, 27 G/s in copies).
+    const bool copies = (!walk_flat && (nslots < P || rs.app == APP_PPR)) || (visits >= (1u << 16) && V <= (1u << 20));
     count_copies = counting && !vregion && copies ? kCountCopies : 1;
     LT_TRY(ensure_pool(std::max<uint64_t>(cap, 1), walk_flat));  // a flat job keeps the queues' limits
     LT_TRY(ensure_outputs(rs, endpoints_out != nullptr, moves_out != nullptr));
@@ -2070,27 +2202,47 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
         return LT_E_ARG;
     }
     if (rs.nq) {
-        std::vector<uint64_t> off(rs.nq + 1, 0);
+        const size_t need = 12 * (size_t)rs.nq + 8;
+        if (query_cap < need) {
+            if (h_query) (void)hipHostFree(h_query);
+            h_query = nullptr;
+            query_cap = 0;
+            LT_HIP(hipHostMalloc((void **)&h_query, need, hipHostMallocDefault));
+            query_cap = need;
+        }
+        uint64_t *off = (uint64_t *)h_query;
+        off[0] = 0;
         for (uint32_t i = 0; i < rs.nq; i++) off[i + 1] = off[i] + rs.q_cnt[i];
-        LT_HIP(hipMemcpy(d_qoff, off.data(), 8 * (rs.nq + 1), hipMemcpyHostToDevice));
-        LT_HIP(hipMemcpy(d_qsrc, rs.q_src, 4 * rs.nq, hipMemcpyHostToDevice));
+        memcpy(off + rs.nq + 1, rs.q_src, 4 * (size_t)rs.nq);
+        LT_HIP(hipMemcpyAsync(d_qoff, off, 8 * ((size_t)rs.nq + 1), hipMemcpyHostToDevice, s_compute));
+        LT_HIP(hipMemcpyAsync(d_qsrc, off + rs.nq + 1, 4 * (size_t)rs.nq, hipMemcpyHostToDevice, s_compute));
         app.q_off = d_qoff;
         app.q_src = d_qsrc;
         app.nq = rs.nq;
     }
-    if (vregion) LT_HIP(hipMemsetAsync(d_vcur, 0, sizeof(*d_vcur) * kLogRegions * kCurStride, s_compute));
-    if (counting) LT_HIP(hipMemsetAsync(d_counts, 0, 4 * (size_t)V * count_copies, s_compute));
-    LT_HIP(hipMemsetAsync(d_stats, 0, 8 * (size_t)kNumStats * kStatSlots, s_compute));
-    if (moves_out) LT_HIP(hipMemsetAsync(d_moves, 0, 4 * rs.total, s_compute));
-    if (rs.paths_out)  // columns after an early stop stay 0xFFFFFFFF
+    const uint64_t nclear = counting ? (uint64_t)V * count_copies : 0;
+    begin_kernel<<<(int)std::min<uint64_t>(8 * num_cu, nclear / 1024 + 2), 256, 0, s_compute>>>(d_counts, nclear, d_stats,
+                                                                                             vregion ? d_vcur : nullptr);
+    LT_HIP(hipGetLastError());
+    // a flat job writes every word of these
+    if (moves_out && !walk_flat) LT_HIP(hipMemsetAsync(d_moves, 0, 4 * rs.total, s_compute));
+    if (rs.paths_out && !walk_flat)  // columns after an early stop stay 0xFFFFFFFF
         LT_HIP(hipMemsetAsync(d_paths, 0xFF, 4 * (size_t)rs.total * (rs.length + 1), s_compute));
+    outs.clear();
+    if (counts_out) outs.push_back({counts_out, d_counts, V});
+    if (endpoints_out) outs.push_back({endpoints_out, d_endpoints, rs.total});
+    if (moves_out) outs.push_back({moves_out, d_moves, rs.total});
+    if (rs.paths_out) outs.push_back({rs.paths_out, d_paths, rs.total * ((uint64_t)rs.length + 1)});
+    uint64_t out_words = 0;
+    for (const OutSeg &o : outs) out_words += o.words;
+    const bool small = out_words <= kSmallOut;
+    ResultHelpers help;
+    if (out_words >= kManyOut) help.most = std::min(4u, std::max(1u, std::thread::hardware_concurrency()) - 1);
 
     double running_ms = 0;
-    if (walk_flat) {
-        const auto t0 = std::chrono::steady_clock::now();
-        LT_TRY(run_flat(rs));
-        running_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-    }
+    auto t_walk = std::chrono::steady_clock::now();
+    job_finished = false;
+    if (walk_flat) LT_TRY(run_flat(rs, help));
     for (uint64_t id0 = walk_flat ? rs.total : 0; id0 < rs.total; id0 += wave) {
         const uint64_t id1 = std::min<uint64_t>(rs.total, id0 + wave);
         // createWalkers: untimed, as in the reference (src/LightTraffic.h:33-44)
@@ -2126,6 +2278,7 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
             LT_TRY(launch_fixup(Consumed{}));
             lo += n;
         }
+        if (id0 == 0) help.start(outs);
         LT_TRY(wait_meta());
         const auto t0 = std::chrono::steady_clock::now();
         w_run = id1 - id0;
@@ -2135,38 +2288,38 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
         const auto t1 = std::chrono::steady_clock::now();
         running_ms += std::chrono::duration<double, std::milli>(t1 - t0).count();
     }
-    if (vregion && !walk_flat) {  // part of the walk's work, so inside the timed region
-        const auto t0 = std::chrono::steady_clock::now();
+    if (!walk_flat) {
         LT_TRY(read_meta());
+        for (uint32_t i = 0; i < P; i++)
+            if (counts[i]) {
+                set_error("partition %u still holds %llu walkers after the run", i, (unsigned long long)counts[i]);
+                return LT_E_INTERNAL;
+            }
+        t_walk = std::chrono::steady_clock::now();
+    }
+    // the counts are part of the walk's work, so inside the timed region
+    if (vregion && !walk_flat) {
         const uint32_t *cur = h_meta + P + 4;
         LT_TRY(count_log(0, *std::max_element(cur, cur + kLogRegions)));
-        LT_HIP(hipStreamSynchronize(s_compute));
-        running_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     }
     if (count_copies > 1) {
-        const auto t0 = std::chrono::steady_clock::now();
         sum_count_copies_kernel<<<std::max(1, 8 * num_cu), 256, 0, s_compute>>>(d_counts, V);
         LT_HIP(hipGetLastError());
-        LT_HIP(hipStreamSynchronize(s_compute));
-        running_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     }
-    if (!walk_flat) LT_TRY(read_meta());
-    for (uint32_t i = 0; !walk_flat && i < P; i++)
-        if (counts[i]) {
-            set_error("partition %u still holds %llu walkers after the run", i, (unsigned long long)counts[i]);
-            return LT_E_INTERNAL;
-        }
-
-    // reduce (app/pagerank.cu:71-74): results back to the host, untimed
-    if (counts_out) LT_HIP(hipMemcpy(counts_out, d_counts, 4 * (size_t)V, hipMemcpyDeviceToHost));
-    if (endpoints_out) LT_HIP(hipMemcpy(endpoints_out, d_endpoints, 4 * rs.total, hipMemcpyDeviceToHost));
-    if (moves_out) LT_HIP(hipMemcpy(moves_out, d_moves, 4 * rs.total, hipMemcpyDeviceToHost));
-    if (rs.paths_out)
-        LT_HIP(hipMemcpy(rs.paths_out, d_paths, 4 * (size_t)rs.total * (rs.length + 1), hipMemcpyDeviceToHost));
-    std::vector<unsigned long long> slots_h((size_t)kNumStats * kStatSlots);
-    LT_HIP(hipMemcpy(slots_h.data(), d_stats, 8 * slots_h.size(), hipMemcpyDeviceToHost));
-    unsigned long long hs[kNumStats] = {};
-    for (size_t i = 0; i < slots_h.size(); i++) hs[i % kNumStats] += slots_h[i];
+    // reduce (app/pagerank.cu:71-74): results back to the host, untimed but for
+    // those of a few pages, which the last kernels write
+    if (!job_finished) LT_TRY(finish_job(small));
+    if (!small && !walk_flat) LT_TRY(poll_host(h_out + kOutFlag, out_seq, "results"));
+    if (!walk_flat)
+        running_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_walk).count();
+    if (!small && !job_finished) {
+        LT_TRY(copy_results(help));
+        LT_TRY(poll_host(h_out + kOutFlag, out_seq, "results"));
+    }
+    if (walk_flat) running_ms = h_out[kOutTicks] / (double)wall_khz;
+    outs.clear();
+    unsigned long long hs[kNumStats];
+    for (int i = 0; i < kNumStats; i++) hs[i] = h_out[2 * i] | (unsigned long long)h_out[2 * i + 1] << 32;
     st.running_ms = running_ms;
     st.moves = hs[ST_MOVES];
     st.teleports = hs[ST_TELEPORTS];

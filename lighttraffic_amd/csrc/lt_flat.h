@@ -92,7 +92,10 @@ __global__ __launch_bounds__(kBlock) void flat_walk_kernel(FlatArgs a) {
                 cur = load_col(a.col + b + bounded32(x.y, x.z, d));
                 ct.moves++;
             }
-            if (path && left == 0) path[length] = cur;
+            if (path) {
+                if (left == 0) path[length] = cur;
+                for (uint32_t i = length - left + 1; left > 0 && i <= length; i++) path[i] = 0xFFFFFFFFu;
+            }
             if (a.app.moves_out) a.app.moves_out[id] = length - left;
         }
         if (a.app.endpoints) a.app.endpoints[id] = cur;

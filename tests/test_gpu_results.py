@@ -1,0 +1,39 @@
+"""Results of every size on their way to the host (written by the job's last
+kernels, through the ring of pinned buffers, or into it by the walk), against
+the CPU oracle bit for bit; flat jobs and jobs through the queues."""
+import numpy as np
+import pytest
+
+import lighttraffic_amd as lt
+from oracle import ffi as oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def graph():
+    return lt.Graph.rmat(14, 8)
+
+
+@pytest.mark.parametrize("kw", [{"zerocopy_threshold": 0}, {"num_device_partitions": 3, "span": "resident"}],
+                         ids=["flat", "queues"])
+@pytest.mark.parametrize("w", [65536, 65537, 524288, 1048577, 3 * 1048576 + 77])
+def test_results_by_walker(graph, kw, w):
+    print(f"results w={w} {kw}", flush=True)
+    rp, col = graph.rowptr(), graph.col()
+    part = lt.Partition.build(graph, 32 << 20 if "span" not in kw else 64 << 10)
+    eng = lt.Engine(graph, part, **kw)
+    eng.genericwalk(10000, 3)
+    re, rm, _ = oracle.genericwalk(rp, col, w, 4, threads=16)
+    ends, moves = eng.genericwalk(w, 4, moves=True)
+    assert np.array_equal(ends, re) and np.array_equal(moves, rm)
+    assert np.array_equal(eng.genericwalk(w, 4)[0], re)
+    assert np.array_equal(eng.genericwalk(w, 4, endpoints=False, moves=True)[1], rm)
+    counts, ends = eng.ppr(w, source=3, endpoints=True)
+    rc, re, _ = oracle.ppr(rp, col, w, source=3, endpoints=True, threads=16)
+    assert np.array_equal(counts, rc) and np.array_equal(ends, re)
+    counts, ends = eng.pagerank(w, 2, endpoints=True)
+    rc, re, _ = oracle.pagerank(rp, col, w, 2, endpoints=True, threads=16)
+    assert np.array_equal(counts, rc) and np.array_equal(ends, re)
+    if w < 600000:
+        assert np.array_equal(eng.genericwalk_paths(w, 4), oracle.genericwalk_paths(rp, col, w, 4))
