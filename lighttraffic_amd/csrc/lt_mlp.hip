@@ -63,7 +63,7 @@ __device__ __forceinline__ float to_f32(float x) { return x; }
 __device__ __forceinline__ float to_f32(uint16_t h) { return bf16_to_f32(h); }
 
 // ---- features ----------------------------------------------------------------
-// One workgroup per decision.  Feature j of partition q:
+// Feature j of partition q:
 //  0 log1p(c)/log1p(W)   1 c/max c   2 log1p(c/mean c)   3 resident
 //  4 chosen now          5..11 loaded k decisions ago (k = 0..6)
 //  12 a/(a+P), a = HBM walks since q's last one (recency: Belady's victim is
@@ -74,186 +74,462 @@ constexpr int kRecentFeat = 7;  // recent loads that become features (the state 
 
 __device__ __forceinline__ float age_feature(uint32_t a, uint32_t P) { return (float)a / ((float)a + (float)P); }
 
-__global__ __launch_bounds__(256) void feat_kernel(uint32_t P, const uint32_t *counts, const uint8_t *resident,
-                                                   const uint32_t *age, const int32_t *recent, const int32_t *cur,
-                                                   const float *w_total, const float *vsh, const float *esh,
-                                                   float *X) {
-    const uint32_t b = blockIdx.x;
-    const uint32_t *c = counts + (size_t)b * P;
-    const uint8_t *r = resident + (size_t)b * P;
-    const uint32_t *ag = age + (size_t)b * P;
-    __shared__ float s_max[256], s_sum[256];
-    float mx = 0.f, sm = 0.f;
-    for (uint32_t q = threadIdx.x; q < P; q += blockDim.x) {
-        const float v = (float)c[q];
-        mx = fmaxf(mx, v);
-        sm += v;
-    }
-    s_max[threadIdx.x] = mx;
-    s_sum[threadIdx.x] = sm;
-    __syncthreads();
-    for (uint32_t off = 128; off > 0; off >>= 1) {
-        if (threadIdx.x < off) {
-            s_max[threadIdx.x] = fmaxf(s_max[threadIdx.x], s_max[threadIdx.x + off]);
-            s_sum[threadIdx.x] += s_sum[threadIdx.x + off];
-        }
-        __syncthreads();
-    }
-    const float cmax = fmaxf(s_max[0], 1.f), csum = s_sum[0];
-    const float W = fmaxf(w_total[b], 1.f);
-    const float mean = fmaxf(csum / (float)P, 1.f);
-    const float lw = log1pf(W);
-    for (uint32_t q = threadIdx.x; q < P; q += blockDim.x) {
-        const float v = (float)c[q];
-        float *x = X + ((size_t)b * P + q) * kFeat;
-        x[0] = log1pf(v) / lw;
-        x[1] = v / cmax;
-        x[2] = log1pf(v / mean);
-        x[3] = r[q] ? 1.f : 0.f;
-        x[4] = cur[b] == (int32_t)q ? 1.f : 0.f;
+// Copy of the first two layers' weights, output-major: Wi[j * kFeat + k] =
+// W1[k][j] and Wi[kWiW2 + j * kHidden + k] = W2[k][j], so that the
+// weights of output j come in 16-byte loads.
+constexpr size_t kWiW2 = (size_t)kHidden * kFeat;
+constexpr size_t kWiSize = kWiW2 + (size_t)kHidden * kHidden;
+
+// ---- training ------------------------------------------------------------------
+// One step over M = decisions * P rows in four launches:
+//   train_forward_kernel   features and the three layers, 32 rows per workgroup
+//   loss_kernel            losses and dY, one workgroup per decision
+//   train_backward_kernel  two kinds of workgroups: tiles of 32 rows, dA2 and
+//                          dA1 with their part of every gradient but W2's; and a
+//                          quarter of W2's gradient over a slice of the rows
+//   train_update_kernel    the gradient (partial sums added in a fixed order),
+//                          and Adam
+// Products run on the matrix cores in FP32 (v_mfma_f32_32x32x2_f32: FP32
+// inputs and accumulation, as on the vector units).  Bound: at 32 decisions of
+// 291 partitions the 3.8 GFLOP take 24 us at the FP32 matrix rate; these launches
+// take 33, 11, 53 and 13, and the sixteen of 64 x 64 LDS-tiled vector GEMMs and
+// their split-K sums took 460.  The batch is read in place from pinned memory
+// (121 KB; a copy to the device first measured the same in all, ten separate
+// copies 150 us more).
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int kTileRows = 32;
+constexpr int kLdH = kHidden + 4;  // LDS row of 256 columns: 16-byte aligned, rows 4 banks apart
+constexpr uint32_t kSliceMost = 64;   // slices of the rows in W2's gradient: 4 x 64 workgroups fill the chip
+constexpr uint32_t kGroupMost = 512;  // workgroups of the other kind, two per CU
+constexpr int kSmallParams = (int)kParams - kHidden * kHidden;  // all but W2
+
+// The small gradients' order in a partial row: W1, b1, b2, W3, b3.
+constexpr int kSmB1 = kFeat * kHidden, kSmB2 = kSmB1 + kHidden, kSmW3 = kSmB2 + kHidden, kSmB3 = kSmW3 + kHidden * kOut;
+
+// One batch of decisions in mapped host memory (upload_samples).
+struct Batch {
+    const uint32_t *counts, *age;  // [n][P]
+    const float *keep;             // [n][P]
+    const float *scale;            // [n][3]: walkers, largest count, sum of the counts
+    const int32_t *recent;         // [n][kRecent]
+    const int32_t *cur, *next;     // [n]
+    const float *wa, *wb;          // [n]
+    const uint8_t *resident;       // [n][P]
+};
+
+// Features of partition q; head gives the decision's scalars.
+__device__ __forceinline__ void features(float *x, uint32_t P, uint32_t q, uint32_t count, bool res, uint32_t age,
+                                         float w_total, float max_count, float sum, int32_t cur, const int32_t *recent,
+                                         float vsh, float esh) {
+    const float W = fmaxf(w_total, 1.f);
+    const float cmax = fmaxf(max_count, 1.f);
+    const float mean = fmaxf(sum / (float)P, 1.f);
+    const float v = (float)count;
+    x[0] = log1pf(v) / log1pf(W);
+    x[1] = v / cmax;
+    x[2] = log1pf(v / mean);
+    x[3] = res ? 1.f : 0.f;
+    x[4] = cur == (int32_t)q ? 1.f : 0.f;
 #pragma unroll
-        for (int k = 0; k < kRecentFeat; k++) x[5 + k] = recent[b * kRecent + k] == (int32_t)q ? 1.f : 0.f;
-        x[12] = age_feature(ag[q], P);
-        x[13] = vsh[q];
-        x[14] = esh[q];
-        x[15] = csum / W;
-    }
+    for (int k = 0; k < kRecentFeat; k++) x[5 + k] = recent[k] == (int32_t)q ? 1.f : 0.f;
+    x[12] = age_feature(age, P);
+    x[13] = vsh;
+    x[14] = esh;
+    x[15] = sum / W;
 }
 
-// ---- tiled FP32-accumulate GEMM ------------------------------------------------
-// C[M x N] = op(A)[M x K] * op(B)[K x N], 64x64 tiles, 256 threads, 4x4 per thread.
-// op(A)[m][k] = TA ? A[k*lda+m] : A[m*lda+k];  op(B)[k][n] = TB ? B[n*ldb+k] : B[k*ldb+n].
-// EPI 0: store; 1: relu(acc + bias[n]); 2: acc * (mask[m][n] > 0); 3: acc + bias[n].
-enum { EPI_STORE = 0, EPI_BIAS_RELU = 1, EPI_RELU_GRAD = 2, EPI_BIAS = 3 };
-
-// With gridDim.z > 1 the K range is split: slice z covers [z*kchunk, (z+1)*kchunk)
-// and stores its partial product at C + z*M*ldc (summed by splitk_reduce_kernel).
-template <bool TA, bool TB, typename BT, int EPI>
-__global__ __launch_bounds__(256) void gemm_kernel(int M, int N, int K, const float *A, int lda, const BT *B, int ldb,
-                                                   float *C, int ldc, const BT *bias, const float *mask, int ldm,
-                                                   int kchunk) {
-    constexpr int TM = 64, TN = 64, TK = 16;
-    __shared__ float As[TK][TM + 4];
-    __shared__ float Bs[TK][TN + 4];
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-    const int kb = blockIdx.z * kchunk;
-    const int ke = min(K, kb + kchunk);
-    C += (size_t)blockIdx.z * M * ldc;
-    float acc[4][4] = {};
-    for (int k0 = kb; k0 < ke; k0 += TK) {
-        for (int i = threadIdx.x; i < TM * TK; i += 256) {
-            int mm, kk;
-            if (TA) { mm = i % TM; kk = i / TM; } else { kk = i % TK; mm = i / TK; }
-            const int m = m0 + mm, k = k0 + kk;
-            float v = 0.f;
-            if (m < M && k < ke) v = TA ? A[(size_t)k * lda + m] : A[(size_t)m * lda + k];
-            As[kk][mm] = v;
-        }
-        for (int i = threadIdx.x; i < TN * TK; i += 256) {
-            int nn, kk;
-            if (TB) { kk = i % TK; nn = i / TK; } else { nn = i % TN; kk = i / TN; }
-            const int n = n0 + nn, k = k0 + kk;
-            float v = 0.f;
-            if (n < N && k < ke) v = to_f32(TB ? B[(size_t)n * ldb + k] : B[(size_t)k * ldb + n]);
-            Bs[kk][nn] = v;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < TK; kk++) {
-            float a[4], bb[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) a[i] = As[kk][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; j++) bb[j] = Bs[kk][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[i][j] = fmaf(a[i], bb[j], acc[i][j]);
-        }
-        __syncthreads();
-    }
+__device__ __forceinline__ void unpack8(const uint4 &w, float *f) {
+    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const int m = m0 + ty * 4 + i;
-        if (m >= M) continue;
+        f[2 * i] = __uint_as_float(u[i] << 16);
+        f[2 * i + 1] = __uint_as_float(u[i] & 0xFFFF0000u);
+    }
+}
+
+// acc[t] += A[32 x 256] * B for the wave's two 32-column tiles: A is an LDS
+// tile of kLdH-float rows, B[k][n] = bt[n * 256 + k] (BF16).  In a step of 64 k
+// the lanes of a wave's lower half hold k = 64 s .. +31 and those of its upper
+// half the next 32, for A and B alike: a lane reads 64 bytes of one weight row
+// at a time, and the next step's weights arrive while this one's 64 products
+// run (1.7 us).  The first step's weights the caller loads ahead.
+struct WeightStep {
+    uint4 w0[4], w1[4];
+};
+__device__ __forceinline__ WeightStep first_weights(const uint16_t *bt, int n0) {
+    const int lane = threadIdx.x & 63, i = lane & 31, h = lane >> 5;
+    WeightStep w;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int n = n0 + tx * 4 + j;
-            if (n >= N) continue;
-            float v = acc[i][j];
-            if (EPI == EPI_BIAS_RELU) v = fmaxf(v + to_f32(bias[n]), 0.f);
-            else if (EPI == EPI_BIAS) v = v + to_f32(bias[n]);
-            else if (EPI == EPI_RELU_GRAD) v = mask[(size_t)m * ldm + n] > 0.f ? v : 0.f;
-            C[(size_t)m * ldc + n] = v;
+    for (int c = 0; c < 4; c++) {
+        w.w0[c] = ((const uint4 *)(bt + (size_t)(n0 + i) * kHidden + 32 * h))[c];
+        w.w1[c] = ((const uint4 *)(bt + (size_t)(n0 + 32 + i) * kHidden + 32 * h))[c];
+    }
+    return w;
+}
+__device__ __forceinline__ void mfma_rows(const float *sA, const uint16_t *bt, int n0, const WeightStep &first,
+                                          f32x16 (&acc)[2]) {
+    const int lane = threadIdx.x & 63, i = lane & 31, h = lane >> 5;
+    const uint4 *b0 = (const uint4 *)(bt + (size_t)(n0 + i) * kHidden + 32 * h);
+    const uint4 *b1 = (const uint4 *)(bt + (size_t)(n0 + 32 + i) * kHidden + 32 * h);
+    const float *a = sA + i * kLdH + 32 * h;
+    uint4 w0[4], w1[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        w0[c] = first.w0[c];
+        w1[c] = first.w1[c];
+    }
+#pragma unroll
+    for (int s = 0; s < kHidden / 64; s++) {
+        uint4 v0[4], v1[4];
+        if (s + 1 < kHidden / 64) {
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                v0[c] = b0[8 * (s + 1) + c];
+                v1[c] = b1[8 * (s + 1) + c];
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const float4 lo = *(const float4 *)(a + 64 * s + 8 * c), hi = *(const float4 *)(a + 64 * s + 8 * c + 4);
+            const float av[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+            float f0[8], f1[8];
+            unpack8(w0[c], f0);
+            unpack8(w1[c], f1);
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[j], f0[j], acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[j], f1[j], acc[1], 0, 0, 0);
+            }
+        }
+        if (s + 1 < kHidden / 64) {
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                w0[c] = v0[c];
+                w1[c] = v1[c];
+            }
         }
     }
 }
 
-template <bool TA, bool TB, typename BT, int EPI>
-static void gemm(hipStream_t s, int M, int N, int K, const float *A, int lda, const BT *B, int ldb, float *C, int ldc,
-                 const BT *bias = nullptr, const float *mask = nullptr, int ldm = 0) {
-    dim3 grid((N + 63) / 64, (M + 63) / 64, 1);
-    gemm_kernel<TA, TB, BT, EPI><<<grid, 256, 0, s>>>(M, N, K, A, lda, B, ldb, C, ldc, bias, mask, ldm, K);
+// Row of element r of a 32 x 32 result tile (column = lane % 32).
+__device__ __forceinline__ int tile_row(int r) { return 8 * (r >> 2) + 4 * ((int)(threadIdx.x & 63) >> 5) + (r & 3); }
+
+__global__ __launch_bounds__(256) void train_forward_kernel(uint32_t P, uint32_t M, Batch d, const float *vsh,
+                                                            const float *esh, const uint16_t *Wb, const uint16_t *Wi,
+                                                            uint32_t *counts, float *X, float *A1, float *A2,
+                                                            float *Y) {
+    __shared__ __align__(16) float s_x[kTileRows][kFeat + 1];
+    __shared__ __align__(16) float s_a[kTileRows * kLdH];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = lane & 31, h = lane >> 5;
+    const int n0 = wave * 64;
+    // weights do not wait for the features
+    const uint4 w1[2] = {*(const uint4 *)(Wi + (size_t)(n0 + i) * kFeat + 8 * h),
+                         *(const uint4 *)(Wi + (size_t)(n0 + 32 + i) * kFeat + 8 * h)};
+    const WeightStep w2 = first_weights(Wi + kWiW2, n0);
+    const float bias1[2] = {bf16_to_f32(Wb[kOffB1 + n0 + i]), bf16_to_f32(Wb[kOffB1 + n0 + 32 + i])};
+    const float bias2[2] = {bf16_to_f32(Wb[kOffB2 + n0 + i]), bf16_to_f32(Wb[kOffB2 + n0 + 32 + i])};
+    const uint32_t r0 = blockIdx.x * kTileRows;
+    if (tid < kTileRows) {
+        const uint32_t r = r0 + tid;
+        float x[kFeat];
+#pragma unroll
+        for (int k = 0; k < kFeat; k++) x[k] = 0.f;
+        if (r < M) {
+            const uint32_t b = r / P, q = r - b * P;
+            const uint32_t count = d.counts[r];
+            counts[r] = count;
+            features(x, P, q, count, d.resident[r], d.age[r], d.scale[3 * b], d.scale[3 * b + 1],
+                     d.scale[3 * b + 2], d.cur[b], d.recent + b * kRecent, vsh[q], esh[q]);
+        }
+#pragma unroll
+        for (int k = 0; k < kFeat; k++) s_x[tid][k] = x[k];
+    }
+    __syncthreads();
+    for (int t = tid; t < kTileRows * kFeat; t += 256)
+        if (r0 + t / kFeat < M) X[(size_t)r0 * kFeat + t] = s_x[t / kFeat][t % kFeat];
+    f32x16 acc[2] = {};
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        float f[8];
+        unpack8(w1[t], f);
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(s_x[i][8 * h + j], f[j], acc[t], 0, 0, 0);
+    }
+    const auto layer_out = [&](const float (&bias)[2], float *A) {
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int n = n0 + 32 * t + i;
+            const float bn = bias[t];
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int m = tile_row(r);
+                const float v = fmaxf(acc[t][r] + bn, 0.f);
+                s_a[m * kLdH + n] = v;
+                if (r0 + m < M) A[(size_t)(r0 + m) * kHidden + n] = v;
+            }
+        }
+    };
+    layer_out(bias1, A1);
+    __syncthreads();
+    acc[0] = acc[1] = f32x16{};
+    mfma_rows(s_a, Wi + kWiW2, n0, w2, acc);
+    __syncthreads();
+    layer_out(bias2, A2);
+    __syncthreads();
+    const int row = tid >> 3, part = tid & 7;  // eight threads per row, 4 of every 32 columns each
+    float y0 = 0.f, y1 = 0.f;
+#pragma unroll
+    for (int s = 0; s < kHidden / 32; s++) {
+        const int k = 32 * s + 4 * part;
+        const float4 v = *(const float4 *)(s_a + row * kLdH + k);
+        float w[8];
+        unpack8(*(const uint4 *)(Wb + kOffW3 + k * kOut), w);
+        y0 = fmaf(v.x, w[0], y0);
+        y1 = fmaf(v.x, w[1], y1);
+        y0 = fmaf(v.y, w[2], y0);
+        y1 = fmaf(v.y, w[3], y1);
+        y0 = fmaf(v.z, w[4], y0);
+        y1 = fmaf(v.z, w[5], y1);
+        y0 = fmaf(v.w, w[6], y0);
+        y1 = fmaf(v.w, w[7], y1);
+    }
+#pragma unroll
+    for (int off = 1; off < 8; off <<= 1) {
+        y0 += __shfl_xor(y0, off, 64);
+        y1 += __shfl_xor(y1, off, 64);
+    }
+    if (part == 0 && r0 + row < M)
+        ((float2 *)Y)[r0 + row] = make_float2(y0 + bf16_to_f32(Wb[kOffB3]), y1 + bf16_to_f32(Wb[kOffB3 + 1]));
 }
 
-// out[i] = sum_z part[z*n + i], fixed order (deterministic).
-__global__ void splitk_reduce_kernel(size_t n, int splits, const float *part, float *out) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float s = 0.f;
-    for (int z = 0; z < splits; z++) s += part[(size_t)z * n + i];
-    out[i] = s;
+// dA2[m][n] before the ReLU mask.
+__device__ __forceinline__ float back3(float dy0, float dy1, float w0, float w1) { return fmaf(dy1, w1, dy0 * w0); }
+
+__global__ __launch_bounds__(256, 2) void train_backward_kernel(uint32_t M, uint32_t groups, uint32_t slices,
+                                                             const float *X, const float *A1, const float *A2,
+                                                             const float *dY, const uint16_t *Wb, float *small,
+                                                             float *w2) {
+    __shared__ __align__(16) float s_d2[kTileRows * kLdH];
+    __shared__ __align__(16) float s_d1[kTileRows * kLdH];
+    __shared__ __align__(16) float s_x[kTileRows][kFeat];
+    __shared__ float s_dy[kTileRows][kOut];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = lane & 31, h = lane >> 5;
+    const uint32_t tiles = (M + kTileRows - 1) / kTileRows;
+    if (blockIdx.x < groups) {
+        float g[kFeat] = {}, b1 = 0.f, b2 = 0.f, b3 = 0.f, g0 = 0.f, g1 = 0.f;
+        const float w30 = bf16_to_f32(Wb[kOffW3 + tid * kOut]), w31 = bf16_to_f32(Wb[kOffW3 + tid * kOut + 1]);
+        const int n0 = wave * 64;
+        const WeightStep w2t = first_weights(Wb + kOffW2, n0);
+        for (uint32_t tile = blockIdx.x; tile < tiles; tile += groups) {
+            const uint32_t r0 = tile * kTileRows;
+            const int rows = (int)min((uint32_t)kTileRows, M - r0);
+            // everything the tile reads is on its way before any of it is waited for
+            float a2[kTileRows];
+#pragma unroll
+            for (int m = 0; m < kTileRows; m++) a2[m] = m < rows ? A2[(size_t)(r0 + m) * kHidden + tid] : 0.f;
+            uint32_t on = 0;  // ReLU masks of this lane's 32 elements of dA1
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int m = tile_row(r);
+                    if (m < rows && A1[(size_t)(r0 + m) * kHidden + n0 + 32 * t + i] > 0.f) on |= 1u << (16 * t + r);
+                }
+            for (int t = tid; t < kTileRows * kFeat; t += 256)
+                s_x[t / kFeat][t % kFeat] = t / kFeat < rows ? X[(size_t)r0 * kFeat + t] : 0.f;
+            if (tid < kTileRows * kOut)
+                s_dy[tid / kOut][tid % kOut] = tid / kOut < rows ? dY[(size_t)r0 * kOut + tid] : 0.f;
+            __syncthreads();
+            // thread = column: dA2, and the sums over its rows that need no product
+#pragma unroll
+            for (int m = 0; m < kTileRows; m++) {
+                const float y0 = s_dy[m][0], y1 = s_dy[m][1];
+                const float v = a2[m] > 0.f ? back3(y0, y1, w30, w31) : 0.f;
+                s_d2[m * kLdH + tid] = v;
+                b2 += v;
+                g0 = fmaf(a2[m], y0, g0);
+                g1 = fmaf(a2[m], y1, g1);
+            }
+            if (tid < kOut)
+                for (int m = 0; m < kTileRows; m++) b3 += s_dy[m][tid];
+            __syncthreads();
+            f32x16 acc[2] = {};
+            mfma_rows(s_d2, Wb + kOffW2, n0, w2t, acc);  // dA1[m][j] = sum_n dA2[m][n] W2[j][n]
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    s_d1[tile_row(r) * kLdH + n0 + 32 * t + i] = (on >> (16 * t + r)) & 1u ? acc[t][r] : 0.f;
+            __syncthreads();
+#pragma unroll 8
+            for (int m = 0; m < kTileRows; m++) {
+                const float v = s_d1[m * kLdH + tid];
+                b1 += v;
+#pragma unroll
+                for (int f = 0; f < kFeat; f++) g[f] = fmaf(s_x[m][f], v, g[f]);
+            }
+            __syncthreads();
+        }
+        float *out = small + (size_t)blockIdx.x * kSmallParams;
+#pragma unroll
+        for (int f = 0; f < kFeat; f++) out[f * kHidden + tid] = g[f];
+        out[kSmB1 + tid] = b1;
+        out[kSmB2 + tid] = b2;
+        out[kSmW3 + tid * kOut] = g0;
+        out[kSmW3 + tid * kOut + 1] = g1;
+        if (tid < kOut) out[kSmB3 + tid] = b3;
+        return;
+    }
+    // W2's gradient: slice z of the row tiles, 128 x 128 quarter (k0, n0); each
+    // wave 64 x 64 of it.  The next tile's rows are loaded while this one's
+    // products run.
+    const uint32_t z = (blockIdx.x - groups) >> 2, quarter = (blockIdx.x - groups) & 3;
+    const int k0 = (int)(quarter >> 1) * 128, n0 = (int)(quarter & 1) * 128;
+    const uint32_t t0 = (uint32_t)((uint64_t)tiles * z / slices), t1 = (uint32_t)((uint64_t)tiles * (z + 1) / slices);
+    constexpr int kLdT = 128, kHalf = kTileRows / 2;  // LDS row of a staged tile; its rows per thread
+    float *s_a = s_d2, *s_b = s_d1;
+    const int wk = (wave >> 1) * 64, wn = (wave & 1) * 64;
+    const int c = tid & 127, half = tid >> 7;
+    const float w30 = bf16_to_f32(Wb[kOffW3 + (n0 + c) * kOut]), w31 = bf16_to_f32(Wb[kOffW3 + (n0 + c) * kOut + 1]);
+    float a[kHalf], b[kHalf];
+    float2 dy[kHalf];
+    const auto load = [&](uint32_t t) {
+        const uint32_t r0 = t * kTileRows;
+#pragma unroll
+        for (int m = 0; m < kHalf; m++) {
+            const uint32_t r = r0 + 2 * m + half;
+            const bool in = r < M;
+            a[m] = in ? A1[(size_t)r * kHidden + k0 + c] : 0.f;
+            b[m] = in ? A2[(size_t)r * kHidden + n0 + c] : 0.f;
+            dy[m] = in ? ((const float2 *)dY)[r] : make_float2(0.f, 0.f);
+        }
+    };
+    f32x16 acc[2][2] = {};
+    load(t0);
+    for (uint32_t t = t0; t < t1; t++) {
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < kHalf; m++) {
+            s_a[(2 * m + half) * kLdT + c] = a[m];
+            s_b[(2 * m + half) * kLdT + c] = b[m] > 0.f ? back3(dy[m].x, dy[m].y, w30, w31) : 0.f;
+        }
+        __syncthreads();
+        if (t + 1 < t1) load(t + 1);
+#pragma unroll
+        for (int s = 0; s < kHalf; s++) {
+            const float *ra = s_a + (2 * s + h) * kLdT + wk + i, *rb = s_b + (2 * s + h) * kLdT + wn + i;
+            const float a0 = ra[0], a1 = ra[32], b0 = rb[0], b1 = rb[32];
+            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, acc[0][0], 0, 0, 0);
+            acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b1, acc[0][1], 0, 0, 0);
+            acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b0, acc[1][0], 0, 0, 0);
+            acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, acc[1][1], 0, 0, 0);
+        }
+    }
+    float *out = w2 + (size_t)z * kHidden * kHidden;
+#pragma unroll
+    for (int ta = 0; ta < 2; ta++)
+#pragma unroll
+        for (int tb = 0; tb < 2; tb++)
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                out[(size_t)(k0 + wk + 32 * ta + tile_row(r)) * kHidden + n0 + wn + 32 * tb + i] = acc[ta][tb][r];
 }
 
-// Weight gradient C[M x N] = A^T B with a long K (rows of the batch): K is cut
-// into slices of kSplitK, each slice writes a partial product, then a fixed-order sum.
-constexpr int kSplitK = 256;
-static void gemm_wgrad(hipStream_t s, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C,
-                       float *partial) {
-    const int splits = (K + kSplitK - 1) / kSplitK;
-    dim3 grid((N + 63) / 64, (M + 63) / 64, splits);
-    gemm_kernel<true, false, float, EPI_STORE><<<grid, 256, 0, s>>>(M, N, K, A, lda, B, ldb, partial, N, nullptr,
-                                                                   nullptr, 0, kSplitK);
-    const size_t n = (size_t)M * N;
-    splitk_reduce_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(n, splits, partial, C);
+// Gradient of 32 parameters per workgroup: 8 threads share a parameter's
+// partial sums, added in a fixed order.  With update, Adam on them (their
+// BF16 forms included); host: the gradient goes there too.  The first workgroup
+// adds up the decisions' losses.
+__global__ __launch_bounds__(256) void train_update_kernel(uint32_t groups, uint32_t slices, const float *small,
+                                                           const float *w2, float *G, float *host, float *W,
+                                                           uint16_t *Wb, uint16_t *Wi, float *Mo, float *Vo, int update,
+                                                           float lr, float b1t, float b2t, uint32_t n,
+                                                           const float *losses, float *loss) {
+    __shared__ float s_p[8][32];
+    const int c = threadIdx.x & 31, g = threadIdx.x >> 5;
+    const uint32_t p = blockIdx.x * 32 + c;
+    float sum = 0.f;
+    if (p < kParams) {
+        const bool is_w2 = p >= kOffW2 && p < kOffB2;
+        // partial rows hold the parameters without W2 in the same order
+        const float *q = is_w2 ? w2 + (p - kOffW2) : small + (p < kOffW2 ? p : p - kHidden * kHidden);
+        const size_t ld = is_w2 ? (size_t)kHidden * kHidden : (size_t)kSmallParams;
+        const uint32_t parts = is_w2 ? slices : groups;
+        uint32_t k = g;
+        for (; k + 24 < parts; k += 32) {  // four loads in flight
+            const float x0 = q[k * ld], x1 = q[(k + 8) * ld], x2 = q[(k + 16) * ld], x3 = q[(k + 24) * ld];
+            sum += (x0 + x1) + (x2 + x3);
+        }
+        for (; k < parts; k += 8) sum += q[k * ld];
+    }
+    s_p[g][c] = sum;
+    __syncthreads();
+    if (g == 0 && p < kParams) {
+        float s = 0.f;
+#pragma unroll
+        for (int k = 0; k < 8; k++) s += s_p[k][c];
+        G[p] = s;
+        if (host) host[p] = s;
+        if (update) {
+            const float m = 0.9f * Mo[p] + 0.1f * s;
+            const float v = 0.999f * Vo[p] + 0.001f * s * s;
+            Mo[p] = m;
+            Vo[p] = v;
+            const float w = W[p] - lr * (m / (1.f - b1t)) / (sqrtf(v / (1.f - b2t)) + 1e-8f);
+            W[p] = w;
+            const uint16_t r = f32_to_bf16(w);
+            Wb[p] = r;
+            if (p < kOffB1) Wi[(p % kHidden) * kFeat + p / kHidden] = r;
+            else if (p >= kOffW2 && p < kOffB2)
+                Wi[kWiW2 + ((p - kOffW2) % kHidden) * kHidden + (p - kOffW2) / kHidden] = r;
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+        float l[2] = {0.f, 0.f};
+        for (uint32_t b = threadIdx.x; b < n; b += 64) {
+            l[0] += losses[2 * b];
+            l[1] += losses[2 * b + 1];
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            l[0] += __shfl_xor(l[0], off, 64);
+            l[1] += __shfl_xor(l[1], off, 64);
+        }
+        if (threadIdx.x < 2) loss[threadIdx.x] = l[threadIdx.x];
+    }
 }
 
 // ---- losses -----------------------------------------------------------------
-// One workgroup per decision; writes dY and adds the weighted losses to loss[0..1].
+// One workgroup per decision; writes dY and the decision's weighted losses.
 __global__ __launch_bounds__(256) void loss_kernel(uint32_t P, uint32_t B, const float *Y, const uint32_t *counts,
                                                    const int32_t *next_label, const float *keep_label,
-                                                   const float *wa, const float *wb, float *dY, float *loss) {
+                                                   const float *wa, const float *wb, float *dY, float *losses) {
     const uint32_t b = blockIdx.x;
     const float *y = Y + (size_t)b * P * kOut;
     float *dy = dY + (size_t)b * P * kOut;
     const uint32_t *c = counts + (size_t)b * P;
     const int32_t lab = next_label[b];
     const float a_w = lab >= 0 ? wa[b] : 0.f, b_w = wb[b];
-    __shared__ float s_red[256];
+    __shared__ float s_red[3][4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // softmax over candidates (walkers queued, or the label itself)
     float mx = -INFINITY;
     for (uint32_t q = threadIdx.x; q < P; q += blockDim.x)
         if (c[q] > 0 || (int32_t)q == lab) mx = fmaxf(mx, y[q * kOut]);
-    s_red[threadIdx.x] = mx;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+    if (lane == 0) s_red[0][wave] = mx;
     __syncthreads();
-    for (uint32_t off = 128; off > 0; off >>= 1) {
-        if (threadIdx.x < off) s_red[threadIdx.x] = fmaxf(s_red[threadIdx.x], s_red[threadIdx.x + off]);
-        __syncthreads();
-    }
-    mx = s_red[0];
-    __syncthreads();
+    mx = fmaxf(fmaxf(s_red[0][0], s_red[0][1]), fmaxf(s_red[0][2], s_red[0][3]));
     float se = 0.f;
     for (uint32_t q = threadIdx.x; q < P; q += blockDim.x)
         if (c[q] > 0 || (int32_t)q == lab) se += expf(y[q * kOut] - mx);
-    s_red[threadIdx.x] = se;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) se += __shfl_xor(se, off, 64);
+    if (lane == 0) s_red[1][wave] = se;
     __syncthreads();
-    for (uint32_t off = 128; off > 0; off >>= 1) {
-        if (threadIdx.x < off) s_red[threadIdx.x] += s_red[threadIdx.x + off];
-        __syncthreads();
-    }
-    se = s_red[0];
-    __syncthreads();
+    se = (s_red[1][0] + s_red[1][1]) + (s_red[1][2] + s_red[1][3]);
     float lb = 0.f;
     const float inv_b = 1.f / (float)B;
     for (uint32_t q = threadIdx.x; q < P; q += blockDim.x) {
@@ -268,48 +544,15 @@ __global__ __launch_bounds__(256) void loss_kernel(uint32_t P, uint32_t B, const
         dy[q * kOut] = g0;
         dy[q * kOut + 1] = b_w * 2.f * d * inv_b / (float)P;
     }
-    s_red[threadIdx.x] = lb;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) lb += __shfl_xor(lb, off, 64);
+    if (lane == 0) s_red[2][wave] = lb;
     __syncthreads();
-    for (uint32_t off = 128; off > 0; off >>= 1) {
-        if (threadIdx.x < off) s_red[threadIdx.x] += s_red[threadIdx.x + off];
-        __syncthreads();
-    }
+    lb = (s_red[2][0] + s_red[2][1]) + (s_red[2][2] + s_red[2][3]);
     if (threadIdx.x == 0) {
-        if (a_w > 0.f && se > 0.f) atomicAdd(&loss[0], a_w * (logf(se) + mx - y[lab * kOut]) * inv_b);
-        atomicAdd(&loss[1], s_red[0] * inv_b / (float)P);
+        losses[2 * b] = a_w > 0.f && se > 0.f ? a_w * (logf(se) + mx - y[lab * kOut]) * inv_b : 0.f;
+        losses[2 * b + 1] = lb * inv_b / (float)P;
     }
-}
-
-// db[n] = sum_m dZ[m][n]: slice z of the rows sums into part[z*N + n]
-// (reduced afterwards in fixed order).
-__global__ void colsum_kernel(int M, int N, const float *dZ, float *part, int rows_per_slice) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
-    const int m0 = blockIdx.y * rows_per_slice, m1 = min(M, m0 + rows_per_slice);
-    float s = 0.f;
-    for (int m = m0; m < m1; m++) s += dZ[(size_t)m * N + n];
-    part[(size_t)blockIdx.y * N + n] = s;
-}
-
-static void colsum(hipStream_t s, int M, int N, const float *dZ, float *out, float *partial) {
-    constexpr int kRows = 64;  // rows per slice: many short slices keep every CU busy
-    const int splits = (M + kRows - 1) / kRows;
-    colsum_kernel<<<dim3((N + 255) / 256, splits), 256, 0, s>>>(M, N, dZ, partial, kRows);
-    splitk_reduce_kernel<<<(N + 255) / 256, 256, 0, s>>>((size_t)N, splits, partial, out);
-}
-
-__global__ void adam_kernel(size_t n, float *W, uint16_t *Wb, const float *G, float *Mo, float *Vo, float lr,
-                            float b1t, float b2t) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float g = G[i];
-    const float m = 0.9f * Mo[i] + 0.1f * g;
-    const float v = 0.999f * Vo[i] + 0.001f * g * g;
-    Mo[i] = m;
-    Vo[i] = v;
-    const float w = W[i] - lr * (m / (1.f - b1t)) / (sqrtf(v / (1.f - b2t)) + 1e-8f);
-    W[i] = w;
-    Wb[i] = f32_to_bf16(w);
 }
 
 __global__ void round_kernel(size_t n, const float *W, uint16_t *Wb) {
@@ -317,13 +560,7 @@ __global__ void round_kernel(size_t n, const float *W, uint16_t *Wb) {
     if (i < n) Wb[i] = f32_to_bf16(W[i]);
 }
 
-// ---- fused inference: one decision, 8 partitions per workgroup --------------
-// Inference copy of the first two layers, output-major: Wi[j * kFeat + k] =
-// W1[k][j] and Wi[kWiW2 + j * kHidden + k] = W2[k][j], so that the thread of
-// output j reads its weights with 16-byte loads.
-constexpr size_t kWiW2 = (size_t)kHidden * kFeat;
-constexpr size_t kWiSize = kWiW2 + (size_t)kHidden * kHidden;
-
+// ---- fused inference: one decision, R partitions per workgroup --------------
 __global__ void transpose_infer_weights_kernel(const uint16_t *Wb, uint16_t *Wi) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < kWiW2) {
@@ -363,13 +600,16 @@ static void pack_state_head(int32_t *head, const uint32_t *counts, uint32_t P, c
     memcpy(&head[kHeadW], f, sizeof(f));
 }
 
-// Each workgroup builds the features of 8 partitions (rows) and runs the
+// Each workgroup builds the features of R partitions (rows) and runs the
 // three layers on them.  Each output neuron accumulates its inputs in
-// increasing order in FP32.
+// increasing order in FP32, whatever R.  A decision waits for this kernel: with
+// 8 rows 291 partitions keep 37 of 256 CUs busy for 17 us, with 2 rows 146 for
+// 10.6.  Above kFewRows partitions there are workgroups enough, and 8 rows share
+// the weights (20,000 partitions: 120 us a call either way).
+template <int R>
 __global__ __launch_bounds__(256) void infer_kernel(uint32_t P, const uint8_t *state, const float *vsh,
                                                     const float *esh, const uint16_t *Wb, const uint16_t *Wi,
                                                     float *Y) {
-    constexpr int R = 8;
     __shared__ float s_x[R][kFeat];
     __shared__ float s_h1[R][kHidden];
     __shared__ float s_h2[R][kHidden];
@@ -383,20 +623,8 @@ __global__ __launch_bounds__(256) void infer_kernel(uint32_t P, const uint8_t *s
         const uint32_t q = r0 + j;
         float *x = s_x[j];
         if (q < P) {
-            const float W = fmaxf(__int_as_float(head[kHeadW]), 1.f);
-            const float cmax = fmaxf(__int_as_float(head[kHeadMax]), 1.f), csum = __int_as_float(head[kHeadSum]);
-            const float mean = fmaxf(csum / (float)P, 1.f);
-            const float v = (float)counts[q];
-            x[0] = log1pf(v) / log1pf(W);
-            x[1] = v / cmax;
-            x[2] = log1pf(v / mean);
-            x[3] = res[q] ? 1.f : 0.f;
-            x[4] = head[kHeadCur] == (int32_t)q ? 1.f : 0.f;
-            for (int k = 0; k < kRecentFeat; k++) x[5 + k] = head[k] == (int32_t)q ? 1.f : 0.f;
-            x[12] = age_feature(age[q], P);
-            x[13] = vsh[q];
-            x[14] = esh[q];
-            x[15] = csum / W;
+            features(x, P, q, counts[q], res[q], age[q], __int_as_float(head[kHeadW]), __int_as_float(head[kHeadMax]),
+                     __int_as_float(head[kHeadSum]), head[kHeadCur], head, vsh[q], esh[q]);
         } else {
             for (int k = 0; k < kFeat; k++) x[k] = 0.f;
         }
@@ -451,6 +679,18 @@ __global__ __launch_bounds__(256) void infer_kernel(uint32_t P, const uint8_t *s
     }
 }
 
+constexpr uint32_t kFewRows = 1024;
+static void launch_infer(hipStream_t s, uint32_t P, const uint8_t *state, const float *vsh, const float *esh,
+                         const uint16_t *Wb, const uint16_t *Wi, float *Y) {
+    if (P <= kFewRows) infer_kernel<2><<<(P + 1) / 2, 256, 0, s>>>(P, state, vsh, esh, Wb, Wi, Y);
+    else infer_kernel<8><<<(P + 7) / 8, 256, 0, s>>>(P, state, vsh, esh, Wb, Wi, Y);
+}
+
+// A sequence number for the host, behind what the stream's kernels wrote to it.
+static __global__ void infer_mark_kernel(uint32_t *flag, uint32_t seq) {
+    __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ---- host object ---------------------------------------------------------------
 template <typename T>
 static lt_status dalloc(T **p, size_t n) {
@@ -476,34 +716,37 @@ struct Scorer {
     bool trained = false;
     // training buffers (capacity in decisions)
     uint32_t cap = 0;
-    uint32_t *d_counts = nullptr, *d_age = nullptr;
-    uint8_t *d_res = nullptr;
-    int32_t *d_recent = nullptr, *d_cur = nullptr, *d_next = nullptr;
-    float *d_wtot = nullptr, *d_keep = nullptr, *d_wa = nullptr, *d_wb = nullptr;
-    float *X = nullptr, *A1 = nullptr, *A2 = nullptr, *Y = nullptr, *dY = nullptr, *dA1 = nullptr, *dA2 = nullptr;
-    float *partial = nullptr;  // split-K partial products
-    float *d_loss = nullptr;
+    uint8_t *h_batch = nullptr;  // a batch, pinned and mapped (see Batch)
+    Batch batch{};               // device views of its arrays
+    uint32_t *d_counts = nullptr;
+    float *X = nullptr, *A1 = nullptr, *A2 = nullptr, *Y = nullptr, *dY = nullptr;
+    float *small = nullptr, *w2 = nullptr;  // partial gradients
+    float *d_losses = nullptr;              // per decision
+    float *h_grad = nullptr, *d_grad = nullptr;  // pinned: the two losses, then the gradient
     // inference buffers
     uint8_t *h_stage = nullptr;  // one decision's packed state, pinned and mapped (see infer_kernel)
     float *h_Y = nullptr;        // its scores, written by the kernel into pinned mapped memory
     uint8_t *d_stage = nullptr;  // device views of h_stage and h_Y
     float *d_Y = nullptr;
+    uint32_t infer_seq = 0;         // of the last launch, written behind h_Y's scores
     hipStream_t pending = nullptr;  // stream of the launched inference not yet waited for
     Samples data;
 
     ~Scorer();
     lt_status init(uint32_t P_, const uint32_t *node_off, const uint64_t *edge_off, uint64_t seed);
     lt_status ensure_cap(uint32_t n);
-    lt_status forward_backward(uint32_t nb, bool update, float lr);
+    lt_status forward_backward(uint32_t nb, bool update, float lr, bool grad_out);
+    lt_status wait_infer();
 };
 
 Scorer::~Scorer() {
     if (pending) (void)hipStreamSynchronize(pending);
     if (stream) (void)hipStreamSynchronize(stream);
-    void *ptrs[] = {d_vsh, d_esh, W, G, Mo, Vo, Wb, Wi, d_counts, d_age, d_res, d_recent, d_cur, d_next, d_wtot, d_keep, d_wa,
-                    d_wb, X, A1, A2, Y, dY, dA1, dA2, partial, d_loss};
+    void *ptrs[] = {d_vsh, d_esh, W, G, Mo, Vo, Wb, Wi, d_counts, X, A1, A2, Y, dY, small, w2, d_losses};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    if (h_batch) (void)hipHostFree(h_batch);
+    if (h_grad) (void)hipHostFree(h_grad);
     if (h_stage) (void)hipHostFree(h_stage);
     if (h_Y) (void)hipHostFree(h_Y);
     if (stream) (void)hipStreamDestroy(stream);
@@ -527,8 +770,7 @@ lt_status Scorer::init(uint32_t P_, const uint32_t *node_off, const uint64_t *ed
     MLP_HIP(hipMemcpy(d_vsh, h_vsh.data(), 4 * P, hipMemcpyHostToDevice));
     MLP_HIP(hipMemcpy(d_esh, h_esh.data(), 4 * P, hipMemcpyHostToDevice));
     if ((st = dalloc(&W, kParams)) || (st = dalloc(&G, kParams)) || (st = dalloc(&Mo, kParams)) ||
-        (st = dalloc(&Vo, kParams)) || (st = dalloc(&Wb, kParams)) || (st = dalloc(&Wi, kWiSize)) ||
-        (st = dalloc(&d_loss, 2)))
+        (st = dalloc(&Vo, kParams)) || (st = dalloc(&Wb, kParams)) || (st = dalloc(&Wi, kWiSize)))
         return st;
     // He-style initialisation from a seeded generator; biases zero.
     std::vector<float> w(kParams, 0.f);
@@ -548,64 +790,80 @@ lt_status Scorer::init(uint32_t P_, const uint32_t *node_off, const uint64_t *ed
     MLP_HIP(hipGetLastError());
     wver++;
     MLP_HIP(hipHostMalloc((void **)&h_stage, state_bytes(P), hipHostMallocMapped | hipHostMallocCoherent));
-    MLP_HIP(hipHostMalloc((void **)&h_Y, sizeof(float) * P * kOut, hipHostMallocMapped | hipHostMallocCoherent));
+    const size_t y_bytes = sizeof(float) * P * kOut + 4;  // scores, sequence number
+    MLP_HIP(hipHostMalloc((void **)&h_Y, y_bytes, hipHostMallocMapped | hipHostMallocCoherent));
+    memset(h_Y, 0, y_bytes);
     MLP_HIP(hipHostGetDevicePointer((void **)&d_stage, h_stage, 0));
     MLP_HIP(hipHostGetDevicePointer((void **)&d_Y, h_Y, 0));
     MLP_HIP(hipStreamSynchronize(stream));
     return LT_OK;
 }
 
+// Buffers for batches of n decisions.  The batch's arrays lie one behind the
+// other in pinned memory, which the forward and loss kernels read in place.
 lt_status Scorer::ensure_cap(uint32_t n) {
     if (n <= cap) return LT_OK;
-    void *ptrs[] = {d_counts, d_age, d_res, d_recent, d_cur, d_next, d_wtot, d_keep, d_wa, d_wb, X, A1, A2, Y, dY, dA1, dA2,
-                    partial};
-    for (void *p : ptrs)
-        if (p) (void)hipFree(p);
-    const size_t rows = (size_t)n * P;
+    cap = 0;
+    for (void **p : {(void **)&d_counts, (void **)&X, (void **)&A1, (void **)&A2, (void **)&Y, (void **)&dY, (void **)&small,
+                     (void **)&w2, (void **)&d_losses}) {
+        if (*p) (void)hipFree(*p);
+        *p = nullptr;
+    }
+    if (h_batch) (void)hipHostFree(h_batch);
+    h_batch = nullptr;
+    const size_t rows = (size_t)n * P, tiles = (rows + kTileRows - 1) / kTileRows;
     lt_status st;
-    if ((st = dalloc(&d_counts, rows)) || (st = dalloc(&d_age, rows)) || (st = dalloc(&d_res, rows)) || (st = dalloc(&d_recent, (size_t)n * kRecent)) ||
-        (st = dalloc(&d_cur, n)) || (st = dalloc(&d_next, n)) || (st = dalloc(&d_wtot, n)) ||
-        (st = dalloc(&d_keep, rows)) || (st = dalloc(&d_wa, n)) || (st = dalloc(&d_wb, n)) ||
-        (st = dalloc(&X, rows * kFeat)) || (st = dalloc(&A1, rows * kHidden)) || (st = dalloc(&A2, rows * kHidden)) ||
-        (st = dalloc(&Y, rows * kOut)) || (st = dalloc(&dY, rows * kOut)) || (st = dalloc(&dA1, rows * kHidden)) ||
-        (st = dalloc(&dA2, rows * kHidden)) ||
-        (st = dalloc(&partial, std::max(((rows + kSplitK - 1) / kSplitK) * (size_t)kHidden * kHidden,
-                                         ((rows + 63) / 64) * (size_t)kHidden))))
+    if ((st = dalloc(&d_counts, rows)) || (st = dalloc(&X, rows * kFeat)) || (st = dalloc(&A1, rows * kHidden)) ||
+        (st = dalloc(&A2, rows * kHidden)) || (st = dalloc(&Y, rows * kOut)) || (st = dalloc(&dY, rows * kOut)) ||
+        (st = dalloc(&small, std::min<size_t>(tiles, kGroupMost) * kSmallParams)) ||
+        (st = dalloc(&w2, std::min<size_t>(tiles, kSliceMost) * kHidden * kHidden)) || (st = dalloc(&d_losses, 2 * (size_t)n)))
         return st;
+    const size_t bytes = 13 * rows + (12 + 4 * kRecent + 16) * (size_t)n;
+    MLP_HIP(hipHostMalloc((void **)&h_batch, bytes, hipHostMallocMapped | hipHostMallocCoherent));
+    uint8_t *d = nullptr;
+    MLP_HIP(hipHostGetDevicePointer((void **)&d, h_batch, 0));
+    batch.counts = (const uint32_t *)d;
+    batch.age = batch.counts + rows;
+    batch.keep = (const float *)(batch.age + rows);
+    batch.scale = batch.keep + rows;
+    batch.recent = (const int32_t *)(batch.scale + 3 * (size_t)n);
+    batch.cur = batch.recent + (size_t)n * kRecent;
+    batch.next = batch.cur + n;
+    batch.wa = (const float *)(batch.next + n);
+    batch.wb = batch.wa + n;
+    batch.resident = (const uint8_t *)(batch.wb + n);
+    if (!h_grad) {
+        MLP_HIP(hipHostMalloc((void **)&h_grad, 4 * (2 + kParams), hipHostMallocMapped | hipHostMallocCoherent));
+        MLP_HIP(hipHostGetDevicePointer((void **)&d_grad, h_grad, 0));
+    }
     cap = n;
     return LT_OK;
 }
 
-// Forward + backward over the first nb decisions of the device buffers; G
-// receives the gradient, d_loss the two losses; with update, one Adam step.
-lt_status Scorer::forward_backward(uint32_t nb, bool update, float lr) {
-    const int M = (int)(nb * P);
-    const int H = kHidden;
+// Forward + backward over the nb decisions of the batch; h_grad receives the two
+// losses and, with grad_out, the gradient; with update, one Adam step.
+lt_status Scorer::forward_backward(uint32_t nb, bool update, float lr, bool grad_out) {
+    const uint32_t M = nb * P, tiles = (M + kTileRows - 1) / kTileRows;
+    const uint32_t groups = std::min(tiles, kGroupMost), slices = std::min(tiles, kSliceMost);
     hipStream_t s = stream;
-    MLP_HIP(hipMemsetAsync(d_loss, 0, 8, s));
-    feat_kernel<<<nb, 256, 0, s>>>(P, d_counts, d_res, d_age, d_recent, d_cur, d_wtot, d_vsh, d_esh, X);
-    // forward with the BF16 weights
-    gemm<false, false, uint16_t, EPI_BIAS_RELU>(s, M, H, kFeat, X, kFeat, Wb + kOffW1, H, A1, H, Wb + kOffB1);
-    gemm<false, false, uint16_t, EPI_BIAS_RELU>(s, M, H, H, A1, H, Wb + kOffW2, H, A2, H, Wb + kOffB2);
-    gemm<false, false, uint16_t, EPI_BIAS>(s, M, kOut, H, A2, H, Wb + kOffW3, kOut, Y, kOut, Wb + kOffB3);
-    loss_kernel<<<nb, 256, 0, s>>>(P, nb, Y, d_counts, d_next, d_keep, d_wa, d_wb, dY, d_loss);
-    // backward
-    gemm_wgrad(s, H, kOut, M, A2, H, dY, kOut, G + kOffW3, partial);
-    colsum(s, M, kOut, dY, G + kOffB3, partial);
-    gemm<false, true, uint16_t, EPI_RELU_GRAD>(s, M, H, kOut, dY, kOut, Wb + kOffW3, kOut, dA2, H, nullptr, A2, H);
-    gemm_wgrad(s, H, H, M, A1, H, dA2, H, G + kOffW2, partial);
-    colsum(s, M, H, dA2, G + kOffB2, partial);
-    gemm<false, true, uint16_t, EPI_RELU_GRAD>(s, M, H, H, dA2, H, Wb + kOffW2, H, dA1, H, nullptr, A1, H);
-    gemm_wgrad(s, kFeat, H, M, X, kFeat, dA1, H, G + kOffW1, partial);
-    colsum(s, M, H, dA1, G + kOffB1, partial);
-    MLP_HIP(hipGetLastError());
+    if (wi_ver != wver) {
+        transpose_infer_weights_kernel<<<(unsigned)((kWiSize + 255) / 256), 256, 0, s>>>(Wb, Wi);
+        wi_ver = wver;
+    }
+    train_forward_kernel<<<tiles, 256, 0, s>>>(P, M, batch, d_vsh, d_esh, Wb, Wi, d_counts, X, A1, A2, Y);
+    loss_kernel<<<nb, 256, 0, s>>>(P, nb, Y, d_counts, batch.next, batch.keep, batch.wa, batch.wb, dY, d_losses);
+    train_backward_kernel<<<groups + 4 * slices, 256, 0, s>>>(M, groups, slices, X, A1, A2, dY, Wb, small, w2);
+    float b1t = 0.f, b2t = 0.f;
     if (update) {
         adam_t++;
-        const float b1t = powf(0.9f, (float)adam_t), b2t = powf(0.999f, (float)adam_t);
-        adam_kernel<<<(kParams + 255) / 256, 256, 0, s>>>(kParams, W, Wb, G, Mo, Vo, lr, b1t, b2t);
-        MLP_HIP(hipGetLastError());
-        wver++;
+        b1t = powf(0.9f, (float)adam_t);
+        b2t = powf(0.999f, (float)adam_t);
+        wi_ver = ++wver;  // the update writes Wi as well
     }
+    train_update_kernel<<<(unsigned)((kParams + 31) / 32), 256, 0, s>>>(groups, slices, small, w2, G,
+                                                                       grad_out ? d_grad + 2 : nullptr, W, Wb, Wi, Mo, Vo,
+                                                                       update ? 1 : 0, lr, b1t, b2t, nb, d_losses, d_grad);
+    MLP_HIP(hipGetLastError());
     return LT_OK;
 }
 
@@ -628,10 +886,8 @@ bool scorer_trained(const Scorer *s) { return s && s->trained; }
 // whose kernel may still be reading the staged state.
 lt_status scorer_infer_launch(Scorer *s, const DecisionState &d, void *stream_v) {
     hipStream_t st = stream_v ? (hipStream_t)stream_v : s->stream;
-    if (s->pending) {
-        MLP_HIP(hipStreamSynchronize(s->pending));
-        s->pending = nullptr;
-    }
+    lt_status rc = s->wait_infer();
+    if (rc != LT_OK) return rc;
     const uint32_t P = s->P;
     uint8_t *h = s->h_stage;
     pack_state_head((int32_t *)h, d.counts, P, d.recent, d.cur, d.w_total);
@@ -643,9 +899,31 @@ lt_status scorer_infer_launch(Scorer *s, const DecisionState &d, void *stream_v)
         MLP_HIP(hipGetLastError());
         s->wi_ver = s->wver;
     }
-    infer_kernel<<<(P + 7) / 8, 256, 0, st>>>(P, s->d_stage, s->d_vsh, s->d_esh, s->Wb, s->Wi, s->d_Y);
+    launch_infer(st, P, s->d_stage, s->d_vsh, s->d_esh, s->Wb, s->Wi, s->d_Y);
+    infer_mark_kernel<<<1, 1, 0, st>>>((uint32_t *)(s->d_Y + (size_t)P * kOut), ++s->infer_seq);
     MLP_HIP(hipGetLastError());
     s->pending = st;
+    return LT_OK;
+}
+
+// The last launched inference is over: its sequence number is there.  Polled in
+// memory; the stream itself is asked only once in a while.
+lt_status Scorer::wait_infer() {
+    if (!pending) return LT_OK;
+    const hipStream_t st = pending;
+    pending = nullptr;
+    const uint32_t *flag = (const uint32_t *)(h_Y + (size_t)P * kOut);
+    for (uint32_t it = 1; __atomic_load_n(flag, __ATOMIC_ACQUIRE) != infer_seq; it++) {
+        __builtin_ia32_pause();
+        if ((it & 0xFFFFF) == 0) {
+            const hipError_t e = hipStreamQuery(st);
+            if (e == hipErrorNotReady) continue;
+            MLP_HIP(e);
+            if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == infer_seq) break;
+            set_error("scores were not written");
+            return LT_E_INTERNAL;
+        }
+    }
     return LT_OK;
 }
 
@@ -656,11 +934,8 @@ lt_status scorer_infer_wait(Scorer *s, float *out) {
         set_error("no inference in flight");
         return LT_E_INTERNAL;
     }
-    hipError_t e;
-    while ((e = hipStreamQuery(s->pending)) == hipErrorNotReady) {
-    }
-    s->pending = nullptr;
-    MLP_HIP(e);
+    lt_status st = s->wait_infer();
+    if (st != LT_OK) return st;
     memcpy(out, s->h_Y, sizeof(float) * s->P * kOut);
     return LT_OK;
 }
@@ -724,41 +999,41 @@ struct lt_scorer : lt::Scorer {};
 
 using namespace lt;
 
-static lt_status upload_samples(Scorer *s, uint64_t off, uint32_t nb, const uint32_t *counts, const uint8_t *resident,
-                                const uint32_t *age, const int32_t *recent, const int32_t *cur, const float *w_total,
-                                const int32_t *next_label, const float *keep_label, const float *wa, const float *wb,
-                                const std::vector<uint64_t> *order) {
-    const uint32_t P = s->P;
-    std::vector<uint32_t> c((size_t)nb * P), ag((size_t)nb * P);
-    std::vector<uint8_t> r((size_t)nb * P);
-    std::vector<int32_t> rc((size_t)nb * kRecent), cu(nb), nx(nb);
-    std::vector<float> wt(nb), kp((size_t)nb * P), a(nb), b(nb);
-    for (uint32_t i = 0; i < nb; i++) {
+// Writes decisions off .. off + nb (or order[off ..]) to the pinned batch; the
+// step before, which reads it, is over.
+static void stage_batch(Scorer *s, uint64_t off, uint32_t nb, const uint32_t *counts, const uint8_t *resident,
+                        const uint32_t *age, const int32_t *recent, const int32_t *cur, const float *w_total,
+                        const int32_t *next_label, const float *keep_label, const float *wa, const float *wb,
+                        const std::vector<uint64_t> *order) {
+    const size_t P = s->P;
+    const auto at = [&](const void *p) { return s->h_batch + ((const uint8_t *)p - (const uint8_t *)s->batch.counts); };
+    uint32_t *c = (uint32_t *)at(s->batch.counts), *ag = (uint32_t *)at(s->batch.age);
+    float *kp = (float *)at(s->batch.keep), *sc = (float *)at(s->batch.scale);
+    int32_t *rc = (int32_t *)at(s->batch.recent), *cu = (int32_t *)at(s->batch.cur), *nx = (int32_t *)at(s->batch.next);
+    float *a = (float *)at(s->batch.wa), *b = (float *)at(s->batch.wb);
+    uint8_t *r = at(s->batch.resident);
+    for (size_t i = 0; i < nb; i++) {
         const uint64_t j = order ? (*order)[off + i] : off + i;
-        memcpy(&c[(size_t)i * P], counts + j * P, 4 * (size_t)P);
-        memcpy(&r[(size_t)i * P], resident + j * P, P);
-        memcpy(&ag[(size_t)i * P], age + j * P, 4 * (size_t)P);
-        memcpy(&rc[(size_t)i * kRecent], recent + j * kRecent, 4 * kRecent);
+        memcpy(c + i * P, counts + j * P, 4 * P);
+        memcpy(r + i * P, resident + j * P, P);
+        memcpy(ag + i * P, age + j * P, 4 * P);
+        memcpy(rc + i * kRecent, recent + j * kRecent, 4 * kRecent);
         cu[i] = cur[j];
         nx[i] = next_label[j];
-        wt[i] = w_total[j];
-        if (keep_label) memcpy(&kp[(size_t)i * P], keep_label + j * P, 4 * (size_t)P);
+        uint32_t mx = 0;
+        uint64_t sum = 0;
+        for (size_t q = 0; q < P; q++) {
+            mx = std::max(mx, counts[j * P + q]);
+            sum += counts[j * P + q];
+        }
+        sc[3 * i] = w_total[j];
+        sc[3 * i + 1] = (float)mx;
+        sc[3 * i + 2] = (float)sum;
+        if (keep_label) memcpy(kp + i * P, keep_label + j * P, 4 * P);
+        else memset(kp + i * P, 0, 4 * P);
         a[i] = wa ? wa[j] : 1.f;
         b[i] = (wb && keep_label) ? wb[j] : 0.f;
     }
-    hipStream_t st = s->stream;
-    MLP_HIP(hipMemcpyAsync(s->d_counts, c.data(), 4 * c.size(), hipMemcpyHostToDevice, st));
-    MLP_HIP(hipMemcpyAsync(s->d_res, r.data(), r.size(), hipMemcpyHostToDevice, st));
-    MLP_HIP(hipMemcpyAsync(s->d_age, ag.data(), 4 * ag.size(), hipMemcpyHostToDevice, st));
-    MLP_HIP(hipMemcpyAsync(s->d_recent, rc.data(), 4 * rc.size(), hipMemcpyHostToDevice, st));
-    MLP_HIP(hipMemcpyAsync(s->d_cur, cu.data(), 4 * cu.size(), hipMemcpyHostToDevice, st));
-    MLP_HIP(hipMemcpyAsync(s->d_next, nx.data(), 4 * nx.size(), hipMemcpyHostToDevice, st));
-    MLP_HIP(hipMemcpyAsync(s->d_wtot, wt.data(), 4 * wt.size(), hipMemcpyHostToDevice, st));
-    MLP_HIP(hipMemcpyAsync(s->d_keep, kp.data(), 4 * kp.size(), hipMemcpyHostToDevice, st));
-    MLP_HIP(hipMemcpyAsync(s->d_wa, a.data(), 4 * a.size(), hipMemcpyHostToDevice, st));
-    MLP_HIP(hipMemcpyAsync(s->d_wb, b.data(), 4 * b.size(), hipMemcpyHostToDevice, st));
-    MLP_HIP(hipStreamSynchronize(st));  // the host vectors die at return
-    return LT_OK;
 }
 
 extern "C" {
@@ -791,13 +1066,11 @@ lt_status lt_scorer_loss_grad(lt_scorer *s, uint64_t n, const uint32_t *counts, 
     }
     lt_status st = s->ensure_cap((uint32_t)n);
     if (st != LT_OK) return st;
-    if ((st = upload_samples(s, 0, (uint32_t)n, counts, resident, age, recent, cur, w_total, next_label, keep_label,
-                             wa, wb, nullptr)) != LT_OK)
-        return st;
-    if ((st = s->forward_backward((uint32_t)n, false, 0.f)) != LT_OK) return st;
-    if (loss_out) MLP_HIP(hipMemcpyAsync(loss_out, s->d_loss, 8, hipMemcpyDeviceToHost, s->stream));
-    if (grad_out) MLP_HIP(hipMemcpyAsync(grad_out, s->G, 4 * kParams, hipMemcpyDeviceToHost, s->stream));
+    stage_batch(s, 0, (uint32_t)n, counts, resident, age, recent, cur, w_total, next_label, keep_label, wa, wb, nullptr);
+    if ((st = s->forward_backward((uint32_t)n, false, 0.f, grad_out != nullptr)) != LT_OK) return st;
     MLP_HIP(hipStreamSynchronize(s->stream));
+    if (loss_out) memcpy(loss_out, s->h_grad, 8);
+    if (grad_out) memcpy(grad_out, s->h_grad + 2, 4 * kParams);
     return LT_OK;
 }
 
@@ -819,13 +1092,10 @@ lt_status lt_scorer_train(lt_scorer *s, uint64_t n, const uint32_t *counts, cons
         double acc[2] = {0, 0};
         uint32_t steps = 0;
         for (uint64_t off = 0; off + batch <= n; off += batch) {
-            if ((st = upload_samples(s, off, batch, counts, resident, age, recent, cur, w_total, next_label,
-                                     keep_label, wa, wb, &order)) != LT_OK)
-                return st;
-            if ((st = s->forward_backward(batch, true, lr)) != LT_OK) return st;
-            float l[2];
-            MLP_HIP(hipMemcpyAsync(l, s->d_loss, 8, hipMemcpyDeviceToHost, s->stream));
+            stage_batch(s, off, batch, counts, resident, age, recent, cur, w_total, next_label, keep_label, wa, wb, &order);
+            if ((st = s->forward_backward(batch, true, lr, false)) != LT_OK) return st;
             MLP_HIP(hipStreamSynchronize(s->stream));
+            const float *l = s->h_grad;
             acc[0] += l[0];
             acc[1] += l[1];
             steps++;
@@ -894,7 +1164,7 @@ lt_status lt_scorer_infer_noalloc(lt_scorer *s, const uint32_t *counts, const ui
             nd->wi_ver = s->wver;
         }
     }
-    infer_kernel<<<(P + 7) / 8, 256, 0, st>>>(P, state, s->d_vsh, s->d_esh, s->Wb, (const uint16_t *)Wi, (float *)Y);
+    launch_infer(st, P, state, s->d_vsh, s->d_esh, s->Wb, (const uint16_t *)Wi, (float *)Y);
     MLP_HIP(hipGetLastError());
     MLP_HIP(hipMemcpyAsync(out, Y, sizeof(float) * P * kOut, hipMemcpyDeviceToHost, st));
     MLP_HIP(hipStreamSynchronize(st));
