@@ -146,15 +146,18 @@ struct BlockImages {
 
 struct WalkArgs {
     AppArgs app;
-    SchedState ss;
     Queues q;
     Parts pt;
-    uint32_t src;         // partition whose queue is consumed
-    uint32_t chunk_lo;    // first chunk of the slice
-    uint32_t chunk_hi;    // one past the last chunk of the slice
     const uint64_t *rowptr;  // rowptr slice of src (HBM slot or mapped host)
     const uint32_t *col;     // col slice of src (block headers if words is set)
     const uint32_t *words;   // bit streams of src's packed slot, nullptr for raw columns
+    unsigned long long *stats;
+    uint64_t eb;          // src's first edge
+    uint32_t src;         // partition whose queue is consumed
+    uint32_t nb, ne;      // its first vertex, and the one past its last
+    uint32_t n;           // walkers in its queue
+    uint32_t chunk_lo;    // first chunk of the slice
+    uint32_t chunk_hi;    // one past the last chunk of the slice
     int zerocopy;         // src slice is read over PCIe
     int span_resident;    // keep walking through HBM-resident partitions
     // How a pass appends its leaving walkers to their queues: 0, one queue
@@ -164,7 +167,6 @@ struct WalkArgs {
     // build, src/WalkManager.h:98-118); 2, one reservation per walker (its
     // ONE_LEVEL_QUEUE build, src/WalkManager.h:195-209).
     int append_mode;
-    unsigned long long *stats;
     // Batch (span_resident only): nsrc > 0 consumes the whole queues of
     // srcs[0..nsrc), each entered in the partition table for the launch
     // (resident slots, or views of the pinned host graph for a zero-copy
@@ -172,12 +174,13 @@ struct WalkArgs {
     // being consumed is appended to.  Queue k occupies [voff[k], voff[k+1])
     // of one virtual range, each start a multiple of kChunk.
     uint32_t nsrc;
-    uint32_t srcs[kMaxZcBatch];
-    uint64_t voff[kMaxZcBatch + 1];
     // Spilled walkers (nhost > 0): walkers of src kept in pinned host memory,
     // read by the kernel over PCIe; piece k holds hn[k] <= kChunk walkers at
     // hptr[k] and occupies [k * kChunk, k * kChunk + hn[k]) of the range.
     uint32_t nhost;
+    SchedState ss;        // device-scheduled loop: ss.ds != nullptr names the source
+    uint32_t srcs[kMaxZcBatch];
+    uint64_t voff[kMaxZcBatch + 1];
     const Walker *hptr[kMaxHostPieces];
     uint32_t hn[kMaxHostPieces];
 };

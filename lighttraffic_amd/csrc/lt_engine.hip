@@ -1106,6 +1106,10 @@ lt_status Engine::process(uint32_t p, bool zerocopy, uint64_t walkers) {
     a.pt.lut_shift = lut_shift;
     a.pt.P = P;
     a.src = p;
+    a.nb = part.node_off[p];
+    a.ne = part.node_off[p + 1];
+    a.eb = part.edge_off[p];
+    a.n = (uint32_t)walkers;
     a.zerocopy = zerocopy ? 1 : 0;
     a.span_resident = cfg.span == LT_SPAN_RESIDENT ? 1 : 0;
     a.stats = d_stats;

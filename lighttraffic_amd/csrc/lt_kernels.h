@@ -121,6 +121,20 @@ __device__ __forceinline__ AppendLds carve_lds(uint8_t *smem, uint32_t P, int wp
     return L;
 }
 
+// Inclusive prefix sum over the 64 lanes of a wave with DPP moves: shifts by
+// 1, 2, 4 and 8 within each row of 16 lanes (lanes shifted in from outside
+// the row read 0), then row 0's total is added to row 1 and row 2's to row 3
+// (row_bcast:15), then lane 31's sum to rows 2 and 3 (row_bcast:31).
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true);  // row_shr:1
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true);  // row_shr:2
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true);  // row_shr:4
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true);  // row_shr:8
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false); // row_bcast:15, rows 1, 3
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false); // row_bcast:31, rows 2, 3
+    return x;
+}
+
 // Exclusive scan of in[0..n) into out[], returns the total (all threads).
 __device__ uint32_t block_exclusive_scan(const uint32_t *in, uint32_t *out, uint32_t n, uint32_t *s_wsum) {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
@@ -128,12 +142,7 @@ __device__ uint32_t block_exclusive_scan(const uint32_t *in, uint32_t *out, uint
     const uint32_t beg = min(tid * per, n), end = min(beg + per, n);
     uint32_t sum = 0;
     for (uint32_t i = beg; i < end; i++) sum += in[i];
-    uint32_t x = sum;
-#pragma unroll
-    for (uint32_t off = 1; off < 64; off <<= 1) {
-        const uint32_t y = __shfl_up(x, off, 64);
-        if (lane >= off) x += y;
-    }
+    const uint32_t x = wave_incl_scan(sum);
     if (lane == 63) s_wsum[wave] = x;
     __syncthreads();
     uint32_t before = 0, total = 0;
@@ -292,9 +301,26 @@ __device__ void block_append_hashed(const Queues &q, const AppendLds &L, const W
 // before that link is published links it itself (the CAS loser's chunk goes
 // to the lost list).  Above kDirectMaxP partitions the slots are numbered
 // through a hash table (block_append_hashed).
+//
+// hint: the chunk that held the end of partition threadIdx.x's queue when this
+// thread last looked; a linked chunk stays linked for the launch, so one that
+// is still the end's needs no lookup.
+struct AppendHint {
+    uint32_t k = kEmpty, c = kEmpty;  // chunk number in the queue, chunk id
+};
+
+// First look, while the first walkers walk.  Only for launches of at most a
+// workgroup per CU: those wait for every round trip, while in larger ones the
+// lines, which every append writes, are better left alone.
+__device__ __forceinline__ void first_hint(const Queues &q, uint32_t P, int mode, AppendHint &h) {
+    if (gridDim.x > 256 || P > kDirectMaxP || mode == 2 || threadIdx.x >= P) return;
+    h.k = load_agent(&qlen_of(q, threadIdx.x)) >> kChunkLog2;
+    if (h.k < q.maxc) h.c = load_agent(&q.frame[(size_t)threadIdx.x * q.maxc + h.k]);
+}
+
 template <int WPT>
 __device__ void block_append(const Queues &q, uint32_t P, const AppendLds &L, const Walker (&w)[WPT],
-                             const uint32_t (&dst)[WPT], uint32_t *s_wsum, int mode = 0) {
+                             const uint32_t (&dst)[WPT], uint32_t *s_wsum, AppendHint &hint, int mode = 0) {
     if (mode == 2) {  // uniform
         append_one_level<WPT>(q, w, dst);
         return;
@@ -330,11 +356,17 @@ __device__ void block_append(const Queues &q, uint32_t P, const AppendLds &L, co
     }
     for (uint32_t i = tid; i < P; i += kBlock) {
         const uint32_t b = L.hist[i];
-        if (L.scan[i + 1] != L.scan[i] && (b & (kChunk - 1)) != 0) {
-            const uint32_t c0 = get_chunk(q, i, b >> kChunkLog2);
-            const uint32_t k1 = (b + (L.scan[i + 1] - L.scan[i]) - 1) >> kChunkLog2;
-            L.ch0[i] = c0;
-            if (k1 == (b >> kChunkLog2)) L.ch1[i] = c0;
+        if (L.scan[i + 1] != L.scan[i]) {
+            const uint32_t k0 = b >> kChunkLog2, k1 = (b + (L.scan[i + 1] - L.scan[i]) - 1) >> kChunkLog2;
+            if ((b & (kChunk - 1)) != 0) {
+                const uint32_t c0 = i == tid && k0 == hint.k && hint.c != kEmpty ? hint.c : get_chunk(q, i, k0);
+                L.ch0[i] = c0;
+                if (k1 == k0) L.ch1[i] = c0;
+            }
+            if (i == tid) {
+                hint.k = k1;
+                hint.c = L.ch1[i];
+            }
         }
     }
     __syncthreads();
@@ -371,6 +403,14 @@ struct Counters {
     uint32_t *vbuf = nullptr, *vn = nullptr;  // workgroup visit buffer in LDS and its fill (walk kernels)
 };
 
+// Sum over the 64 lanes, in lane 63: 16 bits at a time, so that no 32-bit
+// sum wraps.  (DPP moves: the six counters took 2 us of each launch's end by
+// 64-bit shuffles.)
+__device__ __forceinline__ unsigned long long wave_sum(uint32_t v) {
+    const uint32_t lo = wave_incl_scan(v & 0xFFFFu), hi = wave_incl_scan(v >> 16);
+    return (unsigned long long)lo + ((unsigned long long)hi << 16);
+}
+
 // Workgroup sum of the counters, added to slot blockIdx.x % kStatSlots, so
 // that workgroups of one launch do not all update one cache line.
 __device__ void flush_counters(const Counters &c, unsigned long long *stats) {
@@ -379,10 +419,8 @@ __device__ void flush_counters(const Counters &c, unsigned long long *stats) {
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int i = 0; i < 6; i++) {
-        unsigned long long x = v[i];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-        if (lane == 0) s_part[wave][i] = x;
+        const unsigned long long x = wave_sum(v[i]);
+        if (lane == 63) s_part[wave][i] = x;
     }
     __syncthreads();
     if (threadIdx.x < 6) {
@@ -587,7 +625,8 @@ __device__ uint32_t walk_residency(Walker &w, const WalkArgs &a, uint32_t src, c
 // contiguously at cw: walk each, then append the survivors to their queues.
 template <int APP, int WPT>
 __device__ __forceinline__ void walk_walkers(const WalkArgs &a, const AppendLds &L, uint32_t *s_wsum, uint32_t src,
-                                            const Span &src_sp, const Walker *cw, uint32_t nvalid, Counters &ct) {
+                                            const Span &src_sp, const Walker *cw, uint32_t nvalid, Counters &ct,
+                                            AppendHint &hint) {
     Walker w[WPT];
     uint32_t dst[WPT];
 #pragma unroll
@@ -614,7 +653,7 @@ __device__ __forceinline__ void walk_walkers(const WalkArgs &a, const AppendLds 
             const uint32_t n = min(*ct.vn, kVisitBuf);
             uint32_t at = 0;
             if (threadIdx.x == kBlock - 1 && n) at = log_reserve(a.app, n);
-            block_append<WPT>(a.q, a.pt.P, L, w, dst, s_wsum, a.append_mode);
+            block_append<WPT>(a.q, a.pt.P, L, w, dst, s_wsum, hint, a.append_mode);
             if (threadIdx.x == kBlock - 1) {
                 s_at = at;
                 *ct.vn = 0;
@@ -625,7 +664,7 @@ __device__ __forceinline__ void walk_walkers(const WalkArgs &a, const AppendLds 
             return;
         }
     }
-    block_append<WPT>(a.q, a.pt.P, L, w, dst, s_wsum, a.append_mode);
+    block_append<WPT>(a.q, a.pt.P, L, w, dst, s_wsum, hint, a.append_mode);
 }
 
 // One workgroup pass: walkers [base, base + kBlock * WPT) of src's queue,
@@ -633,14 +672,15 @@ __device__ __forceinline__ void walk_walkers(const WalkArgs &a, const AppendLds 
 // chunk.
 template <int APP, int WPT>
 __device__ __forceinline__ void walk_pass(const WalkArgs &a, const AppendLds &L, uint32_t *s_wsum, uint32_t src,
-                                          const Span &src_sp, uint64_t base, uint64_t hi64, Counters &ct) {
+                                          const Span &src_sp, uint64_t base, uint64_t hi64, Counters &ct,
+                                          AppendHint &hint) {
     const uint32_t chunk = a.q.frame[(size_t)src * a.q.maxc + (uint32_t)(base >> kChunkLog2)];
     const bool chunk_ok = chunk < a.q.nchunks;
     if (!chunk_ok && threadIdx.x == 0) atomicOr(&a.q.ctl->overflow, 8u);
     const Walker *cw = a.q.slab + (size_t)(chunk_ok ? chunk : 0) * kChunk + (uint32_t)(base & (kChunk - 1));
     const uint64_t left = hi64 > base ? hi64 - base : 0;
     const uint32_t nvalid = chunk_ok ? (uint32_t)min(left, (uint64_t)(kBlock * WPT)) : 0u;
-    walk_walkers<APP, WPT>(a, L, s_wsum, src, src_sp, cw, nvalid, ct);
+    walk_walkers<APP, WPT>(a, L, s_wsum, src, src_sp, cw, nvalid, ct, hint);
 }
 
 // WPT walkers per thread per pass (1, 2 or 4): small queues use 1 so that
@@ -650,6 +690,11 @@ __global__ __launch_bounds__(kBlock) void walk_kernel(WalkArgs a) {
     constexpr int BW = kBlock * WPT;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     __shared__ uint32_t s_wsum[kBlock / 64];
+    // The arguments lie in memory: asked for one line at a time as the code gets
+    // to them, each costs a small launch a round trip of its own.
+    asm volatile("" ::"s"(a.app.seed), "s"(a.app.counts), "s"(a.app.vcur), "s"(a.app.rp_host), "s"(a.q.slab),
+                 "s"(a.q.ctl), "s"(a.q.maxc), "s"(a.pt.node_off), "s"(a.pt.lut_shift), "s"(a.rowptr), "s"(a.src),
+                 "s"(a.nhost), "s"(a.ss.ds));
     const AppendLds L = carve_lds(smem, a.pt.P, WPT);
     Counters ct;
     if constexpr (APP != APP_GENERIC) {
@@ -661,6 +706,8 @@ __global__ __launch_bounds__(kBlock) void walk_kernel(WalkArgs a) {
             ct.vn = &s_vn;
         }
     }
+    AppendHint hint;
+    first_hint(a.q, a.pt.P, a.append_mode, hint);
     if (a.nsrc) {  // batch: the whole queues of several partitions, each in the partition table
         const uint64_t vend = a.voff[a.nsrc];
         for (uint64_t base = (uint64_t)blockIdx.x * BW; base < vend; base += (uint64_t)gridDim.x * BW) {
@@ -676,27 +723,27 @@ __global__ __launch_bounds__(kBlock) void walk_kernel(WalkArgs a) {
             sp.eb = a.pt.edge_off[src];
             sp.zc = a.pt.zc_part[src];
             const uint64_t local = base - a.voff[k], n = qlen_of(a.q, src);
-            if (local < n) walk_pass<APP, WPT>(a, L, s_wsum, src, sp, local, n, ct);  // uniform per workgroup
+            if (local < n) walk_pass<APP, WPT>(a, L, s_wsum, src, sp, local, n, ct, hint);  // uniform per workgroup
         }
         flush_counters(ct, a.stats);
         return;
     }
-    uint32_t src = a.src, chunk_lo = a.chunk_lo, chunk_hi = a.chunk_hi;
+    uint32_t src = a.src, chunk_lo = a.chunk_lo, chunk_hi = a.chunk_hi, n = a.n;
     Span src_sp;
     src_sp.rowptr = a.rowptr;
     src_sp.col = a.col;
     src_sp.words = a.words;
     src_sp.zc = a.zerocopy;
+    src_sp.nb = a.nb;
+    src_sp.ne = a.ne;
+    src_sp.eb = a.eb;
     if (a.nhost) {  // walkers of src spilled to host memory, read over PCIe
-        src_sp.nb = a.pt.node_off[src];
-        src_sp.ne = a.pt.node_off[src + 1];
-        src_sp.eb = a.pt.edge_off[src];
         const uint64_t vend = (uint64_t)a.nhost << kChunkLog2;
         for (uint64_t base = (uint64_t)blockIdx.x * BW; base < vend; base += (uint64_t)gridDim.x * BW) {
             const uint32_t k = (uint32_t)(base >> kChunkLog2), local = (uint32_t)(base & (kChunk - 1));
             if (local < a.hn[k])  // uniform per workgroup
                 walk_walkers<APP, WPT>(a, L, s_wsum, src, src_sp, a.hptr[k] + local,
-                                       min(a.hn[k] - local, (uint32_t)BW), ct);
+                                       min(a.hn[k] - local, (uint32_t)BW), ct, hint);
         }
         flush_counters(ct, a.stats);
         return;
@@ -707,6 +754,10 @@ __global__ __launch_bounds__(kBlock) void walk_kernel(WalkArgs a) {
         src = (uint32_t)c;
         chunk_lo = 0;
         chunk_hi = 0xFFFFFFFFu;
+        n = qlen_of(a.q, src);
+        src_sp.nb = a.pt.node_off[src];
+        src_sp.ne = a.pt.node_off[src + 1];
+        src_sp.eb = a.pt.edge_off[src];
         src_sp.zc = a.ss.ds->zerocopy;
         src_sp.words = nullptr;
         if (src_sp.zc) {
@@ -719,14 +770,10 @@ __global__ __launch_bounds__(kBlock) void walk_kernel(WalkArgs a) {
             src_sp.words = a.pt.words_tab[src];
         }
     }
-    const uint32_t n = qlen_of(a.q, src);
     const uint64_t lo64 = (uint64_t)chunk_lo << kChunkLog2;
     const uint64_t hi64 = min((uint64_t)n, (uint64_t)chunk_hi << kChunkLog2);
-    src_sp.nb = a.pt.node_off[src];
-    src_sp.ne = a.pt.node_off[src + 1];
-    src_sp.eb = a.pt.edge_off[src];
     for (uint64_t base = lo64 + (uint64_t)blockIdx.x * BW; base < hi64; base += (uint64_t)gridDim.x * BW)
-        walk_pass<APP, WPT>(a, L, s_wsum, src, src_sp, base, hi64, ct);
+        walk_pass<APP, WPT>(a, L, s_wsum, src, src_sp, base, hi64, ct, hint);
     flush_counters(ct, a.stats);
 }
 
@@ -753,6 +800,7 @@ __global__ __launch_bounds__(kBlock) void init_kernel(InitArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     __shared__ uint32_t s_wsum[kBlock / 64];
     const AppendLds L = carve_lds(smem, a.pt.P, kWpt);
+    AppendHint hint;
     for (uint64_t base = a.id_lo + (uint64_t)blockIdx.x * kBlockWalkers; base < a.id_hi;
          base += (uint64_t)gridDim.x * kBlockWalkers) {
         Walker w[kWpt];
@@ -794,7 +842,7 @@ __global__ __launch_bounds__(kBlock) void init_kernel(InitArgs a) {
                 finish_walker(w[k], a.app);
             }
         }
-        block_append<kWpt>(a.q, a.pt.P, L, w, dst, s_wsum);
+        block_append<kWpt>(a.q, a.pt.P, L, w, dst, s_wsum, hint);
     }
 }
 
@@ -1128,20 +1176,6 @@ __global__ __launch_bounds__(256) void load_kernel(SchedState ss, Parts pt, Bloc
 //   - the 64 columns of a chunk are stored by consecutive lanes.
 constexpr uint32_t kUnpackChunks = 8;
 
-// Inclusive prefix sum over the 64 lanes of a wave with DPP moves: shifts by
-// 1, 2, 4 and 8 within each row of 16 lanes (lanes shifted in from outside
-// the row read 0), then row 0's total is added to row 1 and row 2's to row 3
-// (row_bcast:15), then lane 31's sum to rows 2 and 3 (row_bcast:31).
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x, uint32_t) {
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true);  // row_shr:1
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true);  // row_shr:2
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true);  // row_shr:4
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true);  // row_shr:8
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false); // row_bcast:15, rows 1, 3
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false); // row_bcast:31, rows 2, 3
-    return x;
-}
-
 __global__ __launch_bounds__(256) void unpack_kernel(const uint8_t *__restrict__ img, uint32_t n, uint64_t m,
                                                      uint64_t nwords, uint32_t vbits,
                                                      const uint64_t *__restrict__ rowptr,
@@ -1197,14 +1231,14 @@ __global__ __launch_bounds__(256) void unpack_kernel(const uint8_t *__restrict__
         const bool valid = lane < cnt;
         const bool anchor = valid && (lane == 0 || starts[lane] || bw == 0xFFu);
         const uint32_t len = valid ? (anchor ? vbits : bw) : 0u;
-        const uint32_t pos = wave_incl_scan(len, lane) - len;
+        const uint32_t pos = wave_incl_scan(len) - len;
         const uint32_t wi = pos >> 5;
         const uint32_t lo_w = __shfl(word, wi, 64);
         const uint32_t hi_w = __shfl(word, (wi + 1) & 63u, 64);
         // bits [pos, pos + len) of the chunk: (hi:lo) >> (pos % 32), low len bits
         const uint32_t bits = __builtin_amdgcn_alignbit(wi + 1 < 64 ? hi_w : 0u, lo_w, pos & 31u);
         const uint32_t v = len >= 32 ? bits : bits & ((1u << len) - 1u);
-        const uint32_t incl = wave_incl_scan(v, lane);
+        const uint32_t incl = wave_incl_scan(v);
         const uint64_t heads = __ballot(anchor) & (lane == 63 ? ~0ull : ((2ull << lane) - 1));
         const uint32_t head = 63u - (uint32_t)__clzll(heads);  // lane 0 is always a head
         const uint32_t before = __shfl(incl, head > 0 ? head - 1 : 0, 64);
