@@ -115,19 +115,11 @@ struct EventTimer {
     }
 };
 
-// Waits for prefetch copies poll their events: a blocking wait adds its
-// wake-up latency to a decision.
-static hipError_t spin_event(hipEvent_t ev) {
-    hipError_t e;
-    while ((e = hipEventQuery(ev)) == hipErrorNotReady) {
-    }
-    return e;
-}
-
 // h_out: kNumStats u64 of event counters, the job's time in ticks of the
-// device's wall clock, the sequence number, those of the ring's buffers, then small
-// results.
-constexpr uint32_t kOutTicks = 2 * kNumStats, kOutFlag = kOutTicks + 1, kOutRing = kOutFlag + 1, kOutData = 64;
+// device's wall clock, the sequence number, those of the ring's buffers, that of the
+// last load finished, then small results.
+constexpr uint32_t kOutTicks = 2 * kNumStats, kOutFlag = kOutTicks + 1, kOutRing = kOutFlag + 1, kOutCopy = 32,
+                   kOutData = 64;
 constexpr uint64_t kManyOut = 1u << 20;  // words: from here on threads help with the results
 
 struct RunSpec {
@@ -289,13 +281,12 @@ struct Engine {
     uint8_t *d_zc_part = nullptr;  // [P] partitions of the running zero-copy batch
     bool rp_resident = false;      // rowptr of the whole graph kept in HBM (zc_rowptr points there)
     uint64_t *d_pk_off = nullptr, *d_pk_size = nullptr;  // device loop with block slots: image table
-    const uint8_t *d_pk_img = nullptr;                     // device view of the pinned images
+    const uint8_t *d_pk_img = nullptr;                     // device view of the pinned images (block slots)
     uint64_t *d_rowptr_all = nullptr;
     uint64_t pending_h2d = 0;      // one-off H2D bytes not yet charged to a run
     uint32_t zc_batch = 1;         // partitions per zero-copy launch
     uint32_t res_batch = 1;        // partitions per launch over resident queues
     uint32_t slice = kSliceChunks;
-    std::vector<hipEvent_t> pool_events;  // reusable prefetch-completion events
     std::vector<float> scores;            // scorer output of the current decision
     bool scores_valid = false;
     uint64_t scores_clock = 0;            // use_clock when the scores were computed
@@ -313,15 +304,17 @@ struct Engine {
 
     // scheduler primitives
     lt_status read_meta();
-    lt_status take_event(hipEvent_t &ev) {
-        if (!pool_events.empty()) {
-            ev = pool_events.back();
-            pool_events.pop_back();
-            return LT_OK;
-        }
-        LT_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-        return LT_OK;
-    }
+    // A load on its way.  Loads finish in order; h_out holds the number of the
+    // last one that a kernel made.
+    struct Load {
+        bool pulled = false;     // by pull_kernel: seq is written when it is over
+        uint32_t seq = 0;
+        hipEvent_t ev = nullptr; // by DMA, with others behind it; else the copy stream itself is asked
+    };
+    uint32_t copy_seq = 0;
+    std::vector<hipEvent_t> pool_events;  // reusable
+    bool loaded(const Load &l) const;
+    lt_status wait_loaded(Load &l);
     bool meta_dirty = true;  // q.packed may be older than the queues
     uint32_t meta_seq = 0;   // of the last launch that writes q.packed
     bool meta_seen = true;   // h_meta holds what that launch wrote
@@ -336,8 +329,21 @@ struct Engine {
     lt_status process_resident(uint32_t c, int kind, uint8_t *prefetched);
     void record(uint32_t p, int kind, int32_t loaded, int32_t evicted);
     lt_status evict(uint32_t p);
-    lt_status load_async(uint32_t p);
+    lt_status load_async(uint32_t p, bool ahead, Load &l);
     lt_status copy_partition(uint32_t p, uint64_t *rp, uint32_t *cp);
+    // Small slices are copied by one kernel instead of two DMAs, whose second
+    // costs 10 us of its own (256 KB: 14 us, 22 by DMAs; 1 MB: 28 and 38).  Larger
+    // ones hold the walk up: beside a kernel that reads the link for 50 to 80
+    // us its launches took twice as long (s23, 4 MB slots: 14.0 ms a job by DMAs, 17.6
+    // so; s20 reference rules, 2 MB: 24.4 and 28.7; s20 ppr, 1 MB: 27.8 and 25.7).
+    static constexpr size_t kPullBytes = 1280u << 10;
+    static constexpr int kPullGrid = 64;
+    bool pulls(uint32_t p) const {
+        const bool packed = pk && pk->size[p];
+        if (packed && !slot_packed) return false;
+        const size_t rbytes = ((size_t)part.node_off[p + 1] - part.node_off[p] + 1) * 8;
+        return rbytes + (packed ? pk->size[p] : (part.edge_off[p + 1] - part.edge_off[p]) * 4) <= kPullBytes;
+    }
     lt_status fetch_partition(uint32_t p, uint64_t *rowptr_out, uint32_t *col_out);
     // Bit streams of p's slot whose column part starts at cp: past the block
     // headers when the slot holds p's block image, nullptr for raw columns.
@@ -620,8 +626,8 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
         LT_TRY(dmalloc(&d_pk_size, P));
         LT_HIP(hipMemcpy(d_pk_off, off.data(), 8 * (size_t)P, hipMemcpyHostToDevice));
         LT_HIP(hipMemcpy(d_pk_size, size.data(), 8 * (size_t)P, hipMemcpyHostToDevice));
-        LT_HIP(hipHostGetDevicePointer((void **)&d_pk_img, pk->host, 0));
     }
+    if (slot_packed) LT_HIP(hipHostGetDevicePointer((void **)&d_pk_img, pk->host, 0));
     if (rp_resident) {
         LT_TRY(dmalloc(&d_rowptr_all, (size_t)V + 1));
         LT_HIP(hipMemcpy(d_rowptr_all, g->rowptr, rp_bytes, hipMemcpyHostToDevice));
@@ -935,10 +941,35 @@ lt_status Engine::evict(uint32_t p) {
     return LT_OK;
 }
 
+bool Engine::loaded(const Load &l) const {
+    if (l.pulled) return (int32_t)(__atomic_load_n(h_out + kOutCopy, __ATOMIC_ACQUIRE) - l.seq) >= 0;
+    return (l.ev ? hipEventQuery(l.ev) : hipStreamQuery(s_copy)) != hipErrorNotReady;
+}
+
+// Polls: a blocking wait adds its wake-up latency to a decision.
+lt_status Engine::wait_loaded(Load &l) {
+    for (uint32_t it = 1; !loaded(l); it++) {
+        __builtin_ia32_pause();
+        if (l.pulled && (it & 0xFFFFF) == 0) {
+            const hipError_t e = hipStreamQuery(s_copy);
+            if (e == hipErrorNotReady) continue;
+            LT_HIP(e);
+            if (loaded(l)) break;
+            set_error("a partition copy did not finish");
+            return LT_E_INTERNAL;
+        }
+    }
+    if (!l.pulled) LT_HIP(l.ev ? hipEventQuery(l.ev) : hipStreamQuery(s_copy));
+    if (l.ev) pool_events.push_back(l.ev);
+    l.ev = nullptr;
+    return LT_OK;
+}
+
 // GPUGraph::loadAsync (src/GraphLoader.h:193-215): rowptr slice at slot offset
 // 0, col slice right after it, both on the copy stream.  The compute stream
-// must not be reading the slot (the caller evicted it after a sync).
-lt_status Engine::load_async(uint32_t p) {
+// must not be reading the slot (the caller evicted it after a sync).  ahead: other
+// loads may follow before this one is waited for.
+lt_status Engine::load_async(uint32_t p, bool ahead, Load &l) {
     if (free_slots.empty()) {
         set_error("no free cache slot for partition %u", p);
         return LT_E_INTERNAL;
@@ -952,6 +983,21 @@ lt_status Engine::load_async(uint32_t p) {
     uint32_t *cp;
     slot_ptrs(p, &rp, &cp);
     LT_TRY(copy_partition(p, rp, cp));
+    l = Load{};
+    l.pulled = pulls(p);
+    if (l.pulled) {  // (behind a DMA such a kernel starts 10 us late)
+        l.seq = ++copy_seq;
+        mark_kernel<<<1, 1, 0, s_copy>>>(d_out + kOutCopy, l.seq);
+        LT_HIP(hipGetLastError());
+    } else if (ahead) {
+        if (pool_events.empty()) {
+            LT_HIP(hipEventCreateWithFlags(&l.ev, hipEventDisableTiming));
+        } else {
+            l.ev = pool_events.back();
+            pool_events.pop_back();
+        }
+        LT_HIP(hipEventRecord(l.ev, s_copy));
+    }
     t_load.end(t, s_copy);
     return LT_OK;
 }
@@ -968,6 +1014,27 @@ lt_status Engine::copy_partition(uint32_t p, uint64_t *rp, uint32_t *cp) {
     const size_t rbytes = ((size_t)ne - nb + 1) * 8, cbytes = (size_t)(ee - eb) * 4;
     const bool packed = pk && pk->size[p];
     uint32_t k = 0;
+    if (pulls(p)) {
+        const size_t body = packed ? pk->size[p] : cbytes;
+        PullArgs a{};
+        const uint32_t *col = zc_col + eb;
+        if (packed) col = (const uint32_t *)(d_pk_img + pk->off[p]);
+        a.src[0] = (const uint32_t *)(zc_rowptr + nb);
+        a.src[1] = col;
+        a.dst[0] = (uint32_t *)rp;
+        a.dst[1] = cp;
+        a.words[0] = rbytes / 4;
+        a.words[1] = body / 4;
+        pull_kernel<<<kPullGrid, 256, 0, s_copy>>>(a);
+        LT_HIP(hipGetLastError());
+        st.h2d_bytes_explicit += body + (rp_resident ? 0 : rbytes);
+        st.h2d_bytes_unpacked += cbytes + (rp_resident ? 0 : rbytes);
+        if (packed) {
+            st.packed_image_bytes += body;
+            st.packed_col_bytes += cbytes;
+        }
+        return LT_OK;
+    }
     if (packed && slot_packed) {  // the block image is the slot's column part
         if (rp_resident) {
             LT_HIP(hipMemcpyAsync(rp, d_rowptr_all + nb, rbytes, hipMemcpyDeviceToDevice, s_copy));
@@ -1073,8 +1140,9 @@ lt_status Engine::launch_walk(const WalkArgs &a, uint64_t walkers, hipStream_t s
                     : walkers >= 2 * fill         ? 2
                                                   : 1;
     const uint64_t bw = (uint64_t)kBlock * wpt;
-    const int grid =
-        (int)std::max<uint64_t>(1, std::min<uint64_t>((walkers + bw - 1) / bw, (uint64_t)walk_grid[app_kind][wpt]));
+    // with loads going on, room for a pull kernel's workgroups beside the walk's
+    const uint64_t most = walk_grid[app_kind][wpt] - (nslots < P && walk_grid[app_kind][wpt] > kPullGrid ? kPullGrid : 0);
+    const int grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((walkers + bw - 1) / bw, most));
     switch (app_kind) {
         case APP_PAGERANK: launch_walk_app<APP_PAGERANK>(a, wpt, grid, lds_bytes(wpt), s); break;
         case APP_PPR: launch_walk_app<APP_PPR>(a, wpt, grid, lds_bytes(wpt), s); break;
@@ -1592,12 +1660,13 @@ lt_status Engine::run_partition(uint32_t p, int32_t &prev_loaded) {
             evicted = victim;
         }
         record(p, 3, (int32_t)p, evicted);
-        LT_TRY(load_async(p));
+        Load load;
+        LT_TRY(load_async(p, false, load));
         st.graph_loading_calls++;
         sched.on_load(p);
         if (cfg.pipeline) {
             // compute resident partitions while the copy is in flight
-            while (hipStreamQuery(s_copy) == hipErrorNotReady) {
+            while (!loaded(load)) {
                 LT_TRY(read_meta());
                 const int32_t c = sched.computed_choice(counts.data(), resident.data(), (int32_t)p, kRefPage);
                 if (c < 0) break;
@@ -1609,7 +1678,7 @@ lt_status Engine::run_partition(uint32_t p, int32_t &prev_loaded) {
             // the pipelined work changed the queues; p's count is re-read below
             LT_TRY(read_meta());
         }
-        LT_HIP(hipStreamSynchronize(s_copy));
+        LT_TRY(wait_loaded(load));
         resident[p] = 1;
         LT_TRY(set_table(p, true));
     } else {
@@ -1655,7 +1724,7 @@ lt_status Engine::scheduler_loop_learned() {
     bool sync = false;
     struct Inflight {
         int32_t part;
-        hipEvent_t done;
+        Load load;
     };
     std::vector<Inflight> inflight;         // prefetch copies in copy-stream order
     std::vector<uint8_t> prefetched(P, 0);  // resident because of a prefetch, not yet picked
@@ -1674,11 +1743,9 @@ lt_status Engine::scheduler_loop_learned() {
     auto retire = [&](int32_t upto) -> lt_status {
         while (!inflight.empty()) {
             Inflight f = inflight.front();
-            const bool must = upto >= 0;
-            if (must) LT_HIP(spin_event(f.done));
-            else if (hipEventQuery(f.done) != hipSuccess) break;
+            if (upto < 0 && !loaded(f.load)) break;
+            LT_TRY(wait_loaded(f.load));
             inflight.erase(inflight.begin());
-            pool_events.push_back(f.done);
             pending[f.part] = 0;
             resident[f.part] = 1;
             LT_TRY(set_table((uint32_t)f.part, true));
@@ -1687,9 +1754,9 @@ lt_status Engine::scheduler_loop_learned() {
         return LT_OK;
     };
     // reference pipelining: walk resident partitions while the copy engine works
-    auto pipeline_while_copying = [&](int32_t except) -> lt_status {
+    auto pipeline_while_copying = [&](int32_t except, const Load &load) -> lt_status {
         if (!cfg.pipeline) return LT_OK;
-        while (hipStreamQuery(s_copy) == hipErrorNotReady) {
+        while (!loaded(load)) {
             LT_TRY(read_meta());
             const int32_t p2 = sched.computed_choice(counts.data(), resident.data(), except, kRefPage);
             if (p2 < 0) break;
@@ -1754,8 +1821,8 @@ lt_status Engine::scheduler_loop_learned() {
         } else {
             st.explicit_iterations++;
             if (pending[c]) {
-                if (hipEventQuery(inflight.front().done) != hipSuccess && inflight.front().part == c)
-                    LT_TRY(pipeline_while_copying(c));
+                if (!loaded(inflight.front().load) && inflight.front().part == c)
+                    LT_TRY(pipeline_while_copying(c, inflight.front().load));
                 LT_TRY(retire(c));
             }
             if (resident[c]) {
@@ -1776,11 +1843,12 @@ lt_status Engine::scheduler_loop_learned() {
                     prefetched[evicted] = 0;
                 }
                 record((uint32_t)c, 3, c, evicted);
-                LT_TRY(load_async((uint32_t)c));
+                Load load;
+                LT_TRY(load_async((uint32_t)c, false, load));
                 st.graph_loading_calls++;
                 sched.on_load((uint32_t)c);
-                LT_TRY(pipeline_while_copying(c));
-                LT_HIP(hipStreamSynchronize(s_copy));
+                LT_TRY(pipeline_while_copying(c, load));
+                LT_TRY(wait_loaded(load));
                 resident[c] = 1;
                 LT_TRY(set_table((uint32_t)c, true));
             }
@@ -1834,11 +1902,9 @@ lt_status Engine::scheduler_loop_learned() {
                     }
                 }
                 if (q < 0) break;
-                LT_TRY(load_async((uint32_t)q));
-                hipEvent_t ev;
-                LT_TRY(take_event(ev));
-                LT_HIP(hipEventRecord(ev, s_copy));
-                inflight.push_back({q, ev});
+                Load load;
+                LT_TRY(load_async((uint32_t)q, true, load));
+                inflight.push_back({q, load});
                 pending[q] = 1;
                 st.graph_loading_calls++;
                 sched.on_load((uint32_t)q);
@@ -1912,7 +1978,7 @@ lt_status Engine::scheduler_loop_device() {
     const int dwpt = cfg.walkers_per_thread > 0 ? cfg.walkers_per_thread : 1;
     BlockImages bi{};
     bi.words_tab = d_words_tab;
-    bi.img = d_pk_img;
+    bi.img = slot_packed ? d_pk_img : nullptr;
     bi.off = d_pk_off;
     bi.size = d_pk_size;
     hipGraph_t graph = nullptr;

@@ -1012,6 +1012,36 @@ __global__ void set_tables_kernel(Tables tab, TableBatch b) {
     }
 }
 
+// Copy of a partition's two slices from mapped host memory (or HBM) into a cache
+// slot, 4-byte words: 64 workgroups with eight loads per lane in flight fill
+// the link.
+struct PullArgs {
+    const uint32_t *src[2];
+    uint32_t *dst[2];
+    uint64_t words[2];
+};
+
+__global__ __launch_bounds__(256) void pull_kernel(PullArgs a) {
+    constexpr int kAhead = 8;
+    const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+        const uint32_t *src = a.src[s];
+        uint32_t *dst = a.dst[s];
+        const uint64_t n = a.words[s];
+        uint64_t i = tid;
+        for (; i + (kAhead - 1) * stride < n; i += kAhead * stride) {
+            uint32_t v[kAhead];
+#pragma unroll
+            for (int k = 0; k < kAhead; k++) v[k] = __builtin_nontemporal_load(&src[i + k * stride]);
+#pragma unroll
+            for (int k = 0; k < kAhead; k++) dst[i + k * stride] = v[k];
+        }
+        for (; i < n; i += stride) dst[i] = __builtin_nontemporal_load(&src[i]);
+    }
+}
+
 // Plain streaming copy of n 16-byte vectors (known HBM traffic: 16n read, 16n written).
 __global__ __launch_bounds__(256) void copy_probe_kernel(const uint4 *src, uint4 *dst, uint64_t n) {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
