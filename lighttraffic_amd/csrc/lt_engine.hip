@@ -136,6 +136,18 @@ struct RunSpec {
     uint32_t *paths_out = nullptr;  // genericwalk: u32[total][length + 1] on the host
 };
 
+using WalkFn = void (*)(WalkArgs);
+template <int APP>
+static WalkFn walk_fn_app(int wpt, bool gen) {
+    if (gen) return wpt == 4 ? walk_kernel<APP, 4, true> : wpt == 2 ? walk_kernel<APP, 2, true> : walk_kernel<APP, 1, true>;
+    return wpt == 4 ? walk_kernel<APP, 4, false> : wpt == 2 ? walk_kernel<APP, 2, false> : walk_kernel<APP, 1, false>;
+}
+static WalkFn walk_fn(int app, int wpt, bool gen) {
+    return app == APP_PAGERANK ? walk_fn_app<APP_PAGERANK>(wpt, gen)
+           : app == APP_PPR    ? walk_fn_app<APP_PPR>(wpt, gen)
+                               : walk_fn_app<APP_GENERIC>(wpt, gen);
+}
+
 struct Engine {
     const lt_graph *g = nullptr;
     lt_partition part;
@@ -387,6 +399,7 @@ struct Engine {
     AppArgs app{};
     int app_kind = APP_PAGERANK;
     size_t lds_bytes(int wpt = kWpt) const { return append_lds_bytes(P, wpt); }
+    bool append_gen() const { return P > kDirectMaxP || cfg.append_mode != 0; }
     lt_status launch_walk(const WalkArgs &a, uint64_t walkers, hipStream_t s);
     uint64_t partition_bytes(uint32_t p) const {
         return ((uint64_t)part.node_off[p + 1] - part.node_off[p] + 1) * 8 +
@@ -511,16 +524,10 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
     // Each app's kernels have their own register counts, so their own
     // occupancy: a grid sized by another kernel's would queue workgroups
     // behind the resident ones and finish in a second, partial round.
-    const void *wk[3][5] = {
-        {nullptr, (const void *)walk_kernel<APP_PAGERANK, 1>, (const void *)walk_kernel<APP_PAGERANK, 2>, nullptr,
-         (const void *)walk_kernel<APP_PAGERANK, 4>},
-        {nullptr, (const void *)walk_kernel<APP_PPR, 1>, (const void *)walk_kernel<APP_PPR, 2>, nullptr,
-         (const void *)walk_kernel<APP_PPR, 4>},
-        {nullptr, (const void *)walk_kernel<APP_GENERIC, 1>, (const void *)walk_kernel<APP_GENERIC, 2>, nullptr,
-         (const void *)walk_kernel<APP_GENERIC, 4>}};
     for (int app : {APP_PAGERANK, APP_PPR, APP_GENERIC})
         for (int wpt : {1, 2, 4}) {
-            LT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, wk[app][wpt], kBlock, lds_bytes(wpt)));
+            LT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void *)walk_fn(app, wpt, append_gen()),
+                                                                kBlock, lds_bytes(wpt)));
             walk_grid[app][wpt] = std::max(1, occ) * num_cu;
         }
 
@@ -1125,15 +1132,9 @@ lt_status Engine::fetch_partition(uint32_t p, uint64_t *rowptr_out, uint32_t *co
 // (a thread walks its walkers one after another), 2 or 4 for large slices,
 // where the per-workgroup append cost (histogram, scan, one atomic per
 // destination queue) is spread over more walkers.
-template <int APP>
-static void launch_walk_app(const WalkArgs &a, int wpt, int grid, size_t lds, hipStream_t s) {
-    if (wpt == 4) walk_kernel<APP, 4><<<grid, kBlock, lds, s>>>(a);
-    else if (wpt == 2) walk_kernel<APP, 2><<<grid, kBlock, lds, s>>>(a);
-    else walk_kernel<APP, 1><<<grid, kBlock, lds, s>>>(a);
-}
-
 lt_status Engine::launch_walk(const WalkArgs &a, uint64_t walkers, hipStream_t s) {
-    LT_TRY(flush_tables());
+    // a walk of one source that stays in it reads no table
+    if (a.span_resident || a.nsrc) LT_TRY(flush_tables());
     const uint64_t fill = (uint64_t)num_cu * 4 * 6 * 64;  // threads for ~6 waves per SIMD
     const int wpt = cfg.walkers_per_thread > 0 ? cfg.walkers_per_thread
                     : walkers >= 4 * fill         ? 4
@@ -1143,11 +1144,7 @@ lt_status Engine::launch_walk(const WalkArgs &a, uint64_t walkers, hipStream_t s
     // with loads going on, room for a pull kernel's workgroups beside the walk's
     const uint64_t most = walk_grid[app_kind][wpt] - (nslots < P && walk_grid[app_kind][wpt] > kPullGrid ? kPullGrid : 0);
     const int grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((walkers + bw - 1) / bw, most));
-    switch (app_kind) {
-        case APP_PAGERANK: launch_walk_app<APP_PAGERANK>(a, wpt, grid, lds_bytes(wpt), s); break;
-        case APP_PPR: launch_walk_app<APP_PPR>(a, wpt, grid, lds_bytes(wpt), s); break;
-        default: launch_walk_app<APP_GENERIC>(a, wpt, grid, lds_bytes(wpt), s); break;
-    }
+    walk_fn(app_kind, wpt, append_gen())<<<grid, kBlock, lds_bytes(wpt), s>>>(a);
     LT_HIP(hipGetLastError());
     meta_dirty = true;
     return LT_OK;
@@ -1987,17 +1984,7 @@ lt_status Engine::scheduler_loop_device() {
     for (int it = 0; it < kGraphIters; it++) {
         decide_kernel<<<1, 1024, 0, s_compute>>>(q, a.ss, a.pt, bi);
         load_kernel<<<load_grid, 256, 0, s_compute>>>(a.ss, a.pt, bi);
-        switch (app_kind) {
-            case APP_PAGERANK:
-                launch_walk_app<APP_PAGERANK>(a, dwpt, walk_grid[APP_PAGERANK][dwpt], lds_bytes(dwpt), s_compute);
-                break;
-            case APP_PPR:
-                launch_walk_app<APP_PPR>(a, dwpt, walk_grid[APP_PPR][dwpt], lds_bytes(dwpt), s_compute);
-                break;
-            default:
-                launch_walk_app<APP_GENERIC>(a, dwpt, walk_grid[APP_GENERIC][dwpt], lds_bytes(dwpt), s_compute);
-                break;
-        }
+        walk_fn(app_kind, dwpt, append_gen())<<<walk_grid[app_kind][dwpt], kBlock, lds_bytes(dwpt), s_compute>>>(a);
         fixup_kernel<<<1, kBlock, 0, s_compute>>>(q, Consumed{}, tables(), d_ds);
     }
     hipError_t ce = hipStreamEndCapture(s_compute, &graph);

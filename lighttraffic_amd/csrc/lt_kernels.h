@@ -307,27 +307,42 @@ __device__ void block_append_hashed(const Queues &q, const AppendLds &L, const W
 // is still the end's needs no lookup.
 struct AppendHint {
     uint32_t k = kEmpty, c = kEmpty;  // chunk number in the queue, chunk id
+    uint32_t len = 0;                 // first_hint's length of the queue, until second_hint
+    bool look = false;
 };
 
-// First look, while the first walkers walk.  Only for launches of at most a
-// workgroup per CU: those wait for every round trip, while in larger ones the
-// lines, which every append writes, are better left alone.
+// First look, while the first walkers are fetched and walk (in two steps, so that
+// neither load is waited for).  Only for launches of at most a workgroup per CU:
+// those wait for every round trip, while in larger ones the lines, which every
+// append writes, are better left alone.
 __device__ __forceinline__ void first_hint(const Queues &q, uint32_t P, int mode, AppendHint &h) {
-    if (gridDim.x > 256 || P > kDirectMaxP || mode == 2 || threadIdx.x >= P) return;
-    h.k = load_agent(&qlen_of(q, threadIdx.x)) >> kChunkLog2;
-    if (h.k < q.maxc) h.c = load_agent(&q.frame[(size_t)threadIdx.x * q.maxc + h.k]);
+    h.look = gridDim.x <= 256 && P <= kDirectMaxP && mode != 2;
+    if (h.look && threadIdx.x < P) h.len = load_agent(&qlen_of(q, threadIdx.x));
 }
 
-template <int WPT>
-__device__ void block_append(const Queues &q, uint32_t P, const AppendLds &L, const Walker (&w)[WPT],
-                             const uint32_t (&dst)[WPT], uint32_t *s_wsum, AppendHint &hint, int mode = 0) {
-    if (mode == 2) {  // uniform
-        append_one_level<WPT>(q, w, dst);
-        return;
-    }
-    if (L.hashed) {  // uniform: more partitions than LDS slots
-        block_append_hashed<WPT>(q, L, w, dst, s_wsum, mode);
-        return;
+__device__ __forceinline__ void second_hint(const Queues &q, uint32_t P, AppendHint &h) {
+    if (!h.look) return;  // uniform
+    h.look = false;
+    h.k = h.len >> kChunkLog2;
+    if (threadIdx.x < P && h.k < q.maxc) h.c = load_agent(&q.frame[(size_t)threadIdx.x * q.maxc + h.k]);
+}
+
+//
+// GEN: any partition count and append_mode; otherwise at most kDirectMaxP
+// partitions and append_mode 0.
+template <int WPT, bool GEN>
+__device__ __forceinline__ void block_append(const Queues &q, uint32_t P, const AppendLds &L, const Walker (&w)[WPT],
+                                             const uint32_t (&dst)[WPT], uint32_t *s_wsum, AppendHint &hint,
+                                             int mode = 0) {
+    if constexpr (GEN) {
+        if (mode == 2) {  // uniform
+            append_one_level<WPT>(q, w, dst);
+            return;
+        }
+        if (L.hashed) {  // uniform: more partitions than LDS slots
+            block_append_hashed<WPT>(q, L, w, dst, s_wsum, mode);
+            return;
+        }
     }
     const uint32_t tid = threadIdx.x;
     for (uint32_t i = tid; i < P; i += kBlock) L.hist[i] = 0;
@@ -337,16 +352,30 @@ __device__ void block_append(const Queues &q, uint32_t P, const AppendLds &L, co
     for (int k = 0; k < WPT; k++)
         if (dst[k] != kEmpty) rank[k] = atomicAdd(&L.hist[dst[k]], 1u);
     __syncthreads();
+    // The first reservation is on its way during the scan and the staging.
+    uint32_t b0 = 0;
+    if (tid < P && L.hist[tid]) b0 = atomicAdd(&qlen_of(q, tid), L.hist[tid]);
     const uint32_t total = block_exclusive_scan(L.hist, L.scan, P, s_wsum);
     if (tid == 0) L.scan[P] = total;
     __syncthreads();  // the scan reads hist segments that the loop below overwrites
+    const bool staged = !(GEN && mode == 1);  // uniform; otherwise each walker is stored from its own lane
+    if (staged) {
+#pragma unroll
+        for (int k = 0; k < WPT; k++) {
+            if (dst[k] != kEmpty) {
+                const uint32_t pos = L.scan[dst[k]] + rank[k];
+                L.stage[pos] = w[k];
+                L.dst[pos] = (uint16_t)dst[k];
+            }
+        }
+    }
     // Pass 1: reserve and link the chunks this workgroup owns.  Pass 2 waits
     // for chunks owned by others only after every owned link is published,
     // so no owner ever waits before publishing.
     for (uint32_t i = tid; i < P; i += kBlock) {
         const uint32_t c = L.hist[i];
         if (c) {
-            const uint32_t b = atomicAdd(&qlen_of(q, i), c);
+            const uint32_t b = i == tid ? b0 : atomicAdd(&qlen_of(q, i), c);
             const uint32_t k0 = b >> kChunkLog2, k1 = (b + c - 1) >> kChunkLog2;
             const uint32_t c0 = (b & (kChunk - 1)) == 0 ? alloc_chunk(q, i, k0) : kEmpty;
             L.ch0[i] = c0;
@@ -370,22 +399,13 @@ __device__ void block_append(const Queues &q, uint32_t P, const AppendLds &L, co
         }
     }
     __syncthreads();
-    if (mode == 1) {  // uniform: each walker stored from its own lane
+    if (!staged) {
 #pragma unroll
         for (int k = 0; k < WPT; k++)
             if (dst[k] != kEmpty) store_reserved(q, L, dst[k], rank[k], w[k]);
         __syncthreads();
         return;
     }
-#pragma unroll
-    for (int k = 0; k < WPT; k++) {
-        if (dst[k] != kEmpty) {
-            const uint32_t pos = L.scan[dst[k]] + rank[k];
-            L.stage[pos] = w[k];
-            L.dst[pos] = (uint16_t)dst[k];
-        }
-    }
-    __syncthreads();
     for (uint32_t i = tid; i < total; i += kBlock) {
         const uint32_t part = L.dst[i];
         const uint32_t b = L.hist[part];
@@ -623,7 +643,9 @@ __device__ uint32_t walk_residency(Walker &w, const WalkArgs &a, uint32_t src, c
 
 // One workgroup pass over nvalid <= kBlock * WPT walkers stored
 // contiguously at cw: walk each, then append the survivors to their queues.
-template <int APP, int WPT>
+// The visit log is reserved before the append and written after it, so the
+// reservation's round trip overlaps the append's own.
+template <int APP, int WPT, bool GEN>
 __device__ __forceinline__ void walk_walkers(const WalkArgs &a, const AppendLds &L, uint32_t *s_wsum, uint32_t src,
                                             const Span &src_sp, const Walker *cw, uint32_t nvalid, Counters &ct,
                                             AppendHint &hint) {
@@ -640,20 +662,23 @@ __device__ __forceinline__ void walk_walkers(const WalkArgs &a, const AppendLds 
             w[k].step = 0;
         }
     }
+    second_hint(a.q, a.pt.P, hint);
 #pragma unroll
     for (int k = 0; k < WPT; k++) {
         if ((uint32_t)k * kBlock + threadIdx.x < nvalid) dst[k] = walk_residency<APP>(w[k], a, src, src_sp, ct);
     }
+    uint32_t n = 0, at = 0;
     if constexpr (APP != APP_GENERIC) {  // genericwalk counts no visits
         if (ct.vbuf) {  // uniform
-            // The log is reserved before the append and written after it, so
-            // the reservation's round trip overlaps the append's own.
-            __shared__ uint32_t s_at;
             __syncthreads();
-            const uint32_t n = min(*ct.vn, kVisitBuf);
-            uint32_t at = 0;
+            n = min(*ct.vn, kVisitBuf);
             if (threadIdx.x == kBlock - 1 && n) at = log_reserve(a.app, n);
-            block_append<WPT>(a.q, a.pt.P, L, w, dst, s_wsum, hint, a.append_mode);
+        }
+    }
+    block_append<WPT, GEN>(a.q, a.pt.P, L, w, dst, s_wsum, hint, a.append_mode);
+    if constexpr (APP != APP_GENERIC) {
+        if (ct.vbuf) {  // uniform
+            __shared__ uint32_t s_at;
             if (threadIdx.x == kBlock - 1) {
                 s_at = at;
                 *ct.vn = 0;
@@ -661,31 +686,19 @@ __device__ __forceinline__ void walk_walkers(const WalkArgs &a, const AppendLds 
             __syncthreads();
             for (uint32_t i = threadIdx.x; i < n; i += kBlock) log_store(a.app, s_at + i, ct.vbuf[i]);
             __syncthreads();
-            return;
         }
     }
-    block_append<WPT>(a.q, a.pt.P, L, w, dst, s_wsum, hint, a.append_mode);
-}
-
-// One workgroup pass: walkers [base, base + kBlock * WPT) of src's queue,
-// clipped to hi64; base is a multiple of kBlock * WPT, so the pass reads one
-// chunk.
-template <int APP, int WPT>
-__device__ __forceinline__ void walk_pass(const WalkArgs &a, const AppendLds &L, uint32_t *s_wsum, uint32_t src,
-                                          const Span &src_sp, uint64_t base, uint64_t hi64, Counters &ct,
-                                          AppendHint &hint) {
-    const uint32_t chunk = a.q.frame[(size_t)src * a.q.maxc + (uint32_t)(base >> kChunkLog2)];
-    const bool chunk_ok = chunk < a.q.nchunks;
-    if (!chunk_ok && threadIdx.x == 0) atomicOr(&a.q.ctl->overflow, 8u);
-    const Walker *cw = a.q.slab + (size_t)(chunk_ok ? chunk : 0) * kChunk + (uint32_t)(base & (kChunk - 1));
-    const uint64_t left = hi64 > base ? hi64 - base : 0;
-    const uint32_t nvalid = chunk_ok ? (uint32_t)min(left, (uint64_t)(kBlock * WPT)) : 0u;
-    walk_walkers<APP, WPT>(a, L, s_wsum, src, src_sp, cw, nvalid, ct, hint);
 }
 
 // WPT walkers per thread per pass (1, 2 or 4): small queues use 1 so that
-// enough workgroups exist to fill the chip, large ones 4.
-template <int APP, int WPT>
+// enough workgroups exist to fill the chip, large ones 4.  GEN: see block_append.
+//
+// A small launch waits for one round trip after another, and its code is
+// one of them: every CU fetches what it runs.  So the source of a pass (a slice
+// of one queue, queues of a batch, walkers in host memory, the device's
+// choice) is picked in the loop and the pass itself stands here once, and
+// what only large partition tables or append modes need is a kernel of its own.
+template <int APP, int WPT, bool GEN>
 __global__ __launch_bounds__(kBlock) void walk_kernel(WalkArgs a) {
     constexpr int BW = kBlock * WPT;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -708,72 +721,79 @@ __global__ __launch_bounds__(kBlock) void walk_kernel(WalkArgs a) {
     }
     AppendHint hint;
     first_hint(a.q, a.pt.P, a.append_mode, hint);
+    uint32_t src = a.src;
+    Span sp;
+    sp.rowptr = a.rowptr;
+    sp.col = a.col;
+    sp.words = a.words;
+    sp.zc = a.zerocopy;
+    sp.nb = a.nb;
+    sp.ne = a.ne;
+    sp.eb = a.eb;
+    uint64_t lo = 0, hi;
     if (a.nsrc) {  // batch: the whole queues of several partitions, each in the partition table
-        const uint64_t vend = a.voff[a.nsrc];
-        for (uint64_t base = (uint64_t)blockIdx.x * BW; base < vend; base += (uint64_t)gridDim.x * BW) {
-            uint32_t k = 0;
-            while (k + 1 < a.nsrc && base >= a.voff[k + 1]) k++;
-            const uint32_t src = a.srcs[k];
-            Span sp;  // as a walker entering src reads it (walk_residency)
-            sp.rowptr = a.pt.rowptr_tab[src];
-            sp.col = a.pt.col_tab[src];
-            sp.words = a.pt.words_tab[src];
-            sp.nb = a.pt.node_off[src];
-            sp.ne = a.pt.node_off[src + 1];
-            sp.eb = a.pt.edge_off[src];
-            sp.zc = a.pt.zc_part[src];
-            const uint64_t local = base - a.voff[k], n = qlen_of(a.q, src);
-            if (local < n) walk_pass<APP, WPT>(a, L, s_wsum, src, sp, local, n, ct, hint);  // uniform per workgroup
-        }
-        flush_counters(ct, a.stats);
-        return;
-    }
-    uint32_t src = a.src, chunk_lo = a.chunk_lo, chunk_hi = a.chunk_hi, n = a.n;
-    Span src_sp;
-    src_sp.rowptr = a.rowptr;
-    src_sp.col = a.col;
-    src_sp.words = a.words;
-    src_sp.zc = a.zerocopy;
-    src_sp.nb = a.nb;
-    src_sp.ne = a.ne;
-    src_sp.eb = a.eb;
-    if (a.nhost) {  // walkers of src spilled to host memory, read over PCIe
-        const uint64_t vend = (uint64_t)a.nhost << kChunkLog2;
-        for (uint64_t base = (uint64_t)blockIdx.x * BW; base < vend; base += (uint64_t)gridDim.x * BW) {
-            const uint32_t k = (uint32_t)(base >> kChunkLog2), local = (uint32_t)(base & (kChunk - 1));
-            if (local < a.hn[k])  // uniform per workgroup
-                walk_walkers<APP, WPT>(a, L, s_wsum, src, src_sp, a.hptr[k] + local,
-                                       min(a.hn[k] - local, (uint32_t)BW), ct, hint);
-        }
-        flush_counters(ct, a.stats);
-        return;
-    }
-    if (a.ss.ds) {  // the decision of this iteration was taken on the device
+        hi = a.voff[a.nsrc];
+    } else if (a.nhost) {  // walkers of src spilled to host memory, read over PCIe
+        hi = (uint64_t)a.nhost << kChunkLog2;
+    } else if (a.ss.ds) {  // the decision of this iteration was taken on the device
         const int32_t c = a.ss.ds->choice;
         if (c < 0) return;
         src = (uint32_t)c;
-        chunk_lo = 0;
-        chunk_hi = 0xFFFFFFFFu;
-        n = qlen_of(a.q, src);
-        src_sp.nb = a.pt.node_off[src];
-        src_sp.ne = a.pt.node_off[src + 1];
-        src_sp.eb = a.pt.edge_off[src];
-        src_sp.zc = a.ss.ds->zerocopy;
-        src_sp.words = nullptr;
-        if (src_sp.zc) {
-            src_sp.rowptr = a.ss.zc_rowptr + a.pt.node_off[src];
-            src_sp.col = a.ss.zc_col + a.pt.edge_off[src];
+        hi = qlen_of(a.q, src);
+        sp.nb = a.pt.node_off[src];
+        sp.ne = a.pt.node_off[src + 1];
+        sp.eb = a.pt.edge_off[src];
+        sp.zc = a.ss.ds->zerocopy;
+        sp.words = nullptr;
+        if (sp.zc) {
+            sp.rowptr = a.ss.zc_rowptr + a.pt.node_off[src];
+            sp.col = a.ss.zc_col + a.pt.edge_off[src];
         } else {  // a raw slot, or a block slot whose bit streams decide_kernel entered in the table
             const uint8_t *base = a.ss.slots + (size_t)a.ss.slot_of[src] * a.ss.slot_bytes;
-            src_sp.rowptr = (const uint64_t *)base;
-            src_sp.col = (const uint32_t *)(base + ((uint64_t)a.pt.node_off[src + 1] - a.pt.node_off[src] + 1) * 8);
-            src_sp.words = a.pt.words_tab[src];
+            sp.rowptr = (const uint64_t *)base;
+            sp.col = (const uint32_t *)(base + ((uint64_t)a.pt.node_off[src + 1] - a.pt.node_off[src] + 1) * 8);
+            sp.words = a.pt.words_tab[src];
         }
+    } else {
+        lo = (uint64_t)a.chunk_lo << kChunkLog2;
+        hi = min((uint64_t)a.n, (uint64_t)a.chunk_hi << kChunkLog2);
     }
-    const uint64_t lo64 = (uint64_t)chunk_lo << kChunkLog2;
-    const uint64_t hi64 = min((uint64_t)n, (uint64_t)chunk_hi << kChunkLog2);
-    for (uint64_t base = lo64 + (uint64_t)blockIdx.x * BW; base < hi64; base += (uint64_t)gridDim.x * BW)
-        walk_pass<APP, WPT>(a, L, s_wsum, src, src_sp, base, hi64, ct, hint);
+    // A pass: walkers [base, base + BW) clipped to n; base is a multiple of BW, so
+    // it reads one chunk.
+    for (uint64_t at = lo + (uint64_t)blockIdx.x * BW; at < hi; at += (uint64_t)gridDim.x * BW) {
+        const Walker *cw;
+        uint64_t base = at, n = hi;
+        if (a.nhost) {
+            const uint32_t k = (uint32_t)(at >> kChunkLog2);
+            base = at & (kChunk - 1);
+            n = a.hn[k];
+            if (base >= n) continue;  // uniform per workgroup
+            cw = a.hptr[k] + base;
+        } else {
+            if (a.nsrc) {
+                uint32_t k = 0;
+                while (k + 1 < a.nsrc && at >= a.voff[k + 1]) k++;
+                src = a.srcs[k];
+                base = at - a.voff[k];
+                n = qlen_of(a.q, src);
+                if (base >= n) continue;  // uniform per workgroup
+                sp.rowptr = a.pt.rowptr_tab[src];  // as a walker entering src reads it (walk_residency)
+                sp.col = a.pt.col_tab[src];
+                sp.words = a.pt.words_tab[src];
+                sp.nb = a.pt.node_off[src];
+                sp.ne = a.pt.node_off[src + 1];
+                sp.eb = a.pt.edge_off[src];
+                sp.zc = a.pt.zc_part[src];
+            }
+            const uint32_t chunk = a.q.frame[(size_t)src * a.q.maxc + (uint32_t)(base >> kChunkLog2)];
+            if (chunk >= a.q.nchunks) {  // uniform per workgroup
+                if (threadIdx.x == 0) atomicOr(&a.q.ctl->overflow, 8u);
+                continue;
+            }
+            cw = a.q.slab + (size_t)chunk * kChunk + (uint32_t)(base & (kChunk - 1));
+        }
+        walk_walkers<APP, WPT, GEN>(a, L, s_wsum, src, sp, cw, (uint32_t)min(n - base, (uint64_t)BW), ct, hint);
+    }
     flush_counters(ct, a.stats);
 }
 
@@ -842,7 +862,7 @@ __global__ __launch_bounds__(kBlock) void init_kernel(InitArgs a) {
                 finish_walker(w[k], a.app);
             }
         }
-        block_append<kWpt>(a.q, a.pt.P, L, w, dst, s_wsum, hint);
+        block_append<kWpt, true>(a.q, a.pt.P, L, w, dst, s_wsum, hint);
     }
 }
 

@@ -1,0 +1,30 @@
+"""The two forms of the walk kernel at the partition count between them, and what
+each append mode takes, against the CPU oracle bit for bit."""
+import numpy as np
+import pytest
+
+import lighttraffic_amd as lt
+from oracle import ffi as oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("append_mode", [0, 1, 2])
+@pytest.mark.parametrize("P", [1, 255, 256, 257, 1024, 1025])
+def test_partition_counts(P, append_mode):
+    """One vertex with four neighbours a partition; sources one at a time and in
+    batches, 1, 2 and 4 walkers a thread, all slots or half of them."""
+    print(f"walk forms P={P} append_mode={append_mode}", flush=True)
+    rng = np.random.default_rng(P)
+    g = lt.Graph.from_csr(4 * np.arange(P + 1, dtype=np.uint64), rng.integers(0, P, 4 * P).astype(np.uint32))
+    part = lt.Partition.build(g, 32)
+    assert part.count == P
+    w, l = 9973, 5
+    rc, re, _ = oracle.pagerank(g.rowptr(), g.col(), w, l, endpoints=True, threads=8)
+    for wpt, span in ((1, "partition"), (2, "resident"), (4, "resident")):
+        if P > 300 and span == "partition":
+            continue  # a round a partition: long, and nothing new
+        eng = lt.Engine(g, part, num_device_partitions=max(1, P // 2), span=span, walkers_per_thread=wpt,
+                        resident_batch=16, zc_batch=16, append_mode=append_mode)
+        counts, ends = eng.pagerank(w, l, endpoints=True)
+        assert np.array_equal(counts, rc) and np.array_equal(ends, re)
