@@ -55,8 +55,8 @@ struct Queues {
     uint32_t *free_stack;  // [nchunks]
     PoolCtl *ctl;
     uint32_t *lost;        // [kLostCap]
-    uint32_t *packed;      // [P + 5 + kLogRegions] in mapped host memory: the P queue lengths, PoolCtl, the
-                           // fill of the visit log's regions, and seq once the rest is written
+    uint64_t *packed;      // [P + 4 + kLogRegions] in mapped host memory: the P queue lengths, PoolCtl and
+                           // the fill of the visit log's regions (if there is one), seq in each one's upper half
     uint32_t seq;          // names this launch's write of packed
     const unsigned long long *vcur;  // cursors of the visit log, or nullptr
     uint32_t maxc;         // chunk slots per partition

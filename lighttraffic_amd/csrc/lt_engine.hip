@@ -203,7 +203,8 @@ struct Engine {
     uint64_t wcap = 0;  // walkers the pool is sized for
     Queues q{};
     uint32_t *d_meta = nullptr;   // [P] qlen followed by PoolCtl
-    uint32_t *h_meta = nullptr;   // pinned mirror
+    uint64_t *h_packed = nullptr; // q.packed in pinned memory
+    std::vector<uint32_t> h_meta; // what it last said: queue lengths, PoolCtl, the log's fill
     std::vector<uint64_t> counts; // walkers queued per partition: device queue + spilled to host
     std::vector<uint64_t> dcounts;  // device part of counts (qlen)
 
@@ -425,7 +426,7 @@ Engine::~Engine() {
     dfree(q.free_stack);
     dfree(q.lost);
     dfree(d_meta);
-    if (h_meta) (void)hipHostFree(h_meta);
+    if (h_packed) (void)hipHostFree(h_packed);
     for (Walker *b : hblocks) (void)hipHostFree(b);
     dfree(d_plan);
     if (h_plan) (void)hipHostFree(h_plan);
@@ -643,11 +644,12 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
     }
 
     // queue lengths one 128-byte line apart, then PoolCtl on its own line; the
-    // fix-up kernel packs both into h_meta (pinned, mapped) for the host
+    // fix-up kernel packs both into h_packed (pinned, mapped) for the host
     LT_TRY(dmalloc(&d_meta, (size_t)P * kQStride + kQStride));
-    LT_HIP(hipHostMalloc((void **)&h_meta, 4 * (P + 5 + kLogRegions), hipHostMallocMapped | hipHostMallocCoherent));
-    memset(h_meta, 0, 4 * (P + 5 + kLogRegions));
-    LT_HIP(hipHostGetDevicePointer((void **)&q.packed, h_meta, 0));
+    h_meta.assign(P + 4 + kLogRegions, 0);
+    LT_HIP(hipHostMalloc((void **)&h_packed, 8 * h_meta.size(), hipHostMallocMapped | hipHostMallocCoherent));
+    memset(h_packed, 0, 8 * h_meta.size());
+    LT_HIP(hipHostGetDevicePointer((void **)&q.packed, h_packed, 0));
     q.qlen = d_meta;
     q.ctl = (PoolCtl *)(d_meta + (size_t)P * kQStride);
     q.P = P;
@@ -840,15 +842,19 @@ lt_status Engine::launch_fixup(const Consumed &d) {
     return LT_OK;
 }
 
-// Waits until h_meta holds what the last launch that packs it wrote, and so
-// until the walk before that launch is over.  Every decision waits here; the
-// host polls the number that the kernel writes: launch, fix-up and wait of a
-// small kernel take 10 us so, 27 us when hipStreamQuery is polled and 12 us with
-// hipStreamSynchronize.  A stream that ends or fails without the number being
+// Waits until every word of h_packed is of the last launch that writes it, and
+// so until the walk before that launch is over.  Every decision waits here; the host
+// polls the words' numbers: launch, fix-up and wait of a small kernel take
+// 10 us so, 27 us when hipStreamQuery is polled and 12 us with
+// hipStreamSynchronize.  A stream that ends or fails without a word being
 // written is found by the query made once in a while.
 lt_status Engine::wait_meta() {
     if (meta_seen) return LT_OK;
-    LT_TRY(poll_host(h_meta + P + 4 + kLogRegions, meta_seq, "queue lengths"));
+    const size_t n = P + 4 + (q.vcur ? kLogRegions : 0);
+    for (size_t i = 0; i < n; i++) {
+        LT_TRY(poll_host((const uint32_t *)(h_packed + i) + 1, meta_seq, "queue lengths"));
+        h_meta[i] = (uint32_t)h_packed[i];
+    }
     meta_seen = true;
     return LT_OK;
 }
@@ -877,7 +883,7 @@ lt_status Engine::read_meta() {
         meta_seen = false;
     }
     LT_TRY(wait_meta());
-    const PoolCtl *c = (const PoolCtl *)(h_meta + P);
+    const PoolCtl *c = (const PoolCtl *)&h_meta[P];
     if (c->overflow) {
         set_error("walker queue pool overflow (flags 0x%x, top %u)", c->overflow, c->top);
         return LT_E_INTERNAL;
@@ -887,7 +893,7 @@ lt_status Engine::read_meta() {
         counts[i] = dcounts[i] + hcount[i];
     }
     if (vregion) {  // the log is counted before its fullest region is full
-        const uint32_t *cur = h_meta + P + 4;
+        const uint32_t *cur = &h_meta[P + 4];
         const uint32_t most = *std::max_element(cur, cur + kLogRegions);
         if (most >= vregion / 5 * 4) {
             LT_TRY(count_log(0, most));
@@ -2356,7 +2362,7 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
     }
     // the counts are part of the walk's work, so inside the timed region
     if (vregion && !walk_flat) {
-        const uint32_t *cur = h_meta + P + 4;
+        const uint32_t *cur = &h_meta[P + 4];
         LT_TRY(count_log(0, *std::max_element(cur, cur + kLogRegions)));
     }
     if (count_copies > 1) {

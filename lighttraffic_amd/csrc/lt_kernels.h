@@ -866,89 +866,109 @@ __global__ __launch_bounds__(kBlock) void init_kernel(InitArgs a) {
     }
 }
 
-// Copy the queue lengths and PoolCtl into q.packed for the host, which polls
-// the sequence number behind them (Engine::wait_meta).  Collective over one
-// workgroup; runs after every queue update of the stream.  The words are
-// written through to the host, and every wave waits for its own before the
-// barrier, so the number is written last.
+// Written through to the host.
 __device__ __forceinline__ void to_host(uint32_t *p, uint32_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// The queue lengths, PoolCtl and the log's cursors go to q.packed for the host
+// (Engine::wait_meta), each word with the launch's number beside it: the host
+// takes a word once its number is there, and no lane has to wait for the link to
+// take all others' words before one says that they are there (1.3 us).
+__device__ __forceinline__ void tell_host(const Queues &q, uint32_t i, uint32_t v) {
+    __hip_atomic_store(&q.packed[i], (uint64_t)q.seq << 32 | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__device__ __forceinline__ uint32_t log_fill(const Queues &q, uint32_t r) {
+    return (uint32_t)min(q.vcur[r * kCurStride], 0xFFFFFFFFull);
+}
+
+// Collective over one workgroup; runs after every queue update of the stream.
 __device__ void pack_meta(const Queues &q) {
-    for (uint32_t i = threadIdx.x; i < q.P; i += blockDim.x) to_host(&q.packed[i], qlen_of(q, i));
-    if (threadIdx.x < sizeof(PoolCtl) / 4) to_host(&q.packed[q.P + threadIdx.x], ((const uint32_t *)q.ctl)[threadIdx.x]);
-    if (q.vcur && threadIdx.x < kLogRegions)
-        to_host(&q.packed[q.P + 4 + threadIdx.x], (uint32_t)min(q.vcur[threadIdx.x * kCurStride], 0xFFFFFFFFull));
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (threadIdx.x == 0)
-        __hip_atomic_store(&q.packed[q.P + 4 + kLogRegions], q.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    for (uint32_t i = threadIdx.x; i < q.P; i += blockDim.x) tell_host(q, i, qlen_of(q, i));
+    if (threadIdx.x < sizeof(PoolCtl) / 4) tell_host(q, q.P + threadIdx.x, ((const uint32_t *)q.ctl)[threadIdx.x]);
+    if (q.vcur && threadIdx.x < kLogRegions) tell_host(q, q.P + 4 + threadIdx.x, log_fill(q, threadIdx.x));
 }
 
 __global__ __launch_bounds__(kBlock) void pack_meta_kernel(Queues q) { pack_meta(q); }
 
 // Return the popped-but-unused state of the pool, the lost chunks and the
 // consumed source chunks to the free stack; clear the source queues after their
-// last slice; take a zero-copy batch out of the partition table; pack the queue
-// lengths.  One workgroup.  A batch's sources share one launch: sixteen
-// launches of 4.4 us each followed a walk of sixteen queues before.
+// last slice; take a zero-copy batch out of the partition table; tell the host
+// the queue lengths.  One workgroup, for all sources of a batch's launch.
+//
+// Every round of a job waits for this kernel, a chain of round trips: what it
+// reads by known addresses is read at once, and the host, which needs the
+// lengths only, gets them before the chunks move (its next walk is behind this
+// kernel in the stream).
 __global__ __launch_bounds__(kBlock) void fixup_kernel(Queues q, Consumed d, Tables tab, const DevSched *ds) {
     __shared__ uint32_t s_top, s_nlost, s_off[kMaxZcBatch + 1];
+    const uint32_t tid = threadIdx.x;
     // a device-scheduled iteration consumed the whole queue of its choice
     const int32_t choice = ds ? ds->choice : -1;
     const uint32_t n = ds ? (choice < 0 ? 0u : 1u) : d.n;
     const uint32_t lo = ds ? 0u : d.chunk_lo, most = ds ? 0xFFFFFFFFu : d.chunk_hi;
+    const bool clear = ds || d.last;
     const auto src = [&](uint32_t k) { return ds ? (uint32_t)choice : d.src[k]; };
-    if (threadIdx.x < n) {
-        const uint32_t nch = (qlen_of(q, src(threadIdx.x)) + kChunk - 1) >> kChunkLog2;
+    const PoolCtl c = *q.ctl;
+    const uint32_t len = tid < q.P ? qlen_of(q, tid) : 0u;
+    const uint32_t fill = q.vcur && tid < kLogRegions ? log_fill(q, tid) : 0u;
+    if (tid < n) {
+        const uint32_t nch = (qlen_of(q, src(tid)) + kChunk - 1) >> kChunkLog2;
         const uint32_t hi = min(most, nch);
-        s_off[threadIdx.x + 1] = hi > lo ? hi - lo : 0;
+        s_off[tid + 1] = hi > lo ? hi - lo : 0;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        PoolCtl c = *q.ctl;
-        uint32_t popped = c.popped;
-        if (popped > c.top) popped = c.top;
-        uint32_t nlost = c.nlost < kLostCap ? c.nlost : kLostCap;
+    if (tid == 0) {
+        const uint32_t popped = min(c.popped, c.top);
+        const uint32_t nlost = c.nlost < kLostCap ? c.nlost : kLostCap;
+        PoolCtl after{c.top - popped, 0, 0, c.overflow};
         s_off[0] = 0;
         for (uint32_t k = 0; k < n; k++) s_off[k + 1] += s_off[k];
-        s_top = c.top - popped;
+        s_top = after.top;
         s_nlost = nlost;
-        if (s_top + nlost + s_off[n] > q.nchunks) {
-            q.ctl->overflow |= 16u;
+        if (after.top + nlost + s_off[n] > q.nchunks) {
+            after.overflow |= 16u;
             s_nlost = 0;
             for (uint32_t k = 0; k <= n; k++) s_off[k] = 0;
         }
+        after.top += s_nlost + s_off[n];
+        *q.ctl = after;
+        if (!ds) {
+            tell_host(q, q.P, after.top);
+            tell_host(q, q.P + 1, 0);
+            tell_host(q, q.P + 2, 0);
+            tell_host(q, q.P + 3, after.overflow);
+        }
+    }
+    if (!ds) {  // no host waits for an iteration of the device loop
+        for (uint32_t i = tid; i < q.P; i += kBlock) {
+            uint32_t v = i == tid ? len : qlen_of(q, i);
+#pragma unroll
+            for (uint32_t k = 0; k < kMaxZcBatch; k++) v = clear && k < n && d.src[k] == i ? 0u : v;
+            tell_host(q, i, v);
+        }
+        if (q.vcur && tid < kLogRegions) tell_host(q, q.P + 4 + tid, fill);
     }
     __syncthreads();
     const uint32_t top = s_top, nlost = s_nlost, cnt = s_off[n];
-    for (uint32_t i = threadIdx.x; i < nlost; i += kBlock) q.free_stack[top + i] = q.lost[i];
+    for (uint32_t i = tid; i < nlost; i += kBlock) q.free_stack[top + i] = q.lost[i];
     uint32_t k = 0;
-    for (uint32_t j = threadIdx.x; j < cnt; j += kBlock) {
+    for (uint32_t j = tid; j < cnt; j += kBlock) {
         while (j >= s_off[k + 1]) k++;
         uint32_t *f = &q.frame[(size_t)src(k) * q.maxc + lo + (j - s_off[k])];
         q.free_stack[top + nlost + j] = *f;
         *f = kEmpty;
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        q.ctl->top = top + nlost + cnt;
-        q.ctl->popped = 0;
-        q.ctl->nlost = 0;
-    }
-    if (threadIdx.x < n) {
-        const uint32_t p = src(threadIdx.x);
-        if (ds || d.last) qlen_of(q, p) = 0;
+    if (tid < n) {
+        const uint32_t p = src(tid);
+        if (clear) qlen_of(q, p) = 0;
         if (!ds && d.leave) {
             tab.rowptr[p] = nullptr;
             tab.col[p] = nullptr;
             tab.zc[p] = 0;
         }
     }
-    if (ds) return;  // no host waits for an iteration of the device loop
-    __syncthreads();
-    pack_meta(q);
 }
 
 // Copy the queues of a spill round into host memory: walker i of partition
