@@ -110,11 +110,19 @@ enum StatSlot { ST_MOVES = 0, ST_TELEPORTS, ST_VISITS, ST_RESIDENCIES, ST_ZC_MOV
 struct DevSched {
     int32_t choice;     // partition walked this iteration, -1 = every queue is empty
     int32_t zerocopy;   // walked from host memory
-    int32_t load;       // copied into `slot` first
-    int32_t slot;
+    int32_t load;       // copied into its slot first
     int32_t victim;     // partition evicted for the load, -1 = none
     uint32_t iterations, loads, zc_calls;
     unsigned long long h2d_bytes;
+    // the choice's queue length and slices, for the walk
+    uint32_t n, nb, ne;
+    uint64_t eb;
+    const uint64_t *rowptr;
+    const uint32_t *col, *words;
+    // and what a load copies: rowptr slice and col slice or block image, in
+    // 4-byte words
+    const uint32_t *from[2];
+    uint64_t count[2];
 };
 
 struct SchedState {

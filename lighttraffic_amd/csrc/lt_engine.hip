@@ -835,7 +835,7 @@ lt_status Engine::count_log(uint32_t n, uint32_t most) {
 
 lt_status Engine::launch_fixup(const Consumed &d) {
     q.seq = ++meta_seq;
-    fixup_kernel<<<1, kBlock, 0, s_compute>>>(q, d, tables(), nullptr);
+    fixup_kernel<<<1, kBlock, 0, s_compute>>>(q, d, tables());
     LT_HIP(hipGetLastError());
     meta_dirty = false;
     meta_seen = false;
@@ -1938,12 +1938,12 @@ SchedState Engine::sched_state(bool device) const {
     return ss;
 }
 
-// Device-scheduled loop: per iteration decide_kernel (plain greedy rules in
-// one workgroup), load_kernel (partition copy over PCIe by the GPU itself),
-// walk_kernel and fixup_kernel, all reading the decision from device memory.
-// kGraphIters iterations are captured once into a hipGraph and the graph is
+// Device-scheduled loop: per iteration decide_kernel (the end of the iteration
+// before and the plain greedy rules, in one workgroup), load_kernel (partition copy
+// over PCIe by the GPU itself) and walk_kernel, both reading the decision from
+// device memory.  kGraphIters iterations are captured once into a hipGraph and the graph is
 // relaunched until an iteration finds every queue empty; the host reads one
-// 40-byte record per launch instead of syncing on every decision.
+// record per launch instead of syncing on every decision.
 constexpr int kGraphIters = 32;
 
 lt_status Engine::scheduler_loop_device() {
@@ -1955,7 +1955,7 @@ lt_status Engine::scheduler_loop_device() {
     LT_HIP(hipMemcpyAsync(d_part_in_slot, hp.data(), 4 * nslots, hipMemcpyHostToDevice, s_compute));
     LT_HIP(hipMemcpyAsync(d_resident, resident.data(), P, hipMemcpyHostToDevice, s_compute));
     DevSched zero{};
-    zero.choice = 0;
+    zero.choice = -1;
     LT_HIP(hipMemcpyAsync(d_ds, &zero, sizeof(zero), hipMemcpyHostToDevice, s_compute));
     LT_HIP(hipStreamSynchronize(s_compute));
 
@@ -1975,7 +1975,6 @@ lt_status Engine::scheduler_loop_device() {
     a.span_resident = cfg.span == LT_SPAN_RESIDENT ? 1 : 0;
     a.stats = d_stats;
     a.ss = sched_state(true);
-    const int load_grid = 4 * num_cu;
     // walkers per lane of the captured walk launches: the queue sizes are only
     // known on the device, so the grid is the full occupancy grid of that WPT
     const int dwpt = cfg.walkers_per_thread > 0 ? cfg.walkers_per_thread : 1;
@@ -1988,10 +1987,9 @@ lt_status Engine::scheduler_loop_device() {
     hipGraphExec_t exec = nullptr;
     LT_HIP(hipStreamBeginCapture(s_compute, hipStreamCaptureModeThreadLocal));
     for (int it = 0; it < kGraphIters; it++) {
-        decide_kernel<<<1, 1024, 0, s_compute>>>(q, a.ss, a.pt, bi);
-        load_kernel<<<load_grid, 256, 0, s_compute>>>(a.ss, a.pt, bi);
+        decide_kernel<<<1, kBlock, 0, s_compute>>>(q, a.ss, a.pt, bi);
+        load_kernel<<<num_cu, 256, 0, s_compute>>>(d_ds);
         walk_fn(app_kind, dwpt, append_gen())<<<walk_grid[app_kind][dwpt], kBlock, lds_bytes(dwpt), s_compute>>>(a);
-        fixup_kernel<<<1, kBlock, 0, s_compute>>>(q, Consumed{}, tables(), d_ds);
     }
     hipError_t ce = hipStreamEndCapture(s_compute, &graph);
     if (ce != hipSuccess) {

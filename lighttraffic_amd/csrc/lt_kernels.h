@@ -315,8 +315,8 @@ struct AppendHint {
 // neither load is waited for).  Only for launches of at most a workgroup per CU:
 // those wait for every round trip, while in larger ones the lines, which every
 // append writes, are better left alone.
-__device__ __forceinline__ void first_hint(const Queues &q, uint32_t P, int mode, AppendHint &h) {
-    h.look = gridDim.x <= 256 && P <= kDirectMaxP && mode != 2;
+__device__ __forceinline__ void first_hint(const Queues &q, uint32_t P, int mode, uint64_t passes, AppendHint &h) {
+    h.look = passes <= 256 && P <= kDirectMaxP && mode != 2;
     if (h.look && threadIdx.x < P) h.len = load_agent(&qlen_of(q, threadIdx.x));
 }
 
@@ -699,7 +699,7 @@ __device__ __forceinline__ void walk_walkers(const WalkArgs &a, const AppendLds 
 // choice) is picked in the loop and the pass itself stands here once, and
 // what only large partition tables or append modes need is a kernel of its own.
 template <int APP, int WPT, bool GEN>
-__global__ __launch_bounds__(kBlock) void walk_kernel(WalkArgs a) {
+__global__ __launch_bounds__(kBlock, WPT == 1 && !GEN ? 5 : 4) void walk_kernel(WalkArgs a) {
     constexpr int BW = kBlock * WPT;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     __shared__ uint32_t s_wsum[kBlock / 64];
@@ -719,8 +719,6 @@ __global__ __launch_bounds__(kBlock) void walk_kernel(WalkArgs a) {
             ct.vn = &s_vn;
         }
     }
-    AppendHint hint;
-    first_hint(a.q, a.pt.P, a.append_mode, hint);
     uint32_t src = a.src;
     Span sp;
     sp.rowptr = a.rowptr;
@@ -736,28 +734,24 @@ __global__ __launch_bounds__(kBlock) void walk_kernel(WalkArgs a) {
     } else if (a.nhost) {  // walkers of src spilled to host memory, read over PCIe
         hi = (uint64_t)a.nhost << kChunkLog2;
     } else if (a.ss.ds) {  // the decision of this iteration was taken on the device
-        const int32_t c = a.ss.ds->choice;
-        if (c < 0) return;
-        src = (uint32_t)c;
-        hi = qlen_of(a.q, src);
-        sp.nb = a.pt.node_off[src];
-        sp.ne = a.pt.node_off[src + 1];
-        sp.eb = a.pt.edge_off[src];
-        sp.zc = a.ss.ds->zerocopy;
-        sp.words = nullptr;
-        if (sp.zc) {
-            sp.rowptr = a.ss.zc_rowptr + a.pt.node_off[src];
-            sp.col = a.ss.zc_col + a.pt.edge_off[src];
-        } else {  // a raw slot, or a block slot whose bit streams decide_kernel entered in the table
-            const uint8_t *base = a.ss.slots + (size_t)a.ss.slot_of[src] * a.ss.slot_bytes;
-            sp.rowptr = (const uint64_t *)base;
-            sp.col = (const uint32_t *)(base + ((uint64_t)a.pt.node_off[src + 1] - a.pt.node_off[src] + 1) * 8);
-            sp.words = a.pt.words_tab[src];
-        }
+        const DevSched &ds = *a.ss.ds;
+        if (ds.choice < 0) return;
+        src = (uint32_t)ds.choice;
+        hi = ds.n;
+        sp.rowptr = ds.rowptr;
+        sp.col = ds.col;
+        sp.words = ds.words;
+        sp.zc = ds.zerocopy;
+        sp.nb = ds.nb;
+        sp.ne = ds.ne;
+        sp.eb = ds.eb;
     } else {
         lo = (uint64_t)a.chunk_lo << kChunkLog2;
         hi = min((uint64_t)a.n, (uint64_t)a.chunk_hi << kChunkLog2);
     }
+    if (lo + (uint64_t)blockIdx.x * BW >= hi) return;  // the device loop's grid is sized for any queue
+    AppendHint hint;
+    first_hint(a.q, a.pt.P, a.append_mode, (hi - lo) / BW, hint);
     // A pass: walkers [base, base + BW) clipped to n; base is a multiple of BW, so
     // it reads one chunk.
     for (uint64_t at = lo + (uint64_t)blockIdx.x * BW; at < hi; at += (uint64_t)gridDim.x * BW) {
@@ -901,21 +895,16 @@ __global__ __launch_bounds__(kBlock) void pack_meta_kernel(Queues q) { pack_meta
 // reads by known addresses is read at once, and the host, which needs the
 // lengths only, gets them before the chunks move (its next walk is behind this
 // kernel in the stream).
-__global__ __launch_bounds__(kBlock) void fixup_kernel(Queues q, Consumed d, Tables tab, const DevSched *ds) {
+__global__ __launch_bounds__(kBlock) void fixup_kernel(Queues q, Consumed d, Tables tab) {
     __shared__ uint32_t s_top, s_nlost, s_off[kMaxZcBatch + 1];
     const uint32_t tid = threadIdx.x;
-    // a device-scheduled iteration consumed the whole queue of its choice
-    const int32_t choice = ds ? ds->choice : -1;
-    const uint32_t n = ds ? (choice < 0 ? 0u : 1u) : d.n;
-    const uint32_t lo = ds ? 0u : d.chunk_lo, most = ds ? 0xFFFFFFFFu : d.chunk_hi;
-    const bool clear = ds || d.last;
-    const auto src = [&](uint32_t k) { return ds ? (uint32_t)choice : d.src[k]; };
+    const uint32_t n = d.n, lo = d.chunk_lo;
     const PoolCtl c = *q.ctl;
     const uint32_t len = tid < q.P ? qlen_of(q, tid) : 0u;
     const uint32_t fill = q.vcur && tid < kLogRegions ? log_fill(q, tid) : 0u;
     if (tid < n) {
-        const uint32_t nch = (qlen_of(q, src(tid)) + kChunk - 1) >> kChunkLog2;
-        const uint32_t hi = min(most, nch);
+        const uint32_t nch = (qlen_of(q, d.src[tid]) + kChunk - 1) >> kChunkLog2;
+        const uint32_t hi = min(d.chunk_hi, nch);
         s_off[tid + 1] = hi > lo ? hi - lo : 0;
     }
     __syncthreads();
@@ -934,36 +923,32 @@ __global__ __launch_bounds__(kBlock) void fixup_kernel(Queues q, Consumed d, Tab
         }
         after.top += s_nlost + s_off[n];
         *q.ctl = after;
-        if (!ds) {
-            tell_host(q, q.P, after.top);
-            tell_host(q, q.P + 1, 0);
-            tell_host(q, q.P + 2, 0);
-            tell_host(q, q.P + 3, after.overflow);
-        }
+        tell_host(q, q.P, after.top);
+        tell_host(q, q.P + 1, 0);
+        tell_host(q, q.P + 2, 0);
+        tell_host(q, q.P + 3, after.overflow);
     }
-    if (!ds) {  // no host waits for an iteration of the device loop
-        for (uint32_t i = tid; i < q.P; i += kBlock) {
-            uint32_t v = i == tid ? len : qlen_of(q, i);
+    for (uint32_t i = tid; i < q.P; i += kBlock) {
+        uint32_t v = i == tid ? len : qlen_of(q, i);
 #pragma unroll
-            for (uint32_t k = 0; k < kMaxZcBatch; k++) v = clear && k < n && d.src[k] == i ? 0u : v;
-            tell_host(q, i, v);
-        }
-        if (q.vcur && tid < kLogRegions) tell_host(q, q.P + 4 + tid, fill);
+        for (uint32_t k = 0; k < kMaxZcBatch; k++) v = d.last && k < n && d.src[k] == i ? 0u : v;
+        tell_host(q, i, v);
     }
+    if (q.vcur && tid < kLogRegions) tell_host(q, q.P + 4 + tid, fill);
     __syncthreads();
     const uint32_t top = s_top, nlost = s_nlost, cnt = s_off[n];
     for (uint32_t i = tid; i < nlost; i += kBlock) q.free_stack[top + i] = q.lost[i];
     uint32_t k = 0;
     for (uint32_t j = tid; j < cnt; j += kBlock) {
         while (j >= s_off[k + 1]) k++;
-        uint32_t *f = &q.frame[(size_t)src(k) * q.maxc + lo + (j - s_off[k])];
+        uint32_t *f = &q.frame[(size_t)d.src[k] * q.maxc + lo + (j - s_off[k])];
         q.free_stack[top + nlost + j] = *f;
         *f = kEmpty;
     }
     if (tid < n) {
-        const uint32_t p = src(tid);
-        if (clear) qlen_of(q, p) = 0;
-        if (!ds && d.leave) {
+        const uint32_t p = d.src[tid];
+        if (d.last) qlen_of(q, p) = 0;
+        if (d.leave) {
             tab.rowptr[p] = nullptr;
             tab.col[p] = nullptr;
             tab.zc[p] = 0;
@@ -1061,25 +1046,23 @@ struct PullArgs {
     uint64_t words[2];
 };
 
-__global__ __launch_bounds__(256) void pull_kernel(PullArgs a) {
+__device__ __forceinline__ void pull_words(const uint32_t *src, uint32_t *dst, uint64_t n) {
     constexpr int kAhead = 8;
-    const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (; i + (kAhead - 1) * stride < n; i += kAhead * stride) {
+        uint32_t v[kAhead];
 #pragma unroll
-    for (int s = 0; s < 2; s++) {
-        const uint32_t *src = a.src[s];
-        uint32_t *dst = a.dst[s];
-        const uint64_t n = a.words[s];
-        uint64_t i = tid;
-        for (; i + (kAhead - 1) * stride < n; i += kAhead * stride) {
-            uint32_t v[kAhead];
+        for (int k = 0; k < kAhead; k++) v[k] = __builtin_nontemporal_load(&src[i + k * stride]);
 #pragma unroll
-            for (int k = 0; k < kAhead; k++) v[k] = __builtin_nontemporal_load(&src[i + k * stride]);
-#pragma unroll
-            for (int k = 0; k < kAhead; k++) dst[i + k * stride] = v[k];
-        }
-        for (; i < n; i += stride) dst[i] = __builtin_nontemporal_load(&src[i]);
+        for (int k = 0; k < kAhead; k++) dst[i + k * stride] = v[k];
     }
+    for (; i < n; i += stride) dst[i] = __builtin_nontemporal_load(&src[i]);
+}
+
+__global__ __launch_bounds__(256) void pull_kernel(PullArgs a) {
+#pragma unroll
+    for (int s = 0; s < 2; s++) pull_words(a.src[s], a.dst[s], a.words[s]);
 }
 
 // Plain streaming copy of n 16-byte vectors (known HBM traffic: 16n read, 16n written).
@@ -1105,123 +1088,189 @@ __global__ void fill_u32_kernel(uint32_t *p, size_t n, uint32_t v) {
 }
 
 // ---- device-side scheduling ------------------------------------------------
-// One workgroup decides the iteration with the plain rules: the partition with
-// the most queued walkers (lowest id on ties); walk it in place if resident,
-// read it over PCIe if it holds fewer than zc_threshold walkers, else copy it
-// into a free slot or into the slot of the resident partition with the fewest
-// walkers.  Tables are updated here; the copy is done by load_kernel next.
-__global__ __launch_bounds__(1024) void decide_kernel(Queues q, SchedState ss, Parts pt, BlockImages bi) {
-    __shared__ unsigned long long s_best[1024];
-    __shared__ unsigned long long s_victim[1024];
-    __shared__ uint32_t s_free[1024];
-    const uint32_t tid = threadIdx.x, P = pt.P;
-    unsigned long long best = 0, victim = ~0ull;
-    for (uint32_t p = tid; p < P; p += 1024) {
-        const unsigned long long c = qlen_of(q, p);
-        const unsigned long long key = (c << 32) | (0xFFFFFFFFull - p);
-        if (c > 0 && key > best) best = key;
+// Lowest / highest value of the workgroup.
+template <bool MAX>
+__device__ __forceinline__ unsigned long long block_extreme(unsigned long long v, unsigned long long *s_wave) {
+    for (int off = 32; off > 0; off >>= 1) {
+        const unsigned long long o = __shfl_xor(v, off, 64);
+        v = (MAX ? o > v : o < v) ? o : v;
     }
-    s_best[tid] = best;
+    if ((threadIdx.x & 63u) == 0) s_wave[threadIdx.x >> 6] = v;
     __syncthreads();
-    for (uint32_t off = 512; off > 0; off >>= 1) {
-        if (tid < off && s_best[tid + off] > s_best[tid]) s_best[tid] = s_best[tid + off];
-        __syncthreads();
+    for (int w = 0; w < kBlock / 64; w++) {
+        const unsigned long long o = s_wave[w];
+        v = (MAX ? o > v : o < v) ? o : v;
     }
-    best = s_best[0];
-    DevSched *ds = ss.ds;
+    return v;
+}
+
+// What decide_kernel may need to know of a partition.
+struct PartState {
+    uint32_t len = 0, nb = 0, ne = 0, resident = 0;
+    uint64_t eb = 0, ee = 0;
+    int32_t slot = -1;
+    const uint32_t *words = nullptr;
+};
+
+__device__ __forceinline__ PartState part_state(const Queues &q, const SchedState &ss, const Parts &pt, uint32_t p) {
+    PartState o;
+    o.len = qlen_of(q, p);
+    o.nb = pt.node_off[p];
+    o.ne = pt.node_off[p + 1];
+    o.eb = pt.edge_off[p];
+    o.ee = pt.edge_off[p + 1];
+    o.resident = ss.resident[p];
+    o.slot = ss.slot_of[p];
+    o.words = pt.words_tab[p];
+    return o;
+}
+
+// One workgroup ends the iteration before (its queue's chunks, the popped and the
+// lost ones go back to the free stack, as in fixup_kernel) and decides the next
+// with the plain rules: the partition with the most queued walkers (lowest id
+// on ties); walk it in place if resident, read it over PCIe if it holds fewer
+// than zc_threshold walkers, else copy it into a free slot or into the slot of
+// the resident partition with the fewest walkers.  Tables are updated here; the
+// copy is done by load_kernel next.
+//
+// Nothing but round trips: every thread reads its own partition's state at
+// once, so that the one whose partition is chosen holds all that the copy and the
+// walk need, and these read one record instead of looking it up.
+__global__ __launch_bounds__(kBlock) void decide_kernel(Queues q, SchedState ss, Parts pt, BlockImages bi) {
+    __shared__ unsigned long long s_wave[3][kBlock / 64];
+    __shared__ uint32_t s_prev, s_resident;
+    const uint32_t tid = threadIdx.x, P = pt.P;
+    DevSched d = *ss.ds;
+    const PoolCtl ctl = *q.ctl;
+    PartState own;
+    if (tid < P) own = part_state(q, ss, pt, tid);
+    const int32_t in_slot = tid < ss.nslots ? ss.part_in_slot[tid] : 0;
+    const int32_t prev = d.choice;
+    unsigned long long best = 0;
+    for (uint32_t p = tid; p < P; p += kBlock) {
+        const unsigned long long c = p == tid ? own.len : qlen_of(q, p);
+        if ((int32_t)p == prev) {
+            s_prev = (uint32_t)c;
+        } else if (c) {
+            const unsigned long long key = (c << 32) | (0xFFFFFFFFull - p);
+            best = key > best ? key : best;
+        }
+    }
+    best = block_extreme<true>(best, s_wave[0]);
+    if (prev >= 0) {
+        uint32_t nch = (s_prev + kChunk - 1) >> kChunkLog2, nlost = min(ctl.nlost, kLostCap);
+        const uint32_t top = ctl.top - min(ctl.popped, ctl.top);
+        PoolCtl after{top, 0, 0, ctl.overflow};
+        if (top + nlost + nch > q.nchunks) {
+            after.overflow |= 16u;
+            nlost = nch = 0;
+        }
+        for (uint32_t i = tid; i < nlost; i += kBlock) q.free_stack[top + i] = q.lost[i];
+        for (uint32_t j = tid; j < nch; j += kBlock) {
+            uint32_t *f = &q.frame[(size_t)prev * q.maxc + j];
+            q.free_stack[top + nlost + j] = *f;
+            *f = kEmpty;
+        }
+        if (tid == 0) {
+            after.top += nlost + nch;
+            *q.ctl = after;
+            qlen_of(q, (uint32_t)prev) = 0;
+        }
+    }
+    d.load = 0;
+    d.zerocopy = 0;
+    d.victim = -1;
     if (best == 0) {
         if (tid == 0) {
-            ds->choice = -1;
-            ds->load = 0;
-            ds->zerocopy = 0;
-            ds->victim = -1;
+            d.choice = -1;
+            *ss.ds = d;
         }
         return;
     }
     const uint32_t c = 0xFFFFFFFFu - (uint32_t)(best & 0xFFFFFFFFull);
-    const uint64_t cnt = best >> 32;
-    const bool need_slot = !ss.resident[c] && cnt >= ss.zc_threshold;
-    uint32_t fr = 0xFFFFFFFFu;
-    if (need_slot) {
-        for (uint32_t s = tid; s < ss.nslots; s += 1024)
-            if (ss.part_in_slot[s] < 0 && s < fr) fr = s;
-        for (uint32_t p = tid; p < P; p += 1024) {
-            if (!ss.resident[p] || p == c) continue;
-            const unsigned long long key = ((unsigned long long)qlen_of(q, p) << 32) | p;
-            if (key < victim) victim = key;
-        }
+    const bool chosen = tid == c % kBlock;
+    if (chosen) {
+        if (c != tid) own = part_state(q, ss, pt, c);
+        s_resident = own.resident;
     }
-    s_free[tid] = fr;
-    s_victim[tid] = victim;
     __syncthreads();
-    for (uint32_t off = 512; off > 0; off >>= 1) {
-        if (tid < off) {
-            if (s_free[tid + off] < s_free[tid]) s_free[tid] = s_free[tid + off];
-            if (s_victim[tid + off] < s_victim[tid]) s_victim[tid] = s_victim[tid + off];
+    const bool need_slot = !s_resident && (best >> 32) >= ss.zc_threshold;
+    unsigned long long free_slot = ~0ull, victim = ~0ull;
+    if (need_slot) {
+        for (uint32_t s = tid; s < ss.nslots; s += kBlock)
+            if ((s == tid ? in_slot : ss.part_in_slot[s]) < 0 && s < free_slot) free_slot = s;
+        for (uint32_t p = tid; p < P; p += kBlock) {
+            // (the chosen thread's own state may be another partition's by now)
+            const bool mine = p == tid && !chosen;
+            if (p == c || !(mine ? own.resident : ss.resident[p])) continue;
+            const unsigned long long len = (int32_t)p == prev ? 0 : mine ? own.len : qlen_of(q, p);
+            const unsigned long long key = (len << 32) | p;
+            victim = key < victim ? key : victim;
         }
-        __syncthreads();
+        free_slot = block_extreme<false>(free_slot, s_wave[1]);
+        victim = block_extreme<false>(victim, s_wave[2]);
     }
-    if (tid != 0) return;
-    ds->choice = (int32_t)c;
-    ds->iterations++;
-    ds->victim = -1;
-    ds->load = 0;
-    ds->zerocopy = 0;
-    if (ss.resident[c]) return;
-    if (!need_slot) {
-        ds->zerocopy = 1;
-        ds->zc_calls++;
-        return;
-    }
-    uint32_t slot = s_free[0];
-    if (slot == 0xFFFFFFFFu) {
-        if (s_victim[0] == ~0ull) {  // nothing to evict: read over PCIe instead
-            ds->zerocopy = 1;
-            ds->zc_calls++;
+    if (!chosen) return;
+    const uint64_t n1 = (uint64_t)own.ne - own.nb + 1, m = own.ee - own.eb;
+    d.choice = (int32_t)c;
+    d.iterations++;
+    d.n = own.len;
+    d.nb = own.nb;
+    d.ne = own.ne;
+    d.eb = own.eb;
+    int32_t slot = own.slot;
+    if (!own.resident) {
+        if (!need_slot || (free_slot == ~0ull && victim == ~0ull)) {  // few walkers, or nothing to evict
+            d.zerocopy = 1;
+            d.zc_calls++;
+            d.rowptr = ss.zc_rowptr + own.nb;
+            d.col = ss.zc_col + own.eb;
+            d.words = nullptr;
+            *ss.ds = d;
             return;
         }
-        const uint32_t v = (uint32_t)(s_victim[0] & 0xFFFFFFFFull);
-        slot = (uint32_t)ss.slot_of[v];
-        ss.slot_of[v] = -1;
-        ss.resident[v] = 0;
-        ss.rowptr_tab[v] = nullptr;
-        ss.col_tab[v] = nullptr;
-        bi.words_tab[v] = nullptr;
-        ds->victim = (int32_t)v;
+        slot = (int32_t)free_slot;
+        if (free_slot == ~0ull) {
+            const uint32_t v = (uint32_t)(victim & 0xFFFFFFFFull);
+            slot = ss.slot_of[v];
+            ss.slot_of[v] = -1;
+            ss.resident[v] = 0;
+            ss.rowptr_tab[v] = nullptr;
+            ss.col_tab[v] = nullptr;
+            bi.words_tab[v] = nullptr;
+            d.victim = (int32_t)v;
+        }
     }
     uint8_t *base = ss.slots + (size_t)slot * ss.slot_bytes;
-    const uint64_t n1 = (uint64_t)pt.node_off[c + 1] - pt.node_off[c] + 1;
-    const uint64_t m = pt.edge_off[c + 1] - pt.edge_off[c];
-    ss.slot_of[c] = (int32_t)slot;
-    ss.part_in_slot[slot] = (int32_t)c;
-    ss.resident[c] = 1;
-    ss.rowptr_tab[c] = (const uint64_t *)base;
-    ss.col_tab[c] = (const uint32_t *)(base + n1 * 8);
-    const uint64_t img = bi.img ? bi.size[c] : 0;  // block image bytes, 0 = raw columns
-    bi.words_tab[c] = img ? ss.col_tab[c] + 2 * ((m + kBlockEdges - 1) / kBlockEdges + 1) : nullptr;
-    ds->slot = (int32_t)slot;
-    ds->load = 1;
-    ds->loads++;
-    ds->h2d_bytes += n1 * 8 * ss.rp_host + (img ? img : m * 4);
+    d.rowptr = (const uint64_t *)base;
+    d.col = (const uint32_t *)(base + n1 * 8);
+    d.words = own.words;
+    if (!own.resident) {
+        const uint64_t img = bi.img ? bi.size[c] : 0;  // block image bytes, 0 = raw columns
+        d.words = img ? d.col + 2 * ((m + kBlockEdges - 1) / kBlockEdges + 1) : nullptr;
+        ss.slot_of[c] = slot;
+        ss.part_in_slot[slot] = (int32_t)c;
+        ss.resident[c] = 1;
+        ss.rowptr_tab[c] = d.rowptr;
+        ss.col_tab[c] = d.col;
+        bi.words_tab[c] = d.words;
+        d.load = 1;
+        d.from[0] = (const uint32_t *)(ss.zc_rowptr + own.nb);
+        d.from[1] = img ? (const uint32_t *)(bi.img + bi.off[c]) : ss.zc_col + own.eb;
+        d.count[0] = 2 * n1;
+        d.count[1] = img ? img / 4 : m;
+        d.loads++;
+        d.h2d_bytes += n1 * 8 * ss.rp_host + (img ? img : m * 4);
+    }
+    *ss.ds = d;
 }
 
 // Copy the decided partition from pinned host memory into its slot: rowptr
-// slice, then the col slice or (block slots) the partition's block image, as
-// 4-byte words (grid-stride reads over PCIe).
-__global__ __launch_bounds__(256) void load_kernel(SchedState ss, Parts pt, BlockImages bi) {
-    const DevSched *ds = ss.ds;
+// slice, then the col slice or (block slots) the partition's block image.
+__global__ __launch_bounds__(256) void load_kernel(const DevSched *ds) {
     if (!ds->load) return;
-    const uint32_t c = (uint32_t)ds->choice;
-    const uint64_t n1 = (uint64_t)pt.node_off[c + 1] - pt.node_off[c] + 1;
-    const uint64_t img = bi.img ? bi.size[c] : 0;
-    const uint64_t m = img ? img / 4 : pt.edge_off[c + 1] - pt.edge_off[c];  // words after the rowptr slice
-    uint32_t *dst = (uint32_t *)(ss.slots + (size_t)ds->slot * ss.slot_bytes);
-    const uint32_t *src_r = (const uint32_t *)(ss.zc_rowptr + pt.node_off[c]);
-    const uint32_t *src_c = img ? (const uint32_t *)(bi.img + bi.off[c]) : ss.zc_col + pt.edge_off[c];
-    const uint64_t nr = 2 * n1, total = nr + m;
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride)
-        dst[i] = i < nr ? src_r[i] : src_c[i - nr];
+    pull_words(ds->from[0], (uint32_t *)ds->rowptr, ds->count[0]);
+    pull_words(ds->from[1], (uint32_t *)ds->col, ds->count[1]);
 }
 
 // Unpacks a packed partition image into the col slice of an HBM slot whose

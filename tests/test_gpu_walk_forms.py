@@ -28,3 +28,22 @@ def test_partition_counts(P, append_mode):
                         resident_batch=16, zc_batch=16, append_mode=append_mode)
         counts, ends = eng.pagerank(w, l, endpoints=True)
         assert np.array_equal(counts, rc) and np.array_equal(ends, re)
+
+
+@pytest.mark.parametrize("slots", [1, 3, 400])
+@pytest.mark.parametrize("P", [1, 2, 255, 256, 257, 600])
+def test_device_loop_partition_counts(P, slots):
+    """The device's decisions with a partition a thread, one more, several; few
+    slots (evictions), some, and one for each of most partitions."""
+    print(f"device loop P={P} slots={slots}", flush=True)
+    rng = np.random.default_rng(P)
+    g = lt.Graph.from_csr(4 * np.arange(P + 1, dtype=np.uint64), rng.integers(0, P, 4 * P).astype(np.uint32))
+    part = lt.Partition.build(g, 32)
+    assert part.count == P
+    w, l = 2503, 4
+    rc, re, _ = oracle.pagerank(g.rowptr(), g.col(), w, l, endpoints=True, threads=8)
+    for zc in (0, 5):
+        eng = lt.Engine(g, part, num_device_partitions=min(slots, P), zerocopy_threshold=zc, device_schedule=1)
+        for _ in range(2):
+            counts, ends = eng.pagerank(w, l, endpoints=True)
+            assert np.array_equal(counts, rc) and np.array_equal(ends, re)
