@@ -180,7 +180,7 @@ struct WalkArgs {
     // (resident slots, or views of the pinned host graph for a zero-copy
     // batch), so a walker moving between them keeps walking and no queue
     // being consumed is appended to.  Queue k occupies [voff[k], voff[k+1])
-    // of one virtual range, each start a multiple of kChunk.
+    // of one virtual range, each start a multiple of a pass's walkers.
     uint32_t nsrc;
     // Spilled walkers (nhost > 0): walkers of src kept in pinned host memory,
     // read by the kernel over PCIe; piece k holds hn[k] <= kChunk walkers at

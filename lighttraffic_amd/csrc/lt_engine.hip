@@ -401,7 +401,7 @@ struct Engine {
     int app_kind = APP_PAGERANK;
     size_t lds_bytes(int wpt = kWpt) const { return append_lds_bytes(P, wpt); }
     bool append_gen() const { return P > kDirectMaxP || cfg.append_mode != 0; }
-    lt_status launch_walk(const WalkArgs &a, uint64_t walkers, hipStream_t s);
+    lt_status launch_walk(WalkArgs &a, uint64_t walkers, hipStream_t s);
     uint64_t partition_bytes(uint32_t p) const {
         return ((uint64_t)part.node_off[p + 1] - part.node_off[p] + 1) * 8 +
                (part.edge_off[p + 1] - part.edge_off[p]) * 4;
@@ -1138,7 +1138,7 @@ lt_status Engine::fetch_partition(uint32_t p, uint64_t *rowptr_out, uint32_t *co
 // (a thread walks its walkers one after another), 2 or 4 for large slices,
 // where the per-workgroup append cost (histogram, scan, one atomic per
 // destination queue) is spread over more walkers.
-lt_status Engine::launch_walk(const WalkArgs &a, uint64_t walkers, hipStream_t s) {
+lt_status Engine::launch_walk(WalkArgs &a, uint64_t walkers, hipStream_t s) {
     // a walk of one source that stays in it reads no table
     if (a.span_resident || a.nsrc) LT_TRY(flush_tables());
     const uint64_t fill = (uint64_t)num_cu * 4 * 6 * 64;  // threads for ~6 waves per SIMD
@@ -1149,7 +1149,16 @@ lt_status Engine::launch_walk(const WalkArgs &a, uint64_t walkers, hipStream_t s
     const uint64_t bw = (uint64_t)kBlock * wpt;
     // with loads going on, room for a pull kernel's workgroups beside the walk's
     const uint64_t most = walk_grid[app_kind][wpt] - (nslots < P && walk_grid[app_kind][wpt] > kPullGrid ? kPullGrid : 0);
-    const int grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((walkers + bw - 1) / bw, most));
+    // A batch's queues start a pass each.  (Starting a chunk each, with a grid for the
+    // sum of walkers, left sixteen short queues to one workgroup, one after
+    // another: 300-450 us a launch, two fifths of the s20 ppr job's time.)
+    uint64_t passes = (walkers + bw - 1) / bw;
+    if (a.nsrc) {
+        a.voff[0] = 0;
+        for (uint32_t k = 0; k < a.nsrc; k++) a.voff[k + 1] = a.voff[k] + (counts[a.srcs[k]] + bw - 1) / bw * bw;
+        passes = a.voff[a.nsrc] / bw;
+    }
+    const int grid = (int)std::max<uint64_t>(1, std::min<uint64_t>(passes, most));
     walk_fn(app_kind, wpt, append_gen())<<<grid, kBlock, lds_bytes(wpt), s>>>(a);
     LT_HIP(hipGetLastError());
     meta_dirty = true;
@@ -1507,14 +1516,12 @@ lt_status Engine::walk_batch(const std::vector<uint32_t> &parts, bool zerocopy) 
     d.last = 1;
     d.leave = zerocopy ? 1 : 0;
     a.src = parts[0];
-    a.voff[0] = 0;
     uint64_t total = 0;
     for (uint32_t k = 0; k < d.n; k++) {
         const uint32_t p = parts[k];
         d.src[k] = a.srcs[k] = p;
         if (zerocopy)
             LT_TRY(table_entry(p, zc_rowptr + part.node_off[p], zc_col + part.edge_off[p], nullptr, true));
-        a.voff[k + 1] = a.voff[k] + (counts[p] + kChunk - 1) / kChunk * kChunk;
         total += counts[p];
     }
     EventTimer &phase = zerocopy ? t_zc : t_compute;
