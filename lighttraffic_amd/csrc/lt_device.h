@@ -68,14 +68,21 @@ __host__ __device__ __forceinline__ uint32_t &qlen_of(const Queues &q, uint32_t 
     return q.qlen[(size_t)p * kQStride];
 }
 
+// All that a walker entering a partition needs, in half a line: one gather of
+// each of three 16-byte pieces.
+struct __attribute__((aligned(64))) PartRec {
+    const uint64_t *rowptr;  // HBM slot rowptr, nullptr if not resident
+    const uint32_t *col;     // raw col slice, or the block headers of a packed slot
+    const uint32_t *words;   // bit streams of a packed slot, nullptr for raw columns
+    uint64_t eb;             // first edge
+    uint32_t nb, ne;         // first vertex, and the one past the last
+};
+
 struct Parts {
     const uint32_t *node_off;  // [P+1]
     const uint64_t *edge_off;  // [P+1]
     const uint32_t *lut;       // partition of vertex (j << lut_shift)
-    const uint64_t *const *rowptr_tab;  // [P] HBM slot rowptr, nullptr if not resident
-    const uint32_t *const *col_tab;     // [P] raw col slice, or the block headers of a packed slot
-    const uint32_t *const *words_tab;   // [P] bit streams of a packed slot, nullptr for raw columns
-    const uint8_t *zc_part;             // [P] 1 while the table points p at host memory (zero-copy batch)
+    const PartRec *rec;        // [P]
     uint32_t lut_shift;
     uint32_t P;
 };
@@ -130,8 +137,7 @@ struct SchedState {
     int32_t *slot_of;         // [P] slot or -1
     int32_t *part_in_slot;    // [nslots] partition or -1
     uint8_t *resident;        // [P]
-    const uint64_t **rowptr_tab;  // writable views of Parts' tables
-    const uint32_t **col_tab;
+    PartRec *rec;             // [P] writable view of Parts::rec
     uint8_t *slots;
     uint64_t slot_bytes;
     uint32_t nslots;
@@ -143,10 +149,9 @@ struct SchedState {
 
 // Block slots in the device loop (decide_kernel, load_kernel): partition p's
 // block image is size[p] bytes at img + off[p] (mapped host memory), and its
-// bit streams are entered in words_tab when it is loaded; img == nullptr or
+// bit streams are entered in its record when it is loaded; img == nullptr or
 // size[p] == 0: raw columns.
 struct BlockImages {
-    const uint32_t **words_tab;  // writable view of Parts::words_tab
     const uint8_t *img;
     const uint64_t *off;
     const uint64_t *size;
@@ -166,7 +171,7 @@ struct WalkArgs {
     uint32_t n;           // walkers in its queue
     uint32_t chunk_lo;    // first chunk of the slice
     uint32_t chunk_hi;    // one past the last chunk of the slice
-    int zerocopy;         // src slice is read over PCIe
+    int zerocopy;         // src's slice (or srcs') is read over PCIe
     int span_resident;    // keep walking through HBM-resident partitions
     // How a pass appends its leaving walkers to their queues: 0, one queue
     // reservation per (workgroup, destination) and the walkers staged in LDS
@@ -176,11 +181,11 @@ struct WalkArgs {
     // ONE_LEVEL_QUEUE build, src/WalkManager.h:195-209).
     int append_mode;
     // Batch (span_resident only): nsrc > 0 consumes the whole queues of
-    // srcs[0..nsrc), each entered in the partition table for the launch
-    // (resident slots, or views of the pinned host graph for a zero-copy
-    // batch), so a walker moving between them keeps walking and no queue
-    // being consumed is appended to.  Queue k occupies [voff[k], voff[k+1])
-    // of one virtual range, each start a multiple of a pass's walkers.
+    // srcs[0..nsrc) (the rest of srcs: kEmpty), all resident or, with zerocopy,
+    // all read from the pinned host graph, so a walker moving between them
+    // keeps walking and no queue being consumed is appended to.  Queue k
+    // occupies [voff[k], voff[k+1]) of one virtual range, each start a multiple
+    // of a pass's walkers.
     uint32_t nsrc;
     // Spilled walkers (nhost > 0): walkers of src kept in pinned host memory,
     // read by the kernel over PCIe; piece k holds hn[k] <= kChunk walkers at
@@ -211,18 +216,9 @@ constexpr uint32_t kTableBatch = 32;
 struct TableBatch {
     uint32_t n;
     uint32_t part[kTableBatch];
-    uint8_t zc[kTableBatch];  // 1: the entry points at host memory (zero-copy batch)
     const uint64_t *rowptr[kTableBatch];  // nullptr: not resident
     const uint32_t *col[kTableBatch];
     const uint32_t *words[kTableBatch];
-};
-
-// Where the tables lie.
-struct Tables {
-    const uint64_t **rowptr;
-    const uint32_t **col;
-    const uint32_t **words;
-    uint8_t *zc;
 };
 
 // What a walk launch consumed (fixup_kernel): chunks [chunk_lo, chunk_hi) of
@@ -232,7 +228,6 @@ struct Consumed {
     uint32_t src[kMaxZcBatch];
     uint32_t chunk_lo, chunk_hi;
     int last;    // the queues end with those chunks
-    int leave;   // src[] leave the partition table (zero-copy batch)
 };
 
 struct InitArgs {

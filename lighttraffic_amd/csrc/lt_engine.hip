@@ -164,9 +164,7 @@ struct Engine {
     uint64_t *d_edge_off = nullptr;
     uint32_t *d_lut = nullptr;
     uint32_t lut_shift = 0;
-    const uint64_t **d_rowptr_tab = nullptr;
-    const uint32_t **d_col_tab = nullptr;
-    const uint32_t **d_words_tab = nullptr;  // packed slots (pack_partitions = 2): bit streams
+    PartRec *d_rec = nullptr;
 
     // HBM partition cache
     uint32_t nslots = 0;
@@ -291,7 +289,6 @@ struct Engine {
     DevSched *d_ds = nullptr;
     int32_t *d_slot_of = nullptr, *d_part_in_slot = nullptr;
     uint8_t *d_resident = nullptr;
-    uint8_t *d_zc_part = nullptr;  // [P] partitions of the running zero-copy batch
     bool rp_resident = false;      // rowptr of the whole graph kept in HBM (zc_rowptr points there)
     uint64_t *d_pk_off = nullptr, *d_pk_size = nullptr;  // device loop with block slots: image table
     const uint8_t *d_pk_img = nullptr;                     // device view of the pinned images (block slots)
@@ -335,7 +332,6 @@ struct Engine {
     lt_status wait_meta();
     TableBatch table_due{};  // table updates of the next walk launch
     lt_status flush_tables();
-    Tables tables() const { return {d_rowptr_tab, d_col_tab, d_words_tab, d_zc_part}; }
     lt_status process(uint32_t p, bool zerocopy, uint64_t walkers_hint);
     lt_status process_zc(uint32_t c, const uint8_t *pending);
     lt_status walk_batch(const std::vector<uint32_t> &parts, bool zerocopy);
@@ -377,7 +373,6 @@ struct Engine {
         }
     }
     lt_status set_table(uint32_t p, bool present);
-    lt_status table_entry(uint32_t p, const uint64_t *rp, const uint32_t *cp, const uint32_t *wp, bool zc);
     bool can_run_flat() const;
     lt_status run_flat(const RunSpec &rs, ResultHelpers &help);
     bool job_finished = false;  // run_flat has handed the job's results out
@@ -416,9 +411,7 @@ Engine::~Engine() {
     dfree(d_node_off);
     dfree(d_edge_off);
     dfree(d_lut);
-    dfree(d_rowptr_tab);
-    dfree(d_col_tab);
-    dfree(d_words_tab);
+    dfree(d_rec);
     dfree(d_slots);
     dfree(d_rowptr32);
     dfree(q.slab);
@@ -449,7 +442,6 @@ Engine::~Engine() {
     dfree(d_slot_of);
     dfree(d_part_in_slot);
     dfree(d_resident);
-    dfree(d_zc_part);
     dfree(d_rowptr_all);
     dfree(d_pk_off);
     dfree(d_pk_size);
@@ -545,12 +537,11 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
     for (size_t j = 0; j < nlut; j++) lut[j] = part.find((uint32_t)(j << lut_shift));
     LT_TRY(dmalloc(&d_lut, nlut));
     LT_HIP(hipMemcpy(d_lut, lut.data(), 4 * nlut, hipMemcpyHostToDevice));
-    LT_TRY(dmalloc(&d_rowptr_tab, P));
-    LT_TRY(dmalloc(&d_col_tab, P));
-    LT_HIP(hipMemset(d_rowptr_tab, 0, sizeof(void *) * P));
-    LT_HIP(hipMemset(d_col_tab, 0, sizeof(void *) * P));
-    LT_TRY(dmalloc(&d_words_tab, P));
-    LT_HIP(hipMemset(d_words_tab, 0, sizeof(void *) * P));
+    std::vector<PartRec> rec(P);
+    for (uint32_t p = 0; p < P; p++)
+        rec[p] = {nullptr, nullptr, nullptr, part.edge_off[p], part.node_off[p], part.node_off[p + 1]};
+    LT_TRY(dmalloc(&d_rec, P));
+    LT_HIP(hipMemcpy(d_rec, rec.data(), sizeof(PartRec) * P, hipMemcpyHostToDevice));
 
     // Packed copies: the images are built once per graph and partition table.
     // Format 1 travels gap-coded and is unpacked into raw slots; format 2 is
@@ -660,8 +651,6 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
         LT_TRY(dmalloc(&d_part_in_slot, nslots));
         LT_TRY(dmalloc(&d_resident, P));
     }
-    LT_TRY(dmalloc(&d_zc_part, P));
-    LT_HIP(hipMemset(d_zc_part, 0, P));
     zc_batch = cfg.zc_batch > 0 ? (uint32_t)cfg.zc_batch
                                 : (cfg.policy == LT_SCHED_LEARNED && cfg.span == LT_SPAN_RESIDENT ? kMaxZcBatch : 1);
     zc_batch = std::min(zc_batch, kMaxZcBatch);
@@ -835,7 +824,7 @@ lt_status Engine::count_log(uint32_t n, uint32_t most) {
 
 lt_status Engine::launch_fixup(const Consumed &d) {
     q.seq = ++meta_seq;
-    fixup_kernel<<<1, kBlock, 0, s_compute>>>(q, d, tables());
+    fixup_kernel<<<1, kBlock, 0, s_compute>>>(q, d);
     LT_HIP(hipGetLastError());
     meta_dirty = false;
     meta_seen = false;
@@ -904,22 +893,8 @@ lt_status Engine::read_meta() {
     return LT_OK;
 }
 
+// Queue a table update for the next walk launch that reads tables (flush_tables).
 lt_status Engine::set_table(uint32_t p, bool present) {
-    const uint64_t *rp = nullptr;
-    const uint32_t *cp = nullptr, *wp = nullptr;
-    if (present) {
-        uint64_t *r;
-        uint32_t *c;
-        slot_ptrs(p, &r, &c);
-        rp = r;
-        cp = c;
-        wp = slot_words(p, cp);
-    }
-    return table_entry(p, rp, cp, wp, false);
-}
-
-// Queue a table update for the next walk launch (flush_tables).
-lt_status Engine::table_entry(uint32_t p, const uint64_t *rp, const uint32_t *cp, const uint32_t *wp, bool zc) {
     uint32_t k = 0;
     while (k < table_due.n && table_due.part[k] != p) k++;  // the last update of a partition counts
     if (k == kTableBatch) {
@@ -928,16 +903,22 @@ lt_status Engine::table_entry(uint32_t p, const uint64_t *rp, const uint32_t *cp
     }
     if (k == table_due.n) table_due.n++;
     table_due.part[k] = p;
-    table_due.rowptr[k] = rp;
-    table_due.col[k] = cp;
-    table_due.words[k] = wp;
-    table_due.zc[k] = zc ? 1 : 0;
+    table_due.rowptr[k] = nullptr;
+    table_due.col[k] = table_due.words[k] = nullptr;
+    if (present) {
+        uint64_t *r;
+        uint32_t *c;
+        slot_ptrs(p, &r, &c);
+        table_due.rowptr[k] = r;
+        table_due.col[k] = c;
+        table_due.words[k] = slot_words(p, c);
+    }
     return LT_OK;
 }
 
 lt_status Engine::flush_tables() {
     if (table_due.n == 0) return LT_OK;
-    set_tables_kernel<<<1, 64, 0, s_compute>>>(tables(), table_due);
+    set_tables_kernel<<<1, 64, 0, s_compute>>>(d_rec, table_due);
     LT_HIP(hipGetLastError());
     table_due.n = 0;
     return LT_OK;
@@ -1179,10 +1160,7 @@ lt_status Engine::process(uint32_t p, bool zerocopy, uint64_t walkers) {
     a.pt.node_off = d_node_off;
     a.pt.edge_off = d_edge_off;
     a.pt.lut = d_lut;
-    a.pt.rowptr_tab = d_rowptr_tab;
-    a.pt.col_tab = d_col_tab;
-    a.pt.words_tab = d_words_tab;
-    a.pt.zc_part = d_zc_part;
+    a.pt.rec = d_rec;
     a.pt.lut_shift = lut_shift;
     a.pt.P = P;
     a.src = p;
@@ -1488,11 +1466,10 @@ lt_status Engine::process_resident(uint32_t c, int kind, uint8_t *prefetched) {
 }
 
 // One launch over the whole queues of `parts` (span resident).  Resident
-// partitions are in the partition table already; with zerocopy, the
-// partitions are entered in it as views of the pinned host graph for the
-// launch (and flagged in zc_part for the PCIe byte count).  Either way a
-// walker that moves between them keeps walking, and no queue being consumed
-// is appended to.
+// partitions are in the partition table; of a zero-copy batch the kernel
+// knows the members.  (Entered in the table for the launch as well, they cost a
+// launch of their own before it.)  Either way a walker that moves between them
+// keeps walking, and no queue being consumed is appended to.
 lt_status Engine::walk_batch(const std::vector<uint32_t> &parts, bool zerocopy) {
     WalkArgs a{};
     a.append_mode = cfg.append_mode;
@@ -1501,10 +1478,7 @@ lt_status Engine::walk_batch(const std::vector<uint32_t> &parts, bool zerocopy) 
     a.pt.node_off = d_node_off;
     a.pt.edge_off = d_edge_off;
     a.pt.lut = d_lut;
-    a.pt.rowptr_tab = d_rowptr_tab;
-    a.pt.col_tab = d_col_tab;
-    a.pt.words_tab = d_words_tab;
-    a.pt.zc_part = d_zc_part;
+    a.pt.rec = d_rec;
     a.pt.lut_shift = lut_shift;
     a.pt.P = P;
     a.span_resident = 1;
@@ -1514,14 +1488,13 @@ lt_status Engine::walk_batch(const std::vector<uint32_t> &parts, bool zerocopy) 
     d.n = a.nsrc = (uint32_t)parts.size();
     d.chunk_hi = 0xFFFFFFFFu;
     d.last = 1;
-    d.leave = zerocopy ? 1 : 0;
+    a.zerocopy = zerocopy ? 1 : 0;
+    std::fill(a.srcs, a.srcs + kMaxZcBatch, kEmpty);
     a.src = parts[0];
     uint64_t total = 0;
     for (uint32_t k = 0; k < d.n; k++) {
         const uint32_t p = parts[k];
         d.src[k] = a.srcs[k] = p;
-        if (zerocopy)
-            LT_TRY(table_entry(p, zc_rowptr + part.node_off[p], zc_col + part.edge_off[p], nullptr, true));
         total += counts[p];
     }
     EventTimer &phase = zerocopy ? t_zc : t_compute;
@@ -1933,8 +1906,7 @@ SchedState Engine::sched_state(bool device) const {
     ss.slot_of = d_slot_of;
     ss.part_in_slot = d_part_in_slot;
     ss.resident = d_resident;
-    ss.rowptr_tab = d_rowptr_tab;
-    ss.col_tab = d_col_tab;
+    ss.rec = d_rec;
     ss.slots = d_slots;
     ss.slot_bytes = slot_sz;
     ss.nslots = nslots;
@@ -1973,10 +1945,7 @@ lt_status Engine::scheduler_loop_device() {
     a.pt.node_off = d_node_off;
     a.pt.edge_off = d_edge_off;
     a.pt.lut = d_lut;
-    a.pt.rowptr_tab = d_rowptr_tab;
-    a.pt.col_tab = d_col_tab;
-    a.pt.words_tab = d_words_tab;
-    a.pt.zc_part = d_zc_part;
+    a.pt.rec = d_rec;
     a.pt.lut_shift = lut_shift;
     a.pt.P = P;
     a.span_resident = cfg.span == LT_SPAN_RESIDENT ? 1 : 0;
@@ -1986,7 +1955,6 @@ lt_status Engine::scheduler_loop_device() {
     // known on the device, so the grid is the full occupancy grid of that WPT
     const int dwpt = cfg.walkers_per_thread > 0 ? cfg.walkers_per_thread : 1;
     BlockImages bi{};
-    bi.words_tab = d_words_tab;
     bi.img = slot_packed ? d_pk_img : nullptr;
     bi.off = d_pk_off;
     bi.size = d_pk_size;
@@ -2323,10 +2291,7 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
         ia.pt.node_off = d_node_off;
         ia.pt.edge_off = d_edge_off;
         ia.pt.lut = d_lut;
-        ia.pt.rowptr_tab = d_rowptr_tab;
-        ia.pt.col_tab = d_col_tab;
-        ia.pt.words_tab = d_words_tab;
-        ia.pt.zc_part = d_zc_part;
+        ia.pt.rec = d_rec;
         ia.pt.lut_shift = lut_shift;
         ia.pt.P = P;
         ia.stats = d_stats;

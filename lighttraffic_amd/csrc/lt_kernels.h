@@ -563,8 +563,8 @@ __device__ __forceinline__ void step_ppr(Walker &w, const Span &sp, const AppArg
     if (w.step == 0) return;
     const uint64_t *r = sp.rowptr + (w.cur - sp.nb);
     const uint64_t b = r[0], d = r[1] - b;
+    const u32x4 x = draw(a.seed, walker_id(w), w.step, TAG_PPR);  // (while r is fetched)
     if (d > 0) {
-        const u32x4 x = draw(a.seed, walker_id(w), w.step, TAG_PPR);
         w.cur = span_col(sp, b - sp.eb + bounded(x.y, x.z, d));
         ct.moves++;
         if (sp.zc) { ct.zc_moves++; ct.zc_reads += 1 + a.rp_host; }
@@ -583,8 +583,8 @@ __device__ __forceinline__ void step_generic(Walker &w, const Span &sp, const Ap
     const uint64_t b = r[0], d = r[1] - b;
     uint32_t *path = a.paths ? a.paths + walker_id(w) * ((uint64_t)a.length + 1) : nullptr;
     if (path) path[a.length - w.step] = w.cur;  // the vertex after (length - step) moves
+    const u32x4 x = draw(a.seed, walker_id(w), w.step, TAG_GENERIC);  // (while r is fetched)
     if (d > 0) {
-        const u32x4 x = draw(a.seed, walker_id(w), w.step, TAG_GENERIC);
         w.cur = span_col(sp, b - sp.eb + bounded(x.y, x.z, d));
         ct.moves++;
         if (sp.zc) { ct.zc_moves++; ct.zc_reads += 1 + a.rp_host; }
@@ -611,34 +611,67 @@ __device__ __forceinline__ void finish_walker(const Walker &w, const AppArgs &a)
     if (a.endpoints) a.endpoints[walker_id(w)] = w.cur;
 }
 
+__device__ __forceinline__ bool in_batch(const WalkArgs &a, uint32_t p) {
+    bool in = false;
+#pragma unroll
+    for (uint32_t k = 0; k < kMaxZcBatch; k++) in |= a.srcs[k] == p;
+    return in;
+}
+
+__device__ __forceinline__ void zerocopy_span(const WalkArgs &a, Span &sp) {
+    sp.rowptr = a.ss.zc_rowptr + sp.nb;
+    sp.col = a.ss.zc_col + sp.eb;
+    sp.words = nullptr;
+    sp.zc = 1;
+}
+
 // Walk one residency; returns the destination partition or kEmpty when the
 // walk is over.  With span_resident the walker continues into any partition
-// whose slot is resident (and into the source slice itself).
+// whose slot is resident (and into the source slice itself, and into the others of
+// a zero-copy batch).
+//
+// A launch lasts as long as its longest chain of steps, 50 us where the work
+// of all lanes together is a few: a lane that leaves its span enters the next
+// one in the turn in which the others step, rather than wait for all that stay
+// (s20 ppr 15.9 -> 15.3 ms).  Where leaving the span ends the residency there is
+// nothing to enter, and that loop stands by itself (14.7 ms; s20 reference rules
+// as before, 1 % slower in the common loop).
 template <int APP>
-__device__ uint32_t walk_residency(Walker &w, const WalkArgs &a, uint32_t src, const Span &src_sp, Counters &ct) {
-    Span sp = src_sp;
-    while (true) {
-        while (w.step > 0 && (w.cur - sp.nb) < (sp.ne - sp.nb)) app_step<APP>(w, sp, a.app, ct);
-        if (w.step == 0) {
-            finish_walker(w, a.app);
-            return kEmpty;
-        }
-        const uint32_t p = find_part(a.pt, w.cur);
-        if (!a.span_resident) return p;
-        if (p == src) {
-            sp = src_sp;
-            continue;
-        }
-        const uint64_t *rp = a.pt.rowptr_tab[p];
-        if (!rp) return p;
-        sp.rowptr = rp;
-        sp.col = a.pt.col_tab[p];
-        sp.words = a.pt.words_tab[p];
-        sp.nb = a.pt.node_off[p];
-        sp.ne = a.pt.node_off[p + 1];
-        sp.eb = a.pt.edge_off[p];
-        sp.zc = a.pt.zc_part[p];
+__device__ __forceinline__ uint32_t walk_residency(Walker &w, const WalkArgs &a, uint32_t src, const Span &src_sp,
+                                                   Counters &ct) {
+    if (!a.span_resident) {  // uniform
+        while (w.step > 0 && w.cur - src_sp.nb < src_sp.ne - src_sp.nb) app_step<APP>(w, src_sp, a.app, ct);
+        if (w.step > 0) return find_part(a.pt, w.cur);
+        finish_walker(w, a.app);
+        return kEmpty;
     }
+    Span sp = src_sp;
+    while (w.step > 0) {
+        if ((w.cur - sp.nb) >= (sp.ne - sp.nb)) {
+            uint32_t p = a.pt.lut[w.cur >> a.pt.lut_shift];
+            PartRec r = a.pt.rec[p];
+            while (w.cur >= r.ne) r = a.pt.rec[++p];
+            if (p == src) {
+                sp = src_sp;
+            } else {
+                sp.nb = r.nb;
+                sp.ne = r.ne;
+                sp.eb = r.eb;
+                if (r.rowptr) {
+                    sp.rowptr = r.rowptr;
+                    sp.col = r.col;
+                    sp.words = r.words;
+                    sp.zc = 0;
+                } else {
+                    if (!a.nsrc || !a.zerocopy || !in_batch(a, p)) return p;
+                    zerocopy_span(a, sp);
+                }
+            }
+        }
+        app_step<APP>(w, sp, a.app, ct);
+    }
+    finish_walker(w, a.app);
+    return kEmpty;
 }
 
 // One workgroup pass over nvalid <= kBlock * WPT walkers stored
@@ -771,13 +804,15 @@ __global__ __launch_bounds__(kBlock, WPT == 1 && !GEN ? 5 : 4) void walk_kernel(
                 base = at - a.voff[k];
                 n = qlen_of(a.q, src);
                 if (base >= n) continue;  // uniform per workgroup
-                sp.rowptr = a.pt.rowptr_tab[src];  // as a walker entering src reads it (walk_residency)
-                sp.col = a.pt.col_tab[src];
-                sp.words = a.pt.words_tab[src];
-                sp.nb = a.pt.node_off[src];
-                sp.ne = a.pt.node_off[src + 1];
-                sp.eb = a.pt.edge_off[src];
-                sp.zc = a.pt.zc_part[src];
+                const PartRec r = a.pt.rec[src];  // as a walker entering src reads it (walk_residency)
+                sp.rowptr = r.rowptr;
+                sp.col = r.col;
+                sp.words = r.words;
+                sp.nb = r.nb;
+                sp.ne = r.ne;
+                sp.eb = r.eb;
+                sp.zc = 0;
+                if (a.zerocopy) zerocopy_span(a, sp);
             }
             const uint32_t chunk = a.q.frame[(size_t)src * a.q.maxc + (uint32_t)(base >> kChunkLog2)];
             if (chunk >= a.q.nchunks) {  // uniform per workgroup
@@ -888,14 +923,14 @@ __global__ __launch_bounds__(kBlock) void pack_meta_kernel(Queues q) { pack_meta
 
 // Return the popped-but-unused state of the pool, the lost chunks and the
 // consumed source chunks to the free stack; clear the source queues after their
-// last slice; take a zero-copy batch out of the partition table; tell the host
-// the queue lengths.  One workgroup, for all sources of a batch's launch.
+// last slice; tell the host the queue lengths.  One workgroup, for all sources of
+// a batch's launch.
 //
 // Every round of a job waits for this kernel, a chain of round trips: what it
 // reads by known addresses is read at once, and the host, which needs the
 // lengths only, gets them before the chunks move (its next walk is behind this
 // kernel in the stream).
-__global__ __launch_bounds__(kBlock) void fixup_kernel(Queues q, Consumed d, Tables tab) {
+__global__ __launch_bounds__(kBlock) void fixup_kernel(Queues q, Consumed d) {
     __shared__ uint32_t s_top, s_nlost, s_off[kMaxZcBatch + 1];
     const uint32_t tid = threadIdx.x;
     const uint32_t n = d.n, lo = d.chunk_lo;
@@ -945,15 +980,7 @@ __global__ __launch_bounds__(kBlock) void fixup_kernel(Queues q, Consumed d, Tab
         q.free_stack[top + nlost + j] = *f;
         *f = kEmpty;
     }
-    if (tid < n) {
-        const uint32_t p = d.src[tid];
-        if (d.last) qlen_of(q, p) = 0;
-        if (d.leave) {
-            tab.rowptr[p] = nullptr;
-            tab.col[p] = nullptr;
-            tab.zc[p] = 0;
-        }
-    }
+    if (tid < n && d.last) qlen_of(q, d.src[tid]) = 0;
 }
 
 // Copy the queues of a spill round into host memory: walker i of partition
@@ -1026,14 +1053,13 @@ __global__ void reset_queues_kernel(Queues q, uint32_t P) {
 }
 
 // Partition table updates, all those due before a walk in one launch.
-__global__ void set_tables_kernel(Tables tab, TableBatch b) {
+__global__ void set_tables_kernel(PartRec *rec, TableBatch b) {
     const uint32_t k = threadIdx.x;
     if (k < b.n) {
-        const uint32_t p = b.part[k];
-        tab.rowptr[p] = b.rowptr[k];
-        tab.col[p] = b.col[k];
-        tab.words[p] = b.words[k];
-        tab.zc[p] = b.zc[k];
+        PartRec *r = &rec[b.part[k]];
+        r->rowptr = b.rowptr[k];
+        r->col = b.col[k];
+        r->words = b.words[k];
     }
 }
 
@@ -1115,13 +1141,14 @@ struct PartState {
 __device__ __forceinline__ PartState part_state(const Queues &q, const SchedState &ss, const Parts &pt, uint32_t p) {
     PartState o;
     o.len = qlen_of(q, p);
-    o.nb = pt.node_off[p];
-    o.ne = pt.node_off[p + 1];
-    o.eb = pt.edge_off[p];
+    const PartRec r = pt.rec[p];
+    o.nb = r.nb;
+    o.ne = r.ne;
+    o.eb = r.eb;
+    o.words = r.words;
     o.ee = pt.edge_off[p + 1];
     o.resident = ss.resident[p];
     o.slot = ss.slot_of[p];
-    o.words = pt.words_tab[p];
     return o;
 }
 
@@ -1235,9 +1262,7 @@ __global__ __launch_bounds__(kBlock) void decide_kernel(Queues q, SchedState ss,
             slot = ss.slot_of[v];
             ss.slot_of[v] = -1;
             ss.resident[v] = 0;
-            ss.rowptr_tab[v] = nullptr;
-            ss.col_tab[v] = nullptr;
-            bi.words_tab[v] = nullptr;
+            ss.rec[v].rowptr = nullptr;
             d.victim = (int32_t)v;
         }
     }
@@ -1251,9 +1276,9 @@ __global__ __launch_bounds__(kBlock) void decide_kernel(Queues q, SchedState ss,
         ss.slot_of[c] = slot;
         ss.part_in_slot[slot] = (int32_t)c;
         ss.resident[c] = 1;
-        ss.rowptr_tab[c] = d.rowptr;
-        ss.col_tab[c] = d.col;
-        bi.words_tab[c] = d.words;
+        ss.rec[c].rowptr = d.rowptr;
+        ss.rec[c].col = d.col;
+        ss.rec[c].words = d.words;
         d.load = 1;
         d.from[0] = (const uint32_t *)(ss.zc_rowptr + own.nb);
         d.from[1] = img ? (const uint32_t *)(bi.img + bi.off[c]) : ss.zc_col + own.eb;

@@ -47,3 +47,26 @@ def test_device_loop_partition_counts(P, slots):
         for _ in range(2):
             counts, ends = eng.pagerank(w, l, endpoints=True)
             assert np.array_equal(counts, rc) and np.array_equal(ends, re)
+
+
+@pytest.mark.parametrize("kw", [{}, {"zerocopy_threshold": 1 << 30, "zc_batch": 16}, {"pack_partitions": 2},
+                                {"device_schedule": 1}], ids=["resident", "zerocopy", "blocks", "device"])
+def test_partitions_within_a_lookup_step(kw):
+    """131 075 vertices are looked up four at a time; the first 64 of them and the
+    last fill a partition each."""
+    print(f"lookup {kw}", flush=True)
+    rng = np.random.default_rng(5)
+    deg = np.ones(131075, np.uint64)
+    deg[:64] = deg[-1] = 2000
+    rowptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.uint64)
+    col = rng.integers(0, len(deg), int(rowptr[-1]))
+    col[::3] %= 64
+    g = lt.Graph.from_csr(rowptr, col.astype(np.uint32))
+    part = lt.Partition.build(g, 8100)
+    assert part.count > 200
+    w, l = 30011, 6
+    rc, re, _ = oracle.pagerank(g.rowptr(), g.col(), w, l, endpoints=True, threads=8)
+    eng = lt.Engine(g, part, num_device_partitions=part.count // 2, span="resident",
+                    **{"zerocopy_threshold": 100, "resident_batch": 16, **kw})
+    counts, ends = eng.pagerank(w, l, endpoints=True)
+    assert np.array_equal(counts, rc) and np.array_equal(ends, re)
