@@ -157,6 +157,20 @@ struct BlockImages {
     const uint64_t *size;
 };
 
+// Partition table entries to set: before a walk by a launch of their own, or, if
+// they are few, told to the walk and set by the fix-up behind it.
+constexpr uint32_t kTableBatch = 32, kTableFew = 4;
+template <uint32_t N>
+struct TableEntries {
+    uint32_t n;
+    uint32_t part[N];
+    const uint64_t *rowptr[N];  // nullptr: not resident
+    const uint32_t *col[N];
+    const uint32_t *words[N];
+};
+using TableBatch = TableEntries<kTableBatch>;
+using TableFew = TableEntries<kTableFew>;
+
 struct WalkArgs {
     AppArgs app;
     Queues q;
@@ -191,6 +205,7 @@ struct WalkArgs {
     // read by the kernel over PCIe; piece k holds hn[k] <= kChunk walkers at
     // hptr[k] and occupies [k * kChunk, k * kChunk + hn[k]) of the range.
     uint32_t nhost;
+    TableFew due;         // entries of the partition table that it does not hold yet
     SchedState ss;        // device-scheduled loop: ss.ds != nullptr names the source
     uint32_t srcs[kMaxZcBatch];
     uint64_t voff[kMaxZcBatch + 1];
@@ -211,16 +226,6 @@ struct SpillArgs {
     Walker *const *hptr;     // host chunks, mapped for the device
 };
 
-// Partition table entries to set before a walk.
-constexpr uint32_t kTableBatch = 32;
-struct TableBatch {
-    uint32_t n;
-    uint32_t part[kTableBatch];
-    const uint64_t *rowptr[kTableBatch];  // nullptr: not resident
-    const uint32_t *col[kTableBatch];
-    const uint32_t *words[kTableBatch];
-};
-
 // What a walk launch consumed (fixup_kernel): chunks [chunk_lo, chunk_hi) of
 // src[0]'s queue, or with n > 1 the whole queues of src[0..n).
 struct Consumed {
@@ -228,6 +233,7 @@ struct Consumed {
     uint32_t src[kMaxZcBatch];
     uint32_t chunk_lo, chunk_hi;
     int last;    // the queues end with those chunks
+    TableFew due;  // what the walk was told of the partition table
 };
 
 struct InitArgs {

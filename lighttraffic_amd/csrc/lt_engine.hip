@@ -328,9 +328,10 @@ struct Engine {
     bool meta_dirty = true;  // q.packed may be older than the queues
     uint32_t meta_seq = 0;   // of the last launch that writes q.packed
     bool meta_seen = true;   // h_meta holds what that launch wrote
-    lt_status launch_fixup(const Consumed &d);
+    lt_status launch_fixup(Consumed d);
     lt_status wait_meta();
     TableBatch table_due{};  // table updates of the next walk launch
+    TableFew table_told{};  // of the walk whose fix-up comes next
     lt_status flush_tables();
     lt_status process(uint32_t p, bool zerocopy, uint64_t walkers_hint);
     lt_status process_zc(uint32_t c, const uint8_t *pending);
@@ -822,9 +823,11 @@ lt_status Engine::count_log(uint32_t n, uint32_t most) {
     return LT_OK;
 }
 
-lt_status Engine::launch_fixup(const Consumed &d) {
+lt_status Engine::launch_fixup(Consumed d) {
     q.seq = ++meta_seq;
-    fixup_kernel<<<1, kBlock, 0, s_compute>>>(q, d);
+    d.due = table_told;
+    table_told.n = 0;
+    fixup_kernel<<<1, kBlock, 0, s_compute>>>(q, d, d_rec);
     LT_HIP(hipGetLastError());
     meta_dirty = false;
     meta_seen = false;
@@ -1121,7 +1124,22 @@ lt_status Engine::fetch_partition(uint32_t p, uint64_t *rowptr_out, uint32_t *co
 // destination queue) is spread over more walkers.
 lt_status Engine::launch_walk(WalkArgs &a, uint64_t walkers, hipStream_t s) {
     // a walk of one source that stays in it reads no table
-    if (a.span_resident || a.nsrc) LT_TRY(flush_tables());
+    a.due.n = 0;
+    if (a.span_resident || a.nsrc) {
+        if (table_due.n > kTableFew || table_told.n) {
+            LT_TRY(flush_tables());
+        } else {  // the fix-up behind this walk sets them
+            a.due.n = table_due.n;
+            for (uint32_t k = 0; k < table_due.n; k++) {
+                a.due.part[k] = table_due.part[k];
+                a.due.rowptr[k] = table_due.rowptr[k];
+                a.due.col[k] = table_due.col[k];
+                a.due.words[k] = table_due.words[k];
+            }
+            table_told = a.due;
+            table_due.n = 0;
+        }
+    }
     const uint64_t fill = (uint64_t)num_cu * 4 * 6 * 64;  // threads for ~6 waves per SIMD
     const int wpt = cfg.walkers_per_thread > 0 ? cfg.walkers_per_thread
                     : walkers >= 4 * fill         ? 4

@@ -625,6 +625,19 @@ __device__ __forceinline__ void zerocopy_span(const WalkArgs &a, Span &sp) {
     sp.zc = 1;
 }
 
+// Puts what changed since the launch before, which comes with the arguments, into
+// the record of partition p: a launch that sets two entries holds each round up
+// for 7 us.
+__device__ __forceinline__ void update_rec(const WalkArgs &a, uint32_t p, PartRec &r) {
+    for (uint32_t k = 0; k < a.due.n; k++) {  // uniform
+        if (a.due.part[k] == p) {
+            r.rowptr = a.due.rowptr[k];
+            r.col = a.due.col[k];
+            r.words = a.due.words[k];
+        }
+    }
+}
+
 // Walk one residency; returns the destination partition or kEmpty when the
 // walk is over.  With span_resident the walker continues into any partition
 // whose slot is resident (and into the source slice itself, and into the others of
@@ -651,6 +664,7 @@ __device__ __forceinline__ uint32_t walk_residency(Walker &w, const WalkArgs &a,
             uint32_t p = a.pt.lut[w.cur >> a.pt.lut_shift];
             PartRec r = a.pt.rec[p];
             while (w.cur >= r.ne) r = a.pt.rec[++p];
+            update_rec(a, p, r);
             if (p == src) {
                 sp = src_sp;
             } else {
@@ -804,7 +818,8 @@ __global__ __launch_bounds__(kBlock, WPT == 1 && !GEN ? 5 : 4) void walk_kernel(
                 base = at - a.voff[k];
                 n = qlen_of(a.q, src);
                 if (base >= n) continue;  // uniform per workgroup
-                const PartRec r = a.pt.rec[src];  // as a walker entering src reads it (walk_residency)
+                PartRec r = a.pt.rec[src];  // as a walker entering src reads it (walk_residency)
+                update_rec(a, src, r);
                 sp.rowptr = r.rowptr;
                 sp.col = r.col;
                 sp.words = r.words;
@@ -921,6 +936,17 @@ __device__ void pack_meta(const Queues &q) {
 
 __global__ __launch_bounds__(kBlock) void pack_meta_kernel(Queues q) { pack_meta(q); }
 
+template <uint32_t N>
+__device__ __forceinline__ void set_entries(PartRec *rec, const TableEntries<N> &b) {
+    const uint32_t k = threadIdx.x;
+    if (k < b.n) {
+        PartRec *r = &rec[b.part[k]];
+        r->rowptr = b.rowptr[k];
+        r->col = b.col[k];
+        r->words = b.words[k];
+    }
+}
+
 // Return the popped-but-unused state of the pool, the lost chunks and the
 // consumed source chunks to the free stack; clear the source queues after their
 // last slice; tell the host the queue lengths.  One workgroup, for all sources of
@@ -930,7 +956,7 @@ __global__ __launch_bounds__(kBlock) void pack_meta_kernel(Queues q) { pack_meta
 // reads by known addresses is read at once, and the host, which needs the
 // lengths only, gets them before the chunks move (its next walk is behind this
 // kernel in the stream).
-__global__ __launch_bounds__(kBlock) void fixup_kernel(Queues q, Consumed d) {
+__global__ __launch_bounds__(kBlock) void fixup_kernel(Queues q, Consumed d, PartRec *rec) {
     __shared__ uint32_t s_top, s_nlost, s_off[kMaxZcBatch + 1];
     const uint32_t tid = threadIdx.x;
     const uint32_t n = d.n, lo = d.chunk_lo;
@@ -981,6 +1007,7 @@ __global__ __launch_bounds__(kBlock) void fixup_kernel(Queues q, Consumed d) {
         *f = kEmpty;
     }
     if (tid < n && d.last) qlen_of(q, d.src[tid]) = 0;
+    set_entries(rec, d.due);
 }
 
 // Copy the queues of a spill round into host memory: walker i of partition
@@ -1053,15 +1080,7 @@ __global__ void reset_queues_kernel(Queues q, uint32_t P) {
 }
 
 // Partition table updates, all those due before a walk in one launch.
-__global__ void set_tables_kernel(PartRec *rec, TableBatch b) {
-    const uint32_t k = threadIdx.x;
-    if (k < b.n) {
-        PartRec *r = &rec[b.part[k]];
-        r->rowptr = b.rowptr[k];
-        r->col = b.col[k];
-        r->words = b.words[k];
-    }
-}
+__global__ void set_tables_kernel(PartRec *rec, TableBatch b) { set_entries(rec, b); }
 
 // Copy of a partition's two slices from mapped host memory (or HBM) into a cache
 // slot, 4-byte words: 64 workgroups with eight loads per lane in flight fill

@@ -70,3 +70,20 @@ def test_partitions_within_a_lookup_step(kw):
                     **{"zerocopy_threshold": 100, "resident_batch": 16, **kw})
     counts, ends = eng.pagerank(w, l, endpoints=True)
     assert np.array_equal(counts, rc) and np.array_equal(ends, re)
+
+
+@pytest.mark.parametrize("depth", [1, 2, 3, 8])
+def test_table_entries_told_to_the_walk(depth):
+    """Loads ahead change up to two entries each between launches: as many as a walk
+    is told of, one more, and many."""
+    print(f"table entries depth={depth}", flush=True)
+    g = lt.Graph.rmat(15, 16)
+    part = lt.Partition.build(g, 32 << 10)
+    w, l = 40009, 8
+    rc, re, _ = oracle.pagerank(g.rowptr(), g.col(), w, l, endpoints=True, threads=8)
+    eng = lt.Engine(g, part, num_device_partitions=part.count // 2, span="resident", policy="learned",
+                    prefetch_plain=1, prefetch_depth=depth, zerocopy_threshold=50, resident_batch=16)
+    for _ in range(2):
+        counts, ends = eng.pagerank(w, l, endpoints=True)
+        assert np.array_equal(counts, rc) and np.array_equal(ends, re)
+    assert eng.stats()["prefetch_issued"] > 0
