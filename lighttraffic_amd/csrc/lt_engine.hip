@@ -241,7 +241,6 @@ struct Engine {
     VisitScratch vs{};
     unsigned long long *d_vcur = nullptr;
     uint64_t vlog_cap = 0;                       // entries allocated
-    uint64_t vrun_cap = 0, vpartial_cap = 0;     // words
     uint32_t vregion = 0;                        // entries per region of the running job, 0 = no log
     lt_status ensure_log(uint64_t visits, bool queued);
     lt_status count_log(uint32_t n, uint32_t most);
@@ -374,7 +373,8 @@ struct Engine {
         }
     }
     lt_status set_table(uint32_t p, bool present);
-    bool can_run_flat() const;
+    bool can_run_flat(const RunSpec &rs, uint32_t &missing) const;
+    lt_status load_missing();
     lt_status run_flat(const RunSpec &rs, ResultHelpers &help);
     bool job_finished = false;  // run_flat has handed the job's results out
     lt_status scheduler_loop();
@@ -427,9 +427,6 @@ Engine::~Engine() {
     dfree(d_counts);
     dfree(vl.log);
     dfree(d_vcur);
-    dfree(vs.sorted);
-    dfree(vs.run);
-    dfree(vs.partial);
     dfree(d_endpoints);
     dfree(d_moves);
     dfree(d_paths);
@@ -690,7 +687,14 @@ lt_status Engine::ensure_pool(uint64_t walkers, bool check_only) {
     const uint64_t wchunks = (walkers + kChunk - 1) / kChunk;
     // one launch holds at most `held` source chunks while filling new ones
     const uint64_t held = cfg.device_schedule ? wchunks + 1 : std::min<uint64_t>(slice, wchunks + 1);
-    const uint64_t nchunks = wchunks + P + held + 2 + kLostCap;
+    // A reservation links at most two chunks and so loses at most two, and a launch
+    // makes one for each pass and partition (a pass has kBlock walkers or more; 128: queues
+    // and pieces that end in a short one).  With few partitions that is far below
+    // kLostCap: 46 MB instead of 268 for 90 000 walkers of one, whose allocation took
+    // a new engine's first job half its time.
+    const uint64_t lost = cfg.append_mode == 2 ? kLostCap
+                                               : std::min<uint64_t>(kLostCap, 2 * (uint64_t)P * (walkers / kBlock + 128));
+    const uint64_t nchunks = wchunks + P + held + 2 + lost;
     const uint64_t maxc = wchunks + 2;
     if (nchunks >= 0xFFFFFFF0ull || maxc * kChunk > 0xFFFFFFFFull) {
         set_error("%llu walkers exceed the queue limits; lower -b", (unsigned long long)walkers);
@@ -770,14 +774,18 @@ lt_status Engine::ensure_log(uint64_t visits, bool queued) {
     visits = std::min(visits, kLogMost);
     const uint64_t want = std::min(kLogMost, visits + visits / 4 + (1u << 20)) & ~(uint64_t)(kTile * kLogRegions - 1);
     if (vlog_cap < want) {
+        // The log and what counting a full one takes, in one allocation: one by
+        // one they took a new engine's first job 0.6 ms, with tens of MB or few.
+        const uint64_t tiles = want / kTile + kLogRegions;
+        const uint64_t units = std::max<uint64_t>(nbins <= kFewBins ? std::min<uint64_t>(kFewUnits, tiles * nbins) : 0,
+                                                  std::min<uint64_t>(want / kHistUnit, kHistUnits) + 1 + nbins);
+        const uint64_t words[4] = {want, want / 2, tiles * nbins, units * kBin};  // multiples of 4 but the third
         dfree(vl.log);
-        dfree(vs.sorted);
         vlog_cap = 0;
-        if (dmalloc(&vl.log, want) != LT_OK || dmalloc(&vs.sorted, want) != LT_OK) {
-            dfree(vl.log);
-            dfree(vs.sorted);
-            return LT_OK;
-        }
+        if (dmalloc(&vl.log, words[0] + words[1] + words[2] + 4 + words[3]) != LT_OK) return LT_OK;
+        vs.sorted = (uint16_t *)(vl.log + words[0]);
+        vs.run = vl.log + words[0] + words[1];
+        vs.partial = vs.run + ((words[2] + 3) & ~3ull);
         vlog_cap = want;
     }
     vregion = (uint32_t)(want / kLogRegions);
@@ -795,24 +803,12 @@ lt_status Engine::count_log(uint32_t n, uint32_t most) {
     if (entries == 0) return LT_OK;
     l.tiles = (uint32_t)(((n ? n : entries / kLogRegions) + kTile - 1) / kTile);
     const uint32_t ntiles = n ? l.tiles : l.tiles * kLogRegions;
-    const bool few = nbins <= kFewBins && ntiles * nbins <= 1024;
-    vs.unit = std::max<uint32_t>(kHistUnit, (uint32_t)(entries / 512));
+    const bool few = nbins <= kFewBins && ntiles * nbins <= kFewUnits;
+    vs.unit = std::max<uint32_t>(kHistUnit, (uint32_t)(entries / kHistUnits));
     const uint32_t units = few ? ntiles * nbins : (uint32_t)((entries + vs.unit - 1) / vs.unit) + nbins;
-    if (vpartial_cap < (uint64_t)units * kBin) {
-        dfree(vs.partial);
-        vpartial_cap = 0;
-        LT_TRY(dmalloc(&vs.partial, (size_t)units * kBin));
-        vpartial_cap = (uint64_t)units * kBin;
-    }
     if (few) {
         visit_hist_kernel<false><<<units, kVisitThreads, 0, s_compute>>>(l, vs, nbins, ntiles);
     } else {
-        if (vrun_cap < (uint64_t)nbins * ntiles) {
-            dfree(vs.run);
-            vrun_cap = 0;
-            LT_TRY(dmalloc(&vs.run, (size_t)nbins * ntiles));
-            vrun_cap = (uint64_t)nbins * ntiles;
-        }
         visit_tile_kernel<<<ntiles, kVisitThreads, 4 * kRepl * nbins, s_compute>>>(l, vs, nbins, ntiles);
         visit_scan_kernel<<<nbins, kVisitThreads, 0, s_compute>>>(vs, ntiles);
         visit_scatter_kernel<<<ntiles, kVisitThreads, scatter_lds(nbins), s_compute>>>(l, vs, nbins, ntiles);
@@ -943,8 +939,13 @@ bool Engine::loaded(const Load &l) const {
     return (l.ev ? hipEventQuery(l.ev) : hipStreamQuery(s_copy)) != hipErrorNotReady;
 }
 
-// Polls: a blocking wait adds its wake-up latency to a decision.
+// A pulled load's number and an event are polled; the end of a DMA with nothing
+// behind it is waited for by the runtime.
 lt_status Engine::wait_loaded(Load &l) {
+    if (!l.pulled && !l.ev) {
+        LT_HIP(hipStreamSynchronize(s_copy));
+        return LT_OK;
+    }
     for (uint32_t it = 1; !loaded(l); it++) {
         __builtin_ia32_pause();
         if (l.pulled && (it & 0xFFFFF) == 0) {
@@ -956,9 +957,11 @@ lt_status Engine::wait_loaded(Load &l) {
             return LT_E_INTERNAL;
         }
     }
-    if (!l.pulled) LT_HIP(l.ev ? hipEventQuery(l.ev) : hipStreamQuery(s_copy));
-    if (l.ev) pool_events.push_back(l.ev);
+    if (!l.ev) return LT_OK;
+    const hipError_t e = hipEventQuery(l.ev);
+    pool_events.push_back(l.ev);
     l.ev = nullptr;
+    LT_HIP(e);
     return LT_OK;
 }
 
@@ -2034,12 +2037,60 @@ lt_status Engine::scheduler_loop_device() {
 // allowed to walk through all of them in one launch (span resident with
 // batches, or a single partition), all of them on the device at once, and no
 // decision trace or append ablation asked for.  Edge numbers have to fit 32 bits.
-bool Engine::can_run_flat() const {
+// Partitions not cached yet are loaded first where the queues would load them
+// as well: a job of one partition that is not read in place, or one whose
+// walkers start all over the graph, enough for each missing partition to be worth
+// a chunk of them and not to be read in place.  (Walkers of ppr start at their
+// sources and may never see a partition.)  By queues, a new engine's first job
+// took 0.83 ms on s16 (0.50 so, with no pool of queues to allocate) and 14.4 ms
+// on s22 (12.4).
+bool Engine::can_run_flat(const RunSpec &rs, uint32_t &missing) const {
+    missing = 0;
     if (!flat || g->E > 0xFFFFFFFFull || cfg.record_trace || cfg.append_mode != 0 || spill_on) return false;
     if (P > 1 && (cfg.span != LT_SPAN_RESIDENT || res_batch <= 1)) return false;
-    for (uint32_t p = 0; p < P; p++)
-        if (!resident[p]) return false;
-    return true;
+    for (uint32_t p = 0; p < P; p++) missing += resident[p] ? 0 : 1;
+    if (missing == 0) return true;
+    if (P == 1) return rs.total >= zc_threshold;
+    return rs.app != APP_PPR && rs.total / missing >= std::max<uint64_t>(zc_threshold, kChunk);
+}
+
+lt_status Engine::load_missing() {
+    if (pk) {
+        Load l;
+        for (uint32_t p = 0; p < P; p++)
+            if (!resident[p]) LT_TRY(load_async(p, false, l));
+    } else {  // a flat cache is laid out as the graph: neighbours in one copy
+        hipEvent_t t = t_load.begin(s_copy);
+        for (uint32_t p = 0, end; p < P; p = end) {
+            end = p + 1;
+            if (resident[p]) continue;
+            while (end < P && !resident[end]) end++;
+            const uint32_t nb = part.node_off[p];
+            const uint64_t eb = part.edge_off[p];
+            const size_t rbytes = ((size_t)part.node_off[end] - nb + 1) * 8, cbytes = (part.edge_off[end] - eb) * 4;
+            if (rp_resident) LT_HIP(hipMemcpyAsync(flat_rowptr + nb, d_rowptr_all + nb, rbytes, hipMemcpyDeviceToDevice, s_copy));
+            else LT_HIP(hipMemcpyAsync(flat_rowptr + nb, g->rowptr + nb, rbytes, hipMemcpyHostToDevice, s_copy));
+            LT_HIP(hipMemcpyAsync(flat_col + eb, g->col + eb, cbytes, hipMemcpyHostToDevice, s_copy));
+            const size_t h2d = cbytes + (rp_resident ? 0 : rbytes);
+            st.h2d_bytes_explicit += h2d;
+            st.h2d_bytes_unpacked += h2d;
+            for (uint32_t i = p; i < end; i++) {
+                slot_of[i] = (int32_t)free_slots.back();
+                part_in_slot[free_slots.back()] = (int32_t)i;
+                free_slots.pop_back();
+            }
+        }
+        t_load.end(t, s_copy);
+    }
+    LT_HIP(hipStreamSynchronize(s_copy));
+    for (uint32_t p = 0; p < P; p++) {
+        if (resident[p]) continue;
+        resident[p] = 1;
+        st.graph_loading_calls++;
+        sched.on_load(p);
+        LT_TRY(set_table(p, true));
+    }
+    return LT_OK;
 }
 
 // Eight workgroups per CU: the kernels hold few registers, and the lanes of a
@@ -2220,7 +2271,8 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
     const bool counting = rs.app != APP_GENERIC && counts_out;
     uint64_t visits = rs.total;
     if (rs.app == APP_PAGERANK && __builtin_mul_overflow(rs.total, (uint64_t)rs.length, &visits)) visits = UINT64_MAX;
-    const bool walk_flat = can_run_flat();
+    uint32_t missing;
+    const bool walk_flat = can_run_flat(rs, missing);
     if (counting) LT_TRY(ensure_log(visits, !walk_flat));
     else vregion = 0;
     // Without a log, copies of the counters, one per XCD: where the walkers of
@@ -2296,6 +2348,7 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
     double running_ms = 0;
     auto t_walk = std::chrono::steady_clock::now();
     job_finished = false;
+    if (walk_flat && missing) LT_TRY(load_missing());
     if (walk_flat) LT_TRY(run_flat(rs, help));
     for (uint64_t id0 = walk_flat ? rs.total : 0; id0 < rs.total; id0 += wave) {
         const uint64_t id1 = std::min<uint64_t>(rs.total, id0 + wave);

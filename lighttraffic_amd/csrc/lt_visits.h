@@ -27,6 +27,8 @@ constexpr uint32_t kFewBins = 4;
 constexpr uint32_t kVisitThreads = 1024;
 constexpr uint32_t kTile = 16 * kVisitThreads;  // log entries partitioned by one workgroup
 constexpr uint32_t kHistUnit = 1u << 16;        // entries of a bin counted by one workgroup, at least
+constexpr uint32_t kHistUnits = 512;            // units a log is cut into, at most (and one a bin more)
+constexpr uint32_t kFewUnits = 1024;            // tiles times bins counted without a sort, at most
 constexpr uint32_t kLogRegions = 8;  // one per XCD: workgroup b appends to region b % 8
 constexpr uint32_t kRepl = 4;        // copies of a tile's histogram: R-MAT visits crowd into few
                                      // bins, and lanes that add to one address take turns
