@@ -557,6 +557,16 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
         }
     }
     slot_packed = pk && pk->format == 2;
+    // Blocks pay where they let more partitions stay. Asked for raw slots for all,
+    // the images only travel, and the columns are kept raw, for flat walks: a
+    // move reads one line of columns instead of two one after the other (s20
+    // batched ppr, 5 M walkers: 4.0 ms walked from blocks, 3.5 so).  Not where
+    // the raw columns take more than a quarter of the free memory.
+    if (slot_packed && !cfg.device_schedule && (cfg.num_device_partitions == 0 || cfg.num_device_partitions >= P)) {
+        size_t room = 0, all = 0;
+        LT_HIP(hipMemGetInfo(&room, &all));
+        slot_packed = 8ull * ((uint64_t)V + 1) + 4ull * g->E > room / 4;
+    }
 
     // HBM cache slots (GPUGraph, src/GraphLoader.h:175-176)
     uint64_t slot_bytes = 0;
@@ -598,7 +608,7 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
     else zc_threshold = cfg.policy == LT_SCHED_LEARNED ? part.bytes / 128 : part.bytes / 128 / 2;
     LT_HIP(hipHostGetDevicePointer((void **)&zc_rowptr, g->rowptr, 0));
     LT_HIP(hipHostGetDevicePointer((void **)&zc_col, g->col, 0));
-    if (pk && pk->format == 1) {  // staging buffers for the images unpacked in HBM
+    if (pk && !slot_packed) {  // staging buffers for the images unpacked in HBM
         for (int k = 0; k < 2; k++) {
             LT_TRY(dmalloc(&d_stage[k], pk->max_size));
             LT_HIP(hipEventCreateWithFlags(&stage_free[k], hipEventDisableTiming));
@@ -1064,16 +1074,21 @@ lt_status Engine::copy_partition(uint32_t p, uint64_t *rp, uint32_t *cp) {
     }
     st.h2d_bytes_unpacked += cbytes;
     if (packed) {
-        const uint64_t n = ne - nb, nch = (ee - eb + 63) / 64;
-        const uint64_t nwords = (pk->size[p] - 8 * nch) / 4 - 2;
-        const uint64_t waves = (nch + kUnpackChunks - 1) / kUnpackChunks;
         LT_HIP(hipMemcpyAsync(d_stage[k], pk->host + pk->off[p], pk->size[p], hipMemcpyHostToDevice, s_dma));
         if (s_dma != s_copy) {
             LT_HIP(hipEventRecord(ev_dma, s_dma));
             LT_HIP(hipStreamWaitEvent(s_copy, ev_dma, 0));
         }
-        unpack_kernel<<<(unsigned)((waves + 3) / 4), 256, 0, s_copy>>>(
-            d_stage[k], (uint32_t)n, ee - eb, nwords, pk->vbits, rp, cp);
+        if (pk->format == 2) {
+            const int grid = (int)std::min<uint64_t>(8 * (uint64_t)num_cu, (ee - eb) / 256 + 1);
+            unblock_kernel<<<grid, 256, 0, s_copy>>>((const uint32_t *)d_stage[k], ee - eb, cp);
+        } else {
+            const uint64_t n = ne - nb, nch = (ee - eb + 63) / 64;
+            const uint64_t nwords = (pk->size[p] - 8 * nch) / 4 - 2;
+            const uint64_t waves = (nch + kUnpackChunks - 1) / kUnpackChunks;
+            unpack_kernel<<<(unsigned)((waves + 3) / 4), 256, 0, s_copy>>>(
+                d_stage[k], (uint32_t)n, ee - eb, nwords, pk->vbits, rp, cp);
+        }
         LT_HIP(hipGetLastError());
         LT_HIP(hipEventRecord(stage_free[k], s_copy));
         stage_used[k] = true;
@@ -1094,7 +1109,7 @@ lt_status Engine::copy_partition(uint32_t p, uint64_t *rp, uint32_t *cp) {
 // A partition's slot bytes, built by copy_partition in a scratch buffer and
 // copied back; the cache and the statistics are left as they were.
 lt_status Engine::fetch_partition(uint32_t p, uint64_t *rowptr_out, uint32_t *col_out) {
-    if (slot_packed) {
+    if (pk && pk->format == 2) {
         set_error("fetch of partition %u: slots keep columns packed (pack_partitions = 2)", p);
         return LT_E_ARG;
     }
@@ -2040,8 +2055,10 @@ lt_status Engine::scheduler_loop_device() {
 // Partitions not cached yet are loaded first where the queues would load them
 // as well: a job of one partition that is not read in place, or one whose
 // walkers start all over the graph, enough for each missing partition to be worth
-// a chunk of them and not to be read in place.  (Walkers of ppr start at their
-// sources and may never see a partition.)  By queues, a new engine's first job
+// a chunk of them and not to be read in place.  Walkers of ppr start at their
+// sources and may never see a partition: their jobs load as many as they have
+// sources, or the last eighth, which the queues would read in place in every job
+// (s20 batched ppr: 3.5 ms a job by queues, 1.65 flat).  By queues, a new engine's first job
 // took 0.83 ms on s16 (0.50 so, with no pool of queues to allocate) and 14.4 ms
 // on s22 (12.4).
 bool Engine::can_run_flat(const RunSpec &rs, uint32_t &missing) const {
@@ -2051,7 +2068,8 @@ bool Engine::can_run_flat(const RunSpec &rs, uint32_t &missing) const {
     for (uint32_t p = 0; p < P; p++) missing += resident[p] ? 0 : 1;
     if (missing == 0) return true;
     if (P == 1) return rs.total >= zc_threshold;
-    return rs.app != APP_PPR && rs.total / missing >= std::max<uint64_t>(zc_threshold, kChunk);
+    if (rs.app == APP_PPR && missing > std::max(P / 8, rs.nq)) return false;
+    return rs.total / missing >= std::max<uint64_t>(zc_threshold, kChunk);
 }
 
 lt_status Engine::load_missing() {

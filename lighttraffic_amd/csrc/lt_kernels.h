@@ -1317,6 +1317,18 @@ __global__ __launch_bounds__(256) void load_kernel(const DevSched *ds) {
     pull_words(ds->from[1], (uint32_t *)ds->col, ds->count[1]);
 }
 
+// Columns of a block image, in edge order: a lane an edge, so a block's header and
+// words are read by neighbouring lanes at once.  Bound by the link that the image
+// comes over (55 GB/s), not by this.
+__global__ __launch_bounds__(256) void unblock_kernel(const uint32_t *__restrict__ img, uint64_t m,
+                                                      uint32_t *__restrict__ col) {
+    Span sp{};
+    sp.col = img;
+    sp.words = img + 2 * ((m + kBlockEdges - 1) / kBlockEdges + 1);
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < m; e += stride) col[e] = span_col(sp, e);
+}
+
 // Unpacks a packed partition image into the col slice of an HBM slot whose
 // rowptr slice is already in place (it gives the row boundaries; rowptr[0] is
 // the partition's first global edge).  Image layout: meta u32[2*nch] (nch =

@@ -67,3 +67,24 @@ def test_some_partitions_cached_and_ppr():
     counts, ends = eng.pagerank(w, 3, endpoints=True)
     assert np.array_equal(counts, rc) and np.array_equal(ends, re)
     assert eng.stats()["graph_loading_calls"] == part.count - loaded
+
+
+@pytest.mark.parametrize("few", [1, 0])
+def test_batched_ppr(few):
+    """As many sources as partitions load them all at once; with one less, the
+    queues load them."""
+    print(f"first job batched ppr few={few}", flush=True)
+    g = lt.Graph.rmat(14, 16)
+    part = lt.Partition.build(g, 64 << 10)
+    P = part.count
+    nq = P - few
+    assert nq > P // 8
+    eng = lt.Engine(g, part, span="resident", resident_batch=16, zerocopy_threshold=0)
+    src = np.arange(nq, dtype=np.uint32) * 7
+    cnt = np.full(nq, -(-P * 4096 // nq), np.uint64)
+    re, _ = oracle.ppr_batch(g.rowptr(), g.col(), src, cnt, threads=8)
+    for first in (True, False):
+        assert np.array_equal(eng.ppr_batch(src, cnt), re)
+        st = eng.stats()
+        if first:
+            assert (st["iterations"] == 1 and st["graph_loading_calls"] == P) == (few == 0)
