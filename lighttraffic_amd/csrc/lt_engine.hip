@@ -241,6 +241,7 @@ struct Engine {
     VisitScratch vs{};
     unsigned long long *d_vcur = nullptr;
     uint64_t vlog_cap = 0;                       // entries allocated
+    bool log_asked = false;                      // a job would have used one
     uint32_t vregion = 0;                        // entries per region of the running job, 0 = no log
     lt_status ensure_log(uint64_t visits, bool queued);
     lt_status count_log(uint32_t n, uint32_t most);
@@ -267,7 +268,9 @@ struct Engine {
     size_t query_cap = 0;
     lt_status poll_host(const uint32_t *flag, uint32_t seq, const char *what);
     lt_status finish_job(bool small);
-    lt_status ensure_ring();
+    size_t ring_cap = 0;
+    bool ring_asked = false;  // a job would have used one
+    lt_status ensure_ring(size_t bytes);
     lt_status mark_ring(uint32_t slot);
     lt_status wait_ring(uint32_t slot);
     lt_status copy_results(ResultHelpers &help);
@@ -774,6 +777,12 @@ constexpr uint64_t kLogMost = 1ull << 26;  // entries: 256 MB, and 128 MB sorted
 lt_status Engine::ensure_log(uint64_t visits, bool queued) {
     vregion = 0;
     if (visits < (queued ? kLogVisitsQueued : kLogVisits) || nbins > kMaxBins) return LT_OK;
+    // An engine's first job would pay 0.3-0.5 ms for the allocation, and saves
+    // less where it counts few visits (3 M: 0.1 ms of atomics).
+    if (!vlog_cap && !log_asked && visits < kLogVisitsQueued) {
+        log_asked = true;
+        return LT_OK;
+    }
     if (!d_vcur) {
         const size_t cur = (size_t)kLogRegions * kCurStride;  // cursors, then the bins' totals and first units
         LT_TRY(dmalloc(&d_vcur, cur + nbins + 1));
@@ -2150,11 +2159,11 @@ lt_status Engine::run_flat(const RunSpec &rs, ResultHelpers &help) {
     // the next walkers walk.  (PPR lanes end one by one, and paths are written
     // a word per row: those results stay on the device until the end.)
     const uint32_t nout = (uint32_t)outs.size();
-    const bool ring = app_kind == APP_GENERIC && !a.app.paths && nout && nout * rs.total >= kManyOut;
+    const bool ring = ring_asked && app_kind == APP_GENERIC && !a.app.paths && nout && nout * rs.total >= kManyOut;
     constexpr uint32_t kTwo = kRing / 2;  // a launch takes two buffers: its last walkers leave
                                           // the card half idle for some 10 us
     if (ring) {
-        LT_TRY(ensure_ring());
+        LT_TRY(ensure_ring(kRing * kRingBytes));
         piece = 2 * kRingBytes / 4 / nout;
     }
     const auto drain = [&](uint64_t k) -> lt_status {  // launch k's results to the caller
@@ -2223,10 +2232,15 @@ lt_status Engine::finish_job(bool small) {
     return LT_OK;
 }
 
-lt_status Engine::ensure_ring() {
-    if (h_ring) return LT_OK;
-    LT_HIP(hipHostMalloc((void **)&h_ring, kRing * kRingBytes, hipHostMallocMapped | hipHostMallocCoherent));
+// Pinning takes 0.15 ms a MB: no more of it than a job's results fill.
+lt_status Engine::ensure_ring(size_t bytes) {
+    if (ring_cap >= bytes) return LT_OK;
+    if (h_ring) (void)hipHostFree(h_ring);  // (no job is running)
+    h_ring = nullptr;
+    ring_cap = 0;
+    LT_HIP(hipHostMalloc((void **)&h_ring, bytes, hipHostMallocMapped | hipHostMallocCoherent));
     LT_HIP(hipHostGetDevicePointer((void **)&d_ring, h_ring, 0));
+    ring_cap = bytes;
     return LT_OK;
 }
 
@@ -2242,20 +2256,35 @@ lt_status Engine::wait_ring(uint32_t slot) { return poll_host(h_out + kOutRing +
 // The results in pieces of a ring buffer's size: kernels fill the next buffers
 // while the team copies the oldest one out.
 lt_status Engine::copy_results(ResultHelpers &help) {
-    LT_TRY(ensure_ring());
+    if (!ring_asked) {  // an engine's first large results: pinning costs more than it saves (4 MB: 0.6 and 0.2 ms)
+        ring_asked = true;
+        for (const OutSeg &o : outs)
+            LT_HIP(hipMemcpyAsync(o.dst, o.src, 4 * o.words, hipMemcpyDeviceToHost, s_compute));
+        LT_HIP(hipStreamSynchronize(s_compute));
+        return LT_OK;
+    }
     std::vector<OutSeg> pieces;
+    std::vector<size_t> at;  // place of each in the ring: one behind the other if all fit
+    size_t end = 0;
     for (const OutSeg &o : outs)
-        for (uint64_t at = 0; at < o.words; at += kRingBytes / 4)
-            pieces.push_back({o.dst + at, o.src + at, std::min<uint64_t>(kRingBytes / 4, o.words - at)});
+        for (uint64_t i = 0; i < o.words; i += kRingBytes / 4) {
+            pieces.push_back({o.dst + i, o.src + i, std::min<uint64_t>(kRingBytes / 4, o.words - i)});
+            at.push_back(end);
+            end += (4 * pieces.back().words + 4095) & ~(size_t)4095;
+        }
+    if (pieces.size() > kRing) {
+        end = kRing * kRingBytes;
+        for (size_t i = 0; i < at.size(); i++) at[i] = i % kRing * kRingBytes;
+    }
+    LT_TRY(ensure_ring(end));
     for (size_t issued = 0, out = 0; out < pieces.size(); out++) {
         for (; issued < pieces.size() && issued < out + kRing; issued++) {
-            const uint32_t slot = issued % kRing;
-            fill_ring_kernel<<<64, 256, 0, s_compute>>>(pieces[issued].src, (uint32_t *)(d_ring + slot * kRingBytes),
+            fill_ring_kernel<<<64, 256, 0, s_compute>>>(pieces[issued].src, (uint32_t *)(d_ring + at[issued]),
                                                         pieces[issued].words);
-            LT_TRY(mark_ring(slot));
+            LT_TRY(mark_ring(issued % kRing));
         }
         LT_TRY(wait_ring(out % kRing));
-        help.copiers().copy(pieces[out].dst, h_ring + out % kRing * kRingBytes, 4 * pieces[out].words);
+        help.copiers().copy(pieces[out].dst, h_ring + at[out], 4 * pieces[out].words);
     }
     return LT_OK;
 }
