@@ -92,7 +92,10 @@ typedef struct {
                                        frame-of-reference blocks that stay
                                        packed in the cache slot and are read in
                                        place, so slots are smaller and the
-                                       cache holds more partitions.  A
+                                       cache holds more partitions (raw slots
+                                       asked for all of them: the images
+                                       travel, and the columns are kept raw
+                                       unless memory is short).  A
                                        partition that does not get smaller is
                                        copied as is (default 0: off;
                                        device_schedule: 2 only, 1 is ignored)   */

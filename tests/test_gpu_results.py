@@ -37,3 +37,16 @@ def test_results_by_walker(graph, kw, w):
     assert np.array_equal(counts, rc) and np.array_equal(ends, re)
     if w < 600000:
         assert np.array_equal(eng.genericwalk_paths(w, 4), oracle.genericwalk_paths(rp, col, w, 4))
+
+
+@pytest.mark.parametrize("w", [70001, 524288, 1048577, 3 * 1048576 + 77])
+def test_later_jobs_of_one_engine(graph, w):
+    """The first large results go by plain copies, later ones through a ring that
+    grows with them; both arrays of a flat walk are written into it in launches."""
+    print(f"results of later jobs w={w}", flush=True)
+    rp, col = graph.rowptr(), graph.col()
+    eng = lt.Engine(graph, lt.Partition.build(graph, 32 << 20), zerocopy_threshold=0)
+    for n in (66000, 66001, w, 70000, w):
+        re, rm, _ = oracle.genericwalk(rp, col, n, 4, threads=16)
+        ends, moves = eng.genericwalk(n, 4, moves=True)
+        assert np.array_equal(ends, re) and np.array_equal(moves, rm)
