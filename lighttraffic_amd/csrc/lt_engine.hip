@@ -346,8 +346,8 @@ struct Engine {
     // Small slices are copied by one kernel instead of two DMAs, whose second
     // costs 10 us of its own (256 KB: 14 us, 22 by DMAs; 1 MB: 28 and 38).  Larger
     // ones hold the walk up: beside a kernel that reads the link for 50 to 80
-    // us its launches took twice as long (s23, 4 MB slots: 14.0 ms a job by DMAs, 17.6
-    // so; s20 reference rules, 2 MB: 24.4 and 28.7; s20 ppr, 1 MB: 27.8 and 25.7).
+    // us its launches took twice as long (s23, 4 MB slots: 12.1 ms a job by DMAs, 13.7
+    // so; s20 reference rules, 2 MB: 20.2 and 24.7; s20 ppr, 1 MB: 15.5 and 14.5).
     static constexpr size_t kPullBytes = 1280u << 10;
     static constexpr int kPullGrid = 64;
     bool pulls(uint32_t p) const {
