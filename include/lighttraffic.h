@@ -149,7 +149,12 @@ typedef struct {
 /* Statistics of the last run call.  The first eight fields mirror the lines
  * that Scheduler::timing prints (src/Scheduler.h:440-453). */
 typedef struct {
-    double   running_ms;            /* "Running Time" (walk phase only)          */
+    double   running_ms;            /* "Running Time" (walk phase only), host
+                                       clock: the scheduler loop and the counting
+                                       behind it, or, of a job walked over a graph
+                                       that lies whole in HBM, from its first load
+                                       or launch (which creates the walkers too)
+                                       until its walks are over                  */
     uint64_t iterations;            /* scheduler iterations                      */
     uint64_t explicit_iterations;   /* iterations that used an HBM-resident copy */
     double   graph_loading_ms;  uint64_t graph_loading_calls;
@@ -375,7 +380,7 @@ typedef struct {
     int32_t  split;            /* 0: lt_partition_build(S); 1 (block copies only):
                                   lt_partition_build_blocks(S), slots =
                                   cache_bytes / its partition_bytes             */
-    double   running_ms;       /* the warm job's scheduler-loop time               */
+    double   running_ms;       /* the warm job's lt_stats.running_ms               */
     uint64_t h2d_bytes;        /* its explicit + zero-copied H2D bytes             */
     uint64_t iterations;       /* its scheduler iterations                         */
 } lt_tune_trial;

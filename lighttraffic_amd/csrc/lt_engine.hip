@@ -115,11 +115,9 @@ struct EventTimer {
     }
 };
 
-// h_out: kNumStats u64 of event counters, the job's time in ticks of the
-// device's wall clock, the sequence number, those of the ring's buffers, that of the
-// last load finished, then small results.
-constexpr uint32_t kOutTicks = 2 * kNumStats, kOutFlag = kOutTicks + 1, kOutRing = kOutFlag + 1, kOutCopy = 32,
-                   kOutData = 64;
+// h_out: kNumStats u64 of event counters, the sequence number, those of the
+// ring's buffers, that of the last load finished, then small results.
+constexpr uint32_t kOutFlag = 2 * kNumStats, kOutRing = kOutFlag + 1, kOutCopy = 32, kOutData = 64;
 constexpr uint64_t kManyOut = 1u << 20;  // words: from here on threads help with the results
 
 struct RunSpec {
@@ -260,7 +258,8 @@ struct Engine {
     static constexpr size_t kRingBytes = 2u << 20;
     uint32_t *h_out = nullptr, *d_out = nullptr;  // pinned: event counters, sequence number, small results
     uint32_t out_seq = 0;
-    int wall_khz = 100000;                        // rate of the device's wall clock
+    bool over = false;                            // the running job's walks were seen to be over,
+    std::chrono::steady_clock::time_point t_over; // and when
     uint8_t *h_ring = nullptr, *d_ring = nullptr; // pinned: kRing buffers
     uint32_t ring_seq[kRing] = {};                // of each buffer's last fill
     std::vector<OutSeg> outs;                     // results of the running job
@@ -268,6 +267,8 @@ struct Engine {
     size_t query_cap = 0;
     lt_status poll_host(const uint32_t *flag, uint32_t seq, const char *what);
     lt_status finish_job(bool small);
+    bool walks_over();
+    lt_status wait_walks();
     size_t ring_cap = 0;
     bool ring_asked = false;  // a job would have used one
     lt_status ensure_ring(size_t bytes);
@@ -672,12 +673,10 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
     res_batch = std::min(res_batch, kMaxZcBatch);
     if (cfg.span != LT_SPAN_RESIDENT) res_batch = 1;
     slice = cfg.slice_chunks > 0 ? (uint32_t)cfg.slice_chunks : kSliceChunks;
-    LT_TRY(dmalloc(&d_stats, (size_t)kNumStats * kStatSlots + 1));
+    LT_TRY(dmalloc(&d_stats, (size_t)kNumStats * kStatSlots));
     LT_HIP(hipHostMalloc((void **)&h_out, 4 * (kOutData + kSmallOut), hipHostMallocMapped | hipHostMallocCoherent));
     memset(h_out, 0, 4 * kOutData);
     LT_HIP(hipHostGetDevicePointer((void **)&d_out, h_out, 0));
-    int khz = 0;
-    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0) wall_khz = khz;
     counts.assign(P, 0);
     dcounts.assign(P, 0);
     hq.assign(P, {});
@@ -2201,14 +2200,18 @@ lt_status Engine::run_flat(const RunSpec &rs, ResultHelpers &help) {
     job_finished = ring;
     if (ring) {
         LT_TRY(finish_job(false));
-        for (; drained < k; drained++) LT_TRY(drain(drained));
-        LT_TRY(poll_host(h_out + kOutFlag, out_seq, "results"));
+        for (; drained < k; drained++) {  // the last buffer's copy is behind the walks
+            if (drained + 1 == k) LT_TRY(wait_walks());
+            LT_TRY(drain(drained));
+            walks_over();
+        }
     }
     return LT_OK;
 }
 
 // Last kernels of a job: its small results and event counters into pinned
-// memory; waits for them, and so for the job's walks.
+// memory; waits for them, and so for the job's walks (large results:
+// copy_results does).
 lt_status Engine::finish_job(bool small) {
     if (small && !outs.empty()) {
         SmallOut o{};
@@ -2222,13 +2225,29 @@ lt_status Engine::finish_job(bool small) {
     }
     finish_kernel<<<1, kStatSlots, 0, s_compute>>>(d_stats, d_out, d_out + kOutFlag, ++out_seq);
     LT_HIP(hipGetLastError());
-    if (!small) return LT_OK;  // copy_results first
-    LT_TRY(poll_host(h_out + kOutFlag, out_seq, "results"));
+    if (!small) return LT_OK;
+    LT_TRY(wait_walks());
     const uint32_t *from = h_out + kOutData;
     for (const OutSeg &o : outs) {
         memcpy(o.dst, from, 4 * o.words);
         from += o.words;
     }
+    return LT_OK;
+}
+
+// Whether finish_kernel has been seen to be over.  The first time that it is ends
+// the job's running time, on the host's clock by whichever route it walked.
+bool Engine::walks_over() {
+    if (!over && __atomic_load_n(h_out + kOutFlag, __ATOMIC_ACQUIRE) == out_seq) {
+        over = true;
+        t_over = std::chrono::steady_clock::now();
+    }
+    return over;
+}
+
+lt_status Engine::wait_walks() {
+    if (!over) LT_TRY(poll_host(h_out + kOutFlag, out_seq, "results"));
+    walks_over();
     return LT_OK;
 }
 
@@ -2258,6 +2277,7 @@ lt_status Engine::wait_ring(uint32_t slot) { return poll_host(h_out + kOutRing +
 lt_status Engine::copy_results(ResultHelpers &help) {
     if (!ring_asked) {  // an engine's first large results: pinning costs more than it saves (4 MB: 0.6 and 0.2 ms)
         ring_asked = true;
+        LT_TRY(wait_walks());
         for (const OutSeg &o : outs)
             LT_HIP(hipMemcpyAsync(o.dst, o.src, 4 * o.words, hipMemcpyDeviceToHost, s_compute));
         LT_HIP(hipStreamSynchronize(s_compute));
@@ -2282,7 +2302,9 @@ lt_status Engine::copy_results(ResultHelpers &help) {
             fill_ring_kernel<<<64, 256, 0, s_compute>>>(pieces[issued].src, (uint32_t *)(d_ring + at[issued]),
                                                         pieces[issued].words);
             LT_TRY(mark_ring(issued % kRing));
+            walks_over();
         }
+        LT_TRY(wait_walks());
         LT_TRY(wait_ring(out % kRing));
         help.copiers().copy(pieces[out].dst, h_ring + at[out], 4 * pieces[out].words);
     }
@@ -2394,7 +2416,7 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
 
     double running_ms = 0;
     auto t_walk = std::chrono::steady_clock::now();
-    job_finished = false;
+    job_finished = over = false;
     if (walk_flat && missing) LT_TRY(load_missing());
     if (walk_flat) LT_TRY(run_flat(rs, help));
     for (uint64_t id0 = walk_flat ? rs.total : 0; id0 < rs.total; id0 += wave) {
@@ -2458,16 +2480,10 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
         LT_HIP(hipGetLastError());
     }
     // reduce (app/pagerank.cu:71-74): results back to the host, untimed but for
-    // those of a few pages, which the last kernels write
+    // those that the walks write to the ring
     if (!job_finished) LT_TRY(finish_job(small));
-    if (!small && !walk_flat) LT_TRY(poll_host(h_out + kOutFlag, out_seq, "results"));
-    if (!walk_flat)
-        running_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_walk).count();
-    if (!small && !job_finished) {
-        LT_TRY(copy_results(help));
-        LT_TRY(poll_host(h_out + kOutFlag, out_seq, "results"));
-    }
-    if (walk_flat) running_ms = h_out[kOutTicks] / (double)wall_khz;
+    if (!small && !job_finished) LT_TRY(copy_results(help));
+    running_ms += std::chrono::duration<double, std::milli>(t_over - t_walk).count();
     outs.clear();
     unsigned long long hs[kNumStats];
     for (int i = 0; i < kNumStats; i++) hs[i] = h_out[2 * i] | (unsigned long long)h_out[2 * i + 1] << 32;

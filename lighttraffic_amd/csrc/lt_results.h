@@ -66,12 +66,10 @@ __global__ void mark_kernel(uint32_t *flag, uint32_t seq) {
     __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// The job's event counters summed over their slots into pinned memory, and the
-// time since begin_kernel, then the sequence number that the host polls.  One
-// workgroup, last of the job.
+// The job's event counters summed over their slots into pinned memory, then the
+// sequence number that the host polls.  One workgroup, last of the job.
 __global__ __launch_bounds__(kStatSlots) void finish_kernel(const unsigned long long *stats, uint32_t *out,
                                                             uint32_t *flag, uint32_t seq) {
-    const uint32_t ticks = (uint32_t)(wall_clock64() - stats[kNumStats * kStatSlots]);
     __shared__ unsigned long long s_part[kStatSlots / 64][kNumStats];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
 #pragma unroll
@@ -89,14 +87,13 @@ __global__ __launch_bounds__(kStatSlots) void finish_kernel(const unsigned long 
         to_host(&out[2 * threadIdx.x], (uint32_t)x);
         to_host(&out[2 * threadIdx.x + 1], (uint32_t)(x >> 32));
     }
-    if (threadIdx.x == 0) to_host(&out[2 * kNumStats], ticks);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (threadIdx.x == 0) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Clears what a job accumulates into: counters of visits and events, the visit
-// log's cursors.  Notes the time.
+// log's cursors.
 __global__ __launch_bounds__(256) void begin_kernel(uint32_t *counts, uint64_t n, unsigned long long *stats,
                                                     unsigned long long *vcur) {
     const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -105,7 +102,6 @@ __global__ __launch_bounds__(256) void begin_kernel(uint32_t *counts, uint64_t n
     if (tid < n % 4) counts[n / 4 * 4 + tid] = 0;
     for (uint64_t i = tid; i < (uint64_t)kNumStats * kStatSlots; i += stride) stats[i] = 0;
     if (vcur && tid < kLogRegions) vcur[tid * kCurStride] = 0;
-    if (tid == 0) stats[kNumStats * kStatSlots] = wall_clock64();
 }
 
 // Threads that map the pages of result buffers for writing, whose contents stay

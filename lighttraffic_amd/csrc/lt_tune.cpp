@@ -138,7 +138,7 @@ extern "C" lt_status lt_tune_ppr_batch(const lt_graph *g, uint32_t nq, const uin
     // stage 2: the three fastest and the fastest of each copy mode (block
     // copies on either split), on a sample four times larger
     std::vector<lt_tune_trial> top(trials);
-    // equal times (a flat job's are whole ticks of 10 ns) stay in trial order
+    // equal times stay in trial order
     std::stable_sort(top.begin(), top.end(), [](const lt_tune_trial &a, const lt_tune_trial &b) {
         return a.running_ms < b.running_ms;
     });
