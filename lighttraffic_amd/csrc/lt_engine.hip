@@ -64,6 +64,18 @@ static void dfree(T *&p) {
     p = nullptr;
 }
 
+// Room for n elements, whose old contents go.  cap is what p holds, also after a
+// failure: a later job that needs less must not take the buffer for granted.
+template <typename T>
+static lt_status regrow(T **p, size_t &cap, size_t n) {
+    if (cap >= n && *p) return LT_OK;
+    dfree(*p);
+    cap = 0;
+    const lt_status s = dmalloc(p, n);
+    if (s == LT_OK) cap = n;
+    return s;
+}
+
 // Accumulates HIP-event intervals on one stream (GPUTimer, src/utils/Stopwatch.h:49-104).
 struct EventTimer {
     std::vector<std::pair<hipEvent_t, hipEvent_t>> open;
@@ -251,7 +263,7 @@ struct Engine {
     size_t moves_cap = 0;
     uint64_t *d_qoff = nullptr;
     uint32_t *d_qsrc = nullptr;
-    size_t q_cap = 0;
+    size_t qoff_cap = 0, qsrc_cap = 0;
     unsigned long long *d_stats = nullptr;
     // Results on their way to the caller (lt_results.h).
     static constexpr uint32_t kRing = 4;
@@ -713,6 +725,7 @@ lt_status Engine::ensure_pool(uint64_t walkers, bool check_only) {
         return LT_E_ARG;
     }
     if (check_only) return LT_OK;
+    wcap = 0;  // until all four are there
     dfree(q.slab);
     dfree(q.frame);
     dfree(q.free_stack);
@@ -728,36 +741,13 @@ lt_status Engine::ensure_pool(uint64_t walkers, bool check_only) {
 }
 
 lt_status Engine::ensure_outputs(const RunSpec &rs, bool want_endpoints, bool want_moves) {
-    const size_t ncount = (size_t)V * count_copies;
-    if (counts_cap < ncount) {
-        dfree(d_counts);
-        LT_TRY(dmalloc(&d_counts, ncount));
-        counts_cap = ncount;
-    }
-    if (want_endpoints && endpoints_cap < rs.total) {
-        dfree(d_endpoints);
-        LT_TRY(dmalloc(&d_endpoints, rs.total));
-        endpoints_cap = rs.total;
-    }
-    if (rs.paths_out) {
-        const size_t n = (size_t)rs.total * ((size_t)rs.length + 1);
-        if (paths_cap < n) {
-            dfree(d_paths);
-            LT_TRY(dmalloc(&d_paths, n));
-            paths_cap = n;
-        }
-    }
-    if (want_moves && moves_cap < rs.total) {
-        dfree(d_moves);
-        LT_TRY(dmalloc(&d_moves, rs.total));
-        moves_cap = rs.total;
-    }
-    if (rs.nq && q_cap < rs.nq) {
-        dfree(d_qoff);
-        dfree(d_qsrc);
-        LT_TRY(dmalloc(&d_qoff, rs.nq + 1));
-        LT_TRY(dmalloc(&d_qsrc, rs.nq));
-        q_cap = rs.nq;
+    LT_TRY(regrow(&d_counts, counts_cap, (size_t)V * count_copies));
+    if (want_endpoints) LT_TRY(regrow(&d_endpoints, endpoints_cap, rs.total));
+    if (rs.paths_out) LT_TRY(regrow(&d_paths, paths_cap, (size_t)rs.total * ((size_t)rs.length + 1)));
+    if (want_moves) LT_TRY(regrow(&d_moves, moves_cap, rs.total));
+    if (rs.nq) {
+        LT_TRY(regrow(&d_qoff, qoff_cap, (size_t)rs.nq + 1));
+        LT_TRY(regrow(&d_qsrc, qsrc_cap, rs.nq));
     }
     return LT_OK;
 }
@@ -1329,6 +1319,7 @@ lt_status Engine::spill_round(const std::vector<uint32_t> &victims) {
         dfree(d_plan);
         if (h_plan) (void)hipHostFree(h_plan);
         h_plan = nullptr;
+        plan_cap = 0;
         LT_TRY(dmalloc(&d_plan, bytes));
         LT_HIP(hipHostMalloc((void **)&h_plan, bytes, hipHostMallocDefault));
         plan_cap = bytes;

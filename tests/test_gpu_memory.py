@@ -1,0 +1,114 @@
+"""Jobs whose allocations fail, forced from the host (hipfail/): no failed one
+leaves an engine that later jobs cannot use.  Each child process makes the
+chosen runtime calls fail and checks its jobs against the CPU oracle."""
+import ctypes
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+MALLOC, HOST_MALLOC, MEMCPY_ASYNC = range(3)
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def shim(tmp_path_factory):
+    path = str(tmp_path_factory.mktemp("hipfail") / "libhipfail.so")
+    subprocess.run(["gcc", "-O1", "-fPIC", "-shared", "-o", path, os.path.join(HERE, "hipfail", "hipfail.c"), "-ldl"],
+                   check=True)
+    return path
+
+
+def child(shim, *args):
+    print("memory", *args, flush=True)
+    r = subprocess.run([sys.executable, "-u", os.path.abspath(__file__), shim, *map(str, args)], capture_output=True,
+                       text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.endswith("done\n"), r.stdout[-2000:] + r.stderr[-2000:]
+
+
+@pytest.mark.parametrize("form", ["flat", "queues", "spill", "batch", "device"])
+def test_after_a_failed_allocation(shim, form):
+    """Every device allocation of a job fails in turn, after a smaller job had run."""
+    child(shim, "after", form)
+
+
+# ---- the child process ------------------------------------------------------------
+
+FORMS = {"flat": dict(span="resident", resident_batch=16, zerocopy_threshold=0),
+         "queues": dict(num_device_partitions=3, span="resident"),
+         "spill": dict(num_device_partitions=3, num_device_walkers=9000),
+         "batch": dict(num_device_partitions=3),
+         "device": dict(num_device_partitions=3, device_schedule=1)}
+
+
+class Child:
+    def __init__(self, path):
+        self.lib = ctypes.CDLL(path, mode=ctypes.RTLD_GLOBAL)
+        self.lib.hipfail_failed.restype = self.lib.hipfail_calls.restype = ctypes.c_long
+        sys.path.insert(0, ROOT)
+        import numpy as np
+
+        import lighttraffic_amd as lt
+        from oracle import ffi as oracle
+        self.np, self.lt, self.oracle = np, lt, oracle
+        self.graph = lt.Graph.rmat(13, 8)
+        self.rp, self.col = self.graph.rowptr(), self.graph.col()
+        self.part = lt.Partition.build(self.graph, 32 << 10)
+        assert self.part.count > 8
+
+    def arm(self, kind, skip=0, times=1, least=0, most=1 << 62):
+        self.lib.hipfail_arm(ctypes.c_int(kind), ctypes.c_long(skip), ctypes.c_long(times), ctypes.c_size_t(least),
+                             ctypes.c_size_t(most))
+
+    def disarm(self, kind):
+        n = self.lib.hipfail_failed(kind)
+        self.arm(kind, times=0)
+        return n
+
+    def engine(self, **kw):
+        return self.lt.Engine(self.graph, self.part, **kw)
+
+    def jobs(self, eng, w, batch=False):
+        """Jobs of every kind with w walkers; wrong values raise AssertionError."""
+        np, o, rp, col = self.np, self.oracle, self.rp, self.col
+        if batch:
+            src, cnt = np.arange(7, dtype=np.uint32), np.full(7, w // 7 + 1, np.uint64)
+            assert np.array_equal(eng.ppr_batch(src, cnt), o.ppr_batch(rp, col, src, cnt, threads=8)[0])
+            return
+        counts, ends = eng.pagerank(w, 4, endpoints=True)
+        rc, re, _ = o.pagerank(rp, col, w, 4, endpoints=True, threads=8)
+        assert np.array_equal(counts, rc) and np.array_equal(ends, re)
+        ends, moves = eng.genericwalk(w, 3, moves=True)
+        re, rm, _ = o.genericwalk(rp, col, w, 3, threads=8)
+        assert np.array_equal(ends, re) and np.array_equal(moves, rm)
+        assert np.array_equal(eng.genericwalk_paths(w, 3), o.genericwalk_paths(rp, col, w, 3))
+
+    def after(self, form):
+        small, large, n = 5000, 60000, 0
+        while True:
+            eng = self.engine(**FORMS[form])
+            self.jobs(eng, small, form == "batch")
+            self.arm(MALLOC, skip=n)
+            try:
+                self.jobs(eng, large, form == "batch")
+            except self.lt.LTError as e:
+                assert e.status == 4, e  # LT_E_NOMEM
+            failed = self.disarm(MALLOC)
+            print(form, "allocation", n, "failed" if failed else "was not made", flush=True)
+            for w in (small + 1000, small, large):
+                self.jobs(eng, w, form == "batch")
+            eng.close()
+            if not failed:
+                assert n > 2
+                return
+            n += 1
+
+
+if __name__ == "__main__":
+    c = Child(sys.argv[1])
+    getattr(c, sys.argv[2])(*sys.argv[3:])
+    print("done", flush=True)
