@@ -187,6 +187,7 @@ struct Engine {
     uint64_t *flat_rowptr = nullptr;   // [V+1], in d_slots
     uint32_t *flat_col = nullptr;      // [E], in d_slots
     uint32_t *d_rowptr32 = nullptr;    // [V+1] copy of flat_rowptr once every partition is cached (E < 2^32)
+    bool rowptr32_set = false;         // it has been written
     std::vector<int32_t> slot_of;      // partition -> slot or -1
     std::vector<int32_t> part_in_slot; // slot -> partition or -1
     std::vector<uint32_t> free_slots;
@@ -253,7 +254,9 @@ struct Engine {
     uint64_t vlog_cap = 0;                       // entries allocated
     bool log_asked = false;                      // a job would have used one
     uint32_t vregion = 0;                        // entries per region of the running job, 0 = no log
-    lt_status ensure_log(uint64_t visits, bool queued);
+    bool wants_log(uint64_t visits, bool queued);
+    bool ensure_log(uint64_t visits);
+    void drop_log();
     lt_status count_log(uint32_t n, uint32_t most);
     uint32_t *d_endpoints = nullptr;
     size_t endpoints_cap = 0;
@@ -325,6 +328,8 @@ struct Engine {
     lt_status init(const lt_graph *g_, const lt_partition *p_, const lt_config *c);
     lt_status ensure_pool(uint64_t walkers, bool check_only = false);
     lt_status ensure_outputs(const RunSpec &rs, bool want_endpoints, bool want_moves);
+    lt_status ensure_memory(const RunSpec &rs, uint64_t walkers, bool counting, bool want_endpoints, bool want_moves,
+                            bool &walk_flat);
     lt_status run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoints_out, uint32_t *moves_out);
 
     // scheduler primitives
@@ -761,43 +766,94 @@ lt_status Engine::ensure_outputs(const RunSpec &rs, bool want_endpoints, bool wa
 // vertices) the scatter's LDS does not hold a tile's histogram, and a device
 // that cannot hold a log counts directly.
 constexpr uint64_t kLogVisits = 1u << 18, kLogVisitsQueued = 1u << 24;
-constexpr uint64_t kLogMost = 1ull << 26;  // entries: 256 MB, and 128 MB sorted
+constexpr uint64_t kLogMost = 1ull << 26;  // entries: 256 MB; 0.75 GB with what counting them takes
 
-lt_status Engine::ensure_log(uint64_t visits, bool queued) {
-    vregion = 0;
-    if (visits < (queued ? kLogVisitsQueued : kLogVisits) || nbins > kMaxBins) return LT_OK;
+bool Engine::wants_log(uint64_t visits, bool queued) {
+    if (visits < (queued ? kLogVisitsQueued : kLogVisits) || nbins > kMaxBins) return false;
     // An engine's first job would pay 0.3-0.5 ms for the allocation, and saves
     // less where it counts few visits (3 M: 0.1 ms of atomics).
     if (!vlog_cap && !log_asked && visits < kLogVisitsQueued) {
         log_asked = true;
-        return LT_OK;
+        return false;
     }
-    if (!d_vcur) {
-        const size_t cur = (size_t)kLogRegions * kCurStride;  // cursors, then the bins' totals and first units
-        LT_TRY(dmalloc(&d_vcur, cur + nbins + 1));
-        vs.total = (uint32_t *)(d_vcur + cur);
-        vs.unit_off = vs.total + nbins;
-    }
+    return true;
+}
+
+// Whether there is memory for it.
+bool Engine::ensure_log(uint64_t visits) {
     // regions fill unevenly: a quarter more, and a launch's workgroups' buffers
     visits = std::min(visits, kLogMost);
     const uint64_t want = std::min(kLogMost, visits + visits / 4 + (1u << 20)) & ~(uint64_t)(kTile * kLogRegions - 1);
     if (vlog_cap < want) {
+        drop_log();
+        const size_t cur = (size_t)kLogRegions * kCurStride;  // cursors, then the bins' totals and first units
         // The log and what counting a full one takes, in one allocation: one by
         // one they took a new engine's first job 0.6 ms, with tens of MB or few.
         const uint64_t tiles = want / kTile + kLogRegions;
         const uint64_t units = std::max<uint64_t>(nbins <= kFewBins ? std::min<uint64_t>(kFewUnits, tiles * nbins) : 0,
                                                   std::min<uint64_t>(want / kHistUnit, kHistUnits) + 1 + nbins);
         const uint64_t words[4] = {want, want / 2, tiles * nbins, units * kBin};  // multiples of 4 but the third
-        dfree(vl.log);
-        vlog_cap = 0;
-        if (dmalloc(&vl.log, words[0] + words[1] + words[2] + 4 + words[3]) != LT_OK) return LT_OK;
+        if (dmalloc(&d_vcur, cur + nbins + 1) != LT_OK ||
+            dmalloc(&vl.log, words[0] + words[1] + words[2] + 4 + words[3]) != LT_OK) {
+            drop_log();
+            return false;
+        }
+        vs.total = (uint32_t *)(d_vcur + cur);
+        vs.unit_off = vs.total + nbins;
         vs.sorted = (uint16_t *)(vl.log + words[0]);
         vs.run = vl.log + words[0] + words[1];
         vs.partial = vs.run + ((words[2] + 3) & ~3ull);
         vlog_cap = want;
     }
     vregion = (uint32_t)(want / kLogRegions);
-    return LT_OK;
+    return true;
+}
+
+void Engine::drop_log() {
+    dfree(d_vcur);
+    dfree(vl.log);
+    vlog_cap = 0;
+}
+
+// Device memory of a job.  What it cannot do without comes first; the visit log, the
+// counters' copies and the flat walks' row offsets give way to that, and none of
+// these fails a job that does without.
+lt_status Engine::ensure_memory(const RunSpec &rs, uint64_t walkers, bool counting, bool want_endpoints,
+                                bool want_moves, bool &walk_flat) {
+    uint64_t visits = rs.total;
+    if (rs.app == APP_PAGERANK && __builtin_mul_overflow(rs.total, (uint64_t)rs.length, &visits)) visits = UINT64_MAX;
+    vregion = 0;
+    if (walk_flat && !d_rowptr32 && dmalloc(&d_rowptr32, (size_t)V + 1) != LT_OK) walk_flat = false;
+    bool one = false;  // no copies
+    bool log = counting && wants_log(visits, !walk_flat);
+    while (true) {
+        // Without a log, copies of the counters, one per XCD: where the walkers of
+        // one launch stay in a few partitions (capped cache, PPR around its sources; one
+        // array measured 29 % slower there), and where clearing and adding up the
+        // copies of a small graph costs less than its hot vertices' atomics (5 G/s in
+        // one array, 27 G/s in copies).
+        const bool copies =
+            (!walk_flat && (nslots < P || rs.app == APP_PPR)) || (visits >= (1u << 16) && V <= (1u << 20));
+        count_copies = counting && !log && copies && !one ? kCountCopies : 1;
+        lt_status s = ensure_pool(walkers, walk_flat);  // a flat job keeps the queues' limits
+        if (s == LT_OK) s = ensure_outputs(rs, want_endpoints, want_moves);
+        if (s == LT_OK) {
+            if (!log || ensure_log(visits)) return LT_OK;
+            log = false;
+        } else if (s != LT_E_NOMEM) {
+            return s;
+        } else if (vl.log) {
+            drop_log();
+        } else if (count_copies > 1) {
+            one = true;
+        } else if (d_rowptr32) {
+            dfree(d_rowptr32);
+            rowptr32_set = walk_flat = false;
+            log = log && wants_log(visits, true);
+        } else {
+            return s;
+        }
+    }
 }
 
 // Counts the log into d_counts and empties it: the n entries of a flat job's
@@ -2128,11 +2184,11 @@ constexpr uint64_t kFlatPiece = (uint64_t)kSliceChunks * kChunk;
 // in registers, so the queues are not touched.  Row offsets are read as 32
 // bits, which halves the lines that the hot rows take in L2.
 lt_status Engine::run_flat(const RunSpec &rs, ResultHelpers &help) {
-    if (!d_rowptr32) {  // kept: slots of a flat cache are never evicted
-        LT_TRY(dmalloc(&d_rowptr32, (size_t)V + 1));
+    if (!rowptr32_set) {  // kept: slots of a flat cache are never evicted
         narrow_rowptr_kernel<<<std::min<int>(8 * num_cu, (int)(V / 256 + 1)), 256, 0, s_compute>>>(
             flat_rowptr, d_rowptr32, (size_t)V + 1);
         LT_HIP(hipGetLastError());
+        rowptr32_set = true;
     }
     FlatArgs a{};
     a.app = app;
@@ -2329,21 +2385,10 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
     dev_cap = cap;
     const uint64_t wave = spill_on ? rs.total : cap;
     const bool counting = rs.app != APP_GENERIC && counts_out;
-    uint64_t visits = rs.total;
-    if (rs.app == APP_PAGERANK && __builtin_mul_overflow(rs.total, (uint64_t)rs.length, &visits)) visits = UINT64_MAX;
     uint32_t missing;
-    const bool walk_flat = can_run_flat(rs, missing);
-    if (counting) LT_TRY(ensure_log(visits, !walk_flat));
-    else vregion = 0;
-    // Without a log, copies of the counters, one per XCD: where the walkers of
-    // one launch stay in a few partitions (capped cache, PPR around its sources; one
-    // array measured 29 % slower there), and where clearing and adding up the
-    // copies of a small graph costs less than its hot vertices' atomics (5 G/s in
-    // one array, 27 G/s in copies).
-    const bool copies = (!walk_flat && (nslots < P || rs.app == APP_PPR)) || (visits >= (1u << 16) && V <= (1u << 20));
-    count_copies = counting && !vregion && copies ? kCountCopies : 1;
-    LT_TRY(ensure_pool(std::max<uint64_t>(cap, 1), walk_flat));  // a flat job keeps the queues' limits
-    LT_TRY(ensure_outputs(rs, endpoints_out != nullptr, moves_out != nullptr));
+    bool walk_flat = can_run_flat(rs, missing);
+    LT_TRY(ensure_memory(rs, std::max<uint64_t>(cap, 1), counting, endpoints_out != nullptr, moves_out != nullptr,
+                         walk_flat));
 
     app_kind = rs.app;
     app = AppArgs{};

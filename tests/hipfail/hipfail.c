@@ -43,10 +43,36 @@ static int fails(int kind, size_t bytes) {
     return 1;
 }
 
+/* Device memory: bytes that the engine's library holds, and may hold. */
+static size_t held, limit = (size_t)-1;
+static struct {
+    void *p;
+    size_t n;
+} block[4096];
+void hipfail_limit(size_t bytes) { limit = bytes; }
+size_t hipfail_held(void) { return held; }
+
 /* hipErrorOutOfMemory is 2, hipErrorUnknown 999 */
 int hipMalloc(void **p, size_t n) {
-    if (fails(MALLOC, n)) return 2;
-    return ((int (*)(void **, size_t))runtime("hipMalloc"))(p, n);
+    if (fails(MALLOC, n) || n > limit || held > limit - n) return 2;
+    const int e = ((int (*)(void **, size_t))runtime("hipMalloc"))(p, n);
+    int i = 0;
+    while (!e && block[i].p) i++;
+    if (!e) {
+        block[i].p = *p;
+        block[i].n = n;
+        held += n;
+    }
+    return e;
+}
+int hipFree(void *p) {
+    for (int i = 0; p && i < 4096; i++)
+        if (block[i].p == p) {
+            block[i].p = NULL;
+            held -= block[i].n;
+            break;
+        }
+    return ((int (*)(void *))runtime("hipFree"))(p);
 }
 int hipHostMalloc(void **p, size_t n, unsigned flags) {
     if (fails(HOST_MALLOC, n)) return 2;

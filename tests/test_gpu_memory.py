@@ -36,6 +36,14 @@ def test_after_a_failed_allocation(shim, form):
     child(shim, "after", form)
 
 
+@pytest.mark.parametrize("what", ["log", "kept_log", "offsets"])
+def test_what_only_speeds_a_job_up_gives_way(shim, what):
+    """A job runs in the memory that it cannot do without: no visit log where it would
+    take the outputs' memory, a log of earlier jobs freed for them, and no flat walk
+    where its row offsets do not fit."""
+    child(shim, what)
+
+
 # ---- the child process ------------------------------------------------------------
 
 FORMS = {"flat": dict(span="resident", resident_batch=16, zerocopy_threshold=0),
@@ -48,6 +56,7 @@ FORMS = {"flat": dict(span="resident", resident_batch=16, zerocopy_threshold=0),
 class Child:
     def __init__(self, path):
         self.lib = ctypes.CDLL(path, mode=ctypes.RTLD_GLOBAL)
+        self.lib.hipfail_held.restype = ctypes.c_size_t
         self.lib.hipfail_failed.restype = self.lib.hipfail_calls.restype = ctypes.c_long
         sys.path.insert(0, ROOT)
         import numpy as np
@@ -68,6 +77,12 @@ class Child:
         n = self.lib.hipfail_failed(kind)
         self.arm(kind, times=0)
         return n
+
+    def held(self):
+        return self.lib.hipfail_held()
+
+    def limit(self, n):
+        self.lib.hipfail_limit(ctypes.c_size_t(n))
 
     def engine(self, **kw):
         return self.lt.Engine(self.graph, self.part, **kw)
@@ -106,6 +121,55 @@ class Child:
                 assert n > 2
                 return
             n += 1
+
+    def pagerank(self, eng, w, l):
+        counts, ends = eng.pagerank(w, l, endpoints=True)
+        rc, re, _ = self.oracle.pagerank(self.rp, self.col, w, l, endpoints=True, threads=16)
+        assert self.np.array_equal(counts, rc) and self.np.array_equal(ends, re)
+        return eng.stats()
+
+    W, L = 1200000, 30  # 36 M visits
+
+    def logged(self):
+        """A flat engine with its graph cached, and the bytes that it holds once it
+        has also counted W * L visits through a log."""
+        engines = [self.engine(**FORMS["flat"]) for _ in range(2)]
+        for eng in engines:
+            self.pagerank(eng, self.part.count * 4096, 3)
+            before = self.held()
+        assert self.pagerank(engines[1], self.W, self.L)["iterations"] == 1
+        assert self.held() - before > 1 << 28  # with a log
+        return engines, self.held() - before
+
+    def log(self):
+        (eng, other), most = self.logged()
+        other.close()
+        base = self.held()
+        for less in (1, 4 * self.W, most // 2):
+            self.limit(base + most - less)
+            self.pagerank(eng, self.W, self.L)
+        self.limit(1 << 62)
+        self.pagerank(eng, self.W, self.L)
+        assert self.held() - base == most
+
+    def kept_log(self):
+        (_, eng), _ = self.logged()
+        held = self.held()
+        self.limit(held)
+        assert self.np.array_equal(eng.genericwalk_paths(60000, 9),
+                                   self.oracle.genericwalk_paths(self.rp, self.col, 60000, 9))
+        assert self.held() < held
+        self.pagerank(eng, self.W, self.L)
+
+    def offsets(self):
+        eng = self.engine(**FORMS["flat"])
+        n = 4 * (self.graph.num_node + 1)
+        self.arm(MALLOC, times=1 << 40, least=n, most=n)
+        w = self.part.count * 4096
+        for _ in range(2):
+            assert self.pagerank(eng, w, 4)["iterations"] > 1
+        assert self.disarm(MALLOC) > 0
+        assert self.pagerank(eng, w, 4)["iterations"] == 1
 
 
 if __name__ == "__main__":
