@@ -252,7 +252,7 @@ struct Engine {
     VisitScratch vs{};
     unsigned long long *d_vcur = nullptr;
     uint64_t vlog_cap = 0;                       // entries allocated
-    bool log_asked = false;                      // a job would have used one
+    uint64_t log_missed = 0;                     // visits counted directly for want of one
     uint32_t vregion = 0;                        // entries per region of the running job, 0 = no log
     bool wants_log(uint64_t visits, bool queued);
     bool ensure_log(uint64_t visits);
@@ -767,23 +767,31 @@ lt_status Engine::ensure_outputs(const RunSpec &rs, bool want_endpoints, bool wa
 // that cannot hold a log counts directly.
 constexpr uint64_t kLogVisits = 1u << 18, kLogVisitsQueued = 1u << 24;
 constexpr uint64_t kLogMost = 1ull << 26;  // entries: 256 MB; 0.75 GB with what counting them takes
+// A flat job allocates a log once that many visits were counted without: their
+// atomics have then cost what the allocation takes, 13 to 20 us a million visits
+// and 50 to 600 us.  (Allocated by any engine's second job, it took that one
+// from 90 to 600 us on s16, 0.9 M visits a job, and from 54 to 600 on s14, 0.3 M.)
+constexpr uint64_t kLogPays = 1ull << 25;
+
+// Entries of a job's log: regions fill unevenly, so a quarter more than its visits,
+// and a launch's workgroups' buffers.
+static uint64_t log_entries(uint64_t visits) {
+    visits = std::min(visits, kLogMost);
+    return std::min(kLogMost, visits + visits / 4 + (1u << 20)) & ~(uint64_t)(kTile * kLogRegions - 1);
+}
 
 bool Engine::wants_log(uint64_t visits, bool queued) {
     if (visits < (queued ? kLogVisitsQueued : kLogVisits) || nbins > kMaxBins) return false;
-    // An engine's first job would pay 0.3-0.5 ms for the allocation, and saves
-    // less where it counts few visits (3 M: 0.1 ms of atomics).
-    if (!vlog_cap && !log_asked && visits < kLogVisitsQueued) {
-        log_asked = true;
-        return false;
-    }
+    if (queued || vlog_cap >= log_entries(visits)) return true;
+    log_missed += std::min(visits, kLogPays);
+    if (log_missed < kLogPays) return false;
+    log_missed = 0;
     return true;
 }
 
 // Whether there is memory for it.
 bool Engine::ensure_log(uint64_t visits) {
-    // regions fill unevenly: a quarter more, and a launch's workgroups' buffers
-    visits = std::min(visits, kLogMost);
-    const uint64_t want = std::min(kLogMost, visits + visits / 4 + (1u << 20)) & ~(uint64_t)(kTile * kLogRegions - 1);
+    const uint64_t want = log_entries(visits);
     if (vlog_cap < want) {
         drop_log();
         const size_t cur = (size_t)kLogRegions * kCurStride;  // cursors, then the bins' totals and first units

@@ -44,6 +44,12 @@ def test_what_only_speeds_a_job_up_gives_way(shim, what):
     child(shim, what)
 
 
+def test_a_visit_log_is_allocated_when_it_pays(shim):
+    """Jobs of few visits allocate nothing after an engine's first one, until as many
+    visits were counted directly as cost what a log's allocation does."""
+    child(shim, "later_jobs")
+
+
 # ---- the child process ------------------------------------------------------------
 
 FORMS = {"flat": dict(span="resident", resident_batch=16, zerocopy_threshold=0),
@@ -170,6 +176,27 @@ class Child:
             assert self.pagerank(eng, w, 4)["iterations"] > 1
         assert self.disarm(MALLOC) > 0
         assert self.pagerank(eng, w, 4)["iterations"] == 1
+
+    def later_jobs(self):
+        eng = self.engine(**FORMS["flat"])
+        w, l = 100000, 10  # 1 M visits
+        self.pagerank(eng, w, l)
+        held = self.held()
+        paid = 0
+        for job in range(2, 41):
+            assert self.pagerank(eng, w, l)["iterations"] == 1
+            if self.held() != held:
+                assert not paid and job * w * l >= 1 << 25 > (job - 1) * w * l
+                held, paid = self.held(), job
+        assert paid
+        eng = self.engine(**FORMS["flat"])  # one job of that many
+        self.pagerank(eng, self.part.count * 4096, 2)
+        held = self.held()
+        self.pagerank(eng, self.W, self.L)
+        assert self.held() - held > 1 << 28
+        held = self.held()
+        self.pagerank(eng, w, l)  # small ones use it
+        assert self.held() == held
 
 
 if __name__ == "__main__":

@@ -37,6 +37,20 @@ def test_flat_jobs(V):
         assert np.array_equal(counts, oracle.ppr(g.rowptr(), g.col(), w, source=V - 1, threads=16)[0])
 
 
+@pytest.mark.parametrize("V", [1, 32768, 32769, 65536, 131072, 131073, 500001])
+def test_flat_jobs_of_an_engine_with_a_log(V):
+    """The same behind a job of 34 M visits, which allocates the log that they use."""
+    print(f"visit log kept V={V}", flush=True)
+    g = _ring(V)
+    eng = lt.Engine(g, lt.Partition.build(g, 64 << 20), zerocopy_threshold=0)
+    _check(g, eng, 1 << 20, 32)
+    for w, l in ((262143, 1), (262144, 1), (16384 * 16 + 1, 2), (123457, 10)):
+        _check(g, eng, w, l)
+    for w in (262143, 300000):
+        counts = eng.ppr(w, source=V - 1)
+        assert np.array_equal(counts, oracle.ppr(g.rowptr(), g.col(), w, source=V - 1, threads=16)[0])
+
+
 def test_flat_job_in_pieces():
     """75 M visits: more than one log holds."""
     print("visit log pieces", flush=True)
