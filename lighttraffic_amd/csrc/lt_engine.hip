@@ -130,7 +130,8 @@ struct EventTimer {
 // h_out: kNumStats u64 of event counters, the sequence number, those of the
 // ring's buffers, that of the last load finished, then small results.
 constexpr uint32_t kOutFlag = 2 * kNumStats, kOutRing = kOutFlag + 1, kOutCopy = 32, kOutData = 64;
-constexpr uint64_t kManyOut = 1u << 20;  // words: from here on threads help with the results
+constexpr uint64_t kManyOut = 1u << 20;   // words: from here on threads help with the results,
+constexpr uint64_t kLargeOut = 2u << 20;  // and from here on they go through the large ring
 
 struct RunSpec {
     int app = APP_PAGERANK;
@@ -270,12 +271,13 @@ struct Engine {
     unsigned long long *d_stats = nullptr;
     // Results on their way to the caller (lt_results.h).
     static constexpr uint32_t kRing = 4;
-    static constexpr size_t kRingBytes = 2u << 20;
+    static constexpr size_t kRingBytes = 2u << 20, kRingSmall = 512u << 10;  // of a buffer
     uint32_t *h_out = nullptr, *d_out = nullptr;  // pinned: event counters, sequence number, small results
     uint32_t out_seq = 0;
     bool over = false;                            // the running job's walks were seen to be over,
     std::chrono::steady_clock::time_point t_over; // and when
-    uint8_t *h_ring = nullptr, *d_ring = nullptr; // pinned: kRing buffers
+    uint8_t *h_ring = nullptr, *d_ring = nullptr; // pinned: kRing buffers, in h_out's allocation or h_large
+    uint8_t *h_large = nullptr;
     uint32_t ring_seq[kRing] = {};                // of each buffer's last fill
     std::vector<OutSeg> outs;                     // results of the running job
     uint8_t *h_query = nullptr;                   // pinned staging of the query table
@@ -284,9 +286,9 @@ struct Engine {
     lt_status finish_job(bool small);
     bool walks_over();
     lt_status wait_walks();
-    size_t ring_cap = 0;
-    bool ring_asked = false;  // a job would have used one
-    lt_status ensure_ring(size_t bytes);
+    size_t ring_buf = 0;   // bytes of each buffer
+    size_t ring_seen = 0;  // bytes of the ring that the CPU has read before
+    lt_status pick_ring(uint64_t words, ResultHelpers &help);
     lt_status mark_ring(uint32_t slot);
     lt_status wait_ring(uint32_t slot);
     lt_status copy_results(ResultHelpers &help);
@@ -455,7 +457,7 @@ Engine::~Engine() {
     dfree(d_qsrc);
     dfree(d_stats);
     if (h_out) (void)hipHostFree(h_out);
-    if (h_ring) (void)hipHostFree(h_ring);
+    if (h_large) (void)hipHostFree(h_large);
     if (h_query) (void)hipHostFree(h_query);
     dfree(d_ds);
     dfree(d_slot_of);
@@ -691,9 +693,14 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
     if (cfg.span != LT_SPAN_RESIDENT) res_batch = 1;
     slice = cfg.slice_chunks > 0 ? (uint32_t)cfg.slice_chunks : kSliceChunks;
     LT_TRY(dmalloc(&d_stats, (size_t)kNumStats * kStatSlots));
-    LT_HIP(hipHostMalloc((void **)&h_out, 4 * (kOutData + kSmallOut), hipHostMallocMapped | hipHostMallocCoherent));
+    // pinned memory takes 55 us whatever its size: the small ring lies behind h_out
+    const size_t out_bytes = (4 * (kOutData + kSmallOut) + 4095) & ~(size_t)4095;
+    LT_HIP(hipHostMalloc((void **)&h_out, out_bytes + kRing * kRingSmall, hipHostMallocMapped | hipHostMallocCoherent));
     memset(h_out, 0, 4 * kOutData);
     LT_HIP(hipHostGetDevicePointer((void **)&d_out, h_out, 0));
+    h_ring = (uint8_t *)h_out + out_bytes;
+    d_ring = (uint8_t *)d_out + out_bytes;
+    ring_buf = kRingSmall;
     counts.assign(P, 0);
     dcounts.assign(P, 0);
     hq.assign(P, {});
@@ -2213,13 +2220,10 @@ lt_status Engine::run_flat(const RunSpec &rs, ResultHelpers &help) {
     // the next walkers walk.  (PPR lanes end one by one, and paths are written
     // a word per row: those results stay on the device until the end.)
     const uint32_t nout = (uint32_t)outs.size();
-    const bool ring = ring_asked && app_kind == APP_GENERIC && !a.app.paths && nout && nout * rs.total >= kManyOut;
+    const bool ring = app_kind == APP_GENERIC && !a.app.paths && nout * rs.total >= kLargeOut;
     constexpr uint32_t kTwo = kRing / 2;  // a launch takes two buffers: its last walkers leave
                                           // the card half idle for some 10 us
-    if (ring) {
-        LT_TRY(ensure_ring(kRing * kRingBytes));
-        piece = 2 * kRingBytes / 4 / nout;
-    }
+    if (ring) piece = 2 * kRingBytes / 4 / nout;
     const auto drain = [&](uint64_t k) -> lt_status {  // launch k's results to the caller
         LT_TRY(wait_ring(k % kTwo));
         const uint64_t n = std::min<uint64_t>(piece, rs.total - k * piece);
@@ -2306,15 +2310,26 @@ lt_status Engine::wait_walks() {
     return LT_OK;
 }
 
-// Pinning takes 0.15 ms a MB: no more of it than a job's results fill.
-lt_status Engine::ensure_ring(size_t bytes) {
-    if (ring_cap >= bytes) return LT_OK;
-    if (h_ring) (void)hipHostFree(h_ring);  // (no job is running)
-    h_ring = nullptr;
-    ring_cap = 0;
-    LT_HIP(hipHostMalloc((void **)&h_ring, bytes, hipHostMallocMapped | hipHostMallocCoherent));
-    LT_HIP(hipHostGetDevicePointer((void **)&d_ring, h_ring, 0));
-    ring_cap = bytes;
+// The ring for results of that many words: from 8 MB on the large one, which is allocated
+// then.  The CPU's first read of a page of pinned memory costs 1.4 us (0.36 ms a MB,
+// by four threads 0.12), so helpers read the pages while the job walks; and
+// smaller results are no faster with 8 MB (3.4 to 5.3 MB of results: 256-445 us a job with 2
+// MB, 242-418 with 8, 340-560 by plain copies; 10 to 20 MB: 1.66-2.4 ms, 1.58-2.3
+// and 1.9-2.8).
+lt_status Engine::pick_ring(uint64_t words, ResultHelpers &help) {
+    if (words >= kLargeOut && !h_large) {
+        LT_HIP(hipHostMalloc((void **)&h_large, kRing * kRingBytes, hipHostMallocMapped | hipHostMallocCoherent));
+        h_ring = h_large;
+        LT_HIP(hipHostGetDevicePointer((void **)&d_ring, h_ring, 0));
+        ring_buf = kRingBytes;
+        ring_seen = 0;
+    }
+    const size_t use = std::min<uint64_t>(4 * words, kRing * ring_buf);
+    if (use > ring_seen) {
+        help.fresh = h_ring + ring_seen;
+        help.fresh_bytes = use - ring_seen;
+        ring_seen = use;
+    }
     return LT_OK;
 }
 
@@ -2330,28 +2345,17 @@ lt_status Engine::wait_ring(uint32_t slot) { return poll_host(h_out + kOutRing +
 // The results in pieces of a ring buffer's size: kernels fill the next buffers
 // while the team copies the oldest one out.
 lt_status Engine::copy_results(ResultHelpers &help) {
-    if (!ring_asked) {  // an engine's first large results: pinning costs more than it saves (4 MB: 0.6 and 0.2 ms)
-        ring_asked = true;
-        LT_TRY(wait_walks());
-        for (const OutSeg &o : outs)
-            LT_HIP(hipMemcpyAsync(o.dst, o.src, 4 * o.words, hipMemcpyDeviceToHost, s_compute));
-        LT_HIP(hipStreamSynchronize(s_compute));
-        return LT_OK;
-    }
     std::vector<OutSeg> pieces;
     std::vector<size_t> at;  // place of each in the ring: one behind the other if all fit
     size_t end = 0;
     for (const OutSeg &o : outs)
-        for (uint64_t i = 0; i < o.words; i += kRingBytes / 4) {
-            pieces.push_back({o.dst + i, o.src + i, std::min<uint64_t>(kRingBytes / 4, o.words - i)});
+        for (uint64_t i = 0; i < o.words; i += ring_buf / 4) {
+            pieces.push_back({o.dst + i, o.src + i, std::min<uint64_t>(ring_buf / 4, o.words - i)});
             at.push_back(end);
             end += (4 * pieces.back().words + 4095) & ~(size_t)4095;
         }
-    if (pieces.size() > kRing) {
-        end = kRing * kRingBytes;
-        for (size_t i = 0; i < at.size(); i++) at[i] = i % kRing * kRingBytes;
-    }
-    LT_TRY(ensure_ring(end));
+    if (pieces.size() > kRing)
+        for (size_t i = 0; i < at.size(); i++) at[i] = i % kRing * ring_buf;
     for (size_t issued = 0, out = 0; out < pieces.size(); out++) {
         for (; issued < pieces.size() && issued < out + kRing; issued++) {
             fill_ring_kernel<<<64, 256, 0, s_compute>>>(pieces[issued].src, (uint32_t *)(d_ring + at[issued]),
@@ -2456,12 +2460,16 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
     for (const OutSeg &o : outs) out_words += o.words;
     const bool small = out_words <= kSmallOut;
     ResultHelpers help;
-    if (out_words >= kManyOut) help.most = std::min(4u, std::max(1u, std::thread::hardware_concurrency()) - 1);
+    if (out_words >= kManyOut) help.most = help_most(4);
+    if (!small) LT_TRY(pick_ring(out_words, help));
 
     double running_ms = 0;
     auto t_walk = std::chrono::steady_clock::now();
     job_finished = over = false;
-    if (walk_flat && missing) LT_TRY(load_missing());
+    if (walk_flat && missing) {
+        help.start(outs);
+        LT_TRY(load_missing());
+    }
     if (walk_flat) LT_TRY(run_flat(rs, help));
     for (uint64_t id0 = walk_flat ? rs.total : 0; id0 < rs.total; id0 += wave) {
         const uint64_t id1 = std::min<uint64_t>(rs.total, id0 + wave);

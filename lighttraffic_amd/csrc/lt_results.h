@@ -10,13 +10,15 @@
 // gives the two streams hardware queues of their own, which it did not for the
 // second engine of a process; then they took twice as long as these.)  Fixed-
 // length walks over the flat arrays write their endpoints to the ring themselves.
-// Other threads have fresh pages of the caller's mapped while the job walks.
+// Other threads have fresh pages of the caller's mapped, and read those of a new
+// ring for the first time, while the job walks.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <string.h>
 #include <sys/mman.h>
 
+#include <algorithm>
 #include <atomic>
 #include <memory>
 #include <system_error>
@@ -104,23 +106,24 @@ __global__ __launch_bounds__(256) void begin_kernel(uint32_t *counts, uint64_t n
     if (vcur && tid < kLogRegions) vcur[tid * kCurStride] = 0;
 }
 
-// Threads that map the pages of result buffers for writing, whose contents stay
-// as they are (MADV_POPULATE_WRITE; a kernel without it leaves the faults to the
-// copies).  Joined by wait() or with the object.
+// Threads that read each page of fresh pinned memory once, which maps it for the CPU
+// (madvise does not take it), and map the pages of result buffers for writing,
+// whose contents stay as they are (MADV_POPULATE_WRITE; a kernel without it leaves
+// the faults to the copies).  Joined by wait() or with the object.
 class PageMapper {
   public:
     ~PageMapper() { wait(); }
-    void start(const std::vector<OutSeg> &outs, uint32_t threads) {
-        for (const OutSeg &o : outs) {
-            const uintptr_t lo = ((uintptr_t)o.dst + kAlign - 1) & ~(kAlign - 1);
-            const uintptr_t hi = ((uintptr_t)o.dst + 4 * o.words) & ~(kAlign - 1);
-            for (uintptr_t at = lo; at < hi; at += kStep) work.push_back({at, hi - at < kStep ? hi - at : kStep});
-        }
+    void start(const uint8_t *fresh, size_t fresh_bytes, const std::vector<OutSeg> &outs, uint32_t threads) {
+        add((uintptr_t)fresh, (uintptr_t)fresh + fresh_bytes, kReadStep);
+        reads = work.size();
+        for (const OutSeg &o : outs)
+            add(((uintptr_t)o.dst + kAlign - 1) & ~(kAlign - 1), ((uintptr_t)o.dst + 4 * o.words) & ~(kAlign - 1),
+                kStep);
         try {
             for (uint32_t k = 0; k < threads; k++)
                 team.emplace_back([this] {
                     for (size_t i; (i = next.fetch_add(1)) < work.size();)
-                        if (madvise((void *)work[i].first, work[i].second, kPopulateWrite) != 0) return;
+                        if (!map(i)) return;
                 });
         } catch (const std::system_error &) {
         }
@@ -132,11 +135,22 @@ class PageMapper {
     }
 
   private:
-    static constexpr uintptr_t kAlign = 4096, kStep = 1u << 20;
+    static constexpr uintptr_t kAlign = 4096, kStep = 1u << 20, kReadStep = 64u << 10;
     static constexpr int kPopulateWrite = 23;  // MADV_POPULATE_WRITE of Linux 5.14
     std::vector<std::pair<uintptr_t, size_t>> work;
+    size_t reads = 0;  // of work, the first that are read
     std::atomic<size_t> next{0};
     std::vector<std::thread> team;
+
+    void add(uintptr_t lo, uintptr_t hi, uintptr_t step) {
+        for (uintptr_t at = lo; at < hi; at += step) work.push_back({at, hi - at < step ? hi - at : step});
+    }
+    bool map(size_t i) {
+        const auto &w = work[i];
+        if (i >= reads) return madvise((void *)w.first, w.second, kPopulateWrite) == 0;
+        for (uintptr_t at = w.first; at < w.first + w.second; at += kAlign) (void)*(volatile const uint8_t *)at;
+        return true;
+    }
 };
 
 // A few threads that copy one block of memory at a time, each its share, and
@@ -193,13 +207,25 @@ class CopyTeam {
     }
 };
 
+// At most `wanted` threads beside the caller's, and 4.  (The system is asked once: 20 us.)
+inline uint32_t help_most(size_t wanted) {
+    static const uint32_t cpus = std::max(1u, std::thread::hardware_concurrency());
+    return (uint32_t)std::min<size_t>({wanted, 4, cpus - 1});
+}
+
 // Threads that help with one job's results: none for small ones.
 struct ResultHelpers {
     uint32_t most = 0;
+    const uint8_t *fresh = nullptr;  // pinned memory that the CPU has not read yet
+    size_t fresh_bytes = 0;
+    bool started = false;
     PageMapper mapper;
     std::unique_ptr<CopyTeam> team;
-    void start(const std::vector<OutSeg> &outs) {  // behind the job's first launches
-        if (most) mapper.start(outs, most);
+    void start(const std::vector<OutSeg> &outs) {  // before the job's loads, or behind its first launches
+        if (started) return;
+        started = true;
+        const uint32_t readers = fresh_bytes ? help_most(1 + (fresh_bytes >> 19)) : 0;
+        if (most || readers) mapper.start(fresh, fresh_bytes, most ? outs : std::vector<OutSeg>(), std::max(most, readers));
     }
     CopyTeam &copiers() {  // one thread copies at about 32 GB/s, below the link's rate
         mapper.wait();

@@ -50,6 +50,12 @@ def test_a_visit_log_is_allocated_when_it_pays(shim):
     child(shim, "later_jobs")
 
 
+def test_only_larger_results_pin_memory(shim):
+    """Results of up to 8 MB pin no memory in any job of an engine, larger ones in the
+    first such job only."""
+    child(shim, "rings")
+
+
 # ---- the child process ------------------------------------------------------------
 
 FORMS = {"flat": dict(span="resident", resident_batch=16, zerocopy_threshold=0),
@@ -197,6 +203,16 @@ class Child:
         held = self.held()
         self.pagerank(eng, w, l)  # small ones use it
         assert self.held() == held
+
+    def rings(self):
+        eng = self.engine(**FORMS["flat"])
+        for w, pinned in ((70000, 0), (70000, 0), (900000, 0), (900000, 0), (1 << 20, 1), (1 << 20, 0), (70000, 0),
+                          (1500000, 0)):
+            self.arm(HOST_MALLOC, times=0)
+            ends, moves = eng.genericwalk(w, 3, moves=True)
+            re, rm, _ = self.oracle.genericwalk(self.rp, self.col, w, 3, threads=16)
+            assert self.np.array_equal(ends, re) and self.np.array_equal(moves, rm)
+            assert self.lib.hipfail_calls(HOST_MALLOC) == pinned, w
 
 
 if __name__ == "__main__":

@@ -50,3 +50,17 @@ def test_later_jobs_of_one_engine(graph, w):
         re, rm, _ = oracle.genericwalk(rp, col, n, 4, threads=16)
         ends, moves = eng.genericwalk(n, 4, moves=True)
         assert np.array_equal(ends, re) and np.array_equal(moves, rm)
+
+
+@pytest.mark.parametrize("w", [1 << 19, (1 << 20) - 1, 1 << 20, (1 << 20) + 1, 2097152 + 5])
+def test_results_at_the_rings_edges(graph, w):
+    """One array and two, around the sizes from which the large ring and the walk that
+    writes it are used, after small results and before."""
+    print(f"results at the rings' edges w={w}", flush=True)
+    rp, col = graph.rowptr(), graph.col()
+    eng = lt.Engine(graph, lt.Partition.build(graph, 32 << 20), zerocopy_threshold=0)
+    for n in (66000, w, 131072 + 1, w, 2 * w):
+        re, rm, _ = oracle.genericwalk(rp, col, n, 4, threads=16)
+        ends, moves = eng.genericwalk(n, 4, moves=True)
+        assert np.array_equal(ends, re) and np.array_equal(moves, rm)
+        assert np.array_equal(eng.genericwalk(n, 4)[0], re)
