@@ -288,7 +288,7 @@ struct Engine {
     lt_status wait_walks();
     size_t ring_buf = 0;   // bytes of each buffer
     size_t ring_seen = 0;  // bytes of the ring that the CPU has read before
-    lt_status pick_ring(uint64_t words, ResultHelpers &help);
+    void pick_ring(uint64_t words, ResultHelpers &help);
     lt_status mark_ring(uint32_t slot);
     lt_status wait_ring(uint32_t slot);
     lt_status copy_results(ResultHelpers &help);
@@ -2220,7 +2220,7 @@ lt_status Engine::run_flat(const RunSpec &rs, ResultHelpers &help) {
     // the next walkers walk.  (PPR lanes end one by one, and paths are written
     // a word per row: those results stay on the device until the end.)
     const uint32_t nout = (uint32_t)outs.size();
-    const bool ring = app_kind == APP_GENERIC && !a.app.paths && nout * rs.total >= kLargeOut;
+    const bool ring = app_kind == APP_GENERIC && !a.app.paths && nout * rs.total >= kLargeOut && h_large;
     constexpr uint32_t kTwo = kRing / 2;  // a launch takes two buffers: its last walkers leave
                                           // the card half idle for some 10 us
     if (ring) piece = 2 * kRingBytes / 4 / nout;
@@ -2316,13 +2316,21 @@ lt_status Engine::wait_walks() {
 // smaller results are no faster with 8 MB (3.4 to 5.3 MB of results: 256-445 us a job with 2
 // MB, 242-418 with 8, 340-560 by plain copies; 10 to 20 MB: 1.66-2.4 ms, 1.58-2.3
 // and 1.9-2.8).
-lt_status Engine::pick_ring(uint64_t words, ResultHelpers &help) {
+void Engine::pick_ring(uint64_t words, ResultHelpers &help) {
     if (words >= kLargeOut && !h_large) {
-        LT_HIP(hipHostMalloc((void **)&h_large, kRing * kRingBytes, hipHostMallocMapped | hipHostMallocCoherent));
-        h_ring = h_large;
-        LT_HIP(hipHostGetDevicePointer((void **)&d_ring, h_ring, 0));
-        ring_buf = kRingBytes;
-        ring_seen = 0;
+        uint8_t *d = nullptr;
+        if (hipHostMalloc((void **)&h_large, kRing * kRingBytes, hipHostMallocMapped | hipHostMallocCoherent) ==
+                hipSuccess &&
+            hipHostGetDevicePointer((void **)&d, h_large, 0) == hipSuccess) {
+            h_ring = h_large;
+            d_ring = d;
+            ring_buf = kRingBytes;
+            ring_seen = 0;
+        } else {  // the small one does as well
+            (void)hipGetLastError();
+            if (h_large) (void)hipHostFree(h_large);
+            h_large = nullptr;
+        }
     }
     const size_t use = std::min<uint64_t>(4 * words, kRing * ring_buf);
     if (use > ring_seen) {
@@ -2330,7 +2338,6 @@ lt_status Engine::pick_ring(uint64_t words, ResultHelpers &help) {
         help.fresh_bytes = use - ring_seen;
         ring_seen = use;
     }
-    return LT_OK;
 }
 
 // The ring buffer is full once the stream gets here.
@@ -2430,15 +2437,17 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
             if (h_query) (void)hipHostFree(h_query);
             h_query = nullptr;
             query_cap = 0;
-            LT_HIP(hipHostMalloc((void **)&h_query, need, hipHostMallocDefault));
-            query_cap = need;
+            if (hipHostMalloc((void **)&h_query, need, hipHostMallocDefault) == hipSuccess) query_cap = need;
+            else (void)hipGetLastError();
         }
-        uint64_t *off = (uint64_t *)h_query;
+        std::vector<uint64_t> plain(h_query ? 0 : need / 8 + 1);  // pinned memory is short
+        uint64_t *off = h_query ? (uint64_t *)h_query : plain.data();
         off[0] = 0;
         for (uint32_t i = 0; i < rs.nq; i++) off[i + 1] = off[i] + rs.q_cnt[i];
         memcpy(off + rs.nq + 1, rs.q_src, 4 * (size_t)rs.nq);
         LT_HIP(hipMemcpyAsync(d_qoff, off, 8 * ((size_t)rs.nq + 1), hipMemcpyHostToDevice, s_compute));
         LT_HIP(hipMemcpyAsync(d_qsrc, off + rs.nq + 1, 4 * (size_t)rs.nq, hipMemcpyHostToDevice, s_compute));
+        if (!h_query) LT_HIP(hipStreamSynchronize(s_compute));
         app.q_off = d_qoff;
         app.q_src = d_qsrc;
         app.nq = rs.nq;
@@ -2461,7 +2470,7 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
     const bool small = out_words <= kSmallOut;
     ResultHelpers help;
     if (out_words >= kManyOut) help.most = help_most(4);
-    if (!small) LT_TRY(pick_ring(out_words, help));
+    if (!small) pick_ring(out_words, help);
 
     double running_ms = 0;
     auto t_walk = std::chrono::steady_clock::now();

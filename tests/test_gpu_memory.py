@@ -56,6 +56,12 @@ def test_only_larger_results_pin_memory(shim):
     child(shim, "rings")
 
 
+@pytest.mark.parametrize("what", ["no_ring", "no_query_table"])
+def test_jobs_without_more_pinned_memory(shim, what):
+    """Large results and query tables whose pinned memory cannot be had."""
+    child(shim, what)
+
+
 # ---- the child process ------------------------------------------------------------
 
 FORMS = {"flat": dict(span="resident", resident_batch=16, zerocopy_threshold=0),
@@ -213,6 +219,24 @@ class Child:
             re, rm, _ = self.oracle.genericwalk(self.rp, self.col, w, 3, threads=16)
             assert self.np.array_equal(ends, re) and self.np.array_equal(moves, rm)
             assert self.lib.hipfail_calls(HOST_MALLOC) == pinned, w
+
+    def no_ring(self):
+        for kw in (FORMS["flat"], FORMS["queues"]):
+            eng = self.engine(**kw)
+            self.arm(HOST_MALLOC, times=1 << 40)
+            for w in (70000, 1200000):
+                ends, moves = eng.genericwalk(w, 3, moves=True)
+                re, rm, _ = self.oracle.genericwalk(self.rp, self.col, w, 3, threads=16)
+                assert self.np.array_equal(ends, re) and self.np.array_equal(moves, rm)
+            assert self.disarm(HOST_MALLOC) > 0
+            assert self.np.array_equal(eng.genericwalk(3000000, 3)[0][:w], re)
+
+    def no_query_table(self):
+        eng = self.engine(**FORMS["flat"])
+        self.arm(HOST_MALLOC, times=1 << 40)
+        self.jobs(eng, 5000, batch=True)
+        assert self.disarm(HOST_MALLOC) > 0
+        self.jobs(eng, 5000, batch=True)
 
 
 if __name__ == "__main__":
