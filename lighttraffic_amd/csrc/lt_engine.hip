@@ -185,6 +185,7 @@ struct Engine {
     // One raw slot per partition: the slots are slices of one rowptr and one
     // col array (at most as many bytes), which run_flat walks directly.
     bool flat = false;
+    lt_status alloc_flat();
     uint64_t *flat_rowptr = nullptr;   // [V+1], in d_slots
     uint32_t *flat_col = nullptr;      // [E], in d_slots
     uint32_t *d_rowptr32 = nullptr;    // [V+1] copy of flat_rowptr once every partition is cached (E < 2^32)
@@ -583,12 +584,13 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
     // Blocks pay where they let more partitions stay. Asked for raw slots for all,
     // the images only travel, and the columns are kept raw, for flat walks: a
     // move reads one line of columns instead of two one after the other (s20
-    // batched ppr, 5 M walkers: 4.0 ms walked from blocks, 3.5 so).  Not where
-    // the raw columns take more than a quarter of the free memory.
+    // batched ppr, 5 M walkers: 4.05 ms a job from blocks, 1.65 so).  They take no more
+    // than the slots asked for; not where they take more than a quarter of the
+    // free memory, or cannot be allocated.
     if (slot_packed && !cfg.device_schedule && (cfg.num_device_partitions == 0 || cfg.num_device_partitions >= P)) {
         size_t room = 0, all = 0;
         LT_HIP(hipMemGetInfo(&room, &all));
-        slot_packed = 8ull * ((uint64_t)V + 1) + 4ull * g->E > room / 4;
+        slot_packed = 8ull * ((uint64_t)V + 1) + 4ull * g->E > room / 4 || alloc_flat() != LT_OK;
     }
 
     // HBM cache slots (GPUGraph, src/GraphLoader.h:175-176)
@@ -608,14 +610,8 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
     if (rp_resident && nslots >= rp_slots + 2) nslots -= rp_slots;
     else rp_resident = false;
     flat = nslots == P && !slot_packed && !cfg.device_schedule;
-    if (flat) {
-        const size_t rp_size = (rp_bytes + 255) & ~(size_t)255;
-        LT_TRY(dmalloc(&d_slots, rp_size + 4 * (size_t)g->E));
-        flat_rowptr = (uint64_t *)d_slots;
-        flat_col = (uint32_t *)(d_slots + rp_size);
-    } else {
-        LT_TRY(dmalloc(&d_slots, (size_t)nslots * slot_bytes));
-    }
+    if (!flat) LT_TRY(dmalloc(&d_slots, (size_t)nslots * slot_bytes));
+    else if (!d_slots) LT_TRY(alloc_flat());
     slot_of.assign(P, -1);
     part_in_slot.assign(nslots, -1);
     resident.assign(P, 0);
@@ -711,6 +707,15 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
     t_load.enabled = t_compute.enabled = t_zc.enabled = t_wload.enabled = t_wevict.enabled = timers;
     t_kernel.enabled = t_kzc.enabled = timers;
     sched.init(P, cfg);
+    return LT_OK;
+}
+
+// The slots of a flat cache.
+lt_status Engine::alloc_flat() {
+    const size_t rp_size = (8 * ((size_t)V + 1) + 255) & ~(size_t)255;
+    LT_TRY(dmalloc(&d_slots, rp_size + 4 * (size_t)g->E));
+    flat_rowptr = (uint64_t *)d_slots;
+    flat_col = (uint32_t *)(d_slots + rp_size);
     return LT_OK;
 }
 

@@ -62,6 +62,12 @@ def test_jobs_without_more_pinned_memory(shim, what):
     child(shim, what)
 
 
+@pytest.mark.parametrize("slots", [0, 99])
+def test_block_slots_where_raw_columns_do_not_fit(shim, slots):
+    """Slots for all partitions, in memory that holds their block images only."""
+    child(shim, "blocks", slots)
+
+
 # ---- the child process ------------------------------------------------------------
 
 FORMS = {"flat": dict(span="resident", resident_batch=16, zerocopy_threshold=0),
@@ -237,6 +243,20 @@ class Child:
         self.jobs(eng, 5000, batch=True)
         assert self.disarm(HOST_MALLOC) > 0
         self.jobs(eng, 5000, batch=True)
+
+    def blocks(self, slots):
+        kw = dict(FORMS["flat"], pack_partitions=2, num_device_partitions=int(slots))
+        assert self.part.count <= 99
+        size, n = self.part.slot_layout(self.graph, 2, int(slots))
+        raw = 8 * (self.graph.num_node + 1) + 4 * self.graph.num_edge
+        assert n == self.part.count and n * size < raw
+        self.arm(MALLOC, times=1 << 40, least=raw, most=raw + 255)
+        eng = self.engine(**kw)
+        assert self.disarm(MALLOC) == 1
+        self.jobs(eng, 60000)
+        st = eng.stats()
+        assert st["cache_slots"] == n and st["iterations"] > 1  # by queues
+        self.jobs(self.engine(**kw), 60000)
 
 
 if __name__ == "__main__":
