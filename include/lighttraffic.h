@@ -95,7 +95,9 @@ typedef struct {
                                        cache holds more partitions (raw slots
                                        asked for all of them: the images
                                        travel, and the columns are kept raw
-                                       unless memory is short).  A
+                                       unless they take more than a quarter of
+                                       the free memory or cannot be
+                                       allocated).  A
                                        partition that does not get smaller is
                                        copied as is (default 0: off;
                                        device_schedule: 2 only, 1 is ignored)   */
@@ -275,7 +277,13 @@ lt_status lt_partition_pack_blocks(const lt_graph *g, const lt_partition *p, uin
  * block image over the partitions (256-aligned) and the cache keeps the same
  * bytes, so it holds more slots (at most one per partition).  Lets a caller
  * size the cache before creating an engine; engines report the same count in
- * lt_stats.cache_slots.  No counterpart in the reference. */
+ * lt_stats.cache_slots.  With 2 and raw slots asked for all partitions (0, or
+ * at least as many as there are) these are the least bytes that the engine's
+ * cache takes: where the device has room it keeps the columns raw instead,
+ * 8 * (V + 1) + 4 * E bytes (and up to 255), which the raw slots asked for
+ * hold (pack_partitions above).  Whether it does depends on the memory free
+ * when it is created; slots and results do not.  No counterpart in the
+ * reference. */
 lt_status lt_partition_slot_layout(const lt_graph *g, const lt_partition *p, int32_t pack_partitions,
                                    uint32_t num_device_partitions, uint64_t *slot_bytes, uint32_t *slots);
 /* Greedy contiguous split sized for block slots: each partition's rowptr

@@ -341,7 +341,9 @@ class Partition:
 
     def slot_layout(self, graph, pack_partitions=0, num_device_partitions=0):
         """(slot bytes, slots) of the HBM cache an engine with these settings
-        gets (before rowptr_resident takes its share)."""
+        gets (before rowptr_resident takes its share).  With pack_partitions 2
+        and raw slots for all partitions, the least that it takes: where there
+        is room it keeps the columns raw, within the raw slots asked for."""
         sb, n = _u64(), _u32()
         _check(_lib.lt_partition_slot_layout(graph._h, self._h, pack_partitions, num_device_partitions,
                                              ctypes.byref(sb), ctypes.byref(n)), "lt_partition_slot_layout")

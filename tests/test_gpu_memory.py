@@ -68,6 +68,12 @@ def test_block_slots_where_raw_columns_do_not_fit(shim, slots):
     child(shim, "blocks", slots)
 
 
+def test_the_cache_takes_what_its_layout_says(shim):
+    """The bytes of lt_partition_slot_layout, or with block images and slots for all
+    partitions the raw columns, within the raw slots asked for."""
+    child(shim, "layout")
+
+
 # ---- the child process ------------------------------------------------------------
 
 FORMS = {"flat": dict(span="resident", resident_batch=16, zerocopy_threshold=0),
@@ -257,6 +263,24 @@ class Child:
         st = eng.stats()
         assert st["cache_slots"] == n and st["iterations"] > 1  # by queues
         self.jobs(self.engine(**kw), 60000)
+
+    def layout(self):
+        P, raw = self.part.count, 8 * (self.graph.num_node + 1) + 4 * self.graph.num_edge
+
+        def made(pack, slots, least, most):
+            """Allocations of that size by an engine's creation."""
+            self.arm(MALLOC, times=0, least=least, most=most)
+            self.engine(pack_partitions=pack, num_device_partitions=slots).close()
+            return self.lib.hipfail_calls(MALLOC)
+
+        for pack, slots in ((0, 3), (1, 3), (2, 3), (2, P // 2)):
+            size, n = self.part.slot_layout(self.graph, pack, slots)
+            assert made(pack, slots, n * size, n * size) == 1, (pack, slots)
+        for slots in (0, P, 99):
+            size, n = self.part.slot_layout(self.graph, 2, slots)
+            raw_size, raw_n = self.part.slot_layout(self.graph, 0, slots)
+            assert n == raw_n == P and n * size < raw <= raw + 255 <= raw_n * raw_size
+            assert made(2, slots, raw, raw + 255) == 1 and made(2, slots, raw + 256, 1 << 62) == 0
 
 
 if __name__ == "__main__":
