@@ -345,7 +345,10 @@ struct Engine {
         hipEvent_t ev = nullptr; // by DMA, with others behind it; else the copy stream itself is asked
     };
     uint32_t copy_seq = 0;
-    std::vector<hipEvent_t> pool_events;  // reusable
+    std::vector<hipEvent_t> all_events, pool_events;  // of loads; those not in use
+    uint32_t loading = 0;  // partitions that hold a slot and are not resident yet
+    lt_status arrived(uint32_t p);
+    lt_status drop_loads();
     bool loaded(const Load &l) const;
     lt_status wait_loaded(Load &l);
     bool meta_dirty = true;  // q.packed may be older than the queues
@@ -432,7 +435,7 @@ Engine::~Engine() {
     if (s_compute) (void)hipStreamSynchronize(s_compute);
     if (s_copy) (void)hipStreamSynchronize(s_copy);
     if (s_dma && s_dma != s_copy) (void)hipStreamSynchronize(s_dma);
-    for (auto ev : pool_events) (void)hipEventDestroy(ev);
+    for (auto ev : all_events) (void)hipEventDestroy(ev);
     dfree(d_node_off);
     dfree(d_edge_off);
     dfree(d_lut);
@@ -1049,6 +1052,29 @@ lt_status Engine::wait_loaded(Load &l) {
     return LT_OK;
 }
 
+// p's copy is complete: walks may read its slot.
+lt_status Engine::arrived(uint32_t p) {
+    resident[p] = 1;
+    loading--;
+    return set_table(p, true);
+}
+
+// Takes the slots of loads back that a job which ended with an error did not wait for.
+lt_status Engine::drop_loads() {
+    if (loading == 0) return LT_OK;
+    LT_HIP(hipStreamSynchronize(s_copy));
+    if (s_dma != s_copy) LT_HIP(hipStreamSynchronize(s_dma));
+    for (uint32_t p = 0; p < P; p++) {
+        if (slot_of[p] < 0 || resident[p]) continue;
+        part_in_slot[slot_of[p]] = -1;
+        free_slots.push_back((uint32_t)slot_of[p]);
+        slot_of[p] = -1;
+    }
+    pool_events = all_events;
+    loading = 0;
+    return LT_OK;
+}
+
 // GPUGraph::loadAsync (src/GraphLoader.h:193-215): rowptr slice at slot offset
 // 0, col slice right after it, both on the copy stream.  The compute stream
 // must not be reading the slot (the caller evicted it after a sync).  ahead: other
@@ -1063,6 +1089,7 @@ lt_status Engine::load_async(uint32_t p, bool ahead, Load &l) {
     hipEvent_t t = t_load.begin(s_dma);
     slot_of[p] = (int32_t)s;
     part_in_slot[s] = (int32_t)p;
+    loading++;
     uint64_t *rp;
     uint32_t *cp;
     slot_ptrs(p, &rp, &cp);
@@ -1076,6 +1103,7 @@ lt_status Engine::load_async(uint32_t p, bool ahead, Load &l) {
     } else if (ahead) {
         if (pool_events.empty()) {
             LT_HIP(hipEventCreateWithFlags(&l.ev, hipEventDisableTiming));
+            all_events.push_back(l.ev);
         } else {
             l.ev = pool_events.back();
             pool_events.pop_back();
@@ -1773,8 +1801,7 @@ lt_status Engine::run_partition(uint32_t p, int32_t &prev_loaded) {
             LT_TRY(read_meta());
         }
         LT_TRY(wait_loaded(load));
-        resident[p] = 1;
-        LT_TRY(set_table(p, true));
+        LT_TRY(arrived(p));
     } else {
         record(p, 0, -1, -1);
     }
@@ -1841,8 +1868,7 @@ lt_status Engine::scheduler_loop_learned() {
             LT_TRY(wait_loaded(f.load));
             inflight.erase(inflight.begin());
             pending[f.part] = 0;
-            resident[f.part] = 1;
-            LT_TRY(set_table((uint32_t)f.part, true));
+            LT_TRY(arrived((uint32_t)f.part));
             if (f.part == upto) break;
         }
         return LT_OK;
@@ -1943,8 +1969,7 @@ lt_status Engine::scheduler_loop_learned() {
                 sched.on_load((uint32_t)c);
                 LT_TRY(pipeline_while_copying(c, load));
                 LT_TRY(wait_loaded(load));
-                resident[c] = 1;
-                LT_TRY(set_table((uint32_t)c, true));
+                LT_TRY(arrived((uint32_t)c));
             }
             prev_loaded = c;
         }
@@ -2171,6 +2196,7 @@ lt_status Engine::load_missing() {
                 slot_of[i] = (int32_t)free_slots.back();
                 part_in_slot[free_slots.back()] = (int32_t)i;
                 free_slots.pop_back();
+                loading++;
             }
         }
         t_load.end(t, s_copy);
@@ -2178,10 +2204,9 @@ lt_status Engine::load_missing() {
     LT_HIP(hipStreamSynchronize(s_copy));
     for (uint32_t p = 0; p < P; p++) {
         if (resident[p]) continue;
-        resident[p] = 1;
         st.graph_loading_calls++;
         sched.on_load(p);
-        LT_TRY(set_table(p, true));
+        LT_TRY(arrived(p));
     }
     return LT_OK;
 }
@@ -2384,6 +2409,7 @@ lt_status Engine::copy_results(ResultHelpers &help) {
 
 lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoints_out, uint32_t *moves_out) {
     LT_HIP(hipSetDevice(device));
+    LT_TRY(drop_loads());
     memset(&st, 0, sizeof(st));
     st.cache_slots = nslots;
     spill_h2d_bytes = 0;

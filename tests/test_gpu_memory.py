@@ -74,13 +74,22 @@ def test_the_cache_takes_what_its_layout_says(shim):
     child(shim, "layout")
 
 
+@pytest.mark.parametrize("form", ["flat", "queues", "learned"])
+def test_after_failed_loads(shim, form):
+    """Jobs that end at a partition copy's error, more of them than the cache has slots:
+    the slots are there for the next job."""
+    child(shim, "loads", form)
+
+
 # ---- the child process ------------------------------------------------------------
 
 FORMS = {"flat": dict(span="resident", resident_batch=16, zerocopy_threshold=0),
          "queues": dict(num_device_partitions=3, span="resident"),
          "spill": dict(num_device_partitions=3, num_device_walkers=9000),
          "batch": dict(num_device_partitions=3),
-         "device": dict(num_device_partitions=3, device_schedule=1)}
+         "device": dict(num_device_partitions=3, device_schedule=1),
+         "learned": dict(num_device_partitions=4, span="resident", policy="learned", prefetch_plain=1,
+                         prefetch_depth=2, zerocopy_threshold=0)}
 
 
 class Child:
@@ -281,6 +290,19 @@ class Child:
             raw_size, raw_n = self.part.slot_layout(self.graph, 0, slots)
             assert n == raw_n == P and n * size < raw <= raw + 255 <= raw_n * raw_size
             assert made(2, slots, raw, raw + 255) == 1 and made(2, slots, raw + 256, 1 << 62) == 0
+
+    def loads(self, form):
+        eng = self.engine(pack_partitions=1, **FORMS[form])
+        w = self.part.count * 4096
+        for n in range(2 * self.part.count + 3):
+            self.arm(MEMCPY_ASYNC, skip=n)
+            try:
+                self.pagerank(eng, w, 3)
+            except self.lt.LTError as e:
+                assert e.status == 5, e  # LT_E_HIP
+            self.disarm(MEMCPY_ASYNC)
+        for _ in range(2):
+            self.jobs(eng, w)
 
 
 if __name__ == "__main__":
