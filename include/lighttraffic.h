@@ -342,9 +342,10 @@ lt_status lt_run_ppr_batch(lt_engine *e, uint32_t nq, const uint32_t *sources, c
                            float prob, uint32_t *endpoints_out);
 lt_status lt_engine_stats(const lt_engine *e, lt_stats *out);
 /* Partition part as the engine's partition copy writes it into an HBM cache
- * slot (packed or not, per the engine's config), copied back to the host:
- * rowptr_out u64[n+1], col_out u32[m].  Leaves the cache untouched (no
- * counterpart in the reference; it lets a caller check a slot's bytes). */
+ * slot (copied raw or gap-coded, per the engine's config), copied back to the
+ * host: rowptr_out u64[n+1], col_out u32[m].  LT_E_ARG for block images
+ * (pack_partitions = 2).  Leaves the cache untouched (no counterpart in the
+ * reference; it lets a caller check a slot's bytes). */
 lt_status lt_engine_fetch_partition(lt_engine *e, uint32_t part, uint64_t *rowptr_out, uint32_t *col_out);
 /* Batched-PPR query table (no counterpart in the reference): query q draws
  * Philox(seed; q, 0, TAG_QUERY) = (x0,x1,x2,x3); its source is the row that

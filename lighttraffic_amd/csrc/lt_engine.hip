@@ -1212,7 +1212,7 @@ lt_status Engine::copy_partition(uint32_t p, uint64_t *rp, uint32_t *cp) {
 // copied back; the cache and the statistics are left as they were.
 lt_status Engine::fetch_partition(uint32_t p, uint64_t *rowptr_out, uint32_t *col_out) {
     if (pk && pk->format == 2) {
-        set_error("fetch of partition %u: slots keep columns packed (pack_partitions = 2)", p);
+        set_error("fetch of partition %u: refused with pack_partitions = 2, whose copies are block images", p);
         return LT_E_ARG;
     }
     LT_HIP(hipSetDevice(device));

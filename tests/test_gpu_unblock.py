@@ -43,3 +43,13 @@ def test_jobs(V, slots):
         assert np.array_equal(eng.ppr(w, source=V - 2), pc)
     if slots != "less":
         assert eng.stats()["iterations"] == 1 and eng.stats()["graph_loading_calls"] == 0
+
+
+@pytest.mark.parametrize("slots", [0, 2])
+def test_refused_fetch_says_why(slots):
+    """With slots for all the columns are raw, so the reason is the copies' form."""
+    g = _graph(1000, 5)
+    eng = lt.Engine(g, lt.Partition.build(g, max(1024, g.num_edge * 4 // 6)), num_device_partitions=slots,
+                    pack_partitions=2)
+    with pytest.raises(lt.LTError, match="copies are block images"):
+        eng.fetch_partition(0, eng.partition.node_offsets(), eng.partition.edge_offsets())
