@@ -118,7 +118,6 @@ struct DevSched {
     int32_t choice;     // partition walked this iteration, -1 = every queue is empty
     int32_t zerocopy;   // walked from host memory
     int32_t load;       // copied into its slot first
-    int32_t victim;     // partition evicted for the load, -1 = none
     uint32_t iterations, loads, zc_calls;
     unsigned long long h2d_bytes;
     // the choice's queue length and slices, for the walk

@@ -2186,12 +2186,10 @@ lt_status Engine::load_missing() {
             const uint32_t nb = part.node_off[p];
             const uint64_t eb = part.edge_off[p];
             const size_t rbytes = ((size_t)part.node_off[end] - nb + 1) * 8, cbytes = (part.edge_off[end] - eb) * 4;
-            if (rp_resident) LT_HIP(hipMemcpyAsync(flat_rowptr + nb, d_rowptr_all + nb, rbytes, hipMemcpyDeviceToDevice, s_copy));
-            else LT_HIP(hipMemcpyAsync(flat_rowptr + nb, g->rowptr + nb, rbytes, hipMemcpyHostToDevice, s_copy));
+            LT_HIP(hipMemcpyAsync(flat_rowptr + nb, g->rowptr + nb, rbytes, hipMemcpyHostToDevice, s_copy));
             LT_HIP(hipMemcpyAsync(flat_col + eb, g->col + eb, cbytes, hipMemcpyHostToDevice, s_copy));
-            const size_t h2d = cbytes + (rp_resident ? 0 : rbytes);
-            st.h2d_bytes_explicit += h2d;
-            st.h2d_bytes_unpacked += h2d;
+            st.h2d_bytes_explicit += rbytes + cbytes;
+            st.h2d_bytes_unpacked += rbytes + cbytes;
             for (uint32_t i = p; i < end; i++) {
                 slot_of[i] = (int32_t)free_slots.back();
                 part_in_slot[free_slots.back()] = (int32_t)i;

@@ -1225,7 +1225,6 @@ __global__ __launch_bounds__(kBlock) void decide_kernel(Queues q, SchedState ss,
     }
     d.load = 0;
     d.zerocopy = 0;
-    d.victim = -1;
     if (best == 0) {
         if (tid == 0) {
             d.choice = -1;
@@ -1282,7 +1281,6 @@ __global__ __launch_bounds__(kBlock) void decide_kernel(Queues q, SchedState ss,
             ss.slot_of[v] = -1;
             ss.resident[v] = 0;
             ss.rec[v].rowptr = nullptr;
-            d.victim = (int32_t)v;
         }
     }
     uint8_t *base = ss.slots + (size_t)slot * ss.slot_bytes;

@@ -59,8 +59,6 @@ __host__ __device__ inline uint16_t f32_to_bf16(float x) {
 }
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
-__device__ __forceinline__ float to_f32(float x) { return x; }
-__device__ __forceinline__ float to_f32(uint16_t h) { return bf16_to_f32(h); }
 
 // ---- features ----------------------------------------------------------------
 // Feature j of partition q:
@@ -442,7 +440,7 @@ __global__ __launch_bounds__(256, 2) void train_backward_kernel(uint32_t M, uint
 // BF16 forms included); host: the gradient goes there too.  The first workgroup
 // adds up the decisions' losses.
 __global__ __launch_bounds__(256) void train_update_kernel(uint32_t groups, uint32_t slices, const float *small,
-                                                           const float *w2, float *G, float *host, float *W,
+                                                           const float *w2, float *host, float *W,
                                                            uint16_t *Wb, uint16_t *Wi, float *Mo, float *Vo, int update,
                                                            float lr, float b1t, float b2t, uint32_t n,
                                                            const float *losses, float *loss) {
@@ -469,7 +467,6 @@ __global__ __launch_bounds__(256) void train_update_kernel(uint32_t groups, uint
         float s = 0.f;
 #pragma unroll
         for (int k = 0; k < 8; k++) s += s_p[k][c];
-        G[p] = s;
         if (host) host[p] = s;
         if (update) {
             const float m = 0.9f * Mo[p] + 0.1f * s;
@@ -707,7 +704,7 @@ struct Scorer {
     hipStream_t stream = nullptr;
     float *d_vsh = nullptr, *d_esh = nullptr;
     std::vector<float> h_vsh, h_esh;
-    float *W = nullptr, *G = nullptr, *Mo = nullptr, *Vo = nullptr;
+    float *W = nullptr, *Mo = nullptr, *Vo = nullptr;
     uint16_t *Wb = nullptr;
     uint16_t *Wi = nullptr;     // inference copy of W1, W2 (output-major)
     uint64_t wver = 0, wi_ver = ~0ull;  // bumped on every weight update; Wi is valid for wi_ver
@@ -742,7 +739,7 @@ struct Scorer {
 Scorer::~Scorer() {
     if (pending) (void)hipStreamSynchronize(pending);
     if (stream) (void)hipStreamSynchronize(stream);
-    void *ptrs[] = {d_vsh, d_esh, W, G, Mo, Vo, Wb, Wi, d_counts, X, A1, A2, Y, dY, small, w2, d_losses};
+    void *ptrs[] = {d_vsh, d_esh, W, Mo, Vo, Wb, Wi, d_counts, X, A1, A2, Y, dY, small, w2, d_losses};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (h_batch) (void)hipHostFree(h_batch);
@@ -769,8 +766,8 @@ lt_status Scorer::init(uint32_t P_, const uint32_t *node_off, const uint64_t *ed
     if ((st = dalloc(&d_vsh, P)) || (st = dalloc(&d_esh, P))) return st;
     MLP_HIP(hipMemcpy(d_vsh, h_vsh.data(), 4 * P, hipMemcpyHostToDevice));
     MLP_HIP(hipMemcpy(d_esh, h_esh.data(), 4 * P, hipMemcpyHostToDevice));
-    if ((st = dalloc(&W, kParams)) || (st = dalloc(&G, kParams)) || (st = dalloc(&Mo, kParams)) ||
-        (st = dalloc(&Vo, kParams)) || (st = dalloc(&Wb, kParams)) || (st = dalloc(&Wi, kWiSize)))
+    if ((st = dalloc(&W, kParams)) || (st = dalloc(&Mo, kParams)) || (st = dalloc(&Vo, kParams)) ||
+        (st = dalloc(&Wb, kParams)) || (st = dalloc(&Wi, kWiSize)))
         return st;
     // He-style initialisation from a seeded generator; biases zero.
     std::vector<float> w(kParams, 0.f);
@@ -860,7 +857,7 @@ lt_status Scorer::forward_backward(uint32_t nb, bool update, float lr, bool grad
         b2t = powf(0.999f, (float)adam_t);
         wi_ver = ++wver;  // the update writes Wi as well
     }
-    train_update_kernel<<<(unsigned)((kParams + 31) / 32), 256, 0, s>>>(groups, slices, small, w2, G,
+    train_update_kernel<<<(unsigned)((kParams + 31) / 32), 256, 0, s>>>(groups, slices, small, w2,
                                                                        grad_out ? d_grad + 2 : nullptr, W, Wb, Wi, Mo, Vo,
                                                                        update ? 1 : 0, lr, b1t, b2t, nb, d_losses, d_grad);
     MLP_HIP(hipGetLastError());
