@@ -369,16 +369,20 @@ struct Engine {
     lt_status copy_partition(uint32_t p, uint64_t *rp, uint32_t *cp);
     // Small slices are copied by one kernel instead of two DMAs, whose second
     // costs 10 us of its own (256 KB: 14 us, 22 by DMAs; 1 MB: 28 and 38).  Larger
-    // ones hold the walk up: beside a kernel that reads the link for 50 to 80
-    // us its launches took twice as long (s23, 4 MB slots: 12.1 ms a job by DMAs, 13.7
-    // so; s20 reference rules, 2 MB: 20.2 and 24.7; s20 ppr, 1 MB: 15.5 and 14.5).
-    static constexpr size_t kPullBytes = 1280u << 10;
+    // ones hold the walks beside them up, which wait longer for memory.  In ms a job,
+    // pulled and by DMAs: where walks go through all that is resident, s20 ppr 1 MB 14.5 and
+    // 15.4, 1.25 MB 13.2 and 14.3, s21 pagerank 0.75 MB 10.2 and 11.0, 1.25 MB 6.2 and 6.1,
+    // 1.5 MB 5.3 and 4.9; where a walk stays in one partition and a round has little
+    // else to do, s18 pagerank 64 KB 58 and 61, 128 KB 58 and 61, 256 KB 32.2 and 31.9, s16
+    // 6.7 and 6.9, s20 0.75 MB 55 and 50, 1 MB 40 and 35.
+    static constexpr size_t kPullBytes = 1280u << 10, kPullBytesOne = 256u << 10;
     static constexpr int kPullGrid = 64;
     bool pulls(uint32_t p) const {
         const bool packed = pk && pk->size[p];
         if (packed && !slot_packed) return false;
         const size_t rbytes = ((size_t)part.node_off[p + 1] - part.node_off[p] + 1) * 8;
-        return rbytes + (packed ? pk->size[p] : (part.edge_off[p + 1] - part.edge_off[p]) * 4) <= kPullBytes;
+        return rbytes + (packed ? pk->size[p] : (part.edge_off[p + 1] - part.edge_off[p]) * 4) <=
+               (cfg.span == LT_SPAN_RESIDENT ? kPullBytes : kPullBytesOne);
     }
     lt_status fetch_partition(uint32_t p, uint64_t *rowptr_out, uint32_t *col_out);
     // Bit streams of p's slot whose column part starts at cp: past the block

@@ -9,6 +9,7 @@ from oracle import ffi as oracle
 pytestmark = pytest.mark.gpu
 
 _LINE = 1280 << 10  # bytes of a partition's two slices
+_LINE_ONE = 256 << 10
 
 
 @pytest.mark.parametrize("mode", ["plain", "ahead", "device"])
@@ -16,8 +17,17 @@ _LINE = 1280 << 10  # bytes of a partition's two slices
 def test_slices_around_the_line(over, mode):
     """Five partitions of one vertex and its edges each, four of them with slices
     of the line's bytes, a word or an edge less or more, and of about twice that."""
-    print(f"loads {mode} over={over}", flush=True)
-    deg = (_LINE + over - 16) // 4
+    _slices(_LINE, over, mode)
+
+
+@pytest.mark.parametrize("over", [-4, 0, 4, _LINE_ONE - 12])
+def test_slices_around_the_line_of_walks_in_one_partition(over):
+    _slices(_LINE_ONE, over, "plain")
+
+
+def _slices(line, over, mode):
+    print(f"loads {mode} line={line} over={over}", flush=True)
+    deg = (line + over - 16) // 4
     degs = np.array([deg, deg, 7, deg - 1, deg], np.uint64)
     rng = np.random.default_rng(deg)
     rowptr = np.concatenate([[0], np.cumsum(degs)]).astype(np.uint64)
