@@ -277,8 +277,7 @@ struct Engine {
     uint32_t out_seq = 0;
     bool over = false;                            // the running job's walks were seen to be over,
     std::chrono::steady_clock::time_point t_over; // and when
-    uint8_t *h_ring = nullptr, *d_ring = nullptr; // pinned: kRing buffers, in h_out's allocation or h_large
-    uint8_t *h_large = nullptr;
+    uint8_t *h_ring = nullptr, *d_ring = nullptr; // pinned: kRing buffers
     uint32_t ring_seq[kRing] = {};                // of each buffer's last fill
     std::vector<OutSeg> outs;                     // results of the running job
     uint8_t *h_query = nullptr;                   // pinned staging of the query table
@@ -287,9 +286,10 @@ struct Engine {
     lt_status finish_job(bool small);
     bool walks_over();
     lt_status wait_walks();
-    size_t ring_buf = 0;   // bytes of each buffer
+    size_t ring_buf = 0;   // bytes of each buffer, 0 = no ring
     size_t ring_seen = 0;  // bytes of the ring that the CPU has read before
-    void pick_ring(uint64_t words, ResultHelpers &help);
+    bool ensure_ring(size_t buf);
+    void start_results(ResultHelpers &help);
     lt_status mark_ring(uint32_t slot);
     lt_status wait_ring(uint32_t slot);
     lt_status copy_results(ResultHelpers &help);
@@ -405,7 +405,7 @@ struct Engine {
     }
     lt_status set_table(uint32_t p, bool present);
     bool can_run_flat(const RunSpec &rs, uint32_t &missing) const;
-    lt_status load_missing();
+    lt_status load_missing(ResultHelpers &help);
     lt_status run_flat(const RunSpec &rs, ResultHelpers &help);
     bool job_finished = false;  // run_flat has handed the job's results out
     lt_status scheduler_loop();
@@ -465,7 +465,7 @@ Engine::~Engine() {
     dfree(d_qsrc);
     dfree(d_stats);
     if (h_out) (void)hipHostFree(h_out);
-    if (h_large) (void)hipHostFree(h_large);
+    if (h_ring) (void)hipHostFree(h_ring);
     if (h_query) (void)hipHostFree(h_query);
     dfree(d_ds);
     dfree(d_slot_of);
@@ -696,14 +696,9 @@ lt_status Engine::init(const lt_graph *g_, const lt_partition *p_, const lt_conf
     if (cfg.span != LT_SPAN_RESIDENT) res_batch = 1;
     slice = cfg.slice_chunks > 0 ? (uint32_t)cfg.slice_chunks : kSliceChunks;
     LT_TRY(dmalloc(&d_stats, (size_t)kNumStats * kStatSlots));
-    // pinned memory takes 55 us whatever its size: the small ring lies behind h_out
-    const size_t out_bytes = (4 * (kOutData + kSmallOut) + 4095) & ~(size_t)4095;
-    LT_HIP(hipHostMalloc((void **)&h_out, out_bytes + kRing * kRingSmall, hipHostMallocMapped | hipHostMallocCoherent));
+    LT_HIP(hipHostMalloc((void **)&h_out, 4 * (kOutData + kSmallOut), hipHostMallocMapped | hipHostMallocCoherent));
     memset(h_out, 0, 4 * kOutData);
     LT_HIP(hipHostGetDevicePointer((void **)&d_out, h_out, 0));
-    h_ring = (uint8_t *)h_out + out_bytes;
-    d_ring = (uint8_t *)d_out + out_bytes;
-    ring_buf = kRingSmall;
     counts.assign(P, 0);
     dcounts.assign(P, 0);
     hq.assign(P, {});
@@ -2176,7 +2171,7 @@ bool Engine::can_run_flat(const RunSpec &rs, uint32_t &missing) const {
     return rs.total / missing >= std::max<uint64_t>(zc_threshold, kChunk);
 }
 
-lt_status Engine::load_missing() {
+lt_status Engine::load_missing(ResultHelpers &help) {
     if (pk) {
         Load l;
         for (uint32_t p = 0; p < P; p++)
@@ -2203,6 +2198,7 @@ lt_status Engine::load_missing() {
         }
         t_load.end(t, s_copy);
     }
+    start_results(help);
     LT_HIP(hipStreamSynchronize(s_copy));
     for (uint32_t p = 0; p < P; p++) {
         if (resident[p]) continue;
@@ -2252,7 +2248,11 @@ lt_status Engine::run_flat(const RunSpec &rs, ResultHelpers &help) {
     // the next walkers walk.  (PPR lanes end one by one, and paths are written
     // a word per row: those results stay on the device until the end.)
     const uint32_t nout = (uint32_t)outs.size();
-    const bool ring = app_kind == APP_GENERIC && !a.app.paths && nout * rs.total >= kLargeOut && h_large;
+    bool ring = app_kind == APP_GENERIC && !a.app.paths && nout * rs.total >= kLargeOut;
+    if (ring) {
+        start_results(help);
+        ring = ring_buf == kRingBytes;
+    }
     constexpr uint32_t kTwo = kRing / 2;  // a launch takes two buffers: its last walkers leave
                                           // the card half idle for some 10 us
     if (ring) piece = 2 * kRingBytes / 4 / nout;
@@ -2281,7 +2281,7 @@ lt_status Engine::run_flat(const RunSpec &rs, ResultHelpers &help) {
         st.kernel_launches++;
         if (ring) LT_TRY(mark_ring(k % kTwo));
         if (a.app.vlog) LT_TRY(count_log((uint32_t)((a.id_hi - a.id_lo) * each), 0));
-        if (k == 0) help.start(outs);
+        start_results(help);
     }
     t_compute.end(tp, s_compute);
     w_run = rs.total;
@@ -2342,34 +2342,46 @@ lt_status Engine::wait_walks() {
     return LT_OK;
 }
 
-// The ring for results of that many words: from 8 MB on the large one, which is allocated
-// then.  The CPU's first read of a page of pinned memory costs 1.4 us (0.36 ms a MB,
-// by four threads 0.12), so helpers read the pages while the job walks; and
-// smaller results are no faster with 8 MB (3.4 to 5.3 MB of results: 256-445 us a job with 2
-// MB, 242-418 with 8, 340-560 by plain copies; 10 to 20 MB: 1.66-2.4 ms, 1.58-2.3
-// and 1.9-2.8).
-void Engine::pick_ring(uint64_t words, ResultHelpers &help) {
-    if (words >= kLargeOut && !h_large) {
-        uint8_t *d = nullptr;
-        if (hipHostMalloc((void **)&h_large, kRing * kRingBytes, hipHostMallocMapped | hipHostMallocCoherent) ==
-                hipSuccess &&
-            hipHostGetDevicePointer((void **)&d, h_large, 0) == hipSuccess) {
-            h_ring = h_large;
-            d_ring = d;
-            ring_buf = kRingBytes;
-            ring_seen = 0;
-        } else {  // the small one does as well
-            (void)hipGetLastError();
-            if (h_large) (void)hipHostFree(h_large);
-            h_large = nullptr;
+// A ring of buffers of that many bytes or more, if pinned memory can be had.
+bool Engine::ensure_ring(size_t buf) {
+    if (ring_buf >= buf) return true;
+    uint8_t *h = nullptr, *d = nullptr;
+    if (hipHostMalloc((void **)&h, kRing * buf, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+        hipHostGetDevicePointer((void **)&d, h, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        if (h) (void)hipHostFree(h);
+        return false;
+    }
+    if (h_ring) (void)hipHostFree(h_ring);  // (no job is filling it)
+    h_ring = h;
+    d_ring = d;
+    ring_buf = buf;
+    ring_seen = 0;
+    return true;
+}
+
+// Gets what the job's larger results will want, once the device has something to do:
+// threads, and the ring, from 8 MB of results on the large one.  The ring takes 30
+// to 350 us (at an engine's creation it would take them from every engine), and the
+// CPU's first read of each of its pages 1.4 us (0.36 ms a MB, by four threads 0.12),
+// which helpers do while the job walks.  Smaller results are no faster with 8 MB
+// (3.4 to 5.3 MB of results: 256-445 us a job with 2 MB, 242-418 with 8, 340-560
+// by plain copies; 10 to 20 MB: 1.66-2.4 ms, 1.58-2.3 and 1.9-2.8).
+void Engine::start_results(ResultHelpers &help) {
+    if (help.started) return;
+    uint64_t words = 0;
+    for (const OutSeg &o : outs) words += o.words;
+    if (words > kSmallOut) {
+        if (words < kLargeOut || !ensure_ring(kRingBytes)) ensure_ring(kRingSmall);
+        const size_t use = std::min<uint64_t>(4 * words, kRing * ring_buf);
+        if (use > ring_seen) {
+            help.fresh = h_ring + ring_seen;
+            help.fresh_bytes = use - ring_seen;
+            ring_seen = use;
         }
+        if (words >= kManyOut) help.most = help_most(4);
     }
-    const size_t use = std::min<uint64_t>(4 * words, kRing * ring_buf);
-    if (use > ring_seen) {
-        help.fresh = h_ring + ring_seen;
-        help.fresh_bytes = use - ring_seen;
-        ring_seen = use;
-    }
+    help.start(outs);
 }
 
 // The ring buffer is full once the stream gets here.
@@ -2384,6 +2396,11 @@ lt_status Engine::wait_ring(uint32_t slot) { return poll_host(h_out + kOutRing +
 // The results in pieces of a ring buffer's size: kernels fill the next buffers
 // while the team copies the oldest one out.
 lt_status Engine::copy_results(ResultHelpers &help) {
+    if (!ring_buf) {
+        LT_TRY(wait_walks());
+        for (const OutSeg &o : outs) LT_HIP(hipMemcpy(o.dst, o.src, 4 * o.words, hipMemcpyDeviceToHost));
+        return LT_OK;
+    }
     std::vector<OutSeg> pieces;
     std::vector<size_t> at;  // place of each in the ring: one behind the other if all fit
     size_t end = 0;
@@ -2502,16 +2519,11 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
     for (const OutSeg &o : outs) out_words += o.words;
     const bool small = out_words <= kSmallOut;
     ResultHelpers help;
-    if (out_words >= kManyOut) help.most = help_most(4);
-    if (!small) pick_ring(out_words, help);
 
     double running_ms = 0;
     auto t_walk = std::chrono::steady_clock::now();
     job_finished = over = false;
-    if (walk_flat && missing) {
-        help.start(outs);
-        LT_TRY(load_missing());
-    }
+    if (walk_flat && missing) LT_TRY(load_missing(help));
     if (walk_flat) LT_TRY(run_flat(rs, help));
     for (uint64_t id0 = walk_flat ? rs.total : 0; id0 < rs.total; id0 += wave) {
         const uint64_t id1 = std::min<uint64_t>(rs.total, id0 + wave);
@@ -2545,7 +2557,7 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
             LT_TRY(launch_fixup(Consumed{}));
             lo += n;
         }
-        if (id0 == 0) help.start(outs);
+        start_results(help);
         LT_TRY(wait_meta());
         const auto t0 = std::chrono::steady_clock::now();
         w_run = id1 - id0;

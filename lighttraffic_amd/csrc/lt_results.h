@@ -221,8 +221,7 @@ struct ResultHelpers {
     bool started = false;
     PageMapper mapper;
     std::unique_ptr<CopyTeam> team;
-    void start(const std::vector<OutSeg> &outs) {  // before the job's loads, or behind its first launches
-        if (started) return;
+    void start(const std::vector<OutSeg> &outs) {  // behind the job's first loads or launches
         started = true;
         const uint32_t readers = fresh_bytes ? help_most(1 + (fresh_bytes >> 19)) : 0;
         if (most || readers) mapper.start(fresh, fresh_bytes, most ? outs : std::vector<OutSeg>(), std::max(most, readers));

@@ -51,8 +51,8 @@ def test_a_visit_log_is_allocated_when_it_pays(shim):
 
 
 def test_only_larger_results_pin_memory(shim):
-    """Results of up to 8 MB pin no memory in any job of an engine, larger ones in the
-    first such job only."""
+    """Results of up to 256 KB pin no memory, larger ones and those of 8 MB or more in the
+    first such job of an engine only."""
     child(shim, "rings")
 
 
@@ -233,7 +233,7 @@ class Child:
 
     def rings(self):
         eng = self.engine(**FORMS["flat"])
-        for w, pinned in ((70000, 0), (70000, 0), (900000, 0), (900000, 0), (1 << 20, 1), (1 << 20, 0), (70000, 0),
+        for w, pinned in ((32768, 0), (32769, 1), (70000, 0), (900000, 0), (1 << 20, 1), (1 << 20, 0), (70000, 0),
                           (1500000, 0)):
             self.arm(HOST_MALLOC, times=0)
             ends, moves = eng.genericwalk(w, 3, moves=True)
