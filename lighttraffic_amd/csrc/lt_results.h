@@ -15,27 +15,11 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-#include <string.h>
-#include <sys/mman.h>
-
-#include <algorithm>
-#include <atomic>
-#include <memory>
-#include <system_error>
-#include <thread>
-#include <utility>
-#include <vector>
 
 #include "lt_kernels.h"
+#include "lt_team.h"
 
 namespace lt {
-
-// One result of a job: words of device memory and their place in the caller's.
-struct OutSeg {
-    uint32_t *dst;
-    const uint32_t *src;
-    uint64_t words;
-};
 
 // Results small enough to be written to pinned memory by a kernel.
 constexpr uint64_t kSmallOut = 64 * 1024;  // words
@@ -105,132 +89,5 @@ __global__ __launch_bounds__(256) void begin_kernel(uint32_t *counts, uint64_t n
     for (uint64_t i = tid; i < (uint64_t)kNumStats * kStatSlots; i += stride) stats[i] = 0;
     if (vcur && tid < kLogRegions) vcur[tid * kCurStride] = 0;
 }
-
-// Threads that read each page of fresh pinned memory once, which maps it for the CPU
-// (madvise does not take it), and map the pages of result buffers for writing,
-// whose contents stay as they are (MADV_POPULATE_WRITE; a kernel without it leaves
-// the faults to the copies).  Joined by wait() or with the object.
-class PageMapper {
-  public:
-    ~PageMapper() { wait(); }
-    void start(const uint8_t *fresh, size_t fresh_bytes, const std::vector<OutSeg> &outs, uint32_t threads) {
-        add((uintptr_t)fresh, (uintptr_t)fresh + fresh_bytes, kReadStep);
-        reads = work.size();
-        for (const OutSeg &o : outs)
-            add(((uintptr_t)o.dst + kAlign - 1) & ~(kAlign - 1), ((uintptr_t)o.dst + 4 * o.words) & ~(kAlign - 1),
-                kStep);
-        try {
-            for (uint32_t k = 0; k < threads; k++)
-                team.emplace_back([this] {
-                    for (size_t i; (i = next.fetch_add(1)) < work.size();)
-                        if (!map(i)) return;
-                });
-        } catch (const std::system_error &) {
-        }
-    }
-    void wait() {
-        next.store(work.size());  // the copies map the rest
-        for (auto &t : team) t.join();
-        team.clear();
-    }
-
-  private:
-    static constexpr uintptr_t kAlign = 4096, kStep = 1u << 20, kReadStep = 64u << 10;
-    static constexpr int kPopulateWrite = 23;  // MADV_POPULATE_WRITE of Linux 5.14
-    std::vector<std::pair<uintptr_t, size_t>> work;
-    size_t reads = 0;  // of work, the first that are read
-    std::atomic<size_t> next{0};
-    std::vector<std::thread> team;
-
-    void add(uintptr_t lo, uintptr_t hi, uintptr_t step) {
-        for (uintptr_t at = lo; at < hi; at += step) work.push_back({at, hi - at < step ? hi - at : step});
-    }
-    bool map(size_t i) {
-        const auto &w = work[i];
-        if (i >= reads) return madvise((void *)w.first, w.second, kPopulateWrite) == 0;
-        for (uintptr_t at = w.first; at < w.first + w.second; at += kAlign) (void)*(volatile const uint8_t *)at;
-        return true;
-    }
-};
-
-// A few threads that copy one block of memory at a time, each its share, and
-// end with the object.
-class CopyTeam {
-  public:
-    explicit CopyTeam(uint32_t helpers) {
-        try {
-            for (uint32_t k = 0; k < helpers; k++) team.emplace_back([this, k] { help(k + 1); });
-        } catch (const std::system_error &) {  // no more threads: the team is smaller
-        }
-    }
-    ~CopyTeam() {
-        stop = true;
-        turn.fetch_add(1, std::memory_order_release);
-        for (auto &t : team) t.join();
-    }
-    void copy(void *d, const void *s, size_t bytes) {
-        dst = (uint8_t *)d;
-        src = (const uint8_t *)s;
-        n = bytes;
-        parts = team.size() + 1;
-        done.store(0, std::memory_order_relaxed);
-        turn.fetch_add(1, std::memory_order_release);
-        share(0);
-        while (done.load(std::memory_order_acquire) != team.size()) __builtin_ia32_pause();
-    }
-
-  private:
-    std::vector<std::thread> team;
-    std::atomic<uint32_t> turn{0}, done{0};
-    bool stop = false;
-    uint8_t *dst = nullptr;
-    const uint8_t *src = nullptr;
-    size_t n = 0, parts = 1;
-
-    void share(size_t k) {  // on page boundaries of the block
-        const size_t per = ((n + parts - 1) / parts + 4095) & ~(size_t)4095;
-        const size_t lo = k * per < n ? k * per : n, hi = lo + per < n ? lo + per : n;
-        if (hi > lo) memcpy(dst + lo, src + lo, hi - lo);
-    }
-    void help(size_t k) {
-        for (uint32_t seen = 0;;) {
-            uint32_t t;
-            for (uint32_t spins = 0; (t = turn.load(std::memory_order_acquire)) == seen; spins++) {
-                if (spins < 4096) __builtin_ia32_pause();
-                else std::this_thread::yield();
-            }
-            seen = t;
-            if (stop) return;
-            share(k);
-            done.fetch_add(1, std::memory_order_release);
-        }
-    }
-};
-
-// At most `wanted` threads beside the caller's, and 4.  (The system is asked once: 20 us.)
-inline uint32_t help_most(size_t wanted) {
-    static const uint32_t cpus = std::max(1u, std::thread::hardware_concurrency());
-    return (uint32_t)std::min<size_t>({wanted, 4, cpus - 1});
-}
-
-// Threads that help with one job's results: none for small ones.
-struct ResultHelpers {
-    uint32_t most = 0;
-    const uint8_t *fresh = nullptr;  // pinned memory that the CPU has not read yet
-    size_t fresh_bytes = 0;
-    bool started = false;
-    PageMapper mapper;
-    std::unique_ptr<CopyTeam> team;
-    void start(const std::vector<OutSeg> &outs) {  // behind the job's first loads or launches
-        started = true;
-        const uint32_t readers = fresh_bytes ? help_most(1 + (fresh_bytes >> 19)) : 0;
-        if (most || readers) mapper.start(fresh, fresh_bytes, most ? outs : std::vector<OutSeg>(), std::max(most, readers));
-    }
-    CopyTeam &copiers() {  // one thread copies at about 32 GB/s, below the link's rate
-        mapper.wait();
-        if (!team) team.reset(new CopyTeam(most < 3 ? most : 3));
-        return *team;
-    }
-};
 
 }  // namespace lt
