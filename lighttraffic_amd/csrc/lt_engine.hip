@@ -2248,11 +2248,8 @@ lt_status Engine::run_flat(const RunSpec &rs, ResultHelpers &help) {
     // the next walkers walk.  (PPR lanes end one by one, and paths are written
     // a word per row: those results stay on the device until the end.)
     const uint32_t nout = (uint32_t)outs.size();
-    bool ring = app_kind == APP_GENERIC && !a.app.paths && nout * rs.total >= kLargeOut;
-    if (ring) {
-        start_results(help);
-        ring = ring_buf == kRingBytes;
-    }
+    const bool ring =
+        app_kind == APP_GENERIC && !a.app.paths && nout * rs.total >= kLargeOut && ensure_ring(kRingBytes);
     constexpr uint32_t kTwo = kRing / 2;  // a launch takes two buffers: its last walkers leave
                                           // the card half idle for some 10 us
     if (ring) piece = 2 * kRingBytes / 4 / nout;
