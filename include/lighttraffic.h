@@ -169,7 +169,8 @@ typedef struct {
     uint64_t moves;                 /* neighbour moves (rowptr pair + col read)  */
     uint64_t teleports;             /* pagerank jumps to a uniform vertex        */
     uint64_t visits;                /* visit-counter increments                  */
-    uint64_t residencies;           /* walker records read from a queue          */
+    uint64_t residencies;           /* walker records read from a queue (of jobs
+                                       that need no queues: walkers walked)      */
     uint64_t zerocopy_moves;        /* moves whose graph reads crossed PCIe      */
     uint64_t nominal_steps;         /* w*l*runs (pagerank, genericwalk), w/prob  */
     uint64_t kernel_launches;       /* walk-kernel launches                      */
