@@ -130,8 +130,7 @@ struct EventTimer {
 // h_out: kNumStats u64 of event counters, the sequence number, those of the
 // ring's buffers, that of the last load finished, then small results.
 constexpr uint32_t kOutFlag = 2 * kNumStats, kOutRing = kOutFlag + 1, kOutCopy = 32, kOutData = 64;
-constexpr uint64_t kManyOut = 1u << 20;   // words: from here on threads help with the results,
-constexpr uint64_t kLargeOut = 2u << 20;  // and from here on they go through the large ring
+constexpr uint64_t kManyOut = 1u << 20;  // words: from here on threads help with the results
 
 struct RunSpec {
     int app = APP_PAGERANK;
@@ -286,10 +285,15 @@ struct Engine {
     lt_status finish_job(bool small);
     bool walks_over();
     lt_status wait_walks();
-    size_t ring_buf = 0;   // bytes of each buffer, 0 = no ring
-    size_t ring_seen = 0;  // bytes of the ring that the CPU has read before
-    bool ensure_ring(size_t buf);
-    void start_results(ResultHelpers &help);
+    static constexpr size_t kRingLarge = kRing * kRingBytes;
+    size_t ring_cap = 0;       // bytes of the ring: 0, kRing * kRingSmall or kRingLarge
+    size_t ring_seen = 0;      // of them, read by the CPU before
+    uint64_t ring_words = 0;   // results for the large ring that went through the small one
+    uint8_t *h_next = nullptr, *d_next = nullptr;  // the large ring until next_seen, what was read of it, is all
+    size_t next_seen = 0;
+    bool reading_next = false;  // the running job's helpers read it
+    void start_results(ResultHelpers &help, bool cover);
+    void swap_ring();
     lt_status mark_ring(uint32_t slot);
     lt_status wait_ring(uint32_t slot);
     lt_status copy_results(ResultHelpers &help);
@@ -466,6 +470,7 @@ Engine::~Engine() {
     dfree(d_stats);
     if (h_out) (void)hipHostFree(h_out);
     if (h_ring) (void)hipHostFree(h_ring);
+    if (h_next) (void)hipHostFree(h_next);
     if (h_query) (void)hipHostFree(h_query);
     dfree(d_ds);
     dfree(d_slot_of);
@@ -2198,7 +2203,7 @@ lt_status Engine::load_missing(ResultHelpers &help) {
         }
         t_load.end(t, s_copy);
     }
-    start_results(help);
+    start_results(help, true);
     LT_HIP(hipStreamSynchronize(s_copy));
     for (uint32_t p = 0; p < P; p++) {
         if (resident[p]) continue;
@@ -2248,8 +2253,7 @@ lt_status Engine::run_flat(const RunSpec &rs, ResultHelpers &help) {
     // the next walkers walk.  (PPR lanes end one by one, and paths are written
     // a word per row: those results stay on the device until the end.)
     const uint32_t nout = (uint32_t)outs.size();
-    const bool ring =
-        app_kind == APP_GENERIC && !a.app.paths && nout * rs.total >= kLargeOut && ensure_ring(kRingBytes);
+    const bool ring = app_kind == APP_GENERIC && !a.app.paths && nout * rs.total >= kManyOut && ring_cap == kRingLarge;
     constexpr uint32_t kTwo = kRing / 2;  // a launch takes two buffers: its last walkers leave
                                           // the card half idle for some 10 us
     if (ring) piece = 2 * kRingBytes / 4 / nout;
@@ -2278,7 +2282,7 @@ lt_status Engine::run_flat(const RunSpec &rs, ResultHelpers &help) {
         st.kernel_launches++;
         if (ring) LT_TRY(mark_ring(k % kTwo));
         if (a.app.vlog) LT_TRY(count_log((uint32_t)((a.id_hi - a.id_lo) * each), 0));
-        start_results(help);
+        start_results(help, false);
     }
     t_compute.end(tp, s_compute);
     w_run = rs.total;
@@ -2339,46 +2343,69 @@ lt_status Engine::wait_walks() {
     return LT_OK;
 }
 
-// A ring of buffers of that many bytes or more, if pinned memory can be had.
-bool Engine::ensure_ring(size_t buf) {
-    if (ring_buf >= buf) return true;
-    uint8_t *h = nullptr, *d = nullptr;
-    if (hipHostMalloc((void **)&h, kRing * buf, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
-        hipHostGetDevicePointer((void **)&d, h, 0) != hipSuccess) {
-        (void)hipGetLastError();
-        if (h) (void)hipHostFree(h);
-        return false;
+// Pinned, mapped memory for a ring, if it can be had.
+static bool pin(size_t bytes, uint8_t **h, uint8_t **d) {
+    if (hipHostMalloc((void **)h, bytes, hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess) {
+        if (hipHostGetDevicePointer((void **)d, *h, 0) == hipSuccess) return true;
+        (void)hipHostFree(*h);
     }
-    if (h_ring) (void)hipHostFree(h_ring);  // (no job is filling it)
-    h_ring = h;
-    d_ring = d;
-    ring_buf = buf;
-    ring_seen = 0;
-    return true;
+    (void)hipGetLastError();
+    *h = nullptr;
+    return false;
 }
 
 // Gets what the job's larger results will want, once the device has something to do:
-// threads, and the ring, from 8 MB of results on the large one.  The ring takes 30
-// to 350 us (at an engine's creation it would take them from every engine), and the
-// CPU's first read of each of its pages 1.4 us (0.36 ms a MB, by four threads 0.12),
-// which helpers do while the job walks.  Smaller results are no faster with 8 MB
-// (3.4 to 5.3 MB of results: 256-445 us a job with 2 MB, 242-418 with 8, 340-560
-// by plain copies; 10 to 20 MB: 1.66-2.4 ms, 1.58-2.3 and 1.9-2.8).
-void Engine::start_results(ResultHelpers &help) {
+// threads, and a ring.  Pinning takes 30 to 350 us (at an engine's creation it would
+// take them from every engine), and the CPU's first read of each page 1.4 us (0.36 ms a
+// MB, by four threads 0.12), which helpers do while the job walks.
+//
+// Results of 8 MB go faster through a ring of 8 MB than through 2: 10 to 20 MB in 1.58-2.3
+// ms a job and 1.66-2.4 (1.9-2.8 by plain copies); so do endpoints of flat walks from 4 MB
+// on, which only the large ring takes from the walk itself (6 MB: 0.38 and 0.48 ms);
+// fewer do not (3.4 to 5.3 MB: 242-418 us and 256-445, 340-560 by plain copies).  But
+// reading 8 MB takes a millisecond, three times some jobs.  So a job with no ring yet
+// gets the large one if its loads or rounds cover that (cover); else it comes once
+// as many results went through the small one as lose what pinning costs, and is used
+// when helpers have read all of it, behind the walks of as many jobs as that takes.
+void Engine::start_results(ResultHelpers &help, bool cover) {
     if (help.started) return;
     uint64_t words = 0;
     for (const OutSeg &o : outs) words += o.words;
     if (words > kSmallOut) {
-        if (words < kLargeOut || !ensure_ring(kRingBytes)) ensure_ring(kRingSmall);
-        const size_t use = std::min<uint64_t>(4 * words, kRing * ring_buf);
+        const bool large = words >= (app_kind == APP_GENERIC && !app.paths ? kManyOut : 2 * kManyOut);
+        constexpr uint64_t kRingPays = 8u << 20;  // words: 32 MB, 10 to 18 us a MB
+        if (words >= kManyOut) help.most = help_most(4);
+        if (!h_ring) {
+            if (large && cover && pin(kRingLarge, &h_ring, &d_ring)) ring_cap = kRingLarge;
+            else if (pin(kRing * kRingSmall, &h_ring, &d_ring)) ring_cap = kRing * kRingSmall;
+        }
+        if (large && ring_cap < kRingLarge) {
+            ring_words += words;
+            if (!h_next && (cover || ring_words >= kRingPays) && !pin(kRingLarge, &h_next, &d_next)) ring_words = 0;
+        }
+        const size_t use = std::min<uint64_t>(4 * words, ring_cap);
         if (use > ring_seen) {
             help.fresh = h_ring + ring_seen;
             help.fresh_bytes = use - ring_seen;
             ring_seen = use;
+        } else if (large && h_next) {
+            help.fresh = h_next + next_seen;
+            help.fresh_bytes = kRingLarge - next_seen;
+            reading_next = true;
         }
-        if (words >= kManyOut) help.most = help_most(4);
     }
     help.start(outs);
+}
+
+// The large ring takes over once all of it has been read.  Before a job.
+void Engine::swap_ring() {
+    if (!h_next || next_seen < kRingLarge) return;
+    if (h_ring) (void)hipHostFree(h_ring);
+    h_ring = h_next;
+    d_ring = d_next;
+    ring_cap = ring_seen = kRingLarge;
+    h_next = d_next = nullptr;
+    next_seen = 0;
 }
 
 // The ring buffer is full once the stream gets here.
@@ -2393,22 +2420,25 @@ lt_status Engine::wait_ring(uint32_t slot) { return poll_host(h_out + kOutRing +
 // The results in pieces of a ring buffer's size: kernels fill the next buffers
 // while the team copies the oldest one out.
 lt_status Engine::copy_results(ResultHelpers &help) {
-    if (!ring_buf) {
+    if (!ring_cap) {
         LT_TRY(wait_walks());
         for (const OutSeg &o : outs) LT_HIP(hipMemcpy(o.dst, o.src, 4 * o.words, hipMemcpyDeviceToHost));
         return LT_OK;
     }
+    uint64_t words = 0;
+    for (const OutSeg &o : outs) words += o.words;
+    const size_t buf = ring_cap == kRingLarge && words >= 2 * kManyOut ? kRingBytes : kRingSmall;
     std::vector<OutSeg> pieces;
     std::vector<size_t> at;  // place of each in the ring: one behind the other if all fit
     size_t end = 0;
     for (const OutSeg &o : outs)
-        for (uint64_t i = 0; i < o.words; i += ring_buf / 4) {
-            pieces.push_back({o.dst + i, o.src + i, std::min<uint64_t>(ring_buf / 4, o.words - i)});
+        for (uint64_t i = 0; i < o.words; i += buf / 4) {
+            pieces.push_back({o.dst + i, o.src + i, std::min<uint64_t>(buf / 4, o.words - i)});
             at.push_back(end);
             end += (4 * pieces.back().words + 4095) & ~(size_t)4095;
         }
     if (pieces.size() > kRing)
-        for (size_t i = 0; i < at.size(); i++) at[i] = i % kRing * ring_buf;
+        for (size_t i = 0; i < at.size(); i++) at[i] = i % kRing * buf;
     for (size_t issued = 0, out = 0; out < pieces.size(); out++) {
         for (; issued < pieces.size() && issued < out + kRing; issued++) {
             fill_ring_kernel<<<64, 256, 0, s_compute>>>(pieces[issued].src, (uint32_t *)(d_ring + at[issued]),
@@ -2426,6 +2456,8 @@ lt_status Engine::copy_results(ResultHelpers &help) {
 lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoints_out, uint32_t *moves_out) {
     LT_HIP(hipSetDevice(device));
     LT_TRY(drop_loads());
+    swap_ring();
+    reading_next = false;
     memset(&st, 0, sizeof(st));
     st.cache_slots = nslots;
     spill_h2d_bytes = 0;
@@ -2554,7 +2586,7 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
             LT_TRY(launch_fixup(Consumed{}));
             lo += n;
         }
-        start_results(help);
+        start_results(help, true);
         LT_TRY(wait_meta());
         const auto t0 = std::chrono::steady_clock::now();
         w_run = id1 - id0;
@@ -2587,6 +2619,7 @@ lt_status Engine::run(const RunSpec &rs, uint32_t *counts_out, uint32_t *endpoin
     if (!job_finished) LT_TRY(finish_job(small));
     if (!small && !job_finished) LT_TRY(copy_results(help));
     running_ms += std::chrono::duration<double, std::milli>(t_over - t_walk).count();
+    if (reading_next) next_seen += help.mapper.wait();
     outs.clear();
     unsigned long long hs[kNumStats];
     for (int i = 0; i < kNumStats; i++) hs[i] = h_out[2 * i] | (unsigned long long)h_out[2 * i + 1] << 32;

@@ -47,10 +47,15 @@ class PageMapper {
         } catch (const std::exception &) {  // no more threads, or no memory for one
         }
     }
-    void wait() {
-        next.store(work.size());  // the copies map the rest
+    // Ends it; the bytes of fresh memory that were read.
+    size_t wait() {
+        const size_t taken = next.exchange(work.size());  // the copies map the rest
         for (auto &t : team) t.join();
         team.clear();
+        if (!ended)
+            for (size_t i = 0; i < taken && i < reads; i++) bytes_read += work[i].second;
+        ended = true;
+        return bytes_read;
     }
 
   private:
@@ -58,6 +63,8 @@ class PageMapper {
     static constexpr int kPopulateWrite = 23;  // MADV_POPULATE_WRITE of Linux 5.14
     std::vector<std::pair<uintptr_t, size_t>> work;
     size_t reads = 0;  // of work, the first that are read
+    size_t bytes_read = 0;
+    bool ended = false;
     std::atomic<size_t> next{0};
     std::vector<std::thread> team;
 

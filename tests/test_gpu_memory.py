@@ -51,8 +51,8 @@ def test_a_visit_log_is_allocated_when_it_pays(shim):
 
 
 def test_only_larger_results_pin_memory(shim):
-    """Results of up to 256 KB pin no memory, larger ones and those of 8 MB or more in the
-    first such job of an engine only."""
+    """Results of up to 256 KB pin no memory, larger ones in an engine's first such job
+    only, and once more when 32 MB of results of 4 MB or more went through that ring."""
     child(shim, "rings")
 
 
@@ -233,13 +233,19 @@ class Child:
 
     def rings(self):
         eng = self.engine(**FORMS["flat"])
-        for w, pinned in ((32768, 0), (32769, 1), (70000, 0), (900000, 0), (1 << 20, 1), (1 << 20, 0), (70000, 0),
-                          (1500000, 0)):
+        for _ in range(2):
+            eng.genericwalk(30000, 9)
+
+        def pins(w):
             self.arm(HOST_MALLOC, times=0)
             ends, moves = eng.genericwalk(w, 3, moves=True)
             re, rm, _ = self.oracle.genericwalk(self.rp, self.col, w, 3, threads=16)
             assert self.np.array_equal(ends, re) and self.np.array_equal(moves, rm)
-            assert self.lib.hipfail_calls(HOST_MALLOC) == pinned, w
+            return self.lib.hipfail_calls(HOST_MALLOC)
+
+        assert [pins(w) for w in (32768, 32769, 70000, 900000, 1 << 20, 1 << 20, 70000)] == [0, 1, 0, 0, 0, 0, 0]
+        assert sum(pins(1500000) for _ in range(12)) == 1  # when the first ring is ready and 32 MB went through
+        assert [pins(w) for w in (70000, 1500000, 1 << 21)] == [0, 0, 0]
 
     def no_ring(self):
         for kw in (FORMS["flat"], FORMS["queues"]):
